@@ -1954,72 +1954,3 @@ void launch_form_density(hipStream_t s, const double *C, const double *occ, int 
 
 
 }  // namespace pgxc
-
-// ------------------------------------------------------------------ Becke
-namespace pgxc {
-// Becke partition weight of the owning atom (J. Chem. Phys. 88, 2547 (1988)),
-// as becke0 (ParaGauss modules/grid_module.f90:2442-2497) with the step
-// function mu3 = p(p(p(mu))), p(m) = m (3 - m^2) / 2
-// (autodiff/becke_step_func.f90:84-124), no atomic-size adjustment.
-__device__ __forceinline__ double becke_step(double mu) {
-#pragma unroll
-  for (int k = 0; k < 3; ++k) mu = mu * (3.0 - mu * mu) / 2.0;
-  return mu;
-}
-
-__global__ __launch_bounds__(kThreads) void k_becke(int na, const double *__restrict__ axyz,
-                                                    const double *__restrict__ inv_dist,
-                                                    long npts, const double *__restrict__ pts,
-                                                    const int *__restrict__ owner,
-                                                    const double *__restrict__ wat,
-                                                    double *__restrict__ wout) {
-  const long p = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (p >= npts) return;
-  const double x = pts[p], y = pts[npts + p], z = pts[2 * npts + p];
-  const int own = owner[p];
-  double sum = 0.0, pown = 0.0;
-  for (int i = 0; i < na; ++i) {
-    const double dxi = axyz[3 * i] - x, dyi = axyz[3 * i + 1] - y, dzi = axyz[3 * i + 2] - z;
-    const double ri = sqrt(dxi * dxi + dyi * dyi + dzi * dzi);
-    double pi = 1.0;
-    for (int k = 0; k < na && pi != 0.0; ++k) {
-      if (k == i) continue;
-      const double dxk = axyz[3 * k] - x, dyk = axyz[3 * k + 1] - y, dzk = axyz[3 * k + 2] - z;
-      const double rk = sqrt(dxk * dxk + dyk * dyk + dzk * dzk);
-      const double mu = (ri - rk) * inv_dist[(long)i * na + k];
-      pi *= (1.0 - becke_step(mu)) / 2.0;
-    }
-    sum += pi;
-    if (i == own) pown = pi;
-  }
-  wout[p] = wat[p] * (pown / sum);
-}
-
-// Inverse distances of every pair of centres, inv[i][k] = 1/|R_i - R_k|
-// (0 on the diagonal), one thread per pair; the table k_becke reads.
-__global__ __launch_bounds__(kThreads) void k_inv_dist(int na, const double *__restrict__ axyz,
-                                                       double *__restrict__ inv) {
-  const long q = (long)blockIdx.x * kThreads + threadIdx.x;
-  if (q >= (long)na * na) return;
-  const int i = (int)(q / na), k = (int)(q % na);
-  double v = 0.0;
-  if (i != k) {
-    const double dx = axyz[3 * i] - axyz[3 * k], dy = axyz[3 * i + 1] - axyz[3 * k + 1],
-                 dz = axyz[3 * i + 2] - axyz[3 * k + 2];
-    v = 1.0 / sqrt(dx * dx + dy * dy + dz * dz);
-  }
-  inv[q] = v;
-}
-
-void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv) {
-  const long n = (long)na * na;
-  hipLaunchKernelGGL(k_inv_dist, dim3((unsigned)((n + kThreads - 1) / kThreads)), dim3(kThreads), 0,
-                     s, na, axyz, inv);
-}
-
-void launch_becke(hipStream_t s, int na, const double *axyz, const double *inv_dist, long npts,
-                  const double *pts, const int *owner, const double *wat, double *wout) {
-  hipLaunchKernelGGL(k_becke, dim3((unsigned)((npts + kThreads - 1) / kThreads)), dim3(kThreads),
-                     0, s, na, axyz, inv_dist, npts, pts, owner, wat, wout);
-}
-}  // namespace pgxc

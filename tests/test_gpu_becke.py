@@ -1,0 +1,47 @@
+"""Becke weights on the GPU at the sizes where their kernel takes another way:
+fewer centres than it keeps as nearest ones, as many, a few more, and enough
+that most are left out of the sum; against the numpy partition in FP64."""
+import numpy as np
+import pytest
+
+from pgxc import becke_weights, grid, systems
+
+pytestmark = pytest.mark.gpu
+
+
+def _points(rng, xyz, npts):
+    """Points at and near centres, between them and far outside."""
+    own = rng.integers(0, len(xyz), npts).astype(np.int32)
+    r = 10.0 ** rng.uniform(-6, 2, npts)
+    d = rng.normal(size=(npts, 3))
+    pts = xyz[own] + r[:, None] * d / np.linalg.norm(d, axis=1)[:, None]
+    pts[:len(xyz)] = xyz[own[:len(xyz)]]                      # at a nucleus
+    pts[len(xyz)] = 0.5 * (xyz[0] + xyz[-1])                  # halfway
+    return pts, own
+
+
+@pytest.mark.parametrize("na,npts", [(1, 70), (2, 63), (3, 257), (7, 300), (8, 300), (9, 1025),
+                                     (13, 511), (60, 700)])
+def test_weights_match_numpy(na, npts):
+    if na <= 8:
+        xyz = systems.random_molecule(9, seed=5)[1][:na]
+    else:
+        xyz = systems.random_molecule(na, seed=na)[1]
+    rng = np.random.default_rng(na)
+    pts, own = _points(rng, xyz, npts)
+    wat = rng.uniform(0.1, 2.0, npts)
+    ref = wat if na == 1 else grid.becke_numpy(xyz, pts, own, wat)
+    got = becke_weights(xyz, pts, own, wat)
+    # each weight is w times a quotient of products of na factors in [0, 1]
+    # that both sides form in FP64 from distances of up to 100 bohr over
+    # separations of about 2: 1e-13 per factor's mu, steps of slope up to 27/16
+    assert np.max(np.abs(got - ref) / wat) < 1e-13 * 27 / 16 * na
+    assert np.all(got[:na] >= 0)
+
+
+def test_equidistant_centres():
+    """Eight centres on a cube and its middle: no centre is negligible."""
+    xyz = np.array([[i, j, k] for i in (-2.0, 2.0) for j in (-2.0, 2.0) for k in (-2.0, 2.0)])
+    own = np.arange(8, dtype=np.int32)
+    w = becke_weights(xyz, np.zeros((8, 3)), own, np.full(8, 3.0))
+    assert np.max(np.abs(w - 3.0 / 8)) < 1e-15
