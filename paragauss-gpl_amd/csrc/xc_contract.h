@@ -1,0 +1,277 @@
+// FP64 and FP32 contractions of the XC build on MFMA, for gfx950 (kernel
+// templates; xc_contract_f64.hip and xc_contract_f32.hip instantiate them).
+//
+//   k_density    X = Phi D per 128-point tile, fused rho = sum Phi X,
+//                grad rho = 2 sum dPhi X
+//                (ParaGauss modules/density_calc_module.f90:1478-1577)
+//
+// A 16x16x4 FP64 MFMA holds its SIMD's matrix core for 64 cycles (FP32: 32), so
+// the time is the number of MFMAs: K and the output columns are the tile's own
+// functions, one by one, not runs of 8 or whole column chunks, and 16-column
+// blocks past the last function are skipped.  The operands' loads and LDS
+// traffic are a small share of it and only have to stay ahead.
+#pragma once
+#include <algorithm>
+#include <type_traits>
+
+#include "pgxc_internal.h"
+#include "xc_device.h"
+
+namespace pgxc {
+
+__device__ __forceinline__ int unit_of(const long *__restrict__ base, int nu, long it) {
+  int lo = 0, hi = nu - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (base[mid] <= it) lo = mid; else hi = mid - 1;
+  }
+  return lo;
+}
+
+template <typename T>
+struct V2 {
+  typedef T type __attribute__((ext_vector_type(2)));
+};
+
+// Point of a 16-point block that MFMA row i stands for: chosen so that a
+// lane's four results are four consecutive points 4 (lane / 16) + r (the FP64
+// result has rows lane / 16 + 4 r, the FP32 result those already).
+template <typename T>
+__device__ __forceinline__ int row_point(int i) {
+  return MF<T>::kQuadRows ? i : 4 * (i & 3) + (i >> 2);
+}
+
+constexpr int kDBM = 128;  // points of a density tile
+constexpr int kLPad = 16;  // LDS row padding: the four k rows an MFMA operand
+                           // read touches lie on different banks
+
+// X(m, n) = sum_k Phi[f(k)][m0 + m] D[f(k)][c(n)] for one tile and one chunk of
+// NB 16-column blocks, f and c entries of the tile's function list: four waves,
+// each 32 points x all columns.  Both operands are staged [k][row] as they lie
+// in memory: a wave takes whole k rows (its index is uniform, so their addresses
+// are scalar), a lane two points of Phi and one or two columns of D (symmetric,
+// so row f(k) is read along the columns).  Rows past the list repeat its last
+// function, and their D is 0; columns past it repeat its last one and are not
+// used.  The list entries of a step are read a step ahead of its loads.
+//
+// ST = 2: two LDS stages, one barrier per step; ST = 1: one stage.
+template <typename T, int BN, int VAR>
+struct DensTile {
+  static constexpr int BK = Var<VAR>::BK, ST = Var<VAR>::ST;
+  static constexpr int SA = kDBM + kLPad, SB = BN + kLPad, R = BK / 4;
+  static constexpr int kLds = ST * BK * (SA + SB);
+  typedef typename V2<T>::type v2;
+  typedef typename MF<T>::acc acc_t;
+
+  template <int NB>
+  __device__ static __forceinline__ void run(const T *__restrict__ phi, long Mc,
+                                             const T *__restrict__ D, long NP,
+                                             const uint16_t *__restrict__ fl, int K,
+                                             const uint16_t *__restrict__ cf, int ncol, T *lds,
+                                             acc_t (&acc)[2][NB]) {
+    constexpr bool TWO = NB > 4;  // a second column per lane
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ksteps = (K + BK - 1) / BK;
+    const int c0 = gld(cf + min(lane, ncol - 1)), c1 = TWO ? gld(cf + min(64 + lane, ncol - 1)) : 0;
+    const bool in1 = 64 + lane < BN;
+    v2 ra[R];
+    T rb0[R], rb1[R];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < NB; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    auto list = [&](int kt) { return (int)gld(fl + min(kt * BK + (lane & (BK - 1)), K - 1)); };
+    auto load = [&](int fk) {
+#pragma unroll
+      for (int e = 0; e < R; ++e) {
+        const long f = __builtin_amdgcn_readlane(fk, wave + 4 * e);
+        ra[e] = gld((const v2 *)(phi + f * Mc) + lane);
+        rb0[e] = gld(D + f * NP + c0);
+        if constexpr (TWO) rb1[e] = gld(D + f * NP + c1);
+      }
+    };
+    auto store = [&](int buf, int kt) {
+      T *as = lds + buf * BK * (SA + SB), *bs = as + BK * SA;
+#pragma unroll
+      for (int e = 0; e < R; ++e) {
+        const int r = wave + 4 * e;
+        const bool live = kt * BK + r < K;
+        *(v2 *)(as + r * SA + 2 * lane) = ra[e];
+        bs[r * SB + lane] = live ? rb0[e] : T(0);
+        if constexpr (TWO)
+          if (in1) bs[r * SB + 64 + lane] = live ? rb1[e] : T(0);
+      }
+    };
+    const int ar = 32 * wave + row_point<T>(lane & 15), br = lane & 15, kg = lane >> 4;
+    auto compute = [&](int buf) {
+      const T *as = lds + buf * BK * (SA + SB) + kg * SA + ar;
+      const T *bs = lds + buf * BK * (SA + SB) + BK * SA + kg * SB + br;
+#pragma unroll
+      for (int k4 = 0; k4 < BK / 4; ++k4) {
+        T a[2], b[NB];
+        a[0] = as[4 * k4 * SA];
+        a[1] = as[4 * k4 * SA + 16];
+#pragma unroll
+        for (int j = 0; j < NB; ++j) b[j] = bs[4 * k4 * SB + 16 * j];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) acc[i][j] = MF<T>::mma(a[i], b[j], acc[i][j]);
+      }
+    };
+    int fn = list(0);
+    load(fn);
+    fn = list(1);
+    if constexpr (ST == 2) {
+      store(0, 0);
+      __syncthreads();
+      for (int kt = 0; kt < ksteps; ++kt) {
+        load(fn);  // step kt + 1 (past the end: the last function again, D 0)
+        fn = list(kt + 2);
+        compute(kt & 1);
+        store((kt & 1) ^ 1, kt + 1);
+        __syncthreads();
+      }
+    } else {
+      for (int kt = 0; kt < ksteps; ++kt) {
+        store(0, kt);
+        __syncthreads();
+        load(fn);
+        fn = list(kt + 2);
+        compute(0);
+        __syncthreads();
+      }
+    }
+  }
+};
+
+// Column chunks of a tile of nf functions, BN at most per chunk: as many chunks
+// as BN needs, their 16-column blocks shared out evenly (a chunk of few columns
+// would stage every point of the tile for little work).
+__device__ __forceinline__ int chunk_cols(int nf, int BN) {
+  const int nch = (nf + BN - 1) / BN, nb = (nf + 15) / 16;
+  return 16 * ((nb + nch - 1) / nch);
+}
+
+// Sums of a wave's 32 points over a chunk's columns: part[0] = sum_n Phi X,
+// part[c] = 2 sum_n d_c Phi X.  A lane holds four consecutive points of one
+// column per block: 16-byte loads; the 16 lanes of a block's columns are summed
+// by group_reduce, and the wave holds every column, so nothing crosses waves.
+// Absent columns read the chunk's first function and add nothing.
+template <typename T, int NB, bool GRAD>
+__device__ __forceinline__ void density_sums(typename MF<T>::acc (&acc)[2][NB],
+                                             const T *__restrict__ phi, long Mc, long cs,
+                                             const uint16_t *__restrict__ cf, int ncol,
+                                             double *__restrict__ part) {
+  constexpr int NC = GRAD ? 4 : 1, NV = 4 * (int)sizeof(T) / 16, E = 16 / (int)sizeof(T);
+  typedef T vec __attribute__((ext_vector_type(16 / sizeof(T))));
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int p0 = 32 * wave + 4 * (lane >> 4);
+  const T *ph[NB];
+#pragma unroll
+  for (int j = 0; j < NB; ++j) {
+    const int n = 16 * j + (lane & 15);
+    ph[j] = phi + (long)gld(cf + (n < ncol ? n : 0)) * Mc + p0;
+    if (n >= ncol)
+#pragma unroll
+      for (int i = 0; i < 2; ++i) acc[i][j] = typename MF<T>::acc{0, 0, 0, 0};
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll 1  // one plane's loads in flight at a time: more would spill
+    for (int c = 0; c < NC; ++c) {
+      vec v[NB][NV];
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int q = 0; q < NV; ++q) v[j][q] = gld((const vec *)(ph[j] + c * cs + 16 * i) + q);
+      double t[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) t[r] += (double)v[j][r / E][r % E] * (double)acc[i][j][r];
+      int idx;
+      const double tot = group_reduce<4>(t, lane, idx);
+      if ((lane & 3) == 0) gst(part + (long)c * Mc + p0 + 16 * i + idx, c ? 2.0 * tot : tot);
+    }
+}
+
+// item = (128-point tile, pair of column chunks of its functions).  Bound by
+// the matrix cores and, about equally, the sums' reads of Phi and d Phi (32
+// bytes per point and function, 14 GB at (H2O)32 in FP64).  The kernel before
+// walked whole runs of 8 functions and 96-column chunks (1.4 times the MFMAs)
+// and looked every operand vector up in the run list as it loaded it: FP64
+// density stage of an (H2O)32 build, one lane, 10.8 ms; now 6.5.
+template <typename T, int BN, int VAR, bool GRAD>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const StageList S) {
+  typedef DensTile<T, BN, VAR> G;
+  __shared__ __attribute__((aligned(16))) T lds[G::kLds];
+  __shared__ long slot;
+  for (long L = walk_next(S, -1, &slot); L < S.total;) {
+    const uint64_t t0 = S.tlog ? wall_clock64() : 0;
+    const long it = walk_item(S, L);
+    const int u = unit_of(S.base, S.nu, it);
+    const UnitD &U = S.units[u];
+    const uint32_t e = U.ditems[it - S.base[u]];
+    const int tile = (int)(e >> 8), pair = (int)(e & 255);
+    const long m0 = (long)tile * kDBM, Mc = U.Mc, NP = U.NP;
+    const int off = U.tf_off[tile], nf = U.tf_off[tile + 1] - off;
+    const uint16_t *fl = U.tfl + off;
+    const int cc = chunk_cols(nf, BN), nch = (nf + BN - 1) / BN;
+    const T *phi = (const T *)U.phi + m0, *D = (const T *)U.D;
+    int ahead = 0;
+    for (int ch = 2 * pair; ch < min(2 * pair + 2, nch); ++ch) {
+      const bool last = ch + 1 == min(2 * pair + 2, nch);
+      const uint16_t *cf = fl + ch * cc;
+      const int ncol = min(cc, nf - ch * cc);
+      auto go = [&](auto nb) {
+        constexpr int NB = decltype(nb)::value;
+        typename MF<T>::acc acc[2][NB];
+        __syncthreads();  // the previous chunk's readers of the LDS stages are done
+        G::template run<NB>(phi, Mc, D, NP, fl, nf, cf, ncol, lds, acc);
+        if (last) ahead = walk_ahead(S);
+        density_sums<T, NB, GRAD>(acc, phi, Mc, NP * Mc, cf, ncol, U.part + (long)ch * 4 * Mc + m0);
+      };
+      // built for 2 blocks and from half a chunk up (a tile of more than one
+      // chunk has no fewer in any but its last)
+      const int nb = (ncol + 15) / 16;
+      if (nb <= 2) go(std::integral_constant<int, 2>{});
+      else if (BN == 96 ? nb <= 4 : nb <= BN / 32 + 1) go(std::integral_constant<int, (BN == 96 ? 4 : BN / 32 + 1)>{});
+      else if (BN > 64 && nb <= BN / 16 - 1) go(std::integral_constant<int, (BN > 64 ? BN / 16 - 1 : 4)>{});
+      else go(std::integral_constant<int, BN / 16>{});
+    }
+    item_log(S, it, t0);
+    L = walk_take(S, L, ahead, &slot);
+  }
+}
+
+template <typename T, int BN, int VAR>
+static void density_bn(hipStream_t s, bool grad, const StageList &L) {
+  dim3 g(contraction_grid(L, 2));
+  if (grad)
+    hipLaunchKernelGGL((k_density<T, BN, VAR, true>), g, dim3(kThreads), 0, s, L);
+  else
+    hipLaunchKernelGGL((k_density<T, BN, VAR, false>), g, dim3(kThreads), 0, s, L);
+}
+
+template <typename T, int VAR>
+static void density_var(hipStream_t s, bool grad, int tf, const StageList &L) {
+  switch (tf) {
+    case 64: density_bn<T, 64, VAR>(s, grad, L); break;
+    case 96: density_bn<T, 96, VAR>(s, grad, L); break;
+    default: density_bn<T, 128, VAR>(s, grad, L); break;
+  }
+}
+
+template <typename T>
+void launch_density(hipStream_t s, bool grad, int tf, int var, const StageList &L) {
+  if (!L.total) return;
+  switch (var) {
+    case 1: density_var<T, 1>(s, grad, tf, L); break;
+    case 2: density_var<T, 2>(s, grad, tf, L); break;
+    default: density_var<T, 0>(s, grad, tf, L); break;
+  }
+}
+
+}  // namespace pgxc

@@ -1,0 +1,6 @@
+// FP32 instances of the contraction kernels.
+#include "xc_contract.h"
+
+namespace pgxc {
+template void launch_density<float>(hipStream_t, bool, int, int, const StageList &);
+}  // namespace pgxc

@@ -127,6 +127,12 @@ struct MF<float> {
 __device__ __forceinline__ int mf_col(int lane) { return lane & 15; }
 
 
+// K step and LDS stages of the contraction variants the layout can select
+template <int V> struct Var;
+template <> struct Var<0> { static constexpr int BK = 16, ST = 2; };
+template <> struct Var<1> { static constexpr int BK = 32, ST = 1; };
+template <> struct Var<2> { static constexpr int BK = 32, ST = 2; };
+
 // ---------------------------------------------------------------- screening
 // Order-preserving compaction over the workgroup: threads with act append
 // value to list (after `base` entries); returns the new length.  Every thread
@@ -216,8 +222,7 @@ __device__ __forceinline__ double group_reduce(double (&v)[M], int lane, int &in
 // 16-lane group reduction) and written to part[ch][c][p].  Column n of the
 // chunk is function cfn[n] for n < ncol (absent columns add nothing).  With
 // the FP32 result placement a lane holds four consecutive points of one
-// column, read as one 16-byte load per component; the FP64 placement reads
-// point by point.  A lane's columns are looked up once; the loads of IB row
+// column, read as one 16-byte load per component.  A lane's columns are looked up once; the loads of IB row
 // blocks (IB divides the wave's row blocks) are issued together and
 // unconditionally (an absent column reads function 0 and adds nothing), so
 // their latencies overlap instead of following one another.  Waves as in
@@ -225,14 +230,14 @@ __device__ __forceinline__ double group_reduce(double (&v)[M], int lane, int &in
 // make one partial slot: slot ch + s sums wave columns 2s and 2s + 1, and
 // the first nslots slots are written.
 template <typename T, typename ACC, int BM, int BN, bool GRAD, int IB = 1, int NT = kThreads,
-          int WGN = 2, bool PW = false>
+          int WGN = 2>
 __device__ __forceinline__ void density_epilogue(
     const ACC (&acc)[BM / (NT / 64 / WGN) / 16][BN / WGN / 16], const T *__restrict__ phi,
     long Mc, int NP, long m0, const uint16_t *cfn, int ncol, int ch, double *__restrict__ part,
     double (&red)[WGN][4][BM], int nslots = 1) {
   constexpr int WGM = NT / 64 / WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
   constexpr int NC = GRAD ? 4 : 1, SLOTS = WGN / 2;
-  constexpr bool QUAD = MF<T>::kQuadRows;
+  static_assert(MF<T>::kQuadRows, "a lane's results are four consecutive points");
   static_assert(TM % IB == 0 && WGN % 2 == 0, "whole rounds of row blocks, wave column pairs");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int wm = wave / WGN, wn = wave % WGN;
@@ -245,48 +250,6 @@ __device__ __forceinline__ void density_epilogue(
     live[j] = e < ncol;
     col[j] = live[j] ? (long)cfn[min(e, ncol - 1)] * Mc : 0;
   }
-  if constexpr (PW) {
-    // one component plane at a time (a quarter of the registers of the loads;
-    // each sum is formed in the same order)
-    static_assert(!QUAD, "point-by-point placement");
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      double s[NC][4];
-#pragma unroll
-      for (int c = 0; c < NC; ++c) {
-        T v[TN][4];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const long q0 = col[j] + m0 + wm * WM + i * 16;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[j][r] = gld(phi + c * cs + q0 + MF<T>::row(lane, r));
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[c][r] = 0.0;
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          if (!live[j]) continue;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const double xv = (double)acc[i][j][r];
-            if (c == 0) s[0][r] += (double)v[j][r] * xv;
-            else s[c][r] += 2.0 * (double)v[j][r] * xv;
-          }
-        }
-      }
-      double w[NC * 4];
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) w[c * 4 + r] = s[c][r];
-      int idx;
-      const double tot = group_reduce<NC * 4>(w, lane, idx);
-      if (NC == 4 || (lane & 3) == 0) {
-        const int c = idx / 4, r = idx % 4;
-        red[wn][c][wm * WM + i * 16 + MF<T>::row(lane, r)] = tot;
-      }
-    }
-  } else {
 #pragma unroll
   for (int i0 = 0; i0 < TM; i0 += IB) {
     T v[IB][TN][NC][4];
@@ -295,18 +258,11 @@ __device__ __forceinline__ void density_epilogue(
 #pragma unroll
       for (int j = 0; j < TN; ++j) {
         const long q0 = col[j] + m0 + wm * WM + (i0 + ii) * 16;
-        if constexpr (QUAD) {
-          const long q = q0 + MF<T>::row(lane, 0);
+        const long q = q0 + MF<T>::row(lane, 0);
 #pragma unroll
-          for (int c = 0; c < NC; ++c) {
-            const f4 t = gld((const f4 *)(phi + c * cs + q));
-            v[ii][j][c][0] = t.x; v[ii][j][c][1] = t.y; v[ii][j][c][2] = t.z; v[ii][j][c][3] = t.w;
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) v[ii][j][c][r] = gld(phi + c * cs + q0 + MF<T>::row(lane, r));
+        for (int c = 0; c < NC; ++c) {
+          const f4 t = gld((const f4 *)(phi + c * cs + q));
+          v[ii][j][c][0] = t.x; v[ii][j][c][1] = t.y; v[ii][j][c][2] = t.z; v[ii][j][c][3] = t.w;
         }
       }
 #pragma unroll
@@ -340,7 +296,6 @@ __device__ __forceinline__ void density_epilogue(
         red[wn][c][wm * WM + i * 16 + MF<T>::row(lane, r)] = tot;
       }
     }
-  }
   }
   __syncthreads();
   for (int idx = tid; idx < SLOTS * NC * BM; idx += NT) {

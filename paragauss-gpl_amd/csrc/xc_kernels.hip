@@ -4,8 +4,6 @@
 //
 //   k_basis       basis values and gradients  (ParaGauss modules/orbital_module.f90:1742-1932,
 //                 2421-2619; solid harmonics modules/solid_harmonics_module.f90:369-568)
-//   k_density     X = Phi D on MFMA, fused rho = sum Phi X, grad rho = 2 sum dPhi X
-//                 (modules/density_calc_module.f90:1478-1577)
 //   k_functional  Slater + PW92 + PBE-x + PBE-c in FP64, closed-form derivatives
 //                 (modules/xc_func.f90:187-305 and the term modules)
 //   k_wmat        W = a Phi + b . grad Phi  (modules/xc_hamiltonian.f90:1429-1483)
@@ -800,75 +798,6 @@ __global__ __launch_bounds__(kThreads) void k_wbasis(const UnitD *__restrict__ u
 
 // ----------------------------------------------------------------- density
 constexpr int kDBM = 128;
-
-// K step and LDS stages of the contraction variants the layout can select
-template <int V> struct Var;
-template <> struct Var<0> { static constexpr int BK = 16, ST = 2; };
-template <> struct Var<1> { static constexpr int BK = 32, ST = 1; };
-template <> struct Var<2> { static constexpr int BK = 32, ST = 2; };
-
-// item = (128-point tile, pair of function tiles of its gathered runs) of
-// X = Phi D, then the tile's partial contractions per point, one slot per
-// function tile
-template <typename T, int BN, int VAR, bool GRAD>
-__global__ __launch_bounds__(kThreads)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 || VAR != 2 ? 2 : 1))) void k_density(const StageList S) {
-  constexpr int BM = kDBM, BK = Var<VAR>::BK, ST = Var<VAR>::ST, TM = BM / 32, TN = BN / 32;
-  __shared__ T As[lds_elems<T, BM, BK, ST, false>()];
-  __shared__ __attribute__((aligned(16))) T Bs[lds_elems<T, BN, BK, ST, true>()];
-  __shared__ double red[2][4][BM];
-  __shared__ uint16_t kl[kMaxRuns];
-  __shared__ uint8_t km[kMaxRuns];  // per run of kl: its functions in the tile's list
-  __shared__ uint16_t cl[2 * BN];
-  __shared__ long slot;
-  for (long L = walk_next(S, -1, &slot); L < S.total;) {
-    const uint64_t t0 = S.tlog ? wall_clock64() : 0;
-    const long it = walk_item(S, L);
-    const int u = find_unit(S.base, S.nu, it);
-    const UnitD &U = S.units[u];
-    const uint32_t e = U.ditems[it - S.base[u]];
-    const int tile = (int)(e >> 8), pair = (int)(e & 255);
-    const long m0 = (long)tile * BM, Mc = U.Mc, NP = U.NP;
-    const int off = U.tl_off[tile], c8 = U.tl_off[tile + 1] - off;
-    const int foff = U.tf_off[tile] + 2 * pair * BN, nf = U.tf_off[tile + 1] - foff;
-    __syncthreads();  // the previous item's readers of kl and cl are done
-    for (int i = threadIdx.x; i < min(2 * BN, nf); i += kThreads) cl[i] = gld(U.tfl + foff + i);
-    for (int i = threadIdx.x; i < c8; i += kThreads) km[i] = gld(U.tlm + off + i);
-    lds_list(U.tl + off, c8, kl);
-    const int ksteps = (c8 * kRun + BK - 1) / BK;
-    const T *phi = (const T *)U.phi, *D = (const T *)U.D;
-    int ahead = 0;
-    // the item's two column chunks in turn (the second may be absent)
-    for (int h = 0; h < 2 && h * BN < nf; ++h) {
-      const uint16_t *cfn = cl + h * BN;
-      const int ncol = min(BN, nf - h * BN);
-      // A(m, k) = Phi[f(k)][m0 + m], B(k, n) = D[f(k)][col(n)] = D[col(n)][f(k)]
-      // (D symmetric, so B is k-contiguous along runs): K runs over the
-      // tile's gathered runs, the columns over its functions; A is 0 for the
-      // functions of the runs outside the tile's list (left unwritten by the
-      // basis stage)
-      auto aaddr = [&](int m, int kt, int kk) -> long {
-        const int k = kt * BK + kk;
-        const long f = run_fn(kl, c8, k);
-        return (f < 0 || !((km[k >> 3] >> (k & 7)) & 1u)) ? -1 : f * Mc + m;
-      };
-      auto baddr = [&](int n, int kt, int kk) -> long {
-        const long f = run_fn(kl, c8, kt * BK + kk);
-        return (f < 0 || n >= ncol) ? -1 : (long)cfn[min(n, ncol - 1)] * NP + f;
-      };
-      typename MF<T>::acc acc[TM][TN];
-      gemm_tile<T, BM, BN, BK, ST, false, true>(phi + m0, D, ksteps, aaddr, baddr, As, Bs, acc);
-      if (h == 1 || (h + 1) * BN >= nf) ahead = walk_ahead(S);  // the last chunk
-      // FP64 variants 0 and 1 run two waves per SIMD: their epilogue reads
-      // one component plane at a time to fit the registers
-      constexpr bool PW = sizeof(T) == 8 && VAR != 2;
-      density_epilogue<T, typename MF<T>::acc, BM, BN, GRAD, 1, kThreads, 2, PW>(
-          acc, phi, Mc, U.NP, m0, cfn, ncol, 2 * pair + h, U.part, red);
-    }
-    item_log(S, it, t0);
-    L = walk_take(S, L, ahead, &slot);
-  }
-}
 
 // item = 256-point block of a unit
 template <bool GGA>
@@ -1706,34 +1635,6 @@ void launch_xy(hipStream_t s, int tf, int var, const StageList &L, const double 
   }
 }
 
-template <typename T, int BN, int VAR>
-static void density_bn(hipStream_t s, bool grad, const StageList &L) {
-  dim3 g(contraction_grid(L, 2));
-  if (grad)
-    hipLaunchKernelGGL((k_density<T, BN, VAR, true>), g, dim3(kThreads), 0, s, L);
-  else
-    hipLaunchKernelGGL((k_density<T, BN, VAR, false>), g, dim3(kThreads), 0, s, L);
-}
-
-template <typename T, int VAR>
-static void density_var(hipStream_t s, bool grad, int tf, const StageList &L) {
-  switch (tf) {
-    case 64: density_bn<T, 64, VAR>(s, grad, L); break;
-    case 96: density_bn<T, 96, VAR>(s, grad, L); break;
-    default: density_bn<T, 128, VAR>(s, grad, L); break;
-  }
-}
-
-template <typename T>
-void launch_density(hipStream_t s, bool grad, int tf, int var, const StageList &L) {
-  if (!L.total) return;
-  switch (var) {
-    case 1: density_var<T, 1>(s, grad, tf, L); break;
-    case 2: density_var<T, 2>(s, grad, tf, L); break;
-    default: density_var<T, 0>(s, grad, tf, L); break;
-  }
-}
-
 void launch_functional(hipStream_t s, bool gga, const StageList &L) {
   if (!L.total) return;
   dim3 g(persistent_grid(L.total, 8));
@@ -1849,7 +1750,6 @@ void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, lon
 
 #define PGXC_INST(T)                                                                  \
   template void launch_basis<T>(hipStream_t, bool, const StageList &);               \
-  template void launch_density<T>(hipStream_t, bool, int, int, const StageList &);   \
   template void launch_wmat<T>(hipStream_t, bool, bool, bool, const StageList &);    \
   template void launch_potential<T>(hipStream_t, int, int, const StageList &);
 PGXC_INST(double)
