@@ -138,8 +138,9 @@ int pgxc_create_opt(pgxc_ctx **ctx, int32_t n_atoms, const double *atom_xyz,
                     int64_t npts, int32_t veclen, const pgxc_options *opt);
 
 /* Layout chosen for a context: [0] padded nbas, [1] function tile,
- * [2] points per chunk, [3] chunks, [4] point splits of the potential
- * contraction, [5] padded number of points, [6] FP64 variant, [7] FP32 variant. */
+ * [2] points per chunk, [3] chunks, [4] blocks of 2048 or more points a chunk
+ * is made of (the potential contraction cuts them into shorter splits),
+ * [5] padded number of points, [6] FP64 variant, [7] FP32 variant. */
 int pgxc_layout(const pgxc_ctx *ctx, int64_t *out8);
 
 /*

@@ -73,7 +73,8 @@ struct pgxc_ctx {
   int lmax = 0;  // largest angular momentum of the basis
   int var[2] = {0, 1};  // contraction variant for FP64 and for FP32 builds
   long npts = 0, npad = 0, Mc = 0;
-  int nchunks = 0, nsplit = 1, ntiles = 0;
+  int nchunks = 0, nsplit = 1, ntiles = 0;  // nsplit: the chunk rounding's blocks (pgxc_layout)
+  int nsp = 1;  // point splits of the potential contraction per chunk (setup_screen)
   long nblk_total = 0;
   // device: geometry and basis
   double *grid = nullptr;  // [4][npad] x, y, z, w
@@ -101,13 +102,20 @@ struct pgxc_ctx {
   void *phi_base = nullptr;  // Phi of the current build: chunk k at phi_base + k * phi_stride
   size_t phi_stride = 0;
   int skip_basis = 0;        // the current build reads cached basis values
-  double *part = nullptr, *coef = nullptr, *Hpart = nullptr;
+  double *part = nullptr, *coef = nullptr;
+  // potential partials: slots of one chunk's splits each (hstride doubles),
+  // hslots of them over all lanes; every chunk its own slot, or (hflush) as
+  // many as kPartialBytes hold, summed into HS whenever a lane's are full.
+  // HS: [nseg][NP][NP] their symmetric sums
+  double *Hc = nullptr, *HS = nullptr;
+  long hstride = 0;
+  int hslots = 0, hflush = 0, nseg = 1;
   // open shell (ispin = 2): the fields above and below serve the alpha spin,
   // these the beta spin (allocated with the first open-shell density; the
   // basis values and the work tables are shared)
   int ispin = 1;
   struct Beta {
-    double *P = nullptr, *Pref = nullptr, *part = nullptr, *coef = nullptr, *Hpart = nullptr;
+    double *P = nullptr, *Pref = nullptr, *part = nullptr, *coef = nullptr, *Hc = nullptr, *HS = nullptr;
     double *state = nullptr, *Vstate = nullptr, *Vout = nullptr;
     void *D = nullptr, *W = nullptr;
     size_t w_bytes = 0;
@@ -132,17 +140,16 @@ struct pgxc_ctx {
   // screening and work tables over the padded grid (setup_screen)
   int screen = 0, n8 = 0, nw8 = 0, CH = 0;
   int *nbt = nullptr;
-  uint32_t *sig8 = nullptr, *wbits = nullptr;
+  uint32_t *sig8 = nullptr;
   ScreenShell *sshells = nullptr;
   double flops_screened = 0, flops_dense = 0;  // algorithmic work of one build
   double sum_bn = 0, sum_n2 = 0;  // sums over 128-point tiles of B n_b and n_b^2 (screened)
-  // host and device copies: per tile run lists, per split run unions and
-  // [group][chunk] flags, per chunk density and potential items
+  // host and device copies: per tile run and function lists, per split
+  // function unions, per chunk density and potential items
   std::vector<int> h_tl_off, h_su_off, h_tf_off;
   std::vector<uint16_t> h_tl, h_su, h_tfl;
   std::vector<uint8_t> h_tlm;
-  std::vector<long> h_gcf_off, h_di_off, h_pi_off;
-  std::vector<uint8_t> h_gcf;
+  std::vector<long> h_di_off, h_pi_off;
   std::vector<uint32_t> h_di, h_pi;
   int *tl_off = nullptr, *su_off = nullptr, *tf_off = nullptr;
   uint16_t *tl = nullptr, *su = nullptr, *tfl = nullptr;
@@ -150,16 +157,18 @@ struct pgxc_ctx {
   uint32_t *tfb = nullptr;  // per tile, its functions as a bitmap of nwf words
   int nwf = 0;
   // per entry of a split's function list: bit t set when the function is
-  // in the list of the split's tile t (every bit when a split has more than
-  // 32 tiles)
+  // in the list of the split's tile t
   std::vector<uint32_t> h_sumask;
   uint32_t *sumask = nullptr;
+  // per split: where its partial lies in a slot, the functions' places in its
+  // list, and (per 32 functions, a bit per split) whether it has any of them
+  long *ho = nullptr;
+  uint16_t *pos = nullptr;
+  uint8_t *rbits = nullptr;
   // nuclear gradient work space (first gradient on): Hessian planes and
   // products of one chunk, per-(tile, function) sums
   double *ghess = nullptr, *gXY = nullptr, *gpart = nullptr;
   long gpart_n = 0;
-  long *gcf_off = nullptr;
-  uint8_t *gcf = nullptr;
   uint32_t *di = nullptr, *pi = nullptr;
   // blocks of the basis values some stage reads (see setup_screen): per
   // chunk the basis items (256-point block << 16 | atom range) that touch
@@ -207,8 +216,16 @@ const int kTiles[3] = {64, 96, 128};
 // density / potential lists per (function tile, variant): index 3 * t + v
 constexpr int kLists = 3 * kNumVariants;
 
+struct FoldList {
+  const FoldD *d = nullptr;
+  const long *base = nullptr;
+  int n = 0;
+  long total = 0;
+};
+
 struct StepPlan {
   int nunits = 0;
+  FoldList flush;  // the partials summed after this step (lanes whose slots are full)
   StageList basis, func, func2, wmat, wmat2;  // func2, wmat2: open-shell units
   StageList dens[kLists], pot[kLists];
 };
@@ -225,14 +242,6 @@ struct Plan {
   long model_version = -1;
   int *d_ctr = nullptr;  // queue counters of every contraction list
   long nctr = 0;
-  // H partials, cleared at the start: (buffer, ints, lane); lane 1's on the
-  // second stream, overlapping the first lane's first stages
-  struct HZero {
-    int *p;
-    long n;
-    int lane;
-  };
-  std::vector<HZero> hzero;
   // item log: features of every contraction item (row-major), and per list
   // the device log and the list's first feature row
   std::vector<double> feat;
@@ -243,8 +252,9 @@ struct Plan {
   std::vector<int> lanes;  // lanes in use per molecule when the plan was made
   std::vector<int> spins;  // ispin per molecule when the plan was made
   PackD *d_pack = nullptr;
-  long *d_pack_base = nullptr, *d_prep_base = nullptr, *d_fold_base = nullptr;
-  long pack_total = 0, prep_total = 0, fold_total = 0;
+  long *d_pack_base = nullptr, *d_prep_base = nullptr;
+  long pack_total = 0, prep_total = 0;
+  FoldList fold;
   int nmol = 0;
   char *blob = nullptr;  // device memory holding every list
   hipGraphExec_t graph = nullptr;
@@ -335,18 +345,23 @@ static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int p
       push(0, (double)c8 * kRun, c->NP, true, 2.0 * kScreenTile * cols * c8 * kRun);
     }
   } else {
-    const long spts = c->Mc / c->nsplit, G = spts / kGroup;
+    const long spts = c->Mc / c->nsp;
+    std::vector<uint32_t> cm;  // per chunk of the current split: its tiles
+    long last = -1;
     for (long i = c->h_pi_off[step]; i < c->h_pi_off[step + 1]; ++i) {
       const uint32_t e = c->h_pi[(size_t)i];
-      const long S = (long)step * c->nsplit + (e >> 20);
+      const long S = (long)step * c->nsp + (e >> 20);
       const int ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);
-      const int nu = c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S], nch = (nu + tf - 1) / tf;
-      const uint8_t *fl = c->h_gcf.data() + c->h_gcf_off[(size_t)S];
-      long cnt = 0;
-      for (long g = 0; g < G; ++g) cnt += (fl[g * nch + ci] & fl[g * nch + cj]) != 0;
+      const int so = c->h_su_off[(size_t)S], nu = c->h_su_off[(size_t)S + 1] - so;
+      if (S != last) {
+        cm.assign((size_t)(nu + tf - 1) / tf, 0u);
+        for (int f = 0; f < nu; ++f) cm[(size_t)f / tf] |= c->h_sumask[(size_t)so + f];
+        last = S;
+      }
+      const long cnt = __builtin_popcount(cm[(size_t)ci] & cm[(size_t)cj]) * (long)kScreenTile;
       const double rows = (double)std::min(tf, nu - ci * tf);
       const double cols = (double)std::min(tf, nu - cj * tf);
-      push(1, (double)cnt * kGroup, (double)spts, cnt > 0, 2.0 * rows * cols * cnt * kGroup);
+      push(1, (double)cnt, (double)spts, cnt > 0, 2.0 * rows * cols * cnt);
     }
   }
 }
@@ -485,17 +500,19 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.state = c->state + p0;
       U.epart = c->epart + 2 * (p0 / kThreads);
       U.eterm = c->eterm + 5 * (p0 / kThreads);
-      U.Hpart = c->Hpart + (size_t)lane * c->nsplit * c->NP * c->NP;
+      const int L = lanes_of(c), R = c->hslots / L;  // the lane's share of the slots
+      const size_t hslot = (size_t)(k % L) * R + (k / L) % R;
+      U.Hc = c->Hc + hslot * c->hstride;
+      U.ho = c->ho + (long)k * c->nsp;
       U.Mc = c->Mc;
       U.npad = c->npad;
       U.n_atoms = c->n_atoms;
       U.NP = c->NP;
       U.ntiles = c->ntiles;
-      U.nsplit = c->nsplit;
+      U.nsplit = c->nsp;
       U.incremental = incr[m];
       U.mask = functional;
       U.CH = c->CH;
-      U.nw8 = c->nw8;
       U.ditems = c->di + c->h_di_off[k];
       U.pitems = c->pi + c->h_pi_off[k];
       U.ndi = c->h_di_off[k + 1] - c->h_di_off[k];
@@ -507,13 +524,9 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.tfb = c->tfb + (p0 / kScreenTile) * c->nwf;
       U.tlm = c->tlm;
       U.nwf = c->nwf;
-      U.su_off = c->su_off + (long)k * c->nsplit;
+      U.su_off = c->su_off + (long)k * c->nsp;
       U.su = c->su;
       U.sumask = c->sumask;
-      U.gcf_off = c->gcf_off + (long)k * c->nsplit;
-      U.gcf = c->gcf;
-      U.sig8 = c->sig8 + (p0 / kGroup) * c->nw8;
-      U.wbits = c->wbits + (p0 / kGroup) * c->nw8;
       U.bscreen = dense_basis ? 0 : 1;  // the basis stage writes the blocks read later
       U.bitems = c->bi + c->h_bi_off[k];
       U.bflags = c->bfl + 16 * c->h_bi_off[k];
@@ -525,7 +538,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
         B.part = c->beta.part + (size_t)lane * c->ntiles * 4 * c->Mc;
         B.coef = c->beta.coef + (size_t)lane * 4 * c->Mc;
         B.state = c->beta.state + p0;
-        B.Hpart = c->beta.Hpart + (size_t)lane * c->nsplit * c->NP * c->NP;
+        B.Hc = c->beta.Hc + hslot * c->hstride;
         U.part2 = B.part;
         U.coef2 = B.coef;
         U.state2 = B.state;
@@ -664,7 +677,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     for (int sp = 0; sp < c->ispin; ++sp) {
       PackD Q;
       memset(&Q, 0, sizeof(Q));
-      Q.Hpart = sp ? c->beta.Hpart : c->Hpart;
+      Q.HS = sp ? c->beta.HS : c->HS;
       Q.Vout = sp ? c->beta.Vout : c->Vout;
       Q.Vstate = sp ? c->beta.Vstate : c->Vstate;
       Q.P = sp ? c->beta.P : c->P;
@@ -673,29 +686,97 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       Q.fpos = c->d_fpos;
       Q.n = c->nbas;
       Q.NP = c->NP;
-      Q.nsplit = c->nsplit * lanes_of(c);  // the fold sums the partials of every lane
+      Q.nseg = c->hflush ? lanes_of(c) : c->nseg;
       Q.incremental = incr[m];
       packs.push_back(Q);
-      for (int l = 0; l < lanes_of(c); ++l)
-        plan->hzero.push_back({(int *)(Q.Hpart + (size_t)l * c->nsplit * c->NP * c->NP),
-                               2L * c->nsplit * c->NP * c->NP, l});
     }
   }
   const int npack = (int)packs.size();
-  std::vector<long> pbase(npack + 1, 0), qbase(npack + 1, 0), fbase(npack + 1, 0);
+  std::vector<long> pbase(npack + 1, 0), qbase(npack + 1, 0);
   for (int q = 0; q < npack; ++q) {
     const PackD &Q = packs[q];
     const long npk = Q.n * (Q.n + 1) / 2;
     pbase[q + 1] = pbase[q] + (npk + kThreads - 1) / kThreads;
     qbase[q + 1] = qbase[q] + (Q.NP * Q.NP + kThreads - 1) / kThreads;
-    const long nb = Q.NP / 32;
-    fbase[q + 1] = fbase[q] + nb * (nb + 1) / 2;
   }
+  // sums of the potential partials: after the step that fills a lane's slots
+  // or ends the lane (molecules with more chunks than slots), else all at the
+  // end, in segments of the splits
+  auto fold_of = [&](const pgxc_ctx *c, int sp) {
+    FoldD F;
+    memset(&F, 0, sizeof(F));
+    F.Hc = sp ? c->beta.Hc : c->Hc;
+    F.ho = c->ho;
+    F.su_off = c->su_off;
+    F.pos = c->pos;
+    F.rbits = c->rbits;
+    F.out = sp ? c->beta.HS : c->HS;
+    F.stride = c->hstride;
+    F.NP = c->NP;
+    F.nsplit = c->nsp;
+    F.bytes_c = (c->nsp + 7) / 8;
+    F.nbytes = F.bytes_c * c->nchunks;
+    F.lanes = lanes_of(c);
+    F.slots = c->hslots / F.lanes;
+    return F;
+  };
+  struct FoldOff {
+    size_t d = 0, base = 0;
+    int n = 0;
+    long total = 0;
+  };
+  auto put_folds = [&](const std::vector<FoldD> &fs) {
+    FoldOff o;
+    std::vector<long> fb(fs.size() + 1, 0);
+    for (size_t i = 0; i < fs.size(); ++i) {
+      const long nb = fs[i].NP / 32;
+      fb[i + 1] = fb[i] + nb * (nb + 1) / 2;
+    }
+    o.n = (int)fs.size();
+    o.total = fb.back();
+    o.d = put(fs.data(), sizeof(FoldD) * fs.size());
+    o.base = put(fb.data(), sizeof(long) * fb.size());
+    return o;
+  };
+  std::vector<FoldD> last;
+  std::vector<std::vector<FoldD>> flush((size_t)nsteps);
+  for (int m = 0; m < nm && !energy; ++m) {
+    const pgxc_ctx *c = mols[m];
+    for (int sp = 0; sp < c->ispin; ++sp) {
+      FoldD F = fold_of(c, sp);
+      if (!c->hflush) {
+        F.step = 1;
+        F.nchunks = c->nchunks;
+        F.nseg = c->nseg;
+        double *out = F.out;
+        for (F.seg = 0; F.seg < F.nseg; ++F.seg) {
+          F.out = out + (size_t)F.seg * c->NP * c->NP;
+          last.push_back(F);
+        }
+        continue;
+      }
+      F.step = F.lanes;
+      F.nseg = 1;
+      double *out = F.out;
+      for (int k = 0; k < c->nchunks; ++k) {
+        const int j = k / F.lanes, ln = k % F.lanes;
+        if ((j + 1) % F.slots != 0 && k + F.lanes < c->nchunks) continue;
+        const int j0 = j / F.slots * F.slots;
+        F.out = out + (size_t)ln * c->NP * c->NP;
+        F.chunk0 = j0 * F.lanes + ln;
+        F.nchunks = j - j0 + 1;
+        F.acc = j0 > 0;
+        flush[(size_t)k].push_back(F);
+      }
+    }
+  }
+  const FoldOff last_off = put_folds(last);
+  std::vector<FoldOff> flush_off;
+  for (int k = 0; k < nsteps; ++k) flush_off.push_back(put_folds(flush[(size_t)k]));
   plan->nmol = npack;
   const size_t pack_off = put(packs.data(), sizeof(PackD) * npack);
   const size_t pb_off = put(pbase.data(), sizeof(long) * pbase.size());
   const size_t qb_off = put(qbase.data(), sizeof(long) * qbase.size());
-  const size_t fb_off = put(fbase.data(), sizeof(long) * fbase.size());
   HIPCHK(errc, hipMalloc((void **)&plan->blob, std::max<size_t>(img.size(), 256)));
   HIPCHK(errc, hipMemcpy(plan->blob, img.data(), img.size(), hipMemcpyHostToDevice));
   char *B = plan->blob;
@@ -714,6 +795,14 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     if (P.has_log) plan->logs.push_back({L.tlog, P.total});
     return L;
   };
+  auto mkf = [&](const FoldOff &o) {
+    FoldList f;
+    f.d = (const FoldD *)(B + o.d);
+    f.base = (const long *)(B + o.base);
+    f.n = o.n;
+    f.total = o.total;
+    return f;
+  };
   plan->steps.resize(nsteps);
   for (int k = 0; k < nsteps; ++k) {
     StepPlan &S = plan->steps[k];
@@ -725,13 +814,13 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     S.func2 = mk(pend[k][3 + 2 * kLists]);
     S.wmat2 = mk(pend[k][4 + 2 * kLists]);
     S.nunits = pend[k][0].nu;
+    S.flush = mkf(flush_off[(size_t)k]);
   }
+  plan->fold = mkf(last_off);
   plan->nlanes = plan_lanes;
   plan->d_pack = (PackD *)(B + pack_off);
   plan->d_pack_base = (long *)(B + pb_off);
   plan->d_prep_base = (long *)(B + qb_off);
-  plan->d_fold_base = (long *)(B + fb_off);
-  plan->fold_total = fbase[npack];
   plan->pack_total = pbase[npack];
   plan->prep_total = qbase[npack];
   return PGXC_OK;
@@ -781,18 +870,11 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
   const bool x3 = pl.precision == PGXC_PREC_BF16X3;
   const bool two = pl.nlanes > 1 && pl.steps.size() > 1;
   if (pl.nctr) launch_zero_ints(s, pl.d_ctr, pl.nctr);
-  // potential items add into H: each lane's partials cleared on its stream
-  if (!pl.energy)
-    for (auto &z : pl.hzero)
-      if (z.lane == 0 || !two) launch_zero_ints(s, z.p, z.n);
   launch_prep(s, pl.d_pack, pl.nmol, pl.d_prep_base, pl.prep_total,
               x3 ? 2 : std::is_same<T, double>::value ? 0 : 1, false);
   if (two) {
     (void)hipEventRecord(fork, s);
     (void)hipStreamWaitEvent(s2, fork, 0);
-    if (!pl.energy)
-      for (auto &z : pl.hzero)
-        if (z.lane != 0) launch_zero_ints(s2, z.p, z.n);
   }
   for (size_t k = 0; k < pl.steps.size(); ++k) {
     const StepPlan &S = pl.steps[k];
@@ -838,6 +920,7 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
       launch_potential<T>(t, tf, v, S.pot[li]);
     }
     if (E) (void)hipEventRecord(E[4], t);
+    launch_fold(t, S.flush.d, S.flush.n, S.flush.base, S.flush.total);
   }
   if (two) {
     (void)hipEventRecord(join, s2);
@@ -845,7 +928,7 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
   }
   if (pl.energy) return;
   if (ev) (void)hipEventRecord((*ev)[kEvPack], s);
-  launch_fold(s, pl.d_pack, pl.nmol, pl.d_fold_base, pl.fold_total);
+  launch_fold(s, pl.fold.d, pl.fold.n, pl.fold.base, pl.fold.total);
   launch_pack(s, pl.d_pack, pl.nmol, pl.d_pack_base, pl.pack_total);
   launch_prep(s, pl.d_pack, pl.nmol, pl.d_prep_base, pl.prep_total, 0, true);
   if (ev) (void)hipEventRecord((*ev)[kEvEnd], s);
@@ -1115,6 +1198,17 @@ static int upload(pgxc_ctx *c, V **dst, const std::vector<V> &src) {
   return PGXC_OK;
 }
 
+// potential partials held at a time per molecule and spin, and work items of
+// their sum below which it is cut into segments
+constexpr long kPartialBytes = 4L << 30, kFoldItems = 1536;
+constexpr double kSplitItems = 256.0;  // setup_screen: potential items a chunk has at least
+
+static int alloc_partials(pgxc_ctx *c, double **Hc, double **HS) {
+  int rc = dalloc(c, Hc, (size_t)c->hslots * c->hstride);
+  if (rc) return rc;
+  return dalloc(c, HS, (size_t)std::max(c->nseg, c->nlanes_cap) * c->NP * c->NP);
+}
+
 static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double *exps, bool on) {
   const long ntp = c->npad / kScreenTile, ngr = c->npad / kGroup;
   const double n = (double)c->nbas;
@@ -1124,9 +1218,8 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
   c->screen = on;
   c->nw8 = (c->n8 + 31) / 32;
   const int n8 = c->n8, nw8 = c->nw8;
-  const long G = c->Mc / c->nsplit / kGroup;
   if (n8 > kMaxRuns) return fail(c, PGXC_ERR_UNSUPPORTED, "more than 8192 basis functions (padded)");
-  if (G > kMaxSplitGroups) return fail(c, PGXC_ERR_UNSUPPORTED, "point split above 65536 points");
+  if (c->Mc / c->nsplit > 65536) return fail(c, PGXC_ERR_UNSUPPORTED, "point split above 65536 points");
   std::vector<ScreenShell> ss(sh.size());
   for (size_t i = 0; i < sh.size(); ++i) {
     double amin = exps[sh[i].exp_off];
@@ -1212,137 +1305,87 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
       }
     c->h_tl_off.push_back((int)c->h_tl.size());
   }
+  // Point splits of the potential contraction: kSplitPts points (at most 32
+  // tiles), halved while a chunk has fewer than kSplitItems items (split x pair
+  // of function chunks), one per CU.  A shorter split holds fewer functions its
+  // tiles do not share, but its partial is written and read once.  Whole call at
+  // 1 / 256 / 1024 items: 23-atom LDA build 881 / 743 / 760 us, 14-atom open
+  // shell 1268 / 1180 / 1235, water 326 / 284 / 287, (H2O)16 mixed step 4761 /
+  // 4759 / 5427, (H2O)8 open-shell FP32 step 3547 / 3547 / 3707.
+  {
+    long spts = kSplitPts;
+    const double nt = (double)c->h_tfl.size() / (double)std::max<long>(1, (c->npts + kScreenTile - 1) / kScreenTile);
+    const double nch = std::ceil(1.1 * nt / c->tf);
+    while (spts > kMinSplitPts && (double)(c->Mc / spts) * nch * nch < kSplitItems &&
+           (double)(c->npad / spts) * 4.0 * c->NP <= 268435456.0)  // the places: 256 MiB
+      spts /= 2;
+    c->nsp = (int)(c->Mc / spts);
+  }
   // per split: the union of its tiles' functions (the potential's rows and
-  // columns, in chunks of tf functions), and [group][chunk] flags: whether a
-  // run holding a function of the chunk is live on the group
-  const long NS = (long)c->nchunks * c->nsplit;
-  std::vector<uint32_t> wneed((size_t)ngr * nw8, 0u);
+  // columns, in chunks of tf functions), per entry the split's tiles whose list
+  // holds the function, and the functions' places in it
+  const long NS = (long)c->nchunks * c->nsp, nst = c->Mc / c->nsp / kScreenTile;
+  const int bpc = (c->nsp + 7) / 8;
   c->h_su_off.assign(1, 0);
   c->h_su.clear();
   c->h_sumask.clear();
-  c->h_gcf_off.clear();
-  c->h_gcf.clear();
+  std::vector<long> ho((size_t)NS);
+  std::vector<uint16_t> pos((size_t)NS * c->NP, 0xffff);
+  std::vector<uint8_t> rbits((size_t)(c->NP / 32) * bpc * c->nchunks, 0);
+  c->hstride = 1;
   {
-    const int tf = c->tf;
-    std::vector<uint32_t> fm((size_t)(c->NP + 31) / 32);
-    std::vector<int> cr;  // the distinct runs of one chunk
+    std::vector<uint32_t> tm((size_t)c->NP);
+    long at = 0;
     for (long S = 0; S < NS; ++S) {
-      const long g0 = S * G;
-      std::fill(fm.begin(), fm.end(), 0u);
-      for (long t = g0 / 4; t < (g0 + G) / 4; ++t)
-        for (int i = c->h_tf_off[(size_t)t]; i < c->h_tf_off[(size_t)t + 1]; ++i) {
-          const int f = c->h_tfl[(size_t)i];
-          fm[(size_t)f / 32] |= 1u << (f % 32);
-        }
+      if (S % c->nsp == 0) at = 0;
+      std::fill(tm.begin(), tm.end(), 0u);
+      for (long t = 0; t < nst; ++t)
+        for (int i = c->h_tf_off[(size_t)(S * nst + t)]; i < c->h_tf_off[(size_t)(S * nst + t) + 1]; ++i)
+          tm[c->h_tfl[(size_t)i]] |= 1u << t;
       const size_t u0 = c->h_su.size();
+      const size_t byte = (size_t)(S / c->nsp) * bpc + (size_t)(S % c->nsp) / 8;
       for (int f = 0; f < c->NP; ++f)
-        if ((fm[(size_t)f / 32] >> (f % 32)) & 1u) c->h_su.push_back((uint16_t)f);
+        if (tm[(size_t)f]) {
+          pos[(size_t)S * c->NP + f] = (uint16_t)(c->h_su.size() - u0);
+          rbits[(size_t)(f / 32) * bpc * c->nchunks + byte] |= (uint8_t)(1u << ((S % c->nsp) % 8));
+          c->h_su.push_back((uint16_t)f);
+          c->h_sumask.push_back(tm[(size_t)f]);
+        }
       c->h_su_off.push_back((int)c->h_su.size());
-      // per entry: the split's tiles whose list holds the function
-      const long st0 = g0 / 4, nst = G / 4;
-      for (size_t e = u0; e < c->h_su.size(); ++e) {
-        const int f = c->h_su[e];
-        uint32_t m = 0;
-        if (nst > 32)
-          m = ~0u;
-        else
-          for (long t = 0; t < nst; ++t)
-            m |= ((tfb[(size_t)(st0 + t) * c->nwf + (size_t)f / 32] >> (f % 32)) & 1u) << t;
-        c->h_sumask.push_back(m);
-      }
-      const int nu = (int)(c->h_su.size() - u0), nch = (nu + tf - 1) / tf;
-      c->h_gcf_off.push_back((long)c->h_gcf.size());
-      const size_t gf0 = c->h_gcf.size();
-      c->h_gcf.resize(gf0 + (size_t)G * nch, 0);
-      for (int ch = 0; ch < nch; ++ch) {
-        cr.clear();
-        for (int e = ch * tf; e < std::min(nu, (ch + 1) * tf); ++e) {
-          const int r = c->h_su[u0 + e] / kRun;
-          if (cr.empty() || cr.back() != r) cr.push_back(r);
-        }
-        for (long g = g0; g < g0 + G; ++g) {
-          uint8_t f = 0;
-          for (size_t i = 0; i < cr.size() && !f; ++i) f = (uint8_t)bit(g, cr[i]);
-          c->h_gcf[gf0 + (size_t)(g - g0) * nch + ch] = f;
-          // the potential contraction reads W on this group for every function of a flagged chunk
-          if (f)
-            for (int r : cr) wneed[(size_t)g * nw8 + r / 32] |= 1u << (r % 32);
-        }
-      }
+      ho[(size_t)S] = at;
+      const long ld = round_up((long)(c->h_su.size() - u0), 16);
+      at += ld * ld;
+      c->hstride = std::max(c->hstride, at);
     }
   }
-  if ((rc = upload(c, &c->wbits, wneed))) return rc;
+  if ((rc = upload(c, &c->ho, ho))) return rc;
+  if ((rc = upload(c, &c->pos, pos))) return rc;
+  if ((rc = upload(c, &c->rbits, rbits))) return rc;
   // What the basis stage writes, per (shell, 32-point group): values and
   // gradients of the shells marked on the group's tile, the functions of the
-  // tile's list (the density's operand and epilogue, the W pass and the
-  // potentials read no others: they stage zeros for the rest).  When a point
-  // split spans more than 32 tiles, the potentials' tile masks are off, and
-  // values are also written on the runs of the tile (the density's K) and of
-  // the chunks the potentials read there (wneed).  No stage reads any other
-  // block of a basis-value buffer.
+  // tile's list (the contractions, the density's sums and the W pass read no
+  // others: they stage zeros for the rest).  No stage reads any other block of
+  // a basis-value buffer.
   {
-    std::vector<uint32_t> need((size_t)ngr * 2 * nw8, 0u), tw((size_t)nw8);
-    for (long t = 0; t < ntp; ++t) {
-      std::fill(tw.begin(), tw.end(), 0u);
-      for (int i = c->h_tl_off[(size_t)t]; i < c->h_tl_off[(size_t)t + 1]; ++i)
-        tw[c->h_tl[(size_t)i] >> 5] |= 1u << (c->h_tl[(size_t)i] & 31);
-      for (long g = 4 * t; g < 4 * t + 4; ++g)
-        for (int w = 0; w < nw8; ++w) {
-          need[(size_t)g * 2 * nw8 + w] = tw[(size_t)w] | wneed[(size_t)g * nw8 + w];
-          need[(size_t)g * 2 * nw8 + nw8 + w] = tw[(size_t)w];
-        }
-    }
-    // runs holding each atom range's functions
     const int nr = c->n_ranges;
-    std::vector<uint32_t> rmask((size_t)nr * nw8, 0u);
-    for (int ri = 0; ri < nr; ++ri) {
-      const RangeD &R = c->h_ranges[(size_t)ri];
-      for (int si = R.shell_begin; si < R.shell_begin + R.n_shells; ++si) {
-        const ShellD &d = sh[(size_t)si];
-        const int nf = (2 * d.l + 1) * (d.n_unc + d.n_contr);
-        for (int r = d.func_off / kRun; r <= (d.func_off + nf - 1) / kRun; ++r)
-          rmask[(size_t)ri * nw8 + r / 32] |= 1u << (r % 32);
-      }
-    }
-    std::vector<uint32_t> bi, bfl, bm((size_t)nw8);
-    const bool masked = G / 4 <= 32;
+    std::vector<uint32_t> bi, bfl;
     c->h_bi_off.assign(1, 0);
     const long gpb = kThreads / kGroup;  // groups per basis block
     for (int k = 0; k < c->nchunks; ++k) {
       const long g0 = (long)k * c->Mc / kGroup;
       for (long b = 0; b < c->Mc / kThreads; ++b) {
-        std::fill(bm.begin(), bm.end(), 0u);
-        for (long g = g0 + b * gpb; g < g0 + (b + 1) * gpb; ++g)
-          for (int w = 0; w < nw8; ++w) bm[(size_t)w] |= need[(size_t)g * 2 * nw8 + w];
+        const uint32_t *m0 = smark.data() + (size_t)((g0 + b * gpb) / 4) * nws, *m1 = m0 + nws;
         for (int ri = 0; ri < nr; ++ri) {
-          uint32_t any = 0;
-          for (int w = 0; w < nw8 && !any; ++w) any = bm[(size_t)w] & rmask[(size_t)ri * nw8 + w];
-          if (!any) continue;
-          // per (shell j of the range, group g of the block): values, gradients read
+          // per (shell j of the range, group g of the block): values (words
+          // 0-7) and gradients (8-15) read
           uint32_t fw[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
           const RangeD &R = c->h_ranges[(size_t)ri];
           for (int j = 0; j < R.n_shells; ++j) {
             const int sg = R.shell_begin + j;
-            const ShellD &d = sh[(size_t)sg];
-            const int nf = (2 * d.l + 1) * (d.n_unc + d.n_contr);
-            for (long gg = 0; gg < gpb; ++gg) {
-              const uint32_t *nd = need.data() + (size_t)(g0 + b * gpb + gg) * 2 * nw8;
-              uint32_t v = 0;
-              for (int r = d.func_off / kRun; r <= (d.func_off + nf - 1) / kRun; ++r)
-                v |= nd[r >> 5] >> (r & 31);
-              // gradients: read only for the tile's functions (the density
-              // epilogue's columns, and the W pass's live functions)
-              const long tg = (g0 + b * gpb + gg) / 4;
-              const uint32_t gr = smark[(size_t)tg * nws + sg / 32] >> (sg % 32);
-              const int bit = 8 * j + (int)gg;
-              // values: with the contractions skipping the functions outside
-              // a tile's list (always in the density; in the potentials when a
-              // split spans at most 32 tiles), only those of the shells marked
-              // on the tile
-              fw[bit >> 5] |= ((masked ? gr : v) & 1u) << (bit & 31);
-              fw[8 + (bit >> 5)] |= (gr & 1u) << (bit & 31);
-            }
+            const uint32_t a = (m0[sg / 32] >> (sg % 32)) & 1u, z = (m1[sg / 32] >> (sg % 32)) & 1u;
+            fw[j / 4] |= (0xfu * a | 0xf0u * z) << (8 * (j % 4));
           }
+          for (int w = 0; w < 8; ++w) fw[8 + w] = fw[w];
           if (!(fw[0] | fw[1] | fw[2] | fw[3] | fw[4] | fw[5] | fw[6] | fw[7])) continue;
           bi.push_back((uint32_t)(b << 16 | ri));
           bfl.insert(bfl.end(), fw, fw + 16);
@@ -1352,57 +1395,14 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
     }
     if ((rc = upload(c, &c->bi, bi))) return rc;
     if ((rc = upload(c, &c->bfl, bfl))) return rc;
-    if (getenv("PGXC_DEBUG")) {  // sizes of the screened basis work
-      long live = 0, nv = 0, ng = 0;
-      for (long g = 0; g < ngr; ++g)
-        for (int w = 0; w < nw8; ++w) {
-          live += __builtin_popcount(sig[(size_t)g * nw8 + w]);
-          nv += __builtin_popcount(need[(size_t)g * 2 * nw8 + w]);
-          ng += __builtin_popcount(need[(size_t)g * 2 * nw8 + nw8 + w]);
-        }
-      fprintf(stderr, "pgxc: %ld groups x %d runs; blocks live %ld, values read %ld, gradients read %ld; "
-                      "basis items %zu (of %ld)\n",
-              ngr, n8, live, nv, ng, bi.size(), (long)c->nchunks * (c->Mc / kThreads) * c->n_ranges);
-      // elements (function x point): basis values and gradients written,
-      // W written (runs live or read by the potential) and of those the
-      // ones in the tile's list
-      double ev = 0, eg = 0, ew = 0, ewl = 0;
-      for (size_t i = 0; i < bi.size(); ++i) {
-        const RangeD &R = c->h_ranges[bi[i] & 0xffffu];
-        const uint32_t *fw = bfl.data() + 16 * i;
-        for (int j = 0; j < R.n_shells; ++j) {
-          const ShellD &d = sh[(size_t)(R.shell_begin + j)];
-          const int nf = (2 * d.l + 1) * (d.n_unc + d.n_contr);
-          for (int gg = 0; gg < 8; ++gg) {
-            const int bit = 8 * j + gg;
-            ev += ((fw[bit >> 5] >> (bit & 31)) & 1u) * nf * 32.0;
-            eg += ((fw[8 + (bit >> 5)] >> (bit & 31)) & 1u) * nf * 32.0;
-          }
-        }
-      }
-      for (long g = 0; g < ngr; ++g)
-        for (int r = 0; r < n8; ++r)
-          if (((sig[(size_t)g * nw8 + r / 32] | wneed[(size_t)g * nw8 + r / 32]) >> (r % 32)) & 1u) {
-            ew += kRun * 32.0;
-            for (int f = r * kRun; f < std::min(c->NP, (r + 1) * kRun); ++f)
-              ewl += ((tfb[(size_t)(g / 4) * c->nwf + f / 32] >> (f % 32)) & 1u) * 32.0;
-          }
-      // values if only the tiles' runs were read (no potential chunks)
-      double evt = 0;
-      for (long g = 0; g < ngr; ++g) {
-        const long t = g / 4;
-        std::vector<uint32_t> tw2((size_t)nw8, 0u);
-        for (int i = c->h_tl_off[(size_t)t]; i < c->h_tl_off[(size_t)t + 1]; ++i)
-          tw2[c->h_tl[(size_t)i] >> 5] |= 1u << (c->h_tl[(size_t)i] & 31);
-        for (const ShellD &d : sh) {
-          const int nf = (2 * d.l + 1) * (d.n_unc + d.n_contr);
-          uint32_t v = 0;
-          for (int r = d.func_off / kRun; r <= (d.func_off + nf - 1) / kRun; ++r) v |= tw2[r >> 5] >> (r & 31);
-          evt += (v & 1u) * nf * 32.0;
-        }
-      }
-      fprintf(stderr, "pgxc: elements per build: basis values %.4g (tile runs only %.4g), gradients %.4g; "
-                      "W %.4g, of them in the tiles' lists %.4g\n", ev, evt, eg, ew, ewl);
+    if (getenv("PGXC_DEBUG")) {  // sizes of the screened work
+      double ev = 0, hu = 0;
+      for (size_t t = 0; t + 1 < c->h_tf_off.size(); ++t) ev += (double)kScreenTile * (c->h_tf_off[t + 1] - c->h_tf_off[t]);
+      for (long S = 0; S < NS; ++S) hu += c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S];
+      fprintf(stderr, "pgxc: basis items %zu (of %ld), elements per build %.4g; %ld splits of %ld points, "
+                      "%.1f functions each; partials of a chunk %.4g bytes\n",
+              bi.size(), (long)c->nchunks * (c->Mc / kThreads) * c->n_ranges, ev, NS, c->Mc / c->nsp,
+              hu / NS, 8.0 * c->hstride);
     }
   }
   // work items per chunk
@@ -1420,8 +1420,8 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
         c->h_di.push_back((uint32_t)(t << 8 | pr));
     }
     c->h_di_off.push_back((long)c->h_di.size());
-    for (int sl = 0; sl < c->nsplit; ++sl) {
-      const long S = (long)k * c->nsplit + sl;
+    for (int sl = 0; sl < c->nsp; ++sl) {
+      const long S = (long)k * c->nsp + sl;
       const int nu = c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S], nch = (nu + c->tf - 1) / c->tf;
       for (int ci = 0; ci < nch; ++ci)
         for (int cj = 0; cj < nch; ++cj)
@@ -1437,8 +1437,6 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
   if ((rc = upload(c, &c->su_off, c->h_su_off))) return rc;
   if ((rc = upload(c, &c->su, c->h_su))) return rc;
   if ((rc = upload(c, &c->sumask, c->h_sumask))) return rc;
-  if ((rc = upload(c, &c->gcf_off, c->h_gcf_off))) return rc;
-  if ((rc = upload(c, &c->gcf, c->h_gcf))) return rc;
   if ((rc = upload(c, &c->di, c->h_di))) return rc;
   if ((rc = upload(c, &c->pi, c->h_pi))) return rc;
   return PGXC_OK;
@@ -1695,7 +1693,17 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   const size_t L = (size_t)c->nlanes_cap;
   if ((rc = dalloc(c, &c->part, L * c->ntiles * 4 * c->Mc))) return rc;
   if ((rc = dalloc(c, &c->coef, L * 4 * c->Mc))) return rc;
-  if ((rc = dalloc(c, &c->Hpart, L * c->nsplit * np2))) return rc;
+  // a slot for every chunk where they fit kPartialBytes, else as many per lane
+  // as do (summed whenever they are full); sums in enough segments of the splits
+  // that a small matrix still fills the device
+  const long slot_b = 8 * c->hstride;
+  const long want = round_up(c->nchunks, (long)L);
+  c->hflush = want * slot_b > kPartialBytes;
+  c->hslots = (int)(c->hflush ? std::max<long>(1, kPartialBytes / slot_b / (long)L) * (long)L : want);
+  const long nb32 = c->NP / 32, pairs = nb32 * (nb32 + 1) / 2;
+  const long ns = (long)c->nchunks * c->nsp;
+  c->nseg = (int)std::min<long>({std::max<long>(kFoldItems / pairs, (ns + 63) / 64), (ns + 3) / 4, 32L});
+  if ((rc = alloc_partials(c, &c->Hc, &c->HS))) return rc;
   HIPCHK(c, hipMemset(c->part, 0, L * c->ntiles * 4 * c->Mc * 8));
   HIPCHK(c, hipMemset(c->coef, 0, L * 4 * c->Mc * 8));
   return PGXC_OK;
@@ -1734,7 +1742,7 @@ static int alloc_beta(pgxc_ctx *c) {
   HIPCHK(c, hipMalloc(&B.D, np2 * 8));
   if ((rc = dalloc(c, &B.state, (size_t)S_NSLOT * c->npad)) || (rc = dalloc(c, &B.Vstate, npk)) ||
       (rc = dalloc(c, &B.Vout, npk)) || (rc = dalloc(c, &B.part, L * c->ntiles * 4 * c->Mc)) ||
-      (rc = dalloc(c, &B.coef, L * 4 * c->Mc)) || (rc = dalloc(c, &B.Hpart, L * c->nsplit * np2)))
+      (rc = dalloc(c, &B.coef, L * 4 * c->Mc)) || (rc = alloc_partials(c, &B.Hc, &B.HS)))
     return rc;
   HIPCHK(c, hipMemset(B.P, 0, np2 * 8));
   HIPCHK(c, hipMemset(B.Pref, 0, np2 * 8));
@@ -2226,11 +2234,11 @@ int pgxc_destroy(pgxc_ctx *c) {
     g_cache_bytes[c->device] -= c->phic_bytes[0] + c->phic_bytes[1];
   }
   void *bufs[] = {c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->exps, c->norms, c->contr, c->P, c->Pref,
-                  c->D, c->phi, c->W, c->part, c->coef, c->Hpart, c->state,
+                  c->D, c->phi, c->W, c->part, c->coef, c->Hc, c->HS, c->state,
                   c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos,
-                  c->phic[0], c->phic[1], c->wbits, c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,
-                  c->gcf_off, c->gcf, c->di, c->pi, c->bi, c->bfl, c->ghess, c->gXY, c->gpart, c->beta.P, c->beta.Pref, c->beta.D,
-                  c->beta.W, c->beta.part, c->beta.coef, c->beta.Hpart, c->beta.state,
+                  c->phic[0], c->phic[1], c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,
+                  c->ho, c->pos, c->rbits, c->di, c->pi, c->bi, c->bfl, c->ghess, c->gXY, c->gpart, c->beta.P, c->beta.Pref, c->beta.D,
+                  c->beta.W, c->beta.part, c->beta.coef, c->beta.Hc, c->beta.HS, c->beta.state,
                   c->beta.Vstate, c->beta.Vout, c->eterm};
   for (void *b : bufs) dfree(b);
   for (auto &e : c->ev)

@@ -72,7 +72,8 @@ struct UnitD {
   double *coef2, *state2;
   void *W2;         // and the beta spin's W, written by the same W pass
   double *eterm;    // [Mc/256][5] block sums of the energy terms and the charge
-  double *Hpart;    // [nsplit][NP][NP] potential partials of the molecule
+  double *Hc;       // potential partials of the unit's splits, split s at ho[s]:
+  const long *ho;   // its functions x its functions (padded to blocks of 16)
   // Work of the contractions, over gathered runs of 8 functions and gathered
   // functions (all of them when screening is off).  ditems / pitems: the
   // unit's density items (tile << 8 | pair of column chunks) and potential
@@ -83,13 +84,6 @@ struct UnitD {
   // tile), the density's output columns in chunks of tile functions.
   // su_off / su: per point split of the unit, the union of its tiles'
   // functions, the potential's rows and columns in chunks of tile functions.
-  // gcf_off / gcf: per split, [group][chunk] flags, whether the chunk can be
-  // nonzero on the group (a run holding one of its functions is live there).
-  // sig8: per 32-point group (from the unit's first), nw8 words of run
-  // flags, the runs not cut off on the group.  wbits: the same shape, the
-  // runs the potential contraction reads on the group (the FP64/FP32 W pass
-  // writes W there, 0 where cut off; the split-BF16 W is written for the
-  // tile's functions, the only ones its potential reads).
   const uint32_t *ditems, *pitems;
   const int *tl_off, *su_off, *tf_off;
   const uint16_t *tl, *su, *tfl;
@@ -99,12 +93,10 @@ struct UnitD {
   // basis stage does not write
   const uint8_t *tlm;
   // per entry of su: bit t set when its function is in the list of the
-  // split's tile t, so 0 there (every bit when a split has more than 32 tiles)
+  // split's tile t (a split has at most 32), else W and Phi are not written
+  // there and count as 0
   const uint32_t *sumask;
   int nwf, pad_f;
-  const long *gcf_off;
-  const uint8_t *gcf;
-  const uint32_t *sig8, *wbits;
   // Basis stage over the blocks the other stages read (bscreen = 1; 0: every
   // block).  bitems: basis items (256-point block << 16 | atom range) that
   // write some block, with bflags: 16 words per item, bit 8 j + g of words
@@ -116,20 +108,38 @@ struct UnitD {
   long Mc, npad;
   int n_atoms, n_ranges, NP, ntiles, nsplit, incremental, pad_n;
   uint32_t mask;
-  int CH, nw8;
+  int CH, pad_c;
   long ndi, npi;  // density / potential items of the unit
 };
 
 // Per-molecule descriptors of the operand preparation and the final packing.
 struct PackD {
-  double *Hpart;  // split partials; the fold leaves the symmetric sum in split 0
+  const double *HS;  // [nseg][NP][NP] symmetric sums of partials (lower 32 x 32 tiles)
   double *Vout, *Vstate;
   const double *P;
   double *Pref;
   void *D;
   const int *fpos;  // internal position of each basis function (caller order)
   long n, NP;
-  int nsplit, incremental;
+  int nseg, incremental;
+};
+
+// Sums of a molecule's potential partials (k_fold): chunks chunk0, chunk0 +
+// step, ... (nchunks of them), of their mask bytes the share seg of nseg, into
+// out[NP][NP] (added to it when acc is set).  Chunk k's partials lie in slot
+// (k % lanes) * slots + (k / lanes) % slots of Hc.  pos[split][NP]: a
+// function's place in the split's list (0xffff: absent); rbits[row block of 32
+// functions][nbytes]: a bit per split, whether it has any of the block's
+// functions (bytes_c bytes per chunk).
+struct FoldD {
+  const double *Hc;
+  const long *ho;
+  const int *su_off;
+  const uint16_t *pos;
+  const uint8_t *rbits;
+  double *out;
+  long stride, NP;
+  int nsplit, bytes_c, nbytes, lanes, slots, chunk0, step, nchunks, seg, nseg, acc, pad;
 };
 
 // One launch's items: prefix offsets base[0..nu] over units, optional order.
@@ -175,7 +185,7 @@ template <typename T>
 void launch_potential(hipStream_t s, int tf, int var, const StageList &L);
 void launch_density_bf16x3(hipStream_t s, bool grad, int tf, const StageList &L);
 void launch_potential_bf16x3(hipStream_t s, int tf, const StageList &L);
-void launch_fold(hipStream_t s, const PackD *mols, int nm, const long *base, long total);
+void launch_fold(hipStream_t s, const FoldD *folds, int n, const long *base, long total);
 void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total);
 void launch_zero_ints(hipStream_t s, int *p, long n);
 unsigned contraction_grid(const StageList &L, int per_cu);
@@ -191,8 +201,11 @@ void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, lon
 inline long items_basis(long Mc, int n_ranges) { return (Mc / kThreads) * n_ranges; }
 inline long items_functional(long Mc) { return Mc / kThreads; }
 inline long items_wmat(long Mc, int NP) { return (Mc / (4 * kThreads)) * (NP / 16); }
-// point splits of the potential contraction are whole multiples of this
+// chunks are whole multiples of this many points; point splits of the
+// potential contraction have kSplitPts or fewer (setup_screen picks), so at
+// most 32 tiles
 constexpr int kSplitPts = 2048;
+constexpr int kMinSplitPts = 256;
 
 // ---- screening ------------------------------------------------------------
 // A radial factor is exactly zero where alpha r^2 >= 50 (the cut-off of
@@ -207,7 +220,6 @@ constexpr int kRun = 8;
 constexpr int kScreenTile = 128;       // point tile of the density contraction
 constexpr int kMaxRuns = 1024;         // runs of 8 functions per molecule (NP <= 8192)
 constexpr int kMaxShells = 8192;       // shells per molecule
-constexpr int kMaxSplitGroups = 2048;  // point groups per potential split
 constexpr double kCutoff = 50.0 * (1.0 + 1.0e-6);  // margin: a superset in every precision
 struct ScreenShell {
   double amin;                 // smallest exponent of the shell

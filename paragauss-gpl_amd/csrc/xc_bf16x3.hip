@@ -432,8 +432,8 @@ template <int BT>
 __global__ __launch_bounds__(kThreads) void k_potential_bf16x3(const StageList S) {
   __shared__ __attribute__((aligned(16))) __bf16 lds[2 * XStage<BT, BT>::n];
   __shared__ uint16_t ul[2 * BT];  // the functions of the row chunk, then of the column chunk
-  __shared__ uint16_t gl[kMaxSplitGroups];
-  __shared__ int wtot[4];
+  __shared__ int rb[32], cb[32], nt;
+  __shared__ uint8_t tl[32];
   __shared__ long slot;
   static_assert(kXBK == kGroup, "one K step per 32-point group");
   for (long L = walk_next(S, -1, &slot); L < S.total;) {
@@ -445,14 +445,13 @@ __global__ __launch_bounds__(kThreads) void k_potential_bf16x3(const StageList S
     const int sl = (int)(e >> 20), ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);
     const long Mc = U.Mc;
     const int so = U.su_off[sl], nu = U.su_off[sl + 1] - so;
-    const int nch = (nu + BT - 1) / BT, G = (int)(Mc / U.nsplit) / kGroup;
-    const long kb = (long)sl * G * kGroup;
+    const long kb = (long)sl * (Mc / U.nsplit);
     const int nri = min(BT, nu - ci * BT), nrj = min(BT, nu - cj * BT);
     __syncthreads();  // the previous item's readers of ul / gl are done
     for (int i = threadIdx.x; i < 2 * BT; i += kThreads)
       if (i < BT ? i < nri : i - BT < nrj) ul[i] = gld(U.su + so + (i < BT ? ci * BT + i : cj * BT + i - BT));
-    __syncthreads();
-    const int ng = potential_groups(U.gcf + U.gcf_off[sl], G, nch, ci, cj, gl, wtot);
+    const uint32_t *tmi = U.sumask + so + ci * BT, *tmj = U.sumask + so + cj * BT;
+    const int ng = 4 * potential_tiles<BT>(tmi, nri, tmj, nrj, rb, cb, tl, &nt);
     const uint16_t *ri = ul, *rj = ul + BT;
     const __bf16 *wh = (const __bf16 *)U.W;
     const long pn = (long)U.NP * Mc;
@@ -462,17 +461,24 @@ __global__ __launch_bounds__(kThreads) void k_potential_bf16x3(const StageList S
     PFOperand<BT> opb;
     // rows and columns skip the tiles whose list lacks their function (W and
     // Phi are 0 there)
-    const uint32_t *tmi = U.sumask + so + ci * BT, *tmj = U.sumask + so + cj * BT;
     opa.init({wh, wh + pn}, [&](int m) -> long { return m < nri ? (long)ri[m] * Mc : -1; },
              [&](int m) -> unsigned { return m < nri ? gld(tmi + m) : 0u; }, kb);
     opb.init((const float *)U.phi, [&](int n) -> long { return n < nrj ? (long)rj[n] * Mc : -1; },
              [&](int n) -> unsigned { return n < nrj ? gld(tmj + n) : 0u; }, kb);
-    auto kofs = [&](int kt, int c) -> long { return kb + (long)gl[kt] * kGroup + 8 * c; };
+    auto kofs = [&](int kt, int c) -> long { return kb + 32 * (4 * (int)tl[kt >> 2] + (kt & 3)) + 8 * c; };
     f4 acc[BT / 32][BT / 32];
     gemm_tile_bf16x3<BT, BT, kThreads, 2>(opa, opb, ng, kofs, lds, acc);
     const int ahead = walk_ahead(S);
-    potential_epilogue<float, f4, BT, BT>(acc, U.Hpart + (long)sl * U.NP * U.NP, U.NP, ri, nri, rj,
-                                          nrj);
+    {
+      const int ld = split_ld(nu), wave = threadIdx.x >> 6;
+      const int r0 = (wave >> 1) * (BT / 2), c0 = (wave & 1) * (BT / 2);
+      double *H = U.Hc + U.ho[sl] + (long)(ci * BT + r0) * ld + cj * BT + c0;
+#pragma unroll
+      for (int i = 0; i < BT / 32; ++i)
+#pragma unroll
+        for (int j = 0; j < BT / 32; ++j)
+          if (r0 + 16 * i < nri && c0 + 16 * j < nrj) put_block<float>(acc[i][j], H + (long)16 * i * ld + 16 * j, ld);
+    }
     item_log(S, it, t0);
     L = walk_take(S, L, ahead, &slot);
   }

@@ -4,6 +4,7 @@
 //   k_density    X = Phi D per 128-point tile, fused rho = sum Phi X,
 //                grad rho = 2 sum dPhi X
 //                (ParaGauss modules/density_calc_module.f90:1478-1577)
+//   k_potential  H = W^T Phi per point split (modules/xc_hamiltonian.f90:1528-1531)
 //
 // A 16x16x4 FP64 MFMA holds its SIMD's matrix core for 64 cycles (FP32: 32), so
 // the time is the number of MFMAs: K and the output columns are the tile's own
@@ -271,6 +272,193 @@ void launch_density(hipStream_t s, bool grad, int tf, int var, const StageList &
     case 1: density_var<T, 1>(s, grad, tf, L); break;
     case 2: density_var<T, 2>(s, grad, tf, L); break;
     default: density_var<T, 0>(s, grad, tf, L); break;
+  }
+}
+
+// H(m, n) += sum_p W[f(m)][p] Phi[f(n)][p] over the tiles of one split where
+// both chunks have a function: 256 threads, waves 2 x 2, wave (wm, wn) holding
+// the 16 x 16 blocks (2 i + wm, 2 j + wn), so that the rows and columns past the
+// last function, and the blocks without a function on a tile, are shared
+// evenly.  On a tile only the blocks that have one on both sides are multiplied
+// (a uniform branch over the MFMAs of 16 points).  Both operands are kept
+// [row][k] with rows padded by 16 bytes; a lane reads 16 bytes, E consecutive k,
+// for E MFMAs (MFMA e of a chunk takes k = 4 E c + E g + e in lane group g).
+// Functions not in a tile's list are staged as zeros (their values are not
+// written).
+template <typename T, int BT, int VAR>
+struct PotTile {
+  static constexpr int BK = Var<VAR>::BK, ST = Var<VAR>::ST, E = 16 / (int)sizeof(T);
+  static constexpr int BKP = BK + E, SO = BT * BKP, kLds = 2 * ST * SO, TT = BT / 32;
+  // vectors a row is loaded in: 16 bytes where they share out evenly
+  static constexpr int VE = BT * (BK / E) % kThreads == 0 ? E : E / 2;
+  static constexpr int NV = BK / VE, PER = BT * NV / kThreads, RS = kThreads / NV;
+  static constexpr int SPT = kScreenTile / BK;  // K steps per tile
+  static_assert(PER * kThreads == BT * NV && PER * RS == BT, "whole vectors per thread");
+  typedef T vec __attribute__((ext_vector_type(VE)));
+  typedef T rd __attribute__((ext_vector_type(E)));
+  typedef typename MF<T>::acc acc_t;
+
+  __device__ static __forceinline__ void run(const T *__restrict__ W, const T *__restrict__ phi,
+                                             long Mc, const uint16_t *__restrict__ fr,
+                                             const uint32_t *__restrict__ mr, int nr,
+                                             const uint16_t *__restrict__ fc,
+                                             const uint32_t *__restrict__ mc, int nc,
+                                             const int *rb, const int *cb, const uint8_t *tl,
+                                             int ntl, T *lds, acc_t (&acc)[TT][TT]) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1, kv = tid % NV, r0 = tid / NV;
+    const T *pa[PER], *pb[PER];
+    unsigned ma[PER], mb[PER];
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+      const int r = r0 + RS * e;
+      pa[e] = W + (long)gld(fr + min(r, nr - 1)) * Mc + VE * kv;
+      pb[e] = phi + (long)gld(fc + min(r, nc - 1)) * Mc + VE * kv;
+      ma[e] = r < nr ? gld(mr + r) : 0u;
+      mb[e] = r < nc ? gld(mc + r) : 0u;
+    }
+#pragma unroll
+    for (int i = 0; i < TT; ++i)
+#pragma unroll
+      for (int j = 0; j < TT; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    vec ra[PER], rb_[PER];
+    unsigned ok = 0;  // bits 2 e, 2 e + 1: vector e of W, of Phi is live
+    const int ksteps = ntl * SPT;
+    if (!ksteps) return;
+    auto load = [&](int kt) {
+      const int t = tl[min(kt / SPT, ntl - 1)];
+      const long k = kScreenTile * t + (kt % SPT) * BK;
+      ok = 0;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const bool ga = (ma[e] >> t) & 1u, gb = (mb[e] >> t) & 1u;
+        ra[e] = gld((const vec *)(ga ? pa[e] + k : W));
+        rb_[e] = gld((const vec *)(gb ? pb[e] + k : W));
+        ok |= (unsigned)ga << (2 * e) | (unsigned)gb << (2 * e + 1);
+      }
+    };
+    auto store = [&](int buf) {
+      T *as = lds + 2 * buf * SO, *bs = as + SO;
+#pragma unroll
+      for (int e = 0; e < PER; ++e) {
+        const int o = (r0 + RS * e) * BKP + VE * kv;
+        *(vec *)(as + o) = (ok >> (2 * e)) & 1u ? ra[e] : vec{};
+        *(vec *)(bs + o) = (ok >> (2 * e + 1)) & 1u ? rb_[e] : vec{};
+      }
+    };
+    auto compute = [&](int buf, int kt) {
+      const int t = __builtin_amdgcn_readfirstlane((int)tl[kt / SPT]);
+      const int la = __builtin_amdgcn_readfirstlane(rb[t]) >> wm, lb = __builtin_amdgcn_readfirstlane(cb[t]) >> wn;
+      const T *as = lds + 2 * buf * SO + (16 * wm + (lane & 15)) * BKP + E * (lane >> 4);
+      const T *bs = lds + 2 * buf * SO + SO + (16 * wn + (lane & 15)) * BKP + E * (lane >> 4);
+      constexpr int CH = 1;  // reads per branch
+#pragma unroll
+      for (int c0 = 0; c0 < BK / (4 * E); c0 += CH) {
+        rd a[TT][CH], b[TT][CH];
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+          for (int c = 0; c < CH; ++c) {
+            a[i][c] = *(const rd *)(as + 32 * i * BKP + 4 * E * (c0 + c));
+            b[i][c] = *(const rd *)(bs + 32 * i * BKP + 4 * E * (c0 + c));
+          }
+#pragma unroll
+        for (int i = 0; i < TT; ++i)
+#pragma unroll
+          for (int j = 0; j < TT; ++j)
+            if ((la >> (2 * i)) & (lb >> (2 * j)) & 1) {
+#pragma unroll
+              for (int c = 0; c < CH; ++c)
+#pragma unroll
+                for (int e = 0; e < E; ++e) acc[i][j] = MF<T>::mma(a[i][c][e], b[j][c][e], acc[i][j]);
+            }
+      }
+    };
+    load(0);
+    if constexpr (ST == 2) {
+      store(0);
+      __syncthreads();
+      for (int kt = 0; kt < ksteps; ++kt) {
+        load(kt + 1);  // past the end: the last tile again, not used
+        compute(kt & 1, kt);
+        store((kt & 1) ^ 1);
+        __syncthreads();
+      }
+    } else {
+      for (int kt = 0; kt < ksteps; ++kt) {
+        store(0);
+        __syncthreads();
+        load(kt + 1);
+        compute(0, kt);
+        __syncthreads();
+      }
+    }
+  }
+};
+
+// item = (point split, pair of chunks of its functions); writes its blocks of
+// the split's partial (zeros where no tile has both).  Bound by the matrix
+// cores: the blocks multiplied are 1.25 times sum n^2 at (H2O)32 (whole chunks
+// on the groups where both had a function: 1.83).  FP64 stage of an (H2O)32
+// build, one lane: 10.1 -> 6.1 ms; 23-atom molecule (233 000 points) 852 -> 150
+// us, its 57 splits of 4096 points now 456 of 512.  Variants 0 and 1 keep
+// their LDS stages under 80 KB: two workgroups share a CU and hide each other's
+// waits.
+template <typename T, int BT, int VAR>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_potential(const StageList S) {
+  typedef PotTile<T, BT, VAR> G;
+  __shared__ __attribute__((aligned(16))) T lds[G::kLds];
+  __shared__ int rb[32], cb[32], nt;
+  __shared__ uint8_t tl[32];
+  __shared__ long slot;
+  for (long L = walk_next(S, -1, &slot); L < S.total;) {
+    const uint64_t t0 = S.tlog ? wall_clock64() : 0;
+    const long it = walk_item(S, L);
+    const int u = unit_of(S.base, S.nu, it);
+    const UnitD &U = S.units[u];
+    const uint32_t e = U.pitems[it - S.base[u]];
+    const int sl = (int)(e >> 20), ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);
+    const long Mc = U.Mc, kb = (long)sl * (Mc / U.nsplit);
+    const int so = U.su_off[sl], nu = U.su_off[sl + 1] - so;
+    const int nr = min(BT, nu - ci * BT), nc = min(BT, nu - cj * BT);
+    const uint32_t *mr = U.sumask + so + ci * BT, *mc = U.sumask + so + cj * BT;
+    const int n = potential_tiles<BT>(mr, nr, mc, nc, rb, cb, tl, &nt);
+    typename MF<T>::acc acc[G::TT][G::TT];
+    G::run((const T *)U.W + kb, (const T *)U.phi + kb, Mc, U.su + so + ci * BT, mr, nr,
+           U.su + so + cj * BT, mc, nc, rb, cb, tl, n, lds, acc);
+    const int ahead = walk_ahead(S);
+    const int ld = split_ld(nu), wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
+    double *H = U.Hc + U.ho[sl] + (long)ci * BT * ld + cj * BT;
+#pragma unroll
+    for (int i = 0; i < G::TT; ++i)
+#pragma unroll
+      for (int j = 0; j < G::TT; ++j) {
+        const int r = 16 * (2 * i + wm), c = 16 * (2 * j + wn);
+        if (r < nr && c < nc) put_block<T>(acc[i][j], H + (long)r * ld + c, ld);
+      }
+    item_log(S, it, t0);
+    L = walk_take(S, L, ahead, &slot);
+  }
+}
+
+template <typename T, int VAR>
+static void potential_var(hipStream_t s, int tf, const StageList &L) {
+  dim3 g(contraction_grid(L, 2));
+  switch (tf) {
+    case 64: hipLaunchKernelGGL((k_potential<T, 64, VAR>), g, dim3(kThreads), 0, s, L); break;
+    case 96: hipLaunchKernelGGL((k_potential<T, 96, VAR>), g, dim3(kThreads), 0, s, L); break;
+    default: hipLaunchKernelGGL((k_potential<T, 128, VAR>), g, dim3(kThreads), 0, s, L); break;
+  }
+}
+
+template <typename T>
+void launch_potential(hipStream_t s, int tf, int var, const StageList &L) {
+  if (!L.total) return;
+  switch (var) {
+    case 1: potential_var<T, 1>(s, tf, L); break;
+    case 2: potential_var<T, 2>(s, tf, L); break;
+    default: potential_var<T, 0>(s, tf, L); break;
   }
 }
 

@@ -3,4 +3,5 @@
 
 namespace pgxc {
 template void launch_density<float>(hipStream_t, bool, int, int, const StageList &);
+template void launch_potential<float>(hipStream_t, int, int, const StageList &);
 }  // namespace pgxc

@@ -134,24 +134,6 @@ template <> struct Var<1> { static constexpr int BK = 32, ST = 1; };
 template <> struct Var<2> { static constexpr int BK = 32, ST = 2; };
 
 // ---------------------------------------------------------------- screening
-// Order-preserving compaction over the workgroup: threads with act append
-// value to list (after `base` entries); returns the new length.  Every thread
-// of the workgroup calls it.
-__device__ __forceinline__ int block_compact(bool act, int value, uint16_t *list, int base,
-                                             int *wtot) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const unsigned long long m = __ballot(act);
-  const int before = __popcll(m & ((1ull << lane) - 1ull));
-  if (lane == 0) wtot[wave] = __popcll(m);
-  __syncthreads();
-  int off = base;
-  for (int w = 0; w < wave; ++w) off += wtot[w];
-  if (act) list[off + before] = (uint16_t)value;
-  const int total = base + wtot[0] + wtot[1] + wtot[2] + wtot[3];
-  __syncthreads();
-  return total;
-}
-
 // Copy n list entries into LDS (every thread calls it; ends with a barrier).
 __device__ __forceinline__ void lds_list(const uint16_t *__restrict__ src, int n, uint16_t *dst) {
   for (int i = threadIdx.x; i < n; i += (int)blockDim.x) dst[i] = gld(src + i);
@@ -168,17 +150,41 @@ __device__ __forceinline__ long run_fn(const uint16_t *runs, int n, int e) {
   return r < n ? v : -1;
 }
 
-// Potential item: the groups of its split on which both of its chunks can be
-// nonzero (flags [G][nch]), ascending, into gl.  Returns the count.
-__device__ __forceinline__ int potential_groups(const uint8_t *__restrict__ flags, int G, int nch,
-                                                int ci, int cj, uint16_t *gl, int *wtot) {
-  int cnt = 0;
-  for (int b = 0; b < G; b += kThreads) {
-    const int g = b + (int)threadIdx.x;
-    const bool act = g < G && gld(flags + (long)g * nch + ci) != 0 && gld(flags + (long)g * nch + cj) != 0;
-    cnt = block_compact(act, g, gl, cnt, wtot);
+// Potential item (row chunk x column chunk of a split's functions, both within
+// BT): per 16-function block and 128-point tile of the split (at most 32)
+// whether some function of the block is in the tile's list, as bits of rb[t]
+// (rows) and cb[t] (columns), from the functions' tile masks rm and cm (nr and
+// nc of them); and the tiles where both have one, ascending, in tl.  Returns
+// their number; every thread of the workgroup calls it (rb, cb, tl, n in LDS).
+template <int BT, int NT = kThreads>
+__device__ __forceinline__ int potential_tiles(const uint32_t *__restrict__ rm, int nr,
+                                               const uint32_t *__restrict__ cm, int nc,
+                                               int (&rb)[32], int (&cb)[32], uint8_t (&tl)[32],
+                                               int *n) {
+  __syncthreads();  // the previous item's readers are done
+  if (threadIdx.x < 32) rb[threadIdx.x] = cb[threadIdx.x] = 0;
+  __syncthreads();
+  // 16 lanes a block: each turns its function's mask into its tiles' bits
+  for (int i = threadIdx.x; i < 2 * BT; i += NT) {
+    const int f = i < BT ? i : i - BT;
+    uint32_t m = i < BT ? (f < nr ? gld(rm + f) : 0u) : (f < nc ? gld(cm + f) : 0u);
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) m |= (uint32_t)__shfl_xor((int)m, o);
+    // lane q of the block takes tiles q and q + 16
+    int *d = i < BT ? rb : cb;
+    const int q = f & 15, bit = 1 << (f >> 4);
+    if ((m >> q) & 1u) atomicOr(d + q, bit);
+    if ((m >> (q + 16)) & 1u) atomicOr(d + q + 16, bit);
   }
-  return cnt;
+  __syncthreads();
+  if (threadIdx.x < 64) {
+    const int t = threadIdx.x & 31;
+    const unsigned long long live = __ballot(threadIdx.x < 32 && rb[t] != 0 && cb[t] != 0);
+    if (threadIdx.x < 32 && ((live >> t) & 1ull)) tl[__popcll(live & ((1ull << t) - 1ull))] = (uint8_t)t;
+    if (threadIdx.x == 0) *n = __popcll(live);
+  }
+  __syncthreads();
+  return *n;
 }
 
 // Sum of M per-lane values (M = 4 or 16) over the 16 lanes of each lane
@@ -306,33 +312,16 @@ __device__ __forceinline__ void density_epilogue(
   }
 }
 
-// Epilogue of H = W^T Phi for one gathered row chunk x column chunk: the
-// tile is added into the split's FP64 slot at the functions of its rows
-// (rfn[m], m < nr) and columns (cfn[n], n < nc) (slots are zeroed at the
-// start of a build).
-template <typename T, typename ACC, int BM, int BN>
-__device__ __forceinline__ void potential_epilogue(const ACC (&acc)[BM / 32][BN / 32], double *H,
-                                                   int NP, const uint16_t *rfn, int nr,
-                                                   const uint16_t *cfn, int nc) {
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
+// Functions of a split, padded to whole 16-function blocks: the leading
+// dimension of its potential partial.
+__device__ __forceinline__ int split_ld(int n) { return (n + 15) & ~15; }
+
+// One 16 x 16 block of H = W^T Phi into the split's partial.
+template <typename T>
+__device__ __forceinline__ void put_block(const typename MF<T>::acc &acc, double *H, int ld) {
+  const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int n = wn * WN + j * 16 + mf_col(lane);
-    if (n >= nc) continue;
-    const long col = cfn[n];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int m = wm * WM + i * 16 + MF<T>::row(lane, r);
-        if (m >= nr) continue;
-        const long row = rfn[m];
-        const long q = row * NP + col;
-        gst(H + q, gld(H + q) + (double)acc[i][j][r]);
-      }
-  }
+  for (int r = 0; r < 4; ++r) gst(H + (long)MF<T>::row(lane, r) * ld + mf_col(lane), (double)acc[r]);
 }
 
 }  // namespace pgxc

@@ -7,7 +7,6 @@
 //   k_functional  Slater + PW92 + PBE-x + PBE-c in FP64, closed-form derivatives
 //                 (modules/xc_func.f90:187-305 and the term modules)
 //   k_wmat        W = a Phi + b . grad Phi  (modules/xc_hamiltonian.f90:1429-1483)
-//   k_potential   H = W^T Phi on MFMA, split over points  (:1528-1531)
 //   k_pack        V = H + H^T into the packed lower triangle (:1561-1567)
 #include <type_traits>
 
@@ -1227,12 +1226,9 @@ __global__ __launch_bounds__(kThreads) void k_point_f(long Mc, long npad, uint32
 
 // -------------------------------------------------------------------- W
 // item = (1024-point block, 16-function group), 4 consecutive points of one
-// 32-point group per thread: W = a Phi + b . grad Phi.  SPLIT (split-BF16
-// builds, T = float): W stored as bf16 hi / lo planes.  A run of 8 functions
-// cut off on the group is 0 without reading Phi, and is not written at all
-// where the potential contraction never reads it; inside a live run, a
-// function outside the tile's function list (its shell cut off on the whole
-// tile) is 0 without reading Phi either.
+// 32-point group per thread: W = a Phi + b . grad Phi for the functions of the
+// point's tile (the potential contraction reads no others).  SPLIT (split-BF16
+// builds, T = float): W stored as bf16 hi / lo planes.
 template <typename T, bool GRAD, bool SPLIT, bool TWO>
 __global__ __launch_bounds__(kThreads) void k_wmat(const UnitD *__restrict__ units, int nu,
                                                    const long *__restrict__ base,
@@ -1272,29 +1268,12 @@ __global__ __launch_bounds__(kThreads) void k_wmat(const UnitD *__restrict__ uni
         gst((t4 *)((T *)Wout[sp] + q), w);
       }
     };
-    const uint32_t *sg = U.sig8 + (p / kGroup) * U.nw8, *wn = U.wbits + (p / kGroup) * U.nw8;
     const uint32_t *fb = U.tfb + (p / kScreenTile) * U.nwf;
-    // split-BF16 W is read only by the split-BF16 potential, which skips the
-    // functions outside a tile's list (when a split spans at most 32 tiles):
-    // no zeros are written for them
-    const bool skip = SPLIT && Mc / U.nsplit <= 32 * kScreenTile;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {  // the item's two runs of 8 functions
-      const long r = f0 / kRun + h, fr = r * kRun;
-      const uint32_t bit = 1u << (r & 31);
+      const long fr = f0 + h * kRun;
       const uint32_t fm = gld(fb + (fr >> 5)) >> (fr & 31);  // the run's functions in the tile's list
-      const uint32_t wm = skip ? fm : 0xffu;                 // the run's functions written
-      if (!(gld(sg + (r >> 5)) & bit)) {
-        if (gld(wn + (r >> 5)) & bit) {
-          const double z[4] = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-          for (int k = 0; k < kRun; ++k)
-            if ((wm >> k) & 1u)
-#pragma unroll
-              for (int sp = 0; sp < NS; ++sp) put(sp, (fr + k) * Mc + p, z);
-        }
-        continue;
-      }
+      if (!(fm & 0xffu)) continue;
       double a[NS][4], b0[NS][4] = {}, b1[NS][4] = {}, b2[NS][4] = {};
 #pragma unroll
       for (int sp = 0; sp < NS; ++sp)
@@ -1309,16 +1288,14 @@ __global__ __launch_bounds__(kThreads) void k_wmat(const UnitD *__restrict__ uni
         }
 #pragma unroll 4
       for (int k = 0; k < kRun; ++k) {
-        if (!((wm >> k) & 1u)) continue;
+        if (!((fm >> k) & 1u)) continue;
         const long q = (fr + k) * Mc + p;
-        t4 v0 = {}, v1 = {}, v2 = {}, v3 = {};
-        if ((fm >> k) & 1u) {
-          v0 = gld((const t4 *)(phi + q));
-          if (GRAD) {
-            v1 = gld((const t4 *)(phi + cs + q));
-            v2 = gld((const t4 *)(phi + 2 * cs + q));
-            v3 = gld((const t4 *)(phi + 3 * cs + q));
-          }
+        const t4 v0 = gld((const t4 *)(phi + q));
+        t4 v1 = {}, v2 = {}, v3 = {};
+        if (GRAD) {
+          v1 = gld((const t4 *)(phi + cs + q));
+          v2 = gld((const t4 *)(phi + 2 * cs + q));
+          v3 = gld((const t4 *)(phi + 3 * cs + q));
         }
 #pragma unroll
         for (int sp = 0; sp < NS; ++sp) {
@@ -1335,101 +1312,95 @@ __global__ __launch_bounds__(kThreads) void k_wmat(const UnitD *__restrict__ uni
   }
 }
 
-// --------------------------------------------------------------- potential
-// item = (point split, function tile pair) of H[split] (+)= W^T Phi
-// Variants 0 and 1 keep one LDS stage set under 64 KB: built for two waves
-// per SIMD, two workgroups share a CU and hide each other's waits.
-template <typename T, int BT, int VAR>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_potential(const StageList S) {
-  constexpr int BK = Var<VAR>::BK, ST = Var<VAR>::ST, TT = BT / 32;
-  constexpr int R = kGroup / BK;  // K steps per 32-point group
-  __shared__ __attribute__((aligned(16))) T As[lds_elems<T, BT, BK, ST, true>()];
-  __shared__ __attribute__((aligned(16))) T Bs[lds_elems<T, BT, BK, ST, true>()];
-  __shared__ uint16_t ul[2 * BT];  // the functions of the row chunk, then of the column chunk
-  __shared__ uint32_t cm[BT];      // per column: the split's tiles whose list holds its function
-  __shared__ uint16_t gl[kMaxSplitGroups];
-  __shared__ int wtot[4];
-  __shared__ long slot;
-  for (long L = walk_next(S, -1, &slot); L < S.total;) {
-    const uint64_t t0 = S.tlog ? wall_clock64() : 0;
-    const long it = walk_item(S, L);
-    const int u = find_unit(S.base, S.nu, it);
-    const UnitD &U = S.units[u];
-    const uint32_t e = U.pitems[it - S.base[u]];
-    const int sl = (int)(e >> 20), ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);
-    const long Mc = U.Mc;
-    const int so = U.su_off[sl], nu = U.su_off[sl + 1] - so;
-    const int nch = (nu + BT - 1) / BT, G = (int)(Mc / U.nsplit) / kGroup;
-    const long kb = (long)sl * G * kGroup;  // first point of the split
-    const int nri = min(BT, nu - ci * BT), nrj = min(BT, nu - cj * BT);
-    __syncthreads();  // the previous item's readers of ul / gl are done
-    for (int i = threadIdx.x; i < 2 * BT; i += kThreads)
-      if (i < BT ? i < nri : i - BT < nrj) ul[i] = gld(U.su + so + (i < BT ? ci * BT + i : cj * BT + i - BT));
-    for (int i = threadIdx.x; i < nrj; i += kThreads) cm[i] = gld(U.sumask + so + cj * BT + i);
-    __syncthreads();
-    const int ng = potential_groups(U.gcf + U.gcf_off[sl], G, nch, ci, cj, gl, wtot);
-    const uint16_t *ri = ul, *rj = ul + BT;
-    // A(m, k) = W[f_i(m)][kb + p(k)], B(k, n) = Phi[f_j(n)][kb + p(k)]: rows from
-    // the split's functions, K over the groups where both chunks can be
-    // nonzero; B is 0 on the tiles whose list lacks the column's function
-    // (left unwritten by the basis stage)
-    auto kpt = [&](int kt, int kk) -> long { return (long)gl[kt / R] * kGroup + (kt % R) * BK + kk; };
-    auto aaddr = [&](int m, int kt, int kk) -> long {
-      return m < nri ? (long)ri[min(m, nri - 1)] * Mc + kb + kpt(kt, kk) : -1;
-    };
-    auto baddr = [&](int n, int kt, int kk) -> long {
-      const long k = kpt(kt, kk);
-      return (n < nrj && ((cm[min(n, nrj - 1)] >> ((int)(k >> 7) & 31)) & 1u))
-                 ? (long)rj[min(n, nrj - 1)] * Mc + kb + k : -1;
-    };
-    const T *W = (const T *)U.W, *phi = (const T *)U.phi;
-    typename MF<T>::acc acc[TT][TT];
-    gemm_tile<T, BT, BT, BK, ST, true, true>(W, phi, ng * R, aaddr, baddr, As, Bs, acc);
-    const int ahead = walk_ahead(S);
-    potential_epilogue<T, typename MF<T>::acc, BT, BT>(acc, U.Hpart + (long)sl * U.NP * U.NP,
-                                                       U.NP, ri, nri, rj, nrj);
-    item_log(S, it, t0);
-    L = walk_take(S, L, ahead, &slot);
-  }
-}
-
 // -------------------------------------------------------------------- pack
-// Fold, item = 32 x 32 tile (rb >= cb) of one molecule's internal matrix:
-// S(r, c) = sum_split H(r, c) + sum_split H(c, r) for both the tile and its
-// mirror, read along rows; the mirror's sums change places through LDS.  S
-// replaces split 0's partial on the tile (only this item reads that tile and
-// its mirror, and it writes after every read).
-__global__ __launch_bounds__(kThreads) void k_fold(const PackD *__restrict__ mols, int nm,
+// Fold, item = 32 x 32 tile (rb >= cb): S(r, c) = sum over the listed splits of
+// H(r, c) + H(c, r), each split's H gathered from its partial through the
+// functions' places in it (0 where a split lacks one).  Of every kFoldSplits
+// splits those with functions of both blocks of 32 (their mask bits) are
+// listed in LDS with the places of the two blocks' functions, so the loop over
+// them has only the elements' loads, four splits' at a time, to wait for.  The
+// mirror tile's sums change places through LDS.  Bound by the latency of those
+// loads; a tile all splits hold sets the time, hence the segments of at most
+// 64 splits: (H2O)32, 960 splits, 500 MB, fold and packing 0.30 ms (0.65 with
+// two segments).
+constexpr int kFoldSplits = 64;
+__global__ __launch_bounds__(kThreads) void k_fold(const FoldD *__restrict__ folds, int n,
                                                    const long *__restrict__ base, long total) {
+  typedef uint16_t u8v __attribute__((ext_vector_type(8)));
   __shared__ double t[32][33];
-  const int tid = threadIdx.x;
+  __shared__ __attribute__((aligned(16))) uint16_t pos[kFoldSplits][2][32];
+  __shared__ const double *hp[kFoldSplits];
+  __shared__ int ls[kFoldSplits], ld[kFoldSplits], cnt;
+  const int tid = threadIdx.x, c = tid & 31, r0 = tid >> 5;
   for (long L = blockIdx.x; L < total; L += gridDim.x) {
-    const int m = find_unit(base, nm, L);
-    const PackD &M = mols[m];
+    const int m = find_unit(base, n, L);
+    const FoldD &F = folds[m];
     long e = L - base[m], rb = (long)((sqrt(8.0 * (double)e + 1.0) - 1.0) * 0.5);
     while (rb * (rb + 1) / 2 > e) --rb;
     while ((rb + 1) * (rb + 2) / 2 <= e) ++rb;
-    const long cb = e - rb * (rb + 1) / 2, NP = M.NP, np2 = NP * NP;
+    const long cb = e - rb * (rb + 1) / 2, NP = F.NP;
     double sa[4] = {}, sb[4] = {};
-    for (int s = 0; s < M.nsplit; ++s) {
-      const double *H = M.Hpart + (long)s * np2;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int x = tid + kThreads * i, r = x >> 5, c = x & 31;
-        sa[i] += H[(rb * 32 + r) * NP + cb * 32 + c];
-        sb[i] += H[(cb * 32 + r) * NP + rb * 32 + c];
+    const uint8_t *br = F.rbits + rb * F.nbytes, *bc = F.rbits + cb * F.nbytes;
+    const long ns = (long)F.nchunks * F.nsplit, s1 = ns * (F.seg + 1) / F.nseg;
+    for (long s0 = ns * F.seg / F.nseg; s0 < s1; s0 += kFoldSplits) {
+      if (tid < kFoldSplits) {  // one wave
+        const long s = s0 + tid;
+        const int k = F.chunk0 + (int)(s / F.nsplit) * F.step, sl = (int)(s % F.nsplit);
+        const long at = (long)k * F.bytes_c + sl / 8;
+        const bool live = s < s1 && ((gld(br + at) & gld(bc + at)) >> (sl & 7) & 1);
+        const unsigned long long lv = __ballot(live);
+        const int q = __popcll(lv & ((1ull << tid) - 1ull));
+        if (live) {
+          const long S = (long)k * F.nsplit + sl;
+          ls[q] = (int)S;
+          ld[q] = split_ld(F.su_off[S + 1] - F.su_off[S]);
+          hp[q] = F.Hc + (long)((k % F.lanes) * F.slots + (k / F.lanes) % F.slots) * F.stride + F.ho[S];
+        }
+        if (tid == 0) cnt = __popcll(lv);
       }
+      __syncthreads();
+      const int nl = cnt;
+      for (int i = tid; i < nl * 8; i += kThreads) {  // 16 bytes: 8 places
+        const int q = i >> 3, h = (i >> 2) & 1, v = i & 3;
+        *(u8v *)&pos[q][h][8 * v] = gld((const u8v *)(F.pos + ls[q] * NP + (h ? cb : rb) * 32 + 8 * v));
+      }
+      __syncthreads();
+      for (int q0 = 0; q0 < nl; q0 += 4) {
+        double va[4][4], vb[4][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int q = min(q0 + u, nl - 1);
+          const double *H = hp[q];
+          const int pc = q0 + u < nl ? pos[q][1][c] : 0xffff, qc = q0 + u < nl ? pos[q][0][c] : 0xffff;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int pr = pos[q][0][r0 + 8 * i], qr = pos[q][1][r0 + 8 * i];
+            const bool ga = pr != 0xffff && pc != 0xffff, gb = qr != 0xffff && qc != 0xffff;
+            const double x = gld(H + (ga ? (long)pr * ld[q] + pc : 0));
+            const double y = gld(H + (gb ? (long)qr * ld[q] + qc : 0));
+            va[u][i] = ga ? x : 0.0;
+            vb[u][i] = gb ? y : 0.0;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            sa[i] += va[u][i];
+            sb[i] += vb[u][i];
+          }
+      }
+      __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int x = tid + kThreads * i;
-      t[x >> 5][x & 31] = sb[i];
-    }
+    for (int i = 0; i < 4; ++i) t[r0 + 8 * i][c] = sb[i];
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int x = tid + kThreads * i, r = x >> 5, c = x & 31;
-      M.Hpart[(rb * 32 + r) * NP + cb * 32 + c] = sa[i] + t[c][r];
+      const int r = r0 + 8 * i;
+      double *o = F.out + (rb * 32 + r) * NP + cb * 32 + c;
+      const double v = sa[i] + t[c][r];
+      *o = F.acc ? *o + v : v;
     }
     __syncthreads();
   }
@@ -1437,7 +1408,7 @@ __global__ __launch_bounds__(kThreads) void k_fold(const PackD *__restrict__ mol
 
 // item = 256 packed elements of one molecule (caller's function order):
 // V = base + S at the functions' internal rows (S folded above, symmetric,
-// read from its lower tiles); then the molecule's state for the next
+// read from its lower tiles, summed over its segments); then the molecule's state for the next
 // incremental build: V_state = V.
 __global__ __launch_bounds__(kThreads) void k_pack(const PackD *__restrict__ mols, int nm,
                                                    const long *__restrict__ base, long total) {
@@ -1453,7 +1424,8 @@ __global__ __launch_bounds__(kThreads) void k_pack(const PackD *__restrict__ mol
     const long k = idx - j * (j + 1) / 2;
     const long pj = M.fpos[j], pk = M.fpos[k];  // internal rows of caller functions j, k
     const long r = pj > pk ? pj : pk, c = pj > pk ? pk : pj;
-    const double v = M.Hpart[r * NP + c];
+    double v = 0.0;
+    for (int s = 0; s < M.nseg; ++s) v += M.HS[((long)s * NP + r) * NP + c];
     const double out = M.incremental ? M.Vstate[idx] + v : v;
     M.Vout[idx] = out;
     M.Vstate[idx] = out;
@@ -1700,26 +1672,6 @@ void launch_wmat(hipStream_t s, bool grad, bool split, bool two, const StageList
 #undef PGXC_WMAT
 }
 
-template <typename T, int VAR>
-static void potential_var(hipStream_t s, int tf, const StageList &L) {
-  dim3 g(contraction_grid(L, 2));
-  switch (tf) {
-    case 64: hipLaunchKernelGGL((k_potential<T, 64, VAR>), g, dim3(kThreads), 0, s, L); break;
-    case 96: hipLaunchKernelGGL((k_potential<T, 96, VAR>), g, dim3(kThreads), 0, s, L); break;
-    default: hipLaunchKernelGGL((k_potential<T, 128, VAR>), g, dim3(kThreads), 0, s, L); break;
-  }
-}
-
-template <typename T>
-void launch_potential(hipStream_t s, int tf, int var, const StageList &L) {
-  if (!L.total) return;
-  switch (var) {
-    case 1: potential_var<T, 1>(s, tf, L); break;
-    case 2: potential_var<T, 2>(s, tf, L); break;
-    default: potential_var<T, 0>(s, tf, L); break;
-  }
-}
-
 __global__ __launch_bounds__(kThreads) void k_zero_ints(int *p, long n) {
   for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)gridDim.x * kThreads)
     p[i] = 0;
@@ -1731,9 +1683,9 @@ void launch_zero_ints(hipStream_t s, int *p, long n) {
                      dim3(kThreads), 0, s, p, n);
 }
 
-void launch_fold(hipStream_t s, const PackD *mols, int nm, const long *base, long total) {
+void launch_fold(hipStream_t s, const FoldD *folds, int n, const long *base, long total) {
   if (!total) return;
-  hipLaunchKernelGGL(k_fold, dim3(persistent_grid(total, 8)), dim3(kThreads), 0, s, mols, nm, base, total);
+  hipLaunchKernelGGL(k_fold, dim3(persistent_grid(total, 8)), dim3(kThreads), 0, s, folds, n, base, total);
 }
 
 void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total) {
@@ -1750,8 +1702,7 @@ void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, lon
 
 #define PGXC_INST(T)                                                                  \
   template void launch_basis<T>(hipStream_t, bool, const StageList &);               \
-  template void launch_wmat<T>(hipStream_t, bool, bool, bool, const StageList &);    \
-  template void launch_potential<T>(hipStream_t, int, int, const StageList &);
+  template void launch_wmat<T>(hipStream_t, bool, bool, bool, const StageList &);
 PGXC_INST(double)
 PGXC_INST(float)
 #undef PGXC_INST
