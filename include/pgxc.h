@@ -203,11 +203,11 @@ int pgxc_energy(pgxc_ctx *ctx, uint32_t functional, int32_t precision, double *t
  * computed).  grad (n_atoms x 3, row-major by atom, caller atom order)
  * receives dE_xc/dR (written, not added; the reference stores the negative).
  * Evaluated at the density matrix and potential coefficients of the last
- * build on the context, in FP64 whatever that build's precision: basis
- * values and Hessians per chunk, X = Phi P and (d/dc Phi) P on the screened
- * tiles.  The first call allocates the work space of one chunk (Hessian
- * planes and products, 80 bytes per function and point of a chunk) and the
- * context keeps it.
+ * build on the context, in FP64 whatever that build's precision: the basis
+ * and its second derivatives per point, and two products with P on the
+ * screened tiles.  The first call allocates the work space of one chunk (the
+ * products, 16 bytes per function and point of a chunk, and the sums' parts)
+ * and the context keeps it.
  */
 int pgxc_gradient(pgxc_ctx *ctx, double *grad);
 
@@ -220,7 +220,8 @@ int pgxc_gradient(pgxc_ctx *ctx, double *grad);
  * owner[npts] (caller point order): the atom whose atomic grid holds the
  * point; the grid's weights must be the Becke partition of those atomic
  * grids.  grad (n_atoms x 3) receives dE_xc/dR, at the last build's density
- * and coefficients, FP64.
+ * and coefficients, FP64.  The first call allocates 36 bytes per point and at
+ * most 256 MiB of scratch, which the context keeps.
  */
 int pgxc_gradient_grid(pgxc_ctx *ctx, const int32_t *owner, double *grad);
 

@@ -134,6 +134,7 @@ struct pgxc_ctx {
   std::vector<hipEvent_t> ev;
   Plan *plan = nullptr;
   Plan *plan_e = nullptr;  // energy-only builds (pgxc_energy)
+  Plan *plan_g = nullptr;  // the nuclear gradient's stages
   double *eterm = nullptr;  // [nblk_total][5] energy-term block sums
   double last_terms[5] = {0, 0, 0, 0, 0};
   double exps_per_point = 0;
@@ -165,10 +166,12 @@ struct pgxc_ctx {
   long *ho = nullptr;
   uint16_t *pos = nullptr;
   uint8_t *rbits = nullptr;
-  // nuclear gradient work space (first gradient on): Hessian planes and
-  // products of one chunk, per-(tile, function) sums
-  double *ghess = nullptr, *gXY = nullptr, *gpart = nullptr;
-  long gpart_n = 0;
+  // nuclear gradient work space (first gradient on): products of one chunk
+  // (XZ, two planes) and per-(basis item, atom, wave) sums; with the grid moving
+  // (first such gradient on) gpm, the points' terms, and gmov, the rest
+  double *gXZ = nullptr, *gpart = nullptr, *gsum = nullptr, *gpm = nullptr;
+  char *gmov = nullptr;
+  int *perm_d = nullptr;  // caller index of each internal point
   uint32_t *di = nullptr, *pi = nullptr;
   // blocks of the basis values some stage reads (see setup_screen): per
   // chunk the basis items (256-point block << 16 | atom range) that touch
@@ -176,8 +179,6 @@ struct pgxc_ctx {
   uint32_t *bi = nullptr, *bfl = nullptr;
   std::vector<long> h_bi_off;
   std::vector<int> fpos;          // internal position of each caller function
-  std::vector<int> fatom;         // atom of each internal function position
-  std::vector<long> perm;         // caller index of each internal point
   std::vector<double> axyz;       // atom positions (bohr), caller order
   int *d_fpos = nullptr;
   Sched sched;
@@ -303,7 +304,7 @@ enum ItemKind { K_BASIS, K_FUNC, K_WMAT, K_DENS, K_POT, K_WBASIS };
 long unit_items(const UnitD &U, ItemKind k, int tf) {
   switch (k) {
     case K_BASIS:
-    case K_WBASIS: return U.bscreen ? U.nbi : items_basis(U.Mc, U.n_ranges);
+    case K_WBASIS: return U.nbi;
     case K_FUNC: return items_functional(U.Mc);
     case K_WMAT: return items_wmat(U.Mc, U.NP);
     case K_DENS: return U.ndi;
@@ -370,7 +371,7 @@ static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int p
 static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int precision,
                     const std::vector<int> &incr, const std::vector<double> &unit_prio,
                     long order_version, const Sched &sc, Plan *&plan, pgxc_ctx *errc,
-                    int energy = 0, int dense_basis = 0) {
+                    int energy = 0) {
   const int smode = sc.model ? sc.mode : std::min(sc.mode, (int)PGXC_SCHED_ANALYTIC);
   std::vector<int> lanes, spins;
   for (auto *c : mols) {
@@ -527,9 +528,8 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.su_off = c->su_off + (long)k * c->nsp;
       U.su = c->su;
       U.sumask = c->sumask;
-      U.bscreen = dense_basis ? 0 : 1;  // the basis stage writes the blocks read later
       U.bitems = c->bi + c->h_bi_off[k];
-      U.bflags = c->bfl + 16 * c->h_bi_off[k];
+      U.bflags = c->bfl + 8 * c->h_bi_off[k];
       U.nbi = c->h_bi_off[k + 1] - c->h_bi_off[k];
       if (c->ispin == 2) {  // the beta spin's unit: same points and basis values
         UnitD B = U;
@@ -568,7 +568,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       std::vector<UnitD> bu;
       std::vector<int> bm;
       for (size_t i = 0; i < units.size(); ++i)
-        if (uspin[i] == 0 && (dense_basis || !mols[umol[i]]->skip_basis)) {
+        if (uspin[i] == 0 && !mols[umol[i]]->skip_basis) {
           bu.push_back(units[i]);
           bm.push_back(umol[i]);
         }
@@ -998,7 +998,6 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
       c->phic_failed[e] = 0;
       c->phic_bytes[e] = need;
       held += need;
-      HIPCHK(c, hipMemsetAsync(c->phic[e], 0, need, s));  // padding rows read as zero
       HIPCHK(c, poison_basis(c, c->phic[e], elem, need_phi, c->nchunks, s));
       c->phic_valid[e] = 0;
       c->phic_grad[e] = 0;
@@ -1017,11 +1016,9 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
       c->phi_bytes = need_phi * c->nlanes_cap;
       c->phi_elem = 0;
     }
-    // function rows nbas..NP-1 are never written and must read as zero in the
-    // element type of this build (a buffer last used at another precision
-    // holds that precision's bytes there)
+    // (no stage reads what this build's basis stage does not write: neither the
+    // rows past nbas nor what a build of another precision left)
     if (c->phi_elem != elem) {
-      HIPCHK(c, hipMemsetAsync(c->phi, 0, c->phi_bytes, s));
       c->phi_elem = elem;
       HIPCHK(c, poison_basis(c, c->phi, elem, need_phi, c->nlanes_cap, s));
     }
@@ -1037,6 +1034,7 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
   if (moved) {  // their unit descriptors hold the old pointers
     free_plan(c->plan);
     free_plan(c->plan_e);
+    free_plan(c->plan_g);
   }
   return PGXC_OK;
 }
@@ -1376,19 +1374,17 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
       for (long b = 0; b < c->Mc / kThreads; ++b) {
         const uint32_t *m0 = smark.data() + (size_t)((g0 + b * gpb) / 4) * nws, *m1 = m0 + nws;
         for (int ri = 0; ri < nr; ++ri) {
-          // per (shell j of the range, group g of the block): values (words
-          // 0-7) and gradients (8-15) read
-          uint32_t fw[16] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+          // per (shell j of the range, group g of the block): read
+          uint32_t fw[8] = {0, 0, 0, 0, 0, 0, 0, 0};
           const RangeD &R = c->h_ranges[(size_t)ri];
           for (int j = 0; j < R.n_shells; ++j) {
             const int sg = R.shell_begin + j;
             const uint32_t a = (m0[sg / 32] >> (sg % 32)) & 1u, z = (m1[sg / 32] >> (sg % 32)) & 1u;
             fw[j / 4] |= (0xfu * a | 0xf0u * z) << (8 * (j % 4));
           }
-          for (int w = 0; w < 8; ++w) fw[8 + w] = fw[w];
           if (!(fw[0] | fw[1] | fw[2] | fw[3] | fw[4] | fw[5] | fw[6] | fw[7])) continue;
           bi.push_back((uint32_t)(b << 16 | ri));
-          bfl.insert(bfl.end(), fw, fw + 16);
+          bfl.insert(bfl.end(), fw, fw + 8);
         }
       }
       c->h_bi_off.push_back((long)bi.size());
@@ -1561,9 +1557,6 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   c->nbas = (int)foff;
   c->exps_per_point = (double)eoff;
   function_order(sh, exps, atom_xyz, n_atoms, c->fpos);
-  c->fatom.assign(c->nbas, 0);
-  for (const ShellD &d : sh)
-    for (int j = 0; j < (2 * d.l + 1) * (d.n_unc + d.n_contr); ++j) c->fatom[d.func_off + j] = d.atom;
   // function tile: requested, or the one of 128 / 96 / 64 that pads nbas least
   if (opt && opt->tile) {
     c->tf = opt->tile;
@@ -1645,7 +1638,10 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   // grid in space-filling-curve order, padded with far points of zero weight
   std::vector<long> perm;
   morton_order(grid, npts, npts, 1, perm);
-  c->perm = perm;
+  {
+    std::vector<int> p32(perm.begin(), perm.end());
+    if ((rc = upload(c, &c->perm_d, p32))) return rc;
+  }
   c->axyz.assign(atom_xyz, atom_xyz + 3 * (size_t)n_atoms);
   std::vector<double> g(4 * (size_t)c->npad);
   for (int k = 0; k < 4; ++k)
@@ -1765,6 +1761,7 @@ static int set_spins(pgxc_ctx *c, int ispin) {
   c->have_density = 0;
   free_plan(c->plan);
   free_plan(c->plan_e);
+  free_plan(c->plan_g);
   return PGXC_OK;
 }
 
@@ -1930,98 +1927,75 @@ int pgxc_energy(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ter
   return PGXC_OK;
 }
 
-// The basis-centre term into grad; with pm (device [3][npad], zeroed) also
-// w grad f at every point, summed over spins.
-static int gradient_impl(pgxc_ctx *c, double *grad, double *pm) {
-  if (!c || !grad) return PGXC_ERR_ARG;
-  if (!c->have_state) return fail(c, PGXC_ERR_STATE, "pgxc_gradient before a build on this context");
+// The basis-centre term into c->gsum ([atom][3] on the device, zeroed first);
+// with pm (device [3][npad], zeroed) also w grad f at every point, summed over
+// spins.
+static int gradient_impl(pgxc_ctx *c, double *pm) {
   const uint32_t functional = c->state_functional;
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
   hipStream_t s = c->stream;
   int rc;
   if ((rc = ensure_work(c, 8, PGXC_PREC_FP64, s, true))) return rc;
-  // an FP64 plan for its basis stage: chunk k's values land where its unit
-  // points (the FP64 cache, or the lane's work buffer when there is none)
-  Plan *gp = nullptr;
+  // an FP64 plan for its basis and W stages: chunk k's values land where its
+  // unit points (the FP64 cache, or the lane's work buffer when there is none)
   std::vector<pgxc_ctx *> mols{c};
   std::vector<int> full{0};
-  // every block of the values: the products below read all functions on all points
-  if ((rc = get_plan(mols, functional, PGXC_PREC_FP64, full, {}, -1, c->sched, gp, c, 0, 1)))
+  Sched plain;
+  plain.mode = PGXC_SCHED_STATIC;
+  if ((rc = get_plan(mols, functional, PGXC_PREC_FP64, full, {}, -1, plain, c->plan_g, c))) return rc;
+  const Plan &gp = *c->plan_g;
+  const long Mc = c->Mc, NP = c->NP, cs = NP * Mc, np = c->npad;
+  // the chunk's products and sums stay with the context for later gradients
+  long ni = 1;  // the most basis items of one chunk
+  for (int k = 0; k < c->nchunks; ++k) ni = std::max<long>(ni, c->h_bi_off[k + 1] - c->h_bi_off[k]);
+  if ((rc = dalloc(c, &c->gXZ, 2 * (size_t)cs)) || (rc = dalloc(c, &c->gpart, 12 * (size_t)kRangeAtoms * ni)) ||
+      (rc = dalloc(c, &c->gsum, 3 * (size_t)c->n_atoms)))
     return rc;
-  const long Mc = c->Mc, NP = c->NP, cs = NP * Mc, tpc = Mc / kScreenTile;
-  auto done = [&](int code) {
-    free_plan(gp);
-    return code;
-  };
-  // the chunk's Hessian planes, products and per-(tile, function) sums stay
-  // with the context for later gradients
-  long nlist = 1;  // the most list entries of one chunk
-  for (int k = 0; k < c->nchunks; ++k)
-    nlist = std::max<long>(nlist, c->h_tf_off[(size_t)(k + 1) * tpc] - c->h_tf_off[(size_t)k * tpc]);
-  if (!c->ghess && hipMalloc((void **)&c->ghess, 6 * (size_t)cs * 8) != hipSuccess) c->ghess = nullptr;
-  if (!c->gXY && hipMalloc((void **)&c->gXY, 4 * (size_t)cs * 8) != hipSuccess) c->gXY = nullptr;
-  if (c->gpart_n < 3 * nlist) {
-    dfree(c->gpart);
-    c->gpart_n = 0;
-    if (hipMalloc((void **)&c->gpart, 3 * (size_t)nlist * 8) == hipSuccess) c->gpart_n = 3 * nlist;
-    else c->gpart = nullptr;
-  }
-  if (!c->ghess || !c->gXY || !c->gpart) {
-    (void)hipGetLastError();
-    return done(fail(c, PGXC_ERR_NOMEM, "pgxc_gradient: no device memory for the chunk's Hessian and products"));
-  }
-  double *hess = c->ghess, *XY = c->gXY, *part = c->gpart;
-  std::vector<double> gfn(3 * (size_t)NP, 0.0), hp(3 * (size_t)nlist);
+  HIPCHK(c, hipMemsetAsync(c->gsum, 0, 24 * (size_t)c->n_atoms, s));
   for (int k = 0; k < c->nchunks; ++k) {
     const long p0 = (long)k * Mc;
-    const int lane = k % c->nlanes;
-    const double *phi = (const double *)((const char *)c->phi_base +
-                                         (c->phi_stride ? (size_t)k * c->phi_stride : (size_t)lane * c->phi_lane));
-    launch_basis<double>(s, true, gp->steps[k].basis);
-    launch_basis_hess(s, c->grid + p0, c->grid + c->npad + p0, c->grid + 2 * c->npad + p0, c->atoms,
-                      c->n_atoms, c->shells, c->exps, c->norms, c->contr, (int)NP, Mc, hess);
-    const long l0 = c->h_tf_off[(size_t)k * tpc], nl = c->h_tf_off[(size_t)(k + 1) * tpc] - l0;
+    const StepPlan &S = gp.steps[k];
+    const int lane = c->nchunks > 1 ? k % gp.nlanes : 0;
+    launch_basis<double>(s, true, S.basis);
+    if (gga) {
+      // W = 2 a Phi + b . grad Phi of every spin, at the coefficients of the build
+      for (int sp = 0; sp < c->ispin; ++sp)
+        launch_bracket_coef(s, Mc, (sp ? c->beta.state : c->state) + p0, np,
+                            (sp ? c->beta.coef : c->coef) + (size_t)lane * 4 * Mc);
+      launch_wmat<double>(s, true, false, false, S.wmat);
+      launch_wmat<double>(s, true, false, true, S.wmat2);
+    }
+    const UnitD *unit = c->ispin == 2 ? S.func2.units : S.func.units;
     for (int sp = 0; sp < c->ispin; ++sp) {
-      // X = Phi P, Y_c = (d/dc Phi) P with P of the last build (P_ref),
-      // over the density items of the chunk, for each tile's functions
-      const double *P = sp ? c->beta.Pref : c->Pref;
+      // X = Phi P, Z = W P with P of the last build (P_ref)
       for (int li = 0; li < kLists; ++li)
-        launch_xy(s, kTiles[li / kNumVariants], li % kNumVariants, gp->steps[k].dens[li], P, XY,
-                  gga ? 4 : 1, c->ispin, sp);
-      const double *st = (sp ? c->beta.state : c->state) + p0;
-      const long np = c->npad;
-      launch_grad_fn(s, gga, tpc, c->tf_off + p0 / kScreenTile, c->tfl, (int)NP, Mc, XY, phi, hess,
-                     st + S_A * np, st + S_BX * np, st + S_BY * np, st + S_BZ * np, part);
-      if (pm)
-        launch_grad_pt(s, gga, c->tf_off + p0 / kScreenTile, c->tfl, (int)NP, Mc, XY, phi, hess,
-                       st + S_A * np, st + S_BX * np, st + S_BY * np, st + S_BZ * np, pm + p0, np);
-      if (nl > 0 && (hipMemcpyAsync(hp.data(), part, (size_t)nl * 3 * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-                     hipStreamSynchronize(s) != hipSuccess))
-        return done(fail(c, PGXC_ERR_HIP, "pgxc_gradient: kernel or copy failed"));
-      for (long e = 0; e < nl; ++e)  // tiles in order, each tile's functions in order
-        for (int d = 0; d < 3; ++d) gfn[3 * (size_t)c->h_tfl[(size_t)(l0 + e)] + d] += hp[(size_t)e * 3 + d];
+        launch_xz(s, kTiles[li / kNumVariants], li % kNumVariants, S.dens[li], sp ? c->beta.Pref : c->Pref,
+                  c->gXZ, gga ? 2 : 1, c->ispin, sp);
+      launch_bracket(s, gga, c->lmax, unit, Mc, c->n_ranges, c->gXZ,
+                     (sp ? c->beta.state : c->state) + p0, np, pm ? pm + p0 : nullptr, c->gpart, c->gsum);
     }
   }
-  if (hipGetLastError() != hipSuccess) return done(fail(c, PGXC_ERR_HIP, "pgxc_gradient: launch failed"));
+  if (hipGetLastError() != hipSuccess) return fail(c, PGXC_ERR_HIP, "pgxc_gradient: launch failed");
   mark_basis_cached(c, 8, PGXC_PREC_FP64, true);
-  for (int a = 0; a < 3 * c->n_atoms; ++a) grad[a] = 0.0;
-  for (int i = 0; i < c->nbas; ++i)
-    for (int d = 0; d < 3; ++d) grad[3 * c->fatom[i] + d] += -2.0 * gfn[3 * (size_t)i + d];
-  return done(PGXC_OK);
+  return PGXC_OK;
 }
 
-int pgxc_gradient(pgxc_ctx *c, double *grad) { return gradient_impl(c, grad, nullptr); }
+int pgxc_gradient(pgxc_ctx *c, double *grad) {
+  if (!c || !grad) return PGXC_ERR_ARG;
+  if (!c->have_state) return fail(c, PGXC_ERR_STATE, "pgxc_gradient before a build on this context");
+  int rc = gradient_impl(c, nullptr);
+  if (rc) return rc;
+  HIPCHK(c, hipMemcpyAsync(grad, c->gsum, 24 * (size_t)c->n_atoms, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  return PGXC_OK;
+}
 
 int pgxc_gradient_grid(pgxc_ctx *c, const int32_t *owner, double *grad) {
   if (!c || !owner || !grad) return PGXC_ERR_ARG;
-  const long npts = (long)c->perm.size(), np = c->npad, Mc = c->Mc;
+  const long npts = c->npts, np = c->npad;
   const int na = c->n_atoms;
-  std::vector<int> own((size_t)np, -1);
-  for (long p = 0; p < npts; ++p) {
-    const int a = owner[c->perm[p]];
-    if (a < 0 || a >= na) return fail(c, PGXC_ERR_ARG, "pgxc_gradient_grid: owner out of range");
-    own[p] = a;
-  }
+  for (long p = 0; p < npts; ++p)
+    if (owner[p] < 0 || owner[p] >= na) return fail(c, PGXC_ERR_ARG, "pgxc_gradient_grid: owner out of range");
   std::vector<double> inv((size_t)na * na, 0.0);
   for (int i = 0; i < na; ++i)
     for (int k = 0; k < na; ++k)
@@ -2032,59 +2006,36 @@ int pgxc_gradient_grid(pgxc_ctx *c, const int32_t *owner, double *grad) {
         if (!(d > 0.0)) return fail(c, PGXC_ERR_ARG, "pgxc_gradient_grid: two atoms at one position");
         inv[(size_t)i * na + k] = 1.0 / d;
       }
-  double *pm = nullptr, *d_inv = nullptr, *fp = nullptr, *q = nullptr, *rm = nullptr, *part = nullptr;
-  int *d_own = nullptr;
-  const long nblk = Mc / kThreads;
-  auto done = [&](int code) {
-    dfree(pm);
-    dfree(d_inv);
-    dfree(fp);
-    dfree(q);
-    dfree(rm);
-    dfree(part);
-    dfree(d_own);
-    return code;
-  };
-  if (hipMalloc((void **)&pm, 3 * (size_t)np * 8) != hipSuccess ||
-      hipMalloc((void **)&d_inv, inv.size() * 8) != hipSuccess ||
-      hipMalloc((void **)&fp, (size_t)Mc * 8) != hipSuccess ||
-      hipMalloc((void **)&q, (size_t)na * Mc * 8) != hipSuccess ||
-      hipMalloc((void **)&rm, 3 * (size_t)Mc * 8) != hipSuccess ||
-      hipMalloc((void **)&part, (size_t)nblk * na * 3 * 8) != hipSuccess ||
-      hipMalloc((void **)&d_own, (size_t)np * 4) != hipSuccess)
-    return done(fail(c, PGXC_ERR_NOMEM, "pgxc_gradient_grid: no device memory"));
+  if (!c->have_state) return fail(c, PGXC_ERR_STATE, "pgxc_gradient before a build on this context");
+  // work space, kept with the context: caller owners, owners, f per point,
+  // inverse distances, per-wave cells, sums and centre lists
+  const long waves = becke_grad_waves(na, np);
+  size_t off[8] = {0}, bytes[7] = {4 * (size_t)npts, 4 * (size_t)np, 8 * (size_t)np, 8 * inv.size(),
+                                   512 * (size_t)waves * na, 24 * (size_t)waves * na, 2 * (size_t)waves * na};
+  for (int i = 0; i < 7; ++i) off[i + 1] = off[i] + (size_t)round_up((long)bytes[i], 256);
+  int rc;
+  if ((rc = dalloc(c, &c->gmov, off[7])) || (rc = dalloc(c, &c->gpm, 3 * (size_t)np))) return rc;
+  int *d_caller = (int *)(c->gmov + off[0]), *d_own = (int *)(c->gmov + off[1]);
+  double *fp = (double *)(c->gmov + off[2]), *d_inv = (double *)(c->gmov + off[3]);
+  double *scr = (double *)(c->gmov + off[4]), *part = (double *)(c->gmov + off[5]);
+  uint16_t *list = (uint16_t *)(c->gmov + off[6]);
   hipStream_t s = c->stream;
-  if (hipMemsetAsync(pm, 0, 3 * (size_t)np * 8, s) != hipSuccess ||
-      hipMemcpy(d_inv, inv.data(), inv.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
-      hipMemcpy(d_own, own.data(), own.size() * 4, hipMemcpyHostToDevice) != hipSuccess)
-    return done(fail(c, PGXC_ERR_HIP, "pgxc_gradient_grid: upload"));
+  HIPCHK(c, hipMemsetAsync(c->gpm, 0, 24 * (size_t)np, s));
+  HIPCHK(c, hipMemcpyAsync(d_inv, inv.data(), 8 * inv.size(), hipMemcpyHostToDevice, s));
+  HIPCHK(c, hipMemcpyAsync(d_caller, owner, 4 * (size_t)npts, hipMemcpyHostToDevice, s));
+  launch_gather_owner(s, npts, np, c->perm_d, d_caller, d_own);
   // basis-centre term, and w grad f per point (the points move with their atoms)
-  int rc = gradient_impl(c, grad, pm);
-  if (rc) return done(rc);
-  std::vector<double> hpm(3 * (size_t)np);
-  if (hipMemcpy(hpm.data(), pm, hpm.size() * 8, hipMemcpyDeviceToHost) != hipSuccess)
-    return done(fail(c, PGXC_ERR_HIP, "pgxc_gradient_grid: copy"));
-  for (long p = 0; p < np; ++p)
-    if (own[p] >= 0)
-      for (int d = 0; d < 3; ++d) grad[3 * own[p] + d] += hpm[(size_t)d * np + p];
+  if ((rc = gradient_impl(c, c->gpm))) return rc;
+  launch_owner_sum(s, na, np, d_own, c->gpm, waves, part, c->gsum);
   // Becke weight derivatives times f
   const uint32_t functional = c->state_functional;
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
-  std::vector<double> hp((size_t)nblk * na * 3);
-  for (int k = 0; k < c->nchunks; ++k) {
-    const long p0 = (long)k * Mc;
-    const double *st = c->state + p0, *st2 = c->ispin == 2 ? c->beta.state + p0 : st;
-    launch_point_f(s, gga, c->ispin == 2, functional, Mc, np, st, st2, fp);
-    launch_becke_grad(s, na, c->atoms, d_inv, Mc, c->grid + p0, c->grid + np + p0,
-                      c->grid + 2 * np + p0, c->grid + 3 * np + p0, fp, d_own + p0, q, rm, part);
-    if (hipMemcpyAsync(hp.data(), part, hp.size() * 8, hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-      return done(fail(c, PGXC_ERR_HIP, "pgxc_gradient_grid: weight derivatives failed"));
-    for (long b = 0; b < nblk; ++b)
-      for (int a = 0; a < na; ++a)
-        for (int d = 0; d < 3; ++d) grad[3 * a + d] += hp[((size_t)b * na + a) * 3 + d];
-  }
-  return done(PGXC_OK);
+  launch_point_f(s, gga, c->ispin == 2, functional, np, np, c->state, c->ispin == 2 ? c->beta.state : c->state, fp);
+  launch_becke_grad(s, na, c->atoms, d_inv, np, c->grid, fp, d_own, waves, scr, list, part, c->gsum);
+  if (hipGetLastError() != hipSuccess) return fail(c, PGXC_ERR_HIP, "pgxc_gradient_grid: launch failed");
+  HIPCHK(c, hipMemcpyAsync(grad, c->gsum, 24 * (size_t)na, hipMemcpyDeviceToHost, s));
+  HIPCHK(c, hipStreamSynchronize(s));
+  return PGXC_OK;
 }
 
 int pgxc_last_stats(const pgxc_ctx *c, double *s5) {
@@ -2229,6 +2180,7 @@ int pgxc_destroy(pgxc_ctx *c) {
   if (c->stream2) (void)hipStreamSynchronize(c->stream2);
   free_plan(c->plan);
   free_plan(c->plan_e);
+  free_plan(c->plan_g);
   {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     g_cache_bytes[c->device] -= c->phic_bytes[0] + c->phic_bytes[1];
@@ -2237,7 +2189,7 @@ int pgxc_destroy(pgxc_ctx *c) {
                   c->D, c->phi, c->W, c->part, c->coef, c->Hc, c->HS, c->state,
                   c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos,
                   c->phic[0], c->phic[1], c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,
-                  c->ho, c->pos, c->rbits, c->di, c->pi, c->bi, c->bfl, c->ghess, c->gXY, c->gpart, c->beta.P, c->beta.Pref, c->beta.D,
+                  c->ho, c->pos, c->rbits, c->di, c->pi, c->bi, c->bfl, c->gXZ, c->gpart, c->gsum, c->gpm, c->gmov, c->perm_d, c->beta.P, c->beta.Pref, c->beta.D,
                   c->beta.W, c->beta.part, c->beta.coef, c->beta.Hc, c->beta.HS, c->beta.state,
                   c->beta.Vstate, c->beta.Vout, c->eterm};
   for (void *b : bufs) dfree(b);

@@ -97,14 +97,12 @@ struct UnitD {
   // there and count as 0
   const uint32_t *sumask;
   int nwf, pad_f;
-  // Basis stage over the blocks the other stages read (bscreen = 1; 0: every
-  // block).  bitems: basis items (256-point block << 16 | atom range) that
-  // write some block, with bflags: 16 words per item, bit 8 j + g of words
-  // 0-7 (8-15): the values (gradients) of the range's shell j are read on
-  // group g of the block.
+  // Basis stage over the blocks the other stages read.  bitems: basis items
+  // (256-point block << 16 | atom range) that write some block, block by block,
+  // with bflags: 8 words per item, bit 8 j + g: the values and gradients of the
+  // range's shell j are read on group g of the block.
   const uint32_t *bitems, *bflags;
   long nbi;
-  int bscreen, pad_b;
   long Mc, npad;
   int n_atoms, n_ranges, NP, ntiles, nsplit, incremental, pad_n;
   uint32_t mask;
@@ -198,7 +196,6 @@ void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, lon
                  int mode, bool finish);
 
 // item counts per unit, shared by the planner and the kernels' decoding
-inline long items_basis(long Mc, int n_ranges) { return (Mc / kThreads) * n_ranges; }
 inline long items_functional(long Mc) { return Mc / kThreads; }
 inline long items_wmat(long Mc, int NP) { return (Mc / (4 * kThreads)) * (NP / 16); }
 // chunks are whole multiples of this many points; point splits of the
@@ -235,35 +232,31 @@ void launch_form_density(hipStream_t s, const double *C, const double *occ, int 
                          int nocc, int NP, double *P);
 
 
-// Nuclear gradient, basis-centre term: the basis Hessian planes [6][NP][Mc]
-// (xx, xy, xz, yy, yz, zz) of one chunk, and per 128-point tile and function
-// of its list the sums of grad phi_i (2 a X_i + b . Y_i) + X_i (b . grad)
-// grad phi_i into part[list position][3] (XY = [4][NP][Mc]: X = Phi P, Y_c)
-void launch_basis_hess(hipStream_t s, const double *gx, const double *gy, const double *gz,
-                       const AtomD *atoms, int n_atoms, const ShellD *shells, const double *exps,
-                       const double *norms, const double *contr, int NP, long Mc, double *hess);
-// the gradient's products X = Phi P, Y_c = (d/dc Phi) P over a density list's
-// items (tile x function chunks), written for the tiles' functions only
-void launch_xy(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XY,
+// Nuclear gradient.  launch_xz: X = Phi P (plane 0) and, for nplanes = 2, Z = W P
+// (plane 1) into XZ[plane][f][p] over a density list's items (tile x function
+// chunks), for the tiles' functions only; units u with u % nspin == spin.
+void launch_xz(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XZ,
                int nplanes, int nspin, int spin);
-void launch_grad_fn(hipStream_t s, bool gga, long ntiles, const int *tf_off, const uint16_t *tfl,
-                    int NP, long Mc, const double *XY, const double *phi, const double *hess,
-                    const double *a, const double *bx, const double *by, const double *bz,
-                    double *part);
-// Weight-derivative and point-motion terms (the grid moves with the atoms):
-// pm[d * pstride + p] += 2 sum_i t_d(i, p) (w grad f at each point); f per
-// point from the state (st2: the beta spin's, spin builds); the Becke weight
-// derivatives times w f into part[blk][atom][3] (q: [na][Mc], rm: [3][Mc]
-// scratch; owner -1 for padding points)
-void launch_grad_pt(hipStream_t s, bool gga, const int *tf_off, const uint16_t *tfl, int NP,
-                    long Mc, const double *XY, const double *phi, const double *hess,
-                    const double *a, const double *bx, const double *by, const double *bz,
-                    double *pm, long pstride);
+// coef = 2 a, b from the per-point state; the W pass over it forms Z's operand
+void launch_bracket_coef(hipStream_t s, long Mc, const double *st, long np, double *coef);
+// the basis-centre term of one chunk added to grad[atom][3] (caller atoms), w
+// grad f per point to pm when given; part: 96 doubles per basis item
+void launch_bracket(hipStream_t s, bool gga, int lmax, const UnitD *unit, long Mc, int n_ranges,
+                    const double *XZ, const double *st, long np, double *pm, double *part,
+                    double *grad);
+// With the grid moving: own = owner of each internal point; pm summed by owner;
+// f per point from the state (st2: the beta spin's, spin builds); the Becke
+// weight derivatives times w f (scr: 64 doubles, list: one entry per wave and
+// atom; part: 3 doubles per wave and atom)
+void launch_gather_owner(hipStream_t s, long npts, long np, const int *perm, const int *owner, int *own);
+void launch_owner_sum(hipStream_t s, int na, long np, const int *owner, const double *pm, long waves,
+                      double *part, double *grad);
 void launch_point_f(hipStream_t s, bool gga, bool spin, uint32_t mask, long Mc, long npad,
                     const double *st, const double *st2, double *fp);
-void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long Mc,
-                       const double *gx, const double *gy, const double *gz, const double *gw,
-                       const double *fp, const int *owner, double *q, double *rm, double *part);
+long becke_grad_waves(int na, long np);
+void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long np,
+                       const double *grid, const double *fp, const int *owner, long waves,
+                       double *scr, uint16_t *list, double *part, double *grad);
 
 // Becke partition weights of points owned by atoms (grid generation)
 void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv);

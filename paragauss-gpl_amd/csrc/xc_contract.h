@@ -247,6 +247,81 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const Stag
   }
 }
 
+// The nuclear gradient's products over the density's items, P for D, stored
+// instead of summed: plane 0 X = Phi P, plane 1 Z = W P, at the tile's functions.
+// Bound by the matrix cores: 0.98 ms per (H2O)16 chunk of 245 760 points (X and
+// the three products of the gradient planes on whole runs: 2.8 ms).
+template <int BN, int VAR>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_xz(const StageList S, const double *__restrict__ P,
+                                                                  double *__restrict__ XZ, int nplanes,
+                                                                  int nspin, int spin) {
+  typedef DensTile<double, BN, VAR> G;
+  __shared__ __attribute__((aligned(16))) double lds[G::kLds];
+  for (long L = blockIdx.x; L < S.total; L += gridDim.x) {
+    const long it = (long)xcd_remap((int)L, (int)S.total);
+    const int u = unit_of(S.base, S.nu, it);
+    if (u % nspin != spin) continue;  // uniform over the workgroup
+    const UnitD &U = S.units[u];
+    const uint32_t e = U.ditems[it - S.base[u]];
+    const int tile = (int)(e >> 8), pair = (int)(e & 255);
+    const long m0 = (long)tile * kDBM, Mc = U.Mc, NP = U.NP;
+    const int off = U.tf_off[tile], nf = U.tf_off[tile + 1] - off;
+    const uint16_t *fl = U.tfl + off;
+    const int cc = chunk_cols(nf, BN), nch = (nf + BN - 1) / BN;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (int ch = 2 * pair; ch < min(2 * pair + 2, nch); ++ch) {
+      const uint16_t *cf = fl + ch * cc;
+      const int ncol = min(cc, nf - ch * cc);
+      for (int pl = 0; pl < nplanes; ++pl) {
+        const double *A = (const double *)(pl ? U.W : U.phi) + m0;
+        double *out = XZ + pl * NP * Mc + m0 + 32 * wave + 4 * (lane >> 4);
+        auto go = [&](auto nb) {
+          constexpr int NB = decltype(nb)::value;
+          d4 acc[2][NB];
+          __syncthreads();  // the previous product's readers of the LDS stages are done
+          G::template run<NB>(A, Mc, P, NP, fl, nf, cf, ncol, lds, acc);
+#pragma unroll
+          for (int j = 0; j < NB; ++j) {
+            const int n = 16 * j + (lane & 15);
+            if (n >= ncol) continue;
+            double *o = out + (long)gld(cf + n) * Mc;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {  // four consecutive points
+              gst((V2<double>::type *)(o + 16 * i), V2<double>::type{acc[i][j][0], acc[i][j][1]});
+              gst((V2<double>::type *)(o + 16 * i) + 1, V2<double>::type{acc[i][j][2], acc[i][j][3]});
+            }
+          }
+        };
+        const int nb = (ncol + 15) / 16;
+        if (nb <= BN / 32) go(std::integral_constant<int, BN / 32>{});
+        else go(std::integral_constant<int, BN / 16>{});
+      }
+    }
+  }
+}
+
+template <int BN>
+static void xz_bn(hipStream_t s, int var, const StageList &L, const double *P, double *XZ, int np,
+                  int ns, int sp) {
+  dim3 g((unsigned)std::min<long>(L.total, 512));
+  switch (var) {
+    case 1: hipLaunchKernelGGL((k_xz<BN, 1>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+    case 2: hipLaunchKernelGGL((k_xz<BN, 2>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+    default: hipLaunchKernelGGL((k_xz<BN, 0>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+  }
+}
+
+inline void launch_xz_impl(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XZ,
+                           int nplanes, int nspin, int spin) {
+  if (!L.total) return;
+  switch (tf) {
+    case 64: xz_bn<64>(s, var, L, P, XZ, nplanes, nspin, spin); break;
+    case 96: xz_bn<96>(s, var, L, P, XZ, nplanes, nspin, spin); break;
+    default: xz_bn<128>(s, var, L, P, XZ, nplanes, nspin, spin); break;
+  }
+}
+
 template <typename T, int BN, int VAR>
 static void density_bn(hipStream_t s, bool grad, const StageList &L) {
   dim3 g(contraction_grid(L, 2));

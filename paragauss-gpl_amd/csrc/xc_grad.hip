@@ -1,83 +1,60 @@
-// Nuclear gradient of E_xc, the basis-centre term: ParaGauss's F1
-// (modules/post_scf_module.f90:150-185, stored in grad_xc when weight_grads
-// is off), on a fixed grid:
+// Nuclear gradient of E_xc for gfx950: ParaGauss's F1 (basis centres,
+// modules/post_scf_module.f90:150-185, grad_xc when weight_grads is off) and,
+// with the grid moving, F2 (points and Becke weights).  Per spin
 //
-//   dE/dR_A = -2 sum_p sum_{i on A} [ grad_d phi_i (2 a X_i + b . Y_i)
-//                                     + X_i (b . grad) grad_d phi_i ]
+//   dE/dR_A = -2 sum_p sum_{i on A} t_i(p),
+//   t_i     = grad phi_i (2 a X_i + b . Y_i) + X_i (b . grad) grad phi_i,
 //
-// per spin, with X = Phi P, Y_c = (d/dc Phi) P (plain DGEMMs), a = w dF/drho / 2
-// and b = w (2 dF/dg_ss grad rho_s + dF/dg_ab grad rho_s') the potential
-// coefficients of the build (the second term only for GGA).  This file holds
-// the basis Hessian and the per-function reduction over points.
-#include "pgxc_internal.h"
-#include "xc_device.h"
+// X = Phi P, Y_c = (d/dc Phi) P, a = w dF/drho / 2, b = w (2 dF/dg_ss grad rho_s
+// + dF/dg_ab grad rho_s') of the build (the second term only for GGA).  The
+// bracket's Z = 2 a X + b . Y is one product, Z = W P with W = 2 a Phi + b .
+// grad Phi per point, so a GGA gradient takes two products (X and Z) where X
+// and the three Y_c are four.  The basis functions' second derivatives are
+// formed along b where they are used, never stored.
+#include <algorithm>
+#include <type_traits>
+
+#include "xc_basis.h"
 
 namespace pgxc {
 namespace {
 
-// value, gradient and Hessian (xx, xy, xz, yy, yz, zz) of a function of r
-struct J2 {
-  double v, g[3], h[6];
+// A value and its derivative along the point's b.
+struct Du {
+  double v, d;
 };
-__device__ constexpr int kHc[6] = {0, 0, 0, 1, 1, 2}, kHd[6] = {0, 1, 2, 1, 2, 2};
-// position of the symmetric pair (c, d) in that order
-__device__ __forceinline__ int hidx(int c, int d) {
-  const int lo = c < d ? c : d, hi = c < d ? d : c;
-  return lo == 0 ? hi : lo == 1 ? 2 + hi : 5;
-}
+__device__ __forceinline__ Du operator+(Du a, Du b) { return {a.v + b.v, a.d + b.d}; }
+__device__ __forceinline__ Du operator-(Du a, Du b) { return {a.v - b.v, a.d - b.d}; }
+__device__ __forceinline__ Du operator*(Du a, Du b) { return {a.v * b.v, a.d * b.v + a.v * b.d}; }
+__device__ __forceinline__ Du operator*(double s, Du a) { return {s * a.v, s * a.d}; }
 
-__device__ __forceinline__ J2 jconst(double v) {
-  J2 r;
-  r.v = v;
-  for (int c = 0; c < 3; ++c) r.g[c] = 0.0;
-  for (int k = 0; k < 6; ++k) r.h[k] = 0.0;
-  return r;
-}
-__device__ __forceinline__ J2 jcoord(double x, int c) {  // the coordinate x_c
-  J2 r = jconst(x);
-  r.g[c] = 1.0;
-  return r;
-}
-__device__ __forceinline__ J2 jmul(const J2 &a, const J2 &b) {
-  J2 r;
-  r.v = a.v * b.v;
-  for (int c = 0; c < 3; ++c) r.g[c] = a.g[c] * b.v + a.v * b.g[c];
-  for (int k = 0; k < 6; ++k) {
-    const int c = kHc[k], d = kHd[k];
-    r.h[k] = a.h[k] * b.v + a.g[c] * b.g[d] + a.g[d] * b.g[c] + a.v * b.h[k];
-  }
-  return r;
-}
-__device__ __forceinline__ J2 jaxpby(double s, const J2 &a, double t, const J2 &b) {
-  J2 r;
-  r.v = s * a.v + t * b.v;
-  for (int c = 0; c < 3; ++c) r.g[c] = s * a.g[c] + t * b.g[c];
-  for (int k = 0; k < 6; ++k) r.h[k] = s * a.h[k] + t * b.h[k];
-  return r;
-}
-
-// Solid harmonics up to L as jets: the recursion of the value evaluation
-// (m = 1 z-like, (2m, 2m+1) pairs, top pair by the (x, y) rotation) carried
-// out on value + first + second derivatives.
+// Solid harmonics up to L and their gradients as such pairs: the recursion of
+// the value evaluation (m = 1 z-like, (2m, 2m+1) pairs, top pair by the (x, y)
+// rotation) and its derivatives, carried out on values with a derivative along b.
 template <int L>
-__device__ __forceinline__ void sh_jets(double x, double y, double z, J2 *C) {
-  const J2 X = jcoord(x, 0), Y = jcoord(y, 1), Z = jcoord(z, 2);
-  J2 R2 = jconst(x * x + y * y + z * z);
-  R2.g[0] = 2.0 * x;
-  R2.g[1] = 2.0 * y;
-  R2.g[2] = 2.0 * z;
-  R2.h[0] = R2.h[3] = R2.h[5] = 2.0;
-  C[0] = jconst(1.0);
+__device__ __forceinline__ void sh_along(Du x, Du y, Du z, Du *C, Du *Cx, Du *Cy, Du *Cz) {
+  const Du zero = {0.0, 0.0}, one = {1.0, 0.0};
+  const Du r2 = x * x + y * y + z * z;
+  C[0] = one;
+  Cx[0] = Cy[0] = Cz[0] = zero;
   if constexpr (L >= 1) {
-    C[1] = Z;
-    C[2] = X;
-    C[3] = Y;
+    C[1] = z; C[2] = x; C[3] = y;
+    Cx[1] = zero; Cy[1] = zero; Cz[1] = one;
+    Cx[2] = one; Cy[2] = zero; Cz[2] = zero;
+    Cx[3] = zero; Cy[3] = one; Cz[3] = zero;
   }
+  // u = s z p - t r2 q and its derivatives
+  auto two = [&](int o, double s, int p, double t, int q) {
+    C[o] = s * (z * C[p]) - t * (r2 * C[q]);
+    Cx[o] = s * (z * Cx[p]) - t * (2.0 * (x * C[q]) + r2 * Cx[q]);
+    Cy[o] = s * (z * Cy[p]) - t * (2.0 * (y * C[q]) + r2 * Cy[q]);
+    Cz[o] = s * (C[p] + z * Cz[p]) - t * (2.0 * (z * C[q]) + r2 * Cz[q]);
+  };
 #pragma unroll
   for (int l = 2; l <= L; ++l) {
     const int o = l * l, o1 = (l - 1) * (l - 1), o2 = (l - 2) * (l - 2);
     const double lr = l, l1r = l - 1, ll1r = 2 * l - 1;
-    C[o] = jaxpby(ll1r / lr, jmul(Z, C[o1]), -l1r / lr, jmul(R2, C[o2]));
+    two(o, ll1r / lr, o1, l1r / lr, o2);
 #pragma unroll
     for (int im = 1; im <= l - 2; ++im) {
       const double sim = (double)(im * im);
@@ -85,206 +62,299 @@ __device__ __forceinline__ void sh_jets(double x, double y, double z, J2 *C) {
 #pragma unroll
       for (int k = 0; k < 2; ++k) {
         const int m = 2 * im + k - 1;
-        C[o + m] = jaxpby(ll1r * rlm, jmul(Z, C[o1 + m]), -rl1m * rlm, jmul(R2, C[o2 + m]));
+        two(o + m, ll1r * rlm, o1 + m, rl1m * rlm, o2 + m);
       }
     }
-    {
-      const double rlm = 1.0 / sqrt(lr * lr - (double)((l - 1) * (l - 1)));
+    const double rlm = ll1r / sqrt(lr * lr - l1r * l1r);
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int m = 2 * l - 3 + k;
-        C[o + m] = jaxpby(ll1r * rlm, jmul(Z, C[o1 + m]), 0.0, C[o1 + m]);
-      }
+    for (int k = 0; k < 2; ++k) {
+      const int m = 2 * l - 3 + k;
+      C[o + m] = rlm * (z * C[o1 + m]);
+      Cx[o + m] = rlm * (z * Cx[o1 + m]);
+      Cy[o + m] = rlm * (z * Cy[o1 + m]);
+      Cz[o + m] = rlm * (C[o1 + m] + z * Cz[o1 + m]);
     }
-    {
-      const double rll = sqrt(ll1r / (2.0 * lr));
-      const int i2 = o1 + 2 * l - 3, i1 = o1 + 2 * l - 2;
-      C[o + 2 * l - 1] = jaxpby(rll, jmul(X, C[i2]), -rll, jmul(Y, C[i1]));
-      C[o + 2 * l] = jaxpby(rll, jmul(Y, C[i2]), rll, jmul(X, C[i1]));
-    }
+    const double rll = sqrt(ll1r / (2.0 * lr));
+    const int i2 = o1 + 2 * l - 3, i1 = o1 + 2 * l - 2, a = o + 2 * l - 1, b = o + 2 * l;
+    C[a] = rll * (x * C[i2] - y * C[i1]);
+    Cx[a] = rll * (C[i2] + x * Cx[i2] - y * Cx[i1]);
+    Cy[a] = rll * (x * Cy[i2] - C[i1] - y * Cy[i1]);
+    Cz[a] = rll * (x * Cz[i2] - y * Cz[i1]);
+    C[b] = rll * (y * C[i2] + x * C[i1]);
+    Cx[b] = rll * (y * Cx[i2] + C[i1] + x * Cx[i1]);
+    Cy[b] = rll * (C[i2] + y * Cy[i2] + x * Cy[i1]);
+    Cz[b] = rll * (y * Cz[i2] + x * Cz[i1]);
   }
 }
 
-// Hessian planes of the functions of one shell at one point: phi = C_lm R(r)
-// with R a contraction of norm exp(-alpha r^2) (zero where alpha r^2 >= 50,
-// as the value evaluation)
-template <int L>
-__device__ __forceinline__ void shell_hess(const ShellD &sh, const double *__restrict__ exps,
-                                           const double *__restrict__ norms,
-                                           const double *__restrict__ contr, double x, double y,
-                                           double z, const J2 *C, double *hess, long Mc, long cs,
-                                           long p) {
-  const int ne = sh.n_exp, nu = sh.n_unc, nc = sh.n_contr, nf = nu + nc;
-  const double r2 = x * x + y * y + z * z, xs[3] = {x, y, z};
-  // radial jet of R = sum_e c_e r0_e: grad = R1 x, Hessian = R2 x x^T + R1 I,
-  // R1 = sum c (-2 alpha) r0, R2 = sum c (4 alpha^2) r0
-  auto emit = [&](int f, double R0, double R1, double R2) {
-    J2 R = jconst(R0);
-    for (int c = 0; c < 3; ++c) R.g[c] = R1 * xs[c];
-    for (int k = 0; k < 6; ++k)
-      R.h[k] = R2 * xs[kHc[k]] * xs[kHd[k]] + (kHc[k] == kHd[k] ? R1 : 0.0);
+// One point's inputs of the bracket: X and Z at the point's functions (stride
+// Mc; LDA: Z = 2 a X), b, and where the sum goes.
+struct Bracket {
+  const double *X, *Z;
+  long Mc;
+  double a2, b[3];
+};
+
+// t += sum over the 2 L + 1 functions of a shell's radial function R (at f0,
+// nf apart) of the bracket, with r0 = R, r1 = R'/r, r2 = (R'/r)'/r and bx = b . x
+template <int L, bool GGA>
+__device__ __forceinline__ void bracket_fn(const Bracket &B, long f0, int nf, double r0, double r1,
+                                           double r2, double x, double y, double z, double bx,
+                                           const Du *C, const Du *Cx, const Du *Cy, const Du *Cz,
+                                           double (&t)[3]) {
+  constexpr int o = L * L;
+  double X[2 * L + 1], Z[2 * L + 1];
 #pragma unroll
-    for (int m = 0; m < 2 * L + 1; ++m) {
-      const J2 F = jmul(C[L * L + m], R);
-      const long q = (long)(f + m * nf) * Mc + p;
-      for (int k = 0; k < 6; ++k) hess[k * cs + q] = F.h[k];
+  for (int m = 0; m < 2 * L + 1; ++m) {
+    const long q = (f0 + (long)m * nf) * B.Mc;
+    X[m] = gld(B.X + q);
+    Z[m] = GGA ? gld(B.Z + q) : B.a2 * X[m];
+  }
+  double u0[3] = {0.0, 0.0, 0.0}, u1[3] = {0.0, 0.0, 0.0}, zs = 0.0, xs = 0.0, xg = 0.0;
+#pragma unroll
+  for (int m = 0; m < 2 * L + 1; ++m) {
+    const Du g[3] = {Cx[o + m], Cy[o + m], Cz[o + m]};
+    zs += Z[m] * C[o + m].v;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) u0[d] += Z[m] * g[d].v;
+    if (GGA) {
+      xs += X[m] * C[o + m].v;
+      xg += X[m] * C[o + m].d;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        u0[d] += X[m] * g[d].d;
+        u1[d] += X[m] * g[d].v;
+      }
     }
-  };
+  }
+  const double xx[3] = {x, y, z};
+  double s = r1 * zs;
+  if (GGA) s += r1 * xg + r2 * bx * xs;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    t[d] += r0 * u0[d] + s * xx[d];
+    if (GGA) t[d] += r1 * (bx * u1[d] + B.b[d] * xs);
+  }
+}
+
+template <int L, bool GGA>
+__device__ __forceinline__ void bracket_shell(const Bracket &B, const ShellD &sh, const double *ex,
+                                              const double *nm, const double *ct, double x,
+                                              double y, double z, const Du *C, const Du *Cx,
+                                              const Du *Cy, const Du *Cz, double (&t)[3]) {
+  const int ne = sh.n_exp, nu = sh.n_unc, nc = sh.n_contr, nf = nu + nc;
+  const double rr = x * x + y * y + z * z, bx = GGA ? B.b[0] * x + B.b[1] * y + B.b[2] * z : 0.0;
   double s0[kMaxContr], s1[kMaxContr], s2[kMaxContr];
+#pragma unroll
   for (int k = 0; k < kMaxContr; ++k) s0[k] = s1[k] = s2[k] = 0.0;
   for (int e = 0; e < ne; ++e) {
-    const double alpha = exps[sh.exp_off + e], ar2 = alpha * r2;
+    const double al = ex[e], ar2 = al * rr;
     double r0 = 0.0;
-    if (ar2 < 50.0) r0 = norms[sh.exp_off + e] * exp(-ar2);
-    const double r1 = -2.0 * alpha * r0, rr = 4.0 * alpha * alpha * r0;
-    if (e < nu) emit(sh.func_off + e, r0, r1, rr);
-    for (int k = 0; k < nc; ++k) {
-      const double cf = contr[sh.contr_off + k * ne + e];
-      s0[k] += r0 * cf;
-      s1[k] += r1 * cf;
-      s2[k] += rr * cf;
-    }
-  }
-  for (int k = 0; k < nc; ++k) emit(sh.func_off + nu + k, s0[k], s1[k], s2[k]);
-}
-
-template <int LA>
-__device__ __forceinline__ void atom_hess(const AtomD &at, const ShellD *__restrict__ shells,
-                                          const double *exps, const double *norms,
-                                          const double *contr, double x, double y, double z,
-                                          double *hess, long Mc, long cs, long p) {
-  J2 C[(LA + 1) * (LA + 1)];
-  sh_jets<LA>(x, y, z, C);
-  for (int s = at.shell_begin; s < at.shell_end; ++s) {
-    const ShellD sh = shells[s];
-    switch (sh.l) {
-      case 0: shell_hess<0>(sh, exps, norms, contr, x, y, z, C, hess, Mc, cs, p); break;
-      case 1: if constexpr (LA >= 1) shell_hess<1>(sh, exps, norms, contr, x, y, z, C, hess, Mc, cs, p); break;
-      case 2: if constexpr (LA >= 2) shell_hess<2>(sh, exps, norms, contr, x, y, z, C, hess, Mc, cs, p); break;
-      case 3: if constexpr (LA >= 3) shell_hess<3>(sh, exps, norms, contr, x, y, z, C, hess, Mc, cs, p); break;
-      case 4: if constexpr (LA >= 4) shell_hess<4>(sh, exps, norms, contr, x, y, z, C, hess, Mc, cs, p); break;
-    }
-  }
-}
-
-// item = (256-point block, atom); hess = [6][NP][Mc] of one chunk
-__global__ __launch_bounds__(kThreads) void k_basis_hess(
-    const double *__restrict__ gx, const double *__restrict__ gy, const double *__restrict__ gz,
-    const AtomD *__restrict__ atoms, int n_atoms, const ShellD *__restrict__ shells,
-    const double *__restrict__ exps, const double *__restrict__ norms,
-    const double *__restrict__ contr, int NP, long Mc, double *__restrict__ hess) {
-  const long total = (Mc / kThreads) * n_atoms, cs = (long)NP * Mc;
-  for (long it = blockIdx.x; it < total; it += gridDim.x) {
-    const int atom = (int)(it % n_atoms);
-    const long p = (it / n_atoms) * kThreads + threadIdx.x;
-    const AtomD at = atoms[atom];
-    const double x = gx[p] - at.x, y = gy[p] - at.y, z = gz[p] - at.z;
-    switch (at.lmax) {
-      case 0: atom_hess<0>(at, shells, exps, norms, contr, x, y, z, hess, Mc, cs, p); break;
-      case 1: atom_hess<1>(at, shells, exps, norms, contr, x, y, z, hess, Mc, cs, p); break;
-      case 2: atom_hess<2>(at, shells, exps, norms, contr, x, y, z, hess, Mc, cs, p); break;
-      case 3: atom_hess<3>(at, shells, exps, norms, contr, x, y, z, hess, Mc, cs, p); break;
-      default: atom_hess<4>(at, shells, exps, norms, contr, x, y, z, hess, Mc, cs, p); break;
-    }
-  }
-}
-
-// The gradient bracket of function i at point p (q = i Mc + p) added into t:
-//   t_d += grad_d phi_i (a2 X_i + b . Y_i) + X_i sum_c b_c H_dc phi_i
-template <bool GGA>
-__device__ __forceinline__ void grad_bracket(const double *__restrict__ XY,
-                                             const double *__restrict__ phi,
-                                             const double *__restrict__ hess, long cs, long q,
-                                             double a2, const double (&b)[3], double (&t)[3]) {
-  const double X = XY[q];
-  double s = a2 * X;
-  if (GGA) s += b[0] * XY[cs + q] + b[1] * XY[2 * cs + q] + b[2] * XY[3 * cs + q];
-  for (int d = 0; d < 3; ++d) {
-    double u = phi[(1 + d) * cs + q] * s;
-    if (GGA) {
-      double hb = 0.0;
-      for (int c = 0; c < 3; ++c) hb += b[c] * hess[hidx(c, d) * cs + q];
-      u += X * hb;
-    }
-    t[d] += u;
-  }
-}
-
-// item = one 128-point tile of the chunk: for each function i of its list
-// (tfl[tf_off[t] ..], the functions not cut off on the tile; the others add
-// exact zeros) the tile's sum of
-//   t_d = grad_d phi_i (2 a X_i + b . Y_i) + X_i sum_c b_c H_dc phi_i
-// into part[(list position - pbase) * 3 + d], over its points in a fixed
-// order.  Two functions at a time, one per half of the workgroup (a point
-// per thread).  XY = [4][NP][Mc]: X, then Y_x, Y_y, Y_z (written for the
-// listed functions); phi the chunk's [4][NP][Mc] basis values; a, b the
-// build's per-point coefficients.
-template <bool GGA>
-__global__ __launch_bounds__(kThreads) void k_grad_fn(long ntiles, const int *__restrict__ tf_off,
-                                                      const uint16_t *__restrict__ tfl, int NP,
-                                                      long Mc, const double *__restrict__ XY,
-                                                      const double *__restrict__ phi,
-                                                      const double *__restrict__ hess,
-                                                      const double *__restrict__ a,
-                                                      const double *__restrict__ bx,
-                                                      const double *__restrict__ by,
-                                                      const double *__restrict__ bz,
-                                                      double *__restrict__ part) {
-  static_assert(kThreads == 2 * kScreenTile, "two halves of one tile's points");
-  __shared__ double sh[3][kThreads];
-  const long cs = (long)NP * Mc, pbase = tf_off[0];
-  const int tid = threadIdx.x, half = tid / kScreenTile, pt = tid % kScreenTile;
-  for (long t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const long f0 = tf_off[t];
-    const int nf = tf_off[t + 1] - (int)f0;
-    const long p = t * kScreenTile + pt;
-    const double a2 = 2.0 * a[p];
-    const double b[3] = {GGA ? bx[p] : 0.0, GGA ? by[p] : 0.0, GGA ? bz[p] : 0.0};
-    for (int e0 = 0; e0 < nf; e0 += 2) {
-      const int e = e0 + half;
-      double tt[3] = {0.0, 0.0, 0.0};
-      if (e < nf) grad_bracket<GGA>(XY, phi, hess, cs, (long)tfl[f0 + e] * Mc + p, a2, b, tt);
-      for (int d = 0; d < 3; ++d) sh[d][tid] = tt[d];
-      __syncthreads();
-      for (int st = kScreenTile / 2; st > 0; st >>= 1) {
-        if (pt < st)
-          for (int d = 0; d < 3; ++d) sh[d][tid] += sh[d][tid + st];
-        __syncthreads();
+    if (ar2 < 50.0) r0 = nm[e] * exp(-ar2);  // the value evaluation's cut-off
+    const double r1 = -2.0 * al * r0, r2 = -2.0 * al * r1;
+    if (e < nu) bracket_fn<L, GGA>(B, sh.func_off + e, nf, r0, r1, r2, x, y, z, bx, C, Cx, Cy, Cz, t);
+#pragma unroll
+    for (int k = 0; k < kMaxContr; ++k)
+      if (k < nc) {
+        const double c = ct[k * ne + e];
+        s0[k] += r0 * c;
+        s1[k] += r1 * c;
+        s2[k] += r2 * c;
       }
-      if (pt < 3 && e < nf) part[(f0 + e - pbase) * 3 + pt] = sh[pt][half * kScreenTile];
-      __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < kMaxContr; ++k)
+    if (k < nc)
+      bracket_fn<L, GGA>(B, sh.func_off + nu + k, nf, s0[k], s1[k], s2[k], x, y, z, bx, C, Cx, Cy, Cz, t);
+}
+
+// The brackets of one staged atom's shells at the thread's point.
+template <int LA, bool GGA>
+__device__ __forceinline__ void bracket_atom(const RangeLds<double> &A, int sb, int se, int e0, int c0,
+                                             int grp, const Bracket &B, double x, double y, double z,
+                                             double (&t)[3]) {
+  constexpr int NLM = (LA + 1) * (LA + 1);
+  Du C[NLM], Cx[NLM], Cy[NLM], Cz[NLM];
+  sh_along<LA>({x, B.b[0]}, {y, B.b[1]}, {z, B.b[2]}, C, Cx, Cy, Cz);
+  for (int s = sb; s < se; ++s) {
+    if (!(A.fl[s][grp] & 1)) continue;  // cut off on the point's tile
+    ShellD sh = A.sh[s];
+    sh.l = __builtin_amdgcn_readfirstlane(sh.l);
+    sh.n_exp = __builtin_amdgcn_readfirstlane(sh.n_exp);
+    sh.n_unc = __builtin_amdgcn_readfirstlane(sh.n_unc);
+    sh.n_contr = __builtin_amdgcn_readfirstlane(sh.n_contr);
+    sh.exp_off = __builtin_amdgcn_readfirstlane(sh.exp_off);
+    sh.contr_off = __builtin_amdgcn_readfirstlane(sh.contr_off);
+    sh.func_off = __builtin_amdgcn_readfirstlane(sh.func_off);
+    const double *ex = A.ex + (sh.exp_off - e0), *nm = A.nm + (sh.exp_off - e0);
+    const double *ct = A.ct + (sh.contr_off - c0);
+    switch (sh.l) {
+      case 0: bracket_shell<0, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 1: if constexpr (LA >= 1) bracket_shell<1, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 2: if constexpr (LA >= 2) bracket_shell<2, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 3: if constexpr (LA >= 3) bracket_shell<3, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 4: if constexpr (LA >= 4) bracket_shell<4, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
     }
   }
 }
 
-// item = a point of the chunk: pm[d][p] += 2 sum_i t_d(i, p), the same terms
-// as k_grad_fn summed over functions instead of points: w grad f at the point
-// (the motion of the point with its atom)
-template <bool GGA>
-__global__ __launch_bounds__(kThreads) void k_grad_pt(const int *__restrict__ tf_off,
-                                                      const uint16_t *__restrict__ tfl, int NP,
-                                                      long Mc, const double *__restrict__ XY,
-                                                      const double *__restrict__ phi,
-                                                      const double *__restrict__ hess,
-                                                      const double *__restrict__ a,
-                                                      const double *__restrict__ bx,
-                                                      const double *__restrict__ by,
-                                                      const double *__restrict__ bz,
-                                                      double *__restrict__ pm, long pstride) {
-  const long cs = (long)NP * Mc;
-  for (long p = (long)blockIdx.x * kThreads + threadIdx.x; p < Mc; p += (long)gridDim.x * kThreads) {
-    const double a2 = 2.0 * a[p];
-    double b[3] = {0.0, 0.0, 0.0};
-    if (GGA) {
-      b[0] = bx[p];
-      b[1] = by[p];
-      b[2] = bz[p];
+// Sum of v over the wave's 64 lanes, in every lane, in a fixed order.
+__device__ __forceinline__ double wave_sum(double v) {
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
+  return v;
+}
+
+// item = 256-point block of a chunk's unit: its basis items (block, atom range)
+// in turn, the brackets of every atom's functions that are not cut off summed
+// over each wave's points into part[item][atom of the range][wave][3], and over
+// functions into pm[d][p] += 2 t (w grad f at the point: its motion with its
+// atom) when pm is given.  XZ = [2][NP][Mc] at the tiles' functions; st: the
+// build's coefficients a, b (planes stride np apart).  Bound by the reads of X
+// and Z and the registers of their use (two waves a SIMD; one: 0.80 ms).  Per
+// (H2O)16 chunk of 245 760 points 0.47 ms; storing the six second-derivative
+// planes of every function and point and reading 13 planes back twice, once per
+// sum, took 2.7 ms.
+template <bool GGA, int LMAX>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(LMAX <= 2 ? 2 : 1))) void k_bracket(const UnitD *__restrict__ unit,
+                                                      const double *__restrict__ XZ,
+                                                      const double *__restrict__ st, long np,
+                                                      double *__restrict__ pm,
+                                                      double *__restrict__ part) {
+  __shared__ RangeLds<double> A;
+  const UnitD &U = *unit;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = tid / kGroup;
+  const long Mc = U.Mc, cs = (long)U.NP * Mc;
+  for (long blk = blockIdx.x; blk < Mc / kThreads; blk += gridDim.x) {
+    long i0 = 0, hi = U.nbi;  // the block's items: they are listed block by block
+    while (i0 < hi) {
+      const long mid = (i0 + hi) >> 1;
+      if ((long)(U.bitems[mid] >> 16) < blk) i0 = mid + 1; else hi = mid;
     }
-    double t[3] = {0.0, 0.0, 0.0};
-    const long tile = p / kScreenTile;
-    for (int e = tf_off[tile]; e < tf_off[tile + 1]; ++e)  // the functions not cut off here
-      grad_bracket<GGA>(XY, phi, hess, cs, (long)tfl[e] * Mc + p, a2, b, t);
-    for (int d = 0; d < 3; ++d) pm[d * pstride + p] += 2.0 * t[d];
+    const long p = blk * kThreads + tid;
+    Bracket B;
+    B.X = XZ + p;
+    B.Z = XZ + cs + p;
+    B.Mc = Mc;
+    B.a2 = 2.0 * st[(S_A)*np + p];
+    for (int d = 0; d < 3; ++d) B.b[d] = GGA ? st[(S_BX + d) * np + p] : 0.0;
+    double tp[3] = {0.0, 0.0, 0.0};
+    for (long item = i0; item < U.nbi && (long)(U.bitems[item] >> 16) == blk; ++item) {
+      const BasisItem it = stage_basis_item(U, item, A);
+      const int na = __builtin_amdgcn_readfirstlane(it.n_atoms);
+      for (int a = 0; a < na; ++a) {
+        const int sb = __builtin_amdgcn_readfirstlane(A.s0[a]), se = __builtin_amdgcn_readfirstlane(A.s1[a]);
+        bool any = false;
+        for (int s = sb; s < se; ++s) any = any || (A.fl[s][grp] & 1);
+        double t[3] = {0.0, 0.0, 0.0};
+        if (any) {
+          const double x = it.gx - A.ax[a], y = it.gy - A.ay[a], z = it.gz - A.az[a];
+          switch (__builtin_amdgcn_readfirstlane(A.lm[a])) {
+            case 0: bracket_atom<0, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
+            case 1: bracket_atom<1, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
+            case 2: if constexpr (LMAX >= 2) bracket_atom<2, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
+            default: if constexpr (LMAX >= 4) bracket_atom<4, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
+          }
+        }
+        for (int d = 0; d < 3; ++d) {
+          tp[d] += t[d];
+          const double s = wave_sum(t[d]);
+          if (lane == 0) part[((item * kRangeAtoms + a) * 4 + wave) * 3 + d] = s;
+        }
+      }
+    }
+    if (pm)
+      for (int d = 0; d < 3; ++d) pm[d * np + p] += 2.0 * tp[d];
+  }
+}
+
+// item = atom range: grad[atom][d] -= 2 x the sum of part over the chunk's
+// basis items of the range, in a fixed order (a thread takes every 256th item,
+// then the lanes and the waves are summed)
+__global__ __launch_bounds__(kThreads) void k_bracket_sum(const UnitD *__restrict__ unit,
+                                                          const double *__restrict__ part,
+                                                          double *__restrict__ grad) {
+  constexpr int NV = 3 * kRangeAtoms;
+  __shared__ double sh[kThreads / 64][NV];
+  const UnitD &U = *unit;
+  const int rng = blockIdx.x, tid = threadIdx.x;
+  const RangeD R = U.ranges[rng];
+  double s[NV];
+#pragma unroll
+  for (int v = 0; v < NV; ++v) s[v] = 0.0;
+  for (long i = tid; i < U.nbi; i += kThreads) {
+    if ((int)(U.bitems[i] & 0xffffu) != rng) continue;
+    const double *q = part + i * (4 * NV);
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+      if (v / 3 < R.n_atoms)
+        for (int w = 0; w < 4; ++w) s[v] += q[(v / 3 * 4 + w) * 3 + v % 3];
+  }
+#pragma unroll
+  for (int v = 0; v < NV; ++v) {
+    const double t = wave_sum(s[v]);
+    if ((tid & 63) == 0) sh[tid >> 6][v] = t;
+  }
+  __syncthreads();
+  if (tid < 3 * R.n_atoms)
+    grad[3 * U.ratoms[R.atom_begin + tid / 3] + tid % 3] -=
+        2.0 * ((sh[0][tid] + sh[1][tid]) + (sh[2][tid] + sh[3][tid]));
+}
+
+// coef = 2 a, b of the build (planes stride np apart): the W pass over them
+// gives 2 a Phi + b . grad Phi
+__global__ __launch_bounds__(kThreads) void k_bracket_coef(long Mc, const double *__restrict__ st,
+                                                           long np, double *__restrict__ coef) {
+  for (long p = (long)blockIdx.x * kThreads + threadIdx.x; p < Mc; p += (long)gridDim.x * kThreads) {
+    coef[p] = 2.0 * st[S_A * np + p];
+    for (int d = 0; d < 3; ++d) coef[(1 + d) * Mc + p] = st[(S_BX + d) * np + p];
+  }
+}
+
+// out[j] += sum_i part[i][j], j < m: one workgroup per j, fixed order
+__global__ __launch_bounds__(kThreads) void k_column_sum(long n, int m, const double *__restrict__ part,
+                                                         double *__restrict__ out) {
+  __shared__ double sh[kThreads];
+  const int j = blockIdx.x, tid = threadIdx.x;
+  double s = 0.0;
+  for (long i = tid; i < n; i += kThreads) s += part[i * m + j];
+  sh[tid] = s;
+  __syncthreads();
+  for (int o = kThreads / 2; o > 0; o >>= 1) {
+    if (tid < o) sh[tid] += sh[tid + o];
+    __syncthreads();
+  }
+  if (tid == 0) out[j] += sh[0];
+}
+
+// Adds a wave's three values to the three of atom `a`, kept per wave (only this
+// wave touches them).
+__device__ __forceinline__ void wave_add(double *acc, int a, double v0, double v1, double v2) {
+  const int lane = threadIdx.x & 63;
+  const double s0 = wave_sum(v0), s1 = wave_sum(v1), s2 = wave_sum(v2);
+  if (lane < 3) acc[3 * a + lane] += lane == 0 ? s0 : lane == 1 ? s1 : s2;
+}
+
+// One wave per workgroup: the wave's points in groups of 64, pm summed by owner
+// (the owners of a group in order of first appearance) into part[wave][na][3].
+__global__ __launch_bounds__(64) void k_owner_sum(int na, long np, const int *__restrict__ owner,
+                                                  const double *__restrict__ pm,
+                                                  double *__restrict__ part) {
+  double *acc = part + (long)blockIdx.x * na * 3;
+  const int lane = threadIdx.x;
+  for (int j = lane; j < 3 * na; j += 64) acc[j] = 0.0;
+  __syncthreads();
+  for (long g = blockIdx.x; g < np / 64; g += gridDim.x) {
+    const long p = g * 64 + lane;
+    const int own = owner[p];
+    const double v[3] = {pm[p], pm[np + p], pm[2 * np + p]};
+    unsigned long long left = __ballot(own >= 0);
+    while (left) {
+      const int a = __builtin_amdgcn_readlane(own, __builtin_ctzll(left));
+      const bool mine = own == a;
+      wave_add(acc, a, mine ? v[0] : 0.0, mine ? v[1] : 0.0, mine ? v[2] : 0.0);
+      left &= ~__ballot(mine);
+    }
   }
 }
 
@@ -296,17 +366,22 @@ __global__ __launch_bounds__(kThreads) void k_grad_pt(const int *__restrict__ tf
 //   d log P_C / dR_B = sum_{D != C} sigma(mu_CD) d mu_CD / dR_B
 //   dw / dR_B = w sum_C (delta_CA - P_C / Z) d log P_C / dR_B.
 // s = 0 only at mu = +-1, where s' = 0 too: sigma is taken as 0 there.
-__device__ __forceinline__ void becke_s(double mu, double &s, double &sig) {
+__device__ __forceinline__ void becke_sigma(double mu, double &s, double &sig) {
   const double f1 = mu * (3.0 - mu * mu) / 2.0, f2 = f1 * (3.0 - f1 * f1) / 2.0,
                f3 = f2 * (3.0 - f2 * f2) / 2.0;
   const double d = 1.5 * (1.0 - f2 * f2) * 1.5 * (1.0 - f1 * f1) * 1.5 * (1.0 - mu * mu);
   s = 0.5 * (1.0 - f3);
   sig = s > 0.0 ? -0.5 * d / s : 0.0;
 }
+__device__ __forceinline__ double becke_cell(double mu) {
+  const double f1 = mu * (3.0 - mu * mu) / 2.0, f2 = f1 * (3.0 - f1 * f1) / 2.0;
+  return 0.5 * (1.0 - f2 * (3.0 - f2 * f2) / 2.0);
+}
 
 struct Pt {
   double x, y, z;
 };
+// distance of the point from a centre, and the unit vector from the centre
 __device__ __forceinline__ double dist(const AtomD &A, Pt r, double (&e)[3]) {
   e[0] = r.x - A.x;
   e[1] = r.y - A.y;
@@ -318,174 +393,218 @@ __device__ __forceinline__ double dist(const AtomD &A, Pt r, double (&e)[3]) {
   e[2] *= id;
   return d;
 }
+__device__ __forceinline__ double dist(const AtomD &A, Pt r) {
+  const double x = r.x - A.x, y = r.y - A.y, z = r.z - A.z;
+  return sqrt(x * x + y * y + z * z);
+}
 
-// item = a point: q[C][p] = P_C / Z, and rm[p] = sum_C (delta_CA - q_C)
-// d log P_C / dr (the owner's share through the point's motion)
-__global__ __launch_bounds__(kThreads) void k_becke_q(int na, const AtomD *__restrict__ atoms,
-                                                      const double *__restrict__ inv_dist, long Mc,
-                                                      const double *__restrict__ gx,
-                                                      const double *__restrict__ gy,
-                                                      const double *__restrict__ gz,
-                                                      const int *__restrict__ owner,
-                                                      double *__restrict__ q, double *__restrict__ rm) {
-  for (long p = (long)blockIdx.x * kThreads + threadIdx.x; p < Mc; p += (long)gridDim.x * kThreads) {
-    const int A = owner[p];
-    if (A < 0) {
-      for (int C = 0; C < na; ++C) q[C * Mc + p] = 0.0;
-      for (int d = 0; d < 3; ++d) rm[d * Mc + p] = 0.0;
-      continue;
+// One wave per workgroup, a point per lane, groups of 64 points in turn: the
+// wave's sums over its points of w f d log w / dR into part[wave][na][3].  As the
+// weights themselves, only the centres C whose P_C can matter to a point of the
+// wave (above 2^-64 of the nearest centre's, or the owner) are formed and
+// differentiated: their P in scr[wave][listed centre][64], their indices in
+// list[wave][na].  For each of them every other centre D takes
+// k_C sigma d mu_CD / dR_D, C the same with d mu_CD / dR_C, and the owner
+// d mu_CD / dr through the point's motion.  Bound by FP64 arithmetic; (H2O)16,
+// 48 centres, 966 000 points: 4.9 ms, every pair of centres for every point (in
+// two kernels) 21 ms.
+// LDS: the wave's sums are kept there (na up to kLdsAtoms), else in part.
+constexpr int kNearQ = 8, kFormQ = 4, kLdsAtoms = 1024;
+constexpr double kNegligibleQ = 5.421010862427522e-20;  // 2^-64
+template <bool LDS>
+__global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restrict__ atoms,
+                                                   const double *__restrict__ inv_dist, long np,
+                                                   const double *__restrict__ grid,
+                                                   const double *__restrict__ fp,
+                                                   const int *__restrict__ owner,
+                                                   double *__restrict__ scr,
+                                                   uint16_t *__restrict__ list,
+                                                   double *__restrict__ part) {
+  extern __shared__ double lacc[];  // 3 na
+  double *acc = LDS ? lacc : part + (long)blockIdx.x * na * 3;
+  double *P = scr + (long)blockIdx.x * na * 64;
+  uint16_t *ls = list + (long)blockIdx.x * na;
+  const int lane = threadIdx.x;
+  for (int j = lane; j < 3 * na; j += 64) acc[j] = 0.0;
+  __syncthreads();
+  for (long g = blockIdx.x; g < np / 64; g += gridDim.x) {
+    const long p = g * 64 + lane;
+    const int own = owner[p];
+    const double wf = own >= 0 ? grid[3 * np + p] * fp[p] : 0.0;
+    const bool on = wf != 0.0;
+    if (!__any(on)) continue;
+    const Pt r = {grid[p], grid[np + p], grid[2 * np + p]};
+    // the nearest centres and the nearest one's P, as in the weights
+    double rn[kNearQ];
+    int in[kNearQ];
+#pragma unroll
+    for (int t = 0; t < kNearQ; ++t) {
+      rn[t] = __builtin_inf();
+      in[t] = 0;
     }
-    const Pt r = {gx[p], gy[p], gz[p]};
+    for (int i = 0; i < na; ++i) {
+      double v = dist(atoms[i], r);
+      int id = i;
+      if (!__any(v < rn[kNearQ - 1])) continue;
+#pragma unroll
+      for (int t = 0; t < kNearQ; ++t)
+        if (v < rn[t]) {
+          const double tv = rn[t];
+          const int ti = in[t];
+          rn[t] = v;
+          in[t] = id;
+          v = tv;
+          id = ti;
+        }
+    }
+    double floor_p = 2.0 * kNegligibleQ;  // 2: a centre's cell with itself is 1/2
+    for (int k = 0; k < na; ++k)
+      floor_p *= becke_cell((rn[0] - dist(atoms[k], r)) * inv_dist[(long)in[0] * na + k]);
+    int nl = 0;  // listed centres, the same for the wave
+    for (int i = 0; i < na; ++i) {
+      const double ri = dist(atoms[i], r);
+      double pi = 2.0;
+#pragma unroll
+      for (int t = 0; t < kNearQ; ++t)
+        if (t < na) pi *= becke_cell((ri - rn[t]) * inv_dist[(long)i * na + in[t]]);
+      if (!__any(on && (!(pi <= floor_p) || i == own))) continue;
+      if (lane == 0) ls[nl] = (uint16_t)i;
+      ++nl;
+    }
+    __syncthreads();
     double Z = 0.0;
-    for (int C = 0; C < na; ++C) {
-      double eC[3];
-      const double rC = dist(atoms[C], r, eC);
-      double P = 1.0;
-      for (int D = 0; D < na && P != 0.0; ++D) {
-        if (D == C) continue;
-        double eD[3], s, sig;
-        const double rD = dist(atoms[D], r, eD);
-        becke_s((rC - rD) * inv_dist[(long)C * na + D], s, sig);
-        P *= s;
+    for (int c0 = 0; c0 < nl; c0 += kFormQ) {
+      double ri[kFormQ], pi[kFormQ];
+      int c[kFormQ];
+#pragma unroll
+      for (int m = 0; m < kFormQ; ++m) {
+        c[m] = __builtin_amdgcn_readfirstlane((int)ls[min(c0 + m, nl - 1)]);
+        ri[m] = dist(atoms[c[m]], r);
+        pi[m] = 2.0;
       }
-      q[C * Mc + p] = P;
-      Z += P;
+      for (int k = 0; k < na; ++k) {
+        const double rk = dist(atoms[k], r);
+#pragma unroll
+        for (int m = 0; m < kFormQ; ++m) pi[m] *= becke_cell((ri[m] - rk) * inv_dist[(long)c[m] * na + k]);
+      }
+#pragma unroll
+      for (int m = 0; m < kFormQ; ++m)
+        if (c0 + m < nl) {
+          P[(c0 + m) * 64 + lane] = pi[m];
+          Z += pi[m];
+        }
     }
     const double iz = 1.0 / Z;
-    double g[3] = {0.0, 0.0, 0.0};
-    for (int C = 0; C < na; ++C) {
-      const double qc = q[C * Mc + p] * iz;
-      q[C * Mc + p] = qc;
-      const double k = (C == A ? 1.0 : 0.0) - qc;
-      if (k == 0.0) continue;
-      double eC[3];
-      const double rC = dist(atoms[C], r, eC);
-      for (int D = 0; D < na; ++D) {
-        if (D == C) continue;
-        double eD[3], s, sig;
-        const double rD = dist(atoms[D], r, eD);
-        const double iR = inv_dist[(long)C * na + D];
-        becke_s((rC - rD) * iR, s, sig);
-        for (int d = 0; d < 3; ++d) g[d] += k * sig * (eC[d] - eD[d]) * iR;
+    double rm[3] = {0.0, 0.0, 0.0};
+    for (int c0 = 0; c0 < nl; c0 += kFormQ) {
+      double rc[kFormQ], ec[kFormQ][3], kc[kFormQ], ac[kFormQ][3];
+      int c[kFormQ];
+#pragma unroll
+      for (int m = 0; m < kFormQ; ++m) {
+        const bool there = c0 + m < nl;
+        c[m] = __builtin_amdgcn_readfirstlane((int)ls[min(c0 + m, nl - 1)]);
+        rc[m] = dist(atoms[c[m]], r, ec[m]);
+        kc[m] = on && there ? wf * ((c[m] == own ? 1.0 : 0.0) - P[min(c0 + m, nl - 1) * 64 + lane] * iz) : 0.0;
+        ac[m][0] = ac[m][1] = ac[m][2] = 0.0;
       }
+      for (int D = 0; D < na; ++D) {
+        double eD[3], v[3] = {0.0, 0.0, 0.0};
+        const AtomD &AD = atoms[D];
+        const double rD = dist(AD, r, eD);
+#pragma unroll
+        for (int m = 0; m < kFormQ; ++m) {
+          if (c[m] == D) continue;
+          const double iR = inv_dist[(long)c[m] * na + D], mu = (rc[m] - rD) * iR;
+          double s, sig;
+          becke_sigma(mu, s, sig);
+          const double T = kc[m] != 0.0 ? kc[m] * sig * iR : 0.0, M = T * mu * iR;
+          const AtomD &AC = atoms[c[m]];
+          const double dR[3] = {M * (AC.x - AD.x), M * (AC.y - AD.y), M * (AC.z - AD.z)};
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            v[d] += T * eD[d] + dR[d];
+            ac[m][d] -= T * ec[m][d] + dR[d];
+            rm[d] += T * (ec[m][d] - eD[d]);
+          }
+        }
+        wave_add(acc, D, v[0], v[1], v[2]);
+      }
+#pragma unroll
+      for (int m = 0; m < kFormQ; ++m)
+        if (c0 + m < nl) wave_add(acc, c[m], ac[m][0], ac[m][1], ac[m][2]);
     }
-    for (int d = 0; d < 3; ++d) rm[d * Mc + p] = g[d];
+    // through the points' motion with their owners
+    unsigned long long left = __ballot(on);
+    while (left) {
+      const int a = __builtin_amdgcn_readlane(own, __builtin_ctzll(left));
+      const bool mine = on && own == a;
+      wave_add(acc, a, mine ? rm[0] : 0.0, mine ? rm[1] : 0.0, mine ? rm[2] : 0.0);
+      left &= ~__ballot(mine);
+    }
+    __syncthreads();  // ls is written again
   }
+  if (LDS)
+    for (int j = lane; j < 3 * na; j += 64) part[(long)blockIdx.x * na * 3 + j] = acc[j];
 }
 
-// item = (256-point block, atom B): the block's sum over its points of
-//   w f [ sum_{C != B} (delta_CA - q_C) sigma(mu_CB) d mu_CB / dR_B
-//       + (delta_BA - q_B) sum_{D != B} sigma(mu_BD) d mu_BD / dR_B
-//       + [B == A] rm ]
-// with d mu_CB / dR_B = e_B / R + mu (R_C - R_B) / R^2 and
-// d mu_BD / dR_B = -e_B / R - mu (R_B - R_D) / R^2 (R = |R_C - R_B|, ...),
-// into part[blk][B][3]
-__global__ __launch_bounds__(kThreads) void k_becke_atom(
-    int na, const AtomD *__restrict__ atoms, const double *__restrict__ inv_dist, long Mc,
-    const double *__restrict__ gx, const double *__restrict__ gy, const double *__restrict__ gz,
-    const double *__restrict__ gw, const double *__restrict__ fp, const int *__restrict__ owner,
-    const double *__restrict__ q, const double *__restrict__ rm, double *__restrict__ part) {
-  __shared__ double sh[3][kThreads];
-  const int tid = threadIdx.x;
-  const long total = (Mc / kThreads) * na;
-  for (long it = blockIdx.x; it < total; it += gridDim.x) {
-    const int B = (int)(it % na);
-    const long blk = it / na, p = blk * kThreads + tid;
-    const int A = owner[p];
-    double g[3] = {0.0, 0.0, 0.0};
-    const double wf = gw[p] * fp[p];
-    if (A >= 0 && wf != 0.0) {
-      const Pt r = {gx[p], gy[p], gz[p]};
-      const AtomD &AB = atoms[B];
-      double eB[3];
-      const double rB = dist(AB, r, eB);
-      const double kB = (B == A ? 1.0 : 0.0) - q[B * Mc + p];
-      for (int C = 0; C < na; ++C) {
-        if (C == B) continue;
-        const AtomD &AC = atoms[C];
-        double eC[3], s, sig;
-        const double rC = dist(AC, r, eC);
-        const double iR = inv_dist[(long)C * na + B];
-        const double RCB[3] = {AC.x - AB.x, AC.y - AB.y, AC.z - AB.z};
-        // pair (C, B): B is the second atom
-        const double kC = (C == A ? 1.0 : 0.0) - q[C * Mc + p];
-        const double muCB = (rC - rB) * iR;
-        if (kC != 0.0) {
-          becke_s(muCB, s, sig);
-          for (int d = 0; d < 3; ++d) g[d] += kC * sig * (eB[d] * iR + muCB * RCB[d] * iR * iR);
-        }
-        // pair (B, C): B is the first atom, mu_BC = -mu_CB, R_B - R_C = -RCB
-        if (kB != 0.0) {
-          becke_s(-muCB, s, sig);
-          for (int d = 0; d < 3; ++d) g[d] += kB * sig * (-eB[d] * iR - muCB * RCB[d] * iR * iR);
-        }
-      }
-      if (B == A)
-        for (int d = 0; d < 3; ++d) g[d] += rm[d * Mc + p];
-      for (int d = 0; d < 3; ++d) g[d] *= wf;
-    }
-    for (int d = 0; d < 3; ++d) sh[d][tid] = g[d];
-    __syncthreads();
-    for (int st = kThreads / 2; st > 0; st >>= 1) {
-      if (tid < st)
-        for (int d = 0; d < 3; ++d) sh[d][tid] += sh[d][tid + st];
-      __syncthreads();
-    }
-    if (tid < 3) part[(blk * na + B) * 3 + tid] = sh[tid][0];
-    __syncthreads();
-  }
+// own[internal point] = owner[caller point], -1 for padding
+__global__ __launch_bounds__(kThreads) void k_gather_owner(long npts, long np, const int *__restrict__ perm,
+                                                           const int *__restrict__ owner,
+                                                           int *__restrict__ own) {
+  for (long p = (long)blockIdx.x * kThreads + threadIdx.x; p < np; p += (long)gridDim.x * kThreads)
+    own[p] = p < npts ? owner[perm[p]] : -1;
 }
+
+unsigned grid_of(long items, long cap) { return (unsigned)std::max<long>(1, std::min(items, cap)); }
 
 }  // namespace
 
-void launch_basis_hess(hipStream_t s, const double *gx, const double *gy, const double *gz,
-                       const AtomD *atoms, int n_atoms, const ShellD *shells, const double *exps,
-                       const double *norms, const double *contr, int NP, long Mc, double *hess) {
-  const long total = (Mc / kThreads) * n_atoms;
-  const unsigned g = (unsigned)std::min<long>(total, 256L * 8);
-  hipLaunchKernelGGL(k_basis_hess, dim3(g), dim3(kThreads), 0, s, gx, gy, gz, atoms, n_atoms,
-                     shells, exps, norms, contr, NP, Mc, hess);
+void launch_bracket_coef(hipStream_t s, long Mc, const double *st, long np, double *coef) {
+  hipLaunchKernelGGL(k_bracket_coef, dim3(grid_of(Mc / kThreads, 2048)), dim3(kThreads), 0, s, Mc, st, np, coef);
 }
 
-void launch_grad_fn(hipStream_t s, bool gga, long ntiles, const int *tf_off, const uint16_t *tfl,
-                    int NP, long Mc, const double *XY, const double *phi, const double *hess,
-                    const double *a, const double *bx, const double *by, const double *bz,
-                    double *part) {
-  if (ntiles <= 0) return;
-  const unsigned g = (unsigned)std::min<long>(ntiles, 256L * 8);
-  if (gga)
-    hipLaunchKernelGGL(k_grad_fn<true>, dim3(g), dim3(kThreads), 0, s, ntiles, tf_off, tfl, NP, Mc,
-                       XY, phi, hess, a, bx, by, bz, part);
-  else
-    hipLaunchKernelGGL(k_grad_fn<false>, dim3(g), dim3(kThreads), 0, s, ntiles, tf_off, tfl, NP, Mc,
-                       XY, phi, hess, a, bx, by, bz, part);
+void launch_bracket(hipStream_t s, bool gga, int lmax, const UnitD *unit, long Mc, int n_ranges,
+                    const double *XZ, const double *st, long np, double *pm, double *part,
+                    double *grad) {
+  if (n_ranges <= 0) return;
+  const dim3 g(grid_of(Mc / kThreads, 2048));
+  auto go = [&](auto l) {
+    constexpr int LM = decltype(l)::value;
+    if (gga)
+      hipLaunchKernelGGL((k_bracket<true, LM>), g, dim3(kThreads), 0, s, unit, XZ, st, np, pm, part);
+    else
+      hipLaunchKernelGGL((k_bracket<false, LM>), g, dim3(kThreads), 0, s, unit, XZ, st, np, pm, part);
+  };
+  if (lmax <= 2) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
+  hipLaunchKernelGGL(k_bracket_sum, dim3((unsigned)n_ranges), dim3(kThreads), 0, s, unit, part, grad);
 }
 
-}  // namespace pgxc
-
-namespace pgxc {
-void launch_grad_pt(hipStream_t s, bool gga, const int *tf_off, const uint16_t *tfl, int NP,
-                    long Mc, const double *XY, const double *phi, const double *hess,
-                    const double *a, const double *bx, const double *by, const double *bz,
-                    double *pm, long pstride) {
-  const unsigned g = (unsigned)std::min<long>((Mc + kThreads - 1) / kThreads, 256L * 8);
-  if (gga)
-    hipLaunchKernelGGL(k_grad_pt<true>, dim3(g), dim3(kThreads), 0, s, tf_off, tfl, NP, Mc, XY,
-                       phi, hess, a, bx, by, bz, pm, pstride);
-  else
-    hipLaunchKernelGGL(k_grad_pt<false>, dim3(g), dim3(kThreads), 0, s, tf_off, tfl, NP, Mc, XY,
-                       phi, hess, a, bx, by, bz, pm, pstride);
+long becke_grad_waves(int na, long np) {
+  // one wave each, as many as fill the device a few times over and 256 MiB of
+  // scratch allow
+  const long per = (long)na * (64 * 8 + 2 + 24);
+  return std::max<long>(1, std::min<long>({np / 64, 4096L, (256L << 20) / per}));
 }
 
-void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long Mc,
-                       const double *gx, const double *gy, const double *gz, const double *gw,
-                       const double *fp, const int *owner, double *q, double *rm, double *part) {
-  const unsigned g1 = (unsigned)std::min<long>((Mc + kThreads - 1) / kThreads, 256L * 8);
-  hipLaunchKernelGGL(k_becke_q, dim3(g1), dim3(kThreads), 0, s, na, atoms, inv_dist, Mc, gx, gy,
-                     gz, owner, q, rm);
-  const long total = (Mc / kThreads) * na;
-  const unsigned g2 = (unsigned)std::min<long>(total, 256L * 8);
-  hipLaunchKernelGGL(k_becke_atom, dim3(g2), dim3(kThreads), 0, s, na, atoms, inv_dist, Mc, gx, gy,
-                     gz, gw, fp, owner, q, rm, part);
+void launch_owner_sum(hipStream_t s, int na, long np, const int *owner, const double *pm, long waves,
+                      double *part, double *grad) {
+  hipLaunchKernelGGL(k_owner_sum, dim3((unsigned)waves), dim3(64), 0, s, na, np, owner, pm, part);
+  hipLaunchKernelGGL(k_column_sum, dim3((unsigned)(3 * na)), dim3(kThreads), 0, s, waves, 3 * na, part, grad);
 }
+
+void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long np,
+                       const double *grid, const double *fp, const int *owner, long waves,
+                       double *scr, uint16_t *list, double *part, double *grad) {
+  auto k = na <= kLdsAtoms ? k_becke_grad<true> : k_becke_grad<false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)waves), dim3(64), na <= kLdsAtoms ? 24 * na : 0, s, na, atoms, inv_dist,
+                     np, grid, fp, owner, scr, list, part);
+  hipLaunchKernelGGL(k_column_sum, dim3((unsigned)(3 * na)), dim3(kThreads), 0, s, waves, 3 * na, part, grad);
+}
+
+void launch_gather_owner(hipStream_t s, long npts, long np, const int *perm, const int *owner, int *own) {
+  hipLaunchKernelGGL(k_gather_owner, dim3(grid_of(np / kThreads, 2048)), dim3(kThreads), 0, s, npts, np, perm,
+                     owner, own);
+}
+
 }  // namespace pgxc

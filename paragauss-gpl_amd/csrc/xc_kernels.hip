@@ -11,461 +11,10 @@
 #include <type_traits>
 
 #include "pgxc_internal.h"
+#include "xc_basis.h"
 #include "xc_device.h"
 
 namespace pgxc {
-
-// Widest vector (elements, <= 16 bytes) that splits a BM x BK operand tile
-// evenly over the workgroup and along its contiguous dimension.
-constexpr int pick_vec(int elems, int contig, int maxv) {
-  for (int v = maxv; v > 1; v /= 2)
-    if (elems % (kThreads * v) == 0 && contig % v == 0) return v;
-  return 1;
-}
-
-template <typename T, int N>
-struct VecT {
-  typedef T type __attribute__((ext_vector_type(N)));
-  __device__ static __forceinline__ T get(const type &v, int t) { return v[t]; }
-};
-template <typename T>
-struct VecT<T, 1> {
-  typedef T type;
-  __device__ static __forceinline__ T get(const T &v, int) { return v; }
-};
-
-// Block tile BM x BN over K in steps of BK; 4 waves arranged 2 x 2, wave tile
-// (BM/2) x (BN/2) made of 16x16 MFMA blocks.  ST = 2: two LDS stages, the next
-// slab prefetched into registers while the current one feeds the MFMAs (one
-// barrier per step).  ST = 1: one LDS stage, the next slab's global loads are
-// in flight during the MFMAs (two barriers per step, half the LDS).
-//   AKC: A(m,k) = A[m*sA + k] (k contiguous) else A[m + k*sA]
-//   BKC: B(k,n) = B[n*sB + k] (k contiguous) else B[k*sB + n]
-// LDS layout follows the operands.  Row-contiguous operands (both !KC) are
-// kept [k][row]: the staging writes whole vectors and an MFMA operand is one
-// element per lane.  k-contiguous operands (both KC) are kept [row][k] with
-// rows padded by 16 bytes: the staging again writes the loaded vectors as
-// they are, and each lane reads E = 16 / sizeof(T) consecutive k with one
-// 16-byte read that feeds E MFMAs (MFMA e of a k chunk takes k = 4 E c + E g
-// + e in lane group g, the same for A and B).  Rows 16 bytes apart put the
-// 16-byte reads of 16 lanes on distinct banks.
-template <typename T>
-constexpr int kc_elems() { return 16 / (int)sizeof(T); }
-template <typename T, int BK>
-constexpr int kc_row() { return BK + kc_elems<T>(); }
-template <typename T, int R, int BK, int ST, bool KC>
-constexpr int lds_elems() { return ST * R * (KC ? kc_row<T, BK>() : BK); }
-
-// Operand addressing (gathered rows and K runs): aaddr(i, kt, kk) is the
-// element offset in A of the vector that starts at tile row / column i and
-// local k index kk of K step kt (vectors run along the contiguous dimension),
-// or -1 for a vector of zeros; baddr likewise for B.  Each operand is kept
-// in LDS in its own layout ([row][k] padded when k-contiguous, else
-// [k][row]); with both k-contiguous the MFMAs take E k per 16-byte read,
-// otherwise one element per lane and k.
-template <typename T, int BM, int BN, int BK, int ST, bool AKC, bool BKC, class AAddr,
-          class BAddr>
-__device__ __forceinline__ void gemm_tile(const T *__restrict__ A, const T *__restrict__ B,
-                                          int ksteps, AAddr aaddr, BAddr baddr, T *As, T *Bs,
-                                          typename MF<T>::acc (&acc)[BM / 32][BN / 32]) {
-  constexpr bool KC = AKC && BKC;
-  constexpr int E = kc_elems<T>(), BKP = kc_row<T, BK>();
-  static_assert(!KC || BK % (4 * E) == 0, "k chunk");
-  // elements of one LDS stage of each operand
-  constexpr int SA = AKC ? BM * BKP : BK * BM, SB = BKC ? BN * BKP : BK * BN;
-  constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 16, TN = WN / 16;
-  constexpr int MAXV = 16 / (int)sizeof(T);
-  constexpr int VA = pick_vec(BM * BK, AKC ? BK : BM, MAXV);
-  constexpr int VB = pick_vec(BN * BK, BKC ? BK : BN, MAXV);
-  constexpr int LA = BM * BK / (kThreads * VA), LB = BN * BK / (kThreads * VB);
-  static_assert(LA * kThreads * VA == BM * BK && LB * kThreads * VB == BN * BK, "tile split");
-  typedef VecT<T, VA> VA_t;
-  typedef VecT<T, VB> VB_t;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
-  typename VA_t::type ra[LA];
-  typename VB_t::type rb[LB];
-  unsigned oka = 0, okb = 0;  // bit e: vector e is real (else zeros)
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = typename MF<T>::acc{0, 0, 0, 0};
-
-  if (ksteps <= 0) return;
-  // Loads are unconditional global loads (a vector of zeros reads the
-  // operand's first vector instead, and the zeros are applied when it is
-  // written to LDS), and a step past the last one loads zeros: the pipeline
-  // is straight-line code, so the compiler's wait counts keep the next
-  // step's loads in flight during the MFMAs.
-  auto load = [&](int kt) {
-    const bool live = kt < ksteps;
-    unsigned m = 0;
-#pragma unroll
-    for (int e = 0; e < LA; ++e) {
-      const int idx = tid + kThreads * e;
-      long o;
-      if (AKC) {
-        const int mm = idx / (BK / VA), kv = idx % (BK / VA);
-        o = aaddr(mm, kt, kv * VA);
-      } else {
-        const int mv = idx % (BM / VA), kk = idx / (BM / VA);
-        o = aaddr(mv * VA, kt, kk);
-      }
-      const bool g = live && o >= 0;
-      ra[e] = gld((const typename VA_t::type *)(A + (g ? o : 0)));
-      m |= (unsigned)g << e;
-    }
-    oka = m;
-    m = 0;
-#pragma unroll
-    for (int e = 0; e < LB; ++e) {
-      const int idx = tid + kThreads * e;
-      long o;
-      if (BKC) {
-        const int nn = idx / (BK / VB), kv = idx % (BK / VB);
-        o = baddr(nn, kt, kv * VB);
-      } else {
-        const int nv = idx % (BN / VB), kk = idx / (BN / VB);
-        o = baddr(nv * VB, kt, kk);
-      }
-      const bool g = live && o >= 0;
-      rb[e] = gld((const typename VB_t::type *)(B + (g ? o : 0)));
-      m |= (unsigned)g << e;
-    }
-    okb = m;
-  };
-  auto store = [&](int buf) {
-#pragma unroll
-    for (int e = 0; e < LA; ++e)
-      if (!((oka >> e) & 1u)) ra[e] = typename VA_t::type{};
-#pragma unroll
-    for (int e = 0; e < LB; ++e)
-      if (!((okb >> e) & 1u)) rb[e] = typename VB_t::type{};
-    T *as = As + buf * SA, *bs = Bs + buf * SB;
-#pragma unroll
-    for (int e = 0; e < LA; ++e) {
-      const int idx = tid + kThreads * e;
-      if constexpr (AKC) {  // the vector as loaded, row-major [row][k]
-        const int mm = idx / (BK / VA), kv = idx % (BK / VA);
-        *(typename VA_t::type *)(as + mm * BKP + kv * VA) = ra[e];
-      } else {
-#pragma unroll
-        for (int t = 0; t < VA; ++t) {
-          const int mm = (idx % (BM / VA)) * VA + t, kk = idx / (BM / VA);
-          as[kk * BM + mm] = VA_t::get(ra[e], t);
-        }
-      }
-    }
-#pragma unroll
-    for (int e = 0; e < LB; ++e) {
-      const int idx = tid + kThreads * e;
-      if constexpr (BKC) {
-        const int nn = idx / (BK / VB), kv = idx % (BK / VB);
-        *(typename VB_t::type *)(bs + nn * BKP + kv * VB) = rb[e];
-      } else {
-#pragma unroll
-        for (int t = 0; t < VB; ++t) {
-          const int nn = (idx % (BN / VB)) * VB + t, kk = idx / (BN / VB);
-          bs[kk * BN + nn] = VB_t::get(rb[e], t);
-        }
-      }
-    }
-  };
-  auto compute = [&](int buf) {
-    if constexpr (KC) {
-      typedef typename VecT<T, E>::type VE;
-      const T *as = As + buf * BM * BKP, *bs = Bs + buf * BN * BKP;
-      const int ko = E * (lane >> 4);
-#pragma unroll
-      for (int c = 0; c < BK / (4 * E); ++c) {
-        VE a[TM], b[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-          a[i] = *(const VE *)(as + (wm * WM + i * 16 + (lane & 15)) * BKP + 4 * E * c + ko);
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          b[j] = *(const VE *)(bs + (wn * WN + j * 16 + (lane & 15)) * BKP + 4 * E * c + ko);
-#pragma unroll
-        for (int e = 0; e < E; ++e)
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = MF<T>::mma(a[i][e], b[j][e], acc[i][j]);
-      }
-      return;
-    }
-    const T *as = As + buf * SA, *bs = Bs + buf * SB;
-#pragma unroll
-    for (int k4 = 0; k4 < BK / 4; ++k4) {
-      const int kr = k4 * 4 + (lane >> 4);
-      T a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        const int r = wm * WM + i * 16 + (lane & 15);
-        a[i] = AKC ? as[r * BKP + kr] : as[kr * BM + r];
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const int r = wn * WN + j * 16 + (lane & 15);
-        b[j] = BKC ? bs[r * BKP + kr] : bs[kr * BN + r];
-      }
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = MF<T>::mma(a[i], b[j], acc[i][j]);
-    }
-  };
-
-  if constexpr (ST == 2) {
-    load(0);
-    store(0);
-    __syncthreads();
-    for (int kt = 0; kt < ksteps; ++kt) {
-      const int cur = kt & 1;
-      load(kt + 1);
-      compute(cur);
-      store(cur ^ 1);
-      __syncthreads();
-    }
-  } else {
-    load(0);
-    for (int kt = 0; kt < ksteps; ++kt) {
-      store(0);
-      __syncthreads();
-      load(kt + 1);
-      compute(0);
-      __syncthreads();
-    }
-  }
-}
-
-// --------------------------------------------------------- solid harmonics
-// Racah-normalised real solid harmonics up to L and their gradients, by the
-// reference's recursion in l (m = 1 is z-like, then (2m, 2m+1) pairs, top
-// pair by the (x, y) rotation); gradients by differentiating the recursion.
-template <int L, typename R>
-__device__ __forceinline__ void sh_eval(R x, R y, R z, R *C, R *Cx, R *Cy, R *Cz) {
-  const R r2 = x * x + y * y + z * z;
-  C[0] = R(1);
-  Cx[0] = Cy[0] = Cz[0] = R(0);
-  if constexpr (L >= 1) {
-    C[1] = z; C[2] = x; C[3] = y;
-    Cx[1] = R(0); Cy[1] = R(0); Cz[1] = R(1);
-    Cx[2] = R(1); Cy[2] = R(0); Cz[2] = R(0);
-    Cx[3] = R(0); Cy[3] = R(1); Cz[3] = R(0);
-  }
-  const R dr2x = R(2) * x, dr2y = R(2) * y, dr2z = R(2) * z;
-#pragma unroll
-  for (int l = 2; l <= L; ++l) {
-    const int o = l * l, o1 = (l - 1) * (l - 1), o2 = (l - 2) * (l - 2);
-    const R lr = l, l1r = l - 1, ll1r = 2 * l - 1;
-    C[o] = (ll1r * z * C[o1] - l1r * r2 * C[o2]) / lr;
-    Cx[o] = (ll1r * z * Cx[o1] - l1r * (dr2x * C[o2] + r2 * Cx[o2])) / lr;
-    Cy[o] = (ll1r * z * Cy[o1] - l1r * (dr2y * C[o2] + r2 * Cy[o2])) / lr;
-    Cz[o] = (ll1r * (C[o1] + z * Cz[o1]) - l1r * (dr2z * C[o2] + r2 * Cz[o2])) / lr;
-#pragma unroll
-    for (int im = 1; im <= l - 2; ++im) {
-      const R sim = (R)(im * im);
-      const R rlm = R(1) / sqrt(lr * lr - sim);
-      const R rl1m = sqrt(l1r * l1r - sim);
-      const R a = ll1r * z * rlm, b = rl1m * r2 * rlm;
-      const R daz = ll1r * rlm, db = rl1m * rlm;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int m = 2 * im + k - 1;
-        C[o + m] = a * C[o1 + m] - b * C[o2 + m];
-        Cx[o + m] = a * Cx[o1 + m] - b * Cx[o2 + m] - db * dr2x * C[o2 + m];
-        Cy[o + m] = a * Cy[o1 + m] - b * Cy[o2 + m] - db * dr2y * C[o2 + m];
-        Cz[o + m] = a * Cz[o1 + m] + daz * C[o1 + m] - b * Cz[o2 + m] - db * dr2z * C[o2 + m];
-      }
-    }
-    {
-      const R sim = (R)((l - 1) * (l - 1));
-      const R rlm = R(1) / sqrt(lr * lr - sim);
-      const R a = ll1r * z * rlm, daz = ll1r * rlm;
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const int m = 2 * l - 3 + k;
-        C[o + m] = a * C[o1 + m];
-        Cx[o + m] = a * Cx[o1 + m];
-        Cy[o + m] = a * Cy[o1 + m];
-        Cz[o + m] = a * Cz[o1 + m] + daz * C[o1 + m];
-      }
-    }
-    {
-      const R rll = sqrt(ll1r / (R(2) * lr));
-      const int i2 = o1 + 2 * l - 3, i1 = o1 + 2 * l - 2;
-      C[o + 2 * l - 1] = (x * C[i2] - y * C[i1]) * rll;
-      C[o + 2 * l] = (y * C[i2] + x * C[i1]) * rll;
-      Cx[o + 2 * l - 1] = (C[i2] + x * Cx[i2] - y * Cx[i1]) * rll;
-      Cy[o + 2 * l - 1] = (x * Cy[i2] - C[i1] - y * Cy[i1]) * rll;
-      Cz[o + 2 * l - 1] = (x * Cz[i2] - y * Cz[i1]) * rll;
-      Cx[o + 2 * l] = (y * Cx[i2] + C[i1] + x * Cx[i1]) * rll;
-      Cy[o + 2 * l] = (C[i2] + y * Cy[i2] + x * Cy[i1]) * rll;
-      Cz[o + 2 * l] = (y * Cz[i2] + x * Cz[i1]) * rll;
-    }
-  }
-}
-
-// ------------------------------------------------------------------- basis
-// Evaluation in the output precision T: FP64 for the plain build, FP32 for
-// the mixed builds (whose low-precision error is proportional to ||dP||).
-// Value and gradient of function m of a shell of angular momentum L at one
-// point (r0, r1: the contracted radial factor and its derivative factor);
-// every consumer of basis values forms them with this one expression.
-template <int L, bool GRAD, typename T>
-__device__ __forceinline__ void fn_values(int m, T r0, T r1, T x, T y, T z, const T *C,
-                                          const T *Cx, const T *Cy, const T *Cz, T &v, T &gx,
-                                          T &gy, T &gz) {
-  constexpr int o = L * L;
-  const T sv = C[o + m];
-  v = sv * r0;
-  if (GRAD) {
-    const T hv = sv * r1;
-    gx = x * hv + Cx[o + m] * r0;
-    gy = y * hv + Cy[o + m] * r0;
-    gz = z * hv + Cz[o + m] * r0;
-  }
-}
-
-// Emitter of the basis stage: stores a shell's values (and gradients, when
-// wg) at point p of the [4][NP][Mc] planes.  Global (not flat) stores: a flat
-// store also counts against the LDS wait counter, so every wait for the
-// staged shell data would wait for the stores issued before it.
-template <typename T>
-struct StorePhi {
-  T *phi;
-  long Mc, cs;
-  int p;
-  template <int L, bool GRAD>
-  __device__ __forceinline__ void emit(long f0, int nf, T r0, T r1, T x, T y, T z, const T *C,
-                                       const T *Cx, const T *Cy, const T *Cz, bool wg) const {
-#pragma unroll
-    for (int m = 0; m < 2 * L + 1; ++m) {
-      const long q = (f0 + (long)m * nf) * Mc + p;
-      T v, gx = T(0), gy = T(0), gz = T(0);
-      fn_values<L, false>(m, r0, r1, x, y, z, C, Cx, Cy, Cz, v, gx, gy, gz);
-      gst(phi + q, v);
-      if (GRAD && wg) {
-        fn_values<L, true>(m, r0, r1, x, y, z, C, Cx, Cy, Cz, v, gx, gy, gz);
-        gst(phi + cs + q, gx);
-        gst(phi + 2 * cs + q, gy);
-        gst(phi + 3 * cs + q, gz);
-      }
-    }
-  }
-};
-
-// A range of atoms' basis data staged in LDS for a basis item: the shells,
-// their exponents, norms and contraction coefficients in the evaluation
-// precision, per atom its centre, shell range (relative to the range's
-// first shell) and largest l, and per (shell, 32-point group of the item)
-// what to write: bit 0 the values, bit 1 the gradients.
-template <typename T>
-struct RangeLds {
-  ShellD sh[kRangeShells];
-  T ex[kRangePrims], nm[kRangePrims], ct[kRangeContr];
-  double ax[kRangeAtoms], ay[kRangeAtoms], az[kRangeAtoms];
-  int s0[kRangeAtoms], s1[kRangeAtoms], lm[kRangeAtoms];
-  uint8_t fl[kRangeShells][kThreads / kGroup];
-};
-
-// ex, nm: the shell's primitives; ct: its n_exp x n_contr coefficients.
-// Primitives go in blocks of kPB: the block's exponents, norms and
-// coefficients are read from LDS together (one wait, not one per read), its
-// radial factors formed without a branch per primitive (a block whose
-// primitives are all cut off on the wave's points skips the exponentials),
-// then added into the contractions in primitive order.
-constexpr int kPB = 4;
-template <int L, bool GRAD, typename T, class Put>
-__device__ __forceinline__ void shell_emit(const ShellD &sh, const T *ex, const T *nm, const T *ct,
-                                           T x, T y, T z, T r2, const T *C, const T *Cx,
-                                           const T *Cy, const T *Cz, const Put &put, bool wg) {
-  const int ne = sh.n_exp, nu = sh.n_unc, nc = sh.n_contr, nf = nu + nc;
-  T rc0[kMaxContr], rc1[kMaxContr];
-#pragma unroll
-  for (int k = 0; k < kMaxContr; ++k) rc0[k] = rc1[k] = T(0);
-  for (int e0 = 0; e0 < ne; e0 += kPB) {
-    T al[kPB], ar2[kPB], nv[kPB], r0[kPB], r1[kPB];
-    bool any = false;
-#pragma unroll
-    for (int i = 0; i < kPB; ++i) {
-      const int e = min(e0 + i, ne - 1);  // past the shell: a repeat, never used
-      al[i] = ex[e];
-      nv[i] = nm[e];
-      ar2[i] = al[i] * r2;
-      any = any || (e0 + i < ne && ar2[i] < T(50));
-    }
-    if (__ballot(any)) {
-#pragma unroll
-      for (int i = 0; i < kPB; ++i) {
-        const T v = nv[i] * exp(-ar2[i]);
-        r0[i] = (e0 + i < ne && ar2[i] < T(50)) ? v : T(0);  // primitive cut-off of radial1()
-        r1[i] = (T(-2) * al[i]) * r0[i];
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < kPB; ++i) r0[i] = r1[i] = T(0);
-    }
-#pragma unroll
-    for (int i = 0; i < kPB; ++i)
-      if (e0 + i < nu)
-        put.template emit<L, GRAD>(sh.func_off + e0 + i, nf, r0[i], r1[i], x, y, z, C, Cx, Cy, Cz, wg);
-#pragma unroll
-    for (int k = 0; k < kMaxContr; ++k)
-      if (k < nc) {
-        T c[kPB];
-#pragma unroll
-        for (int i = 0; i < kPB; ++i) c[i] = ct[k * ne + min(e0 + i, ne - 1)];
-#pragma unroll
-        for (int i = 0; i < kPB; ++i)
-          if (e0 + i < ne) {
-            rc0[k] += r0[i] * c[i];
-            rc1[k] += r1[i] * c[i];
-          }
-      }
-  }
-#pragma unroll
-  for (int k = 0; k < kMaxContr; ++k)
-    if (k < nc)
-      put.template emit<L, GRAD>(sh.func_off + nu + k, nf, rc0[k], rc1[k], x, y, z, C, Cx, Cy, Cz, wg);
-}
-
-// One atom's shells sb .. se-1 of the LDS image A at one point (e0, c0: the
-// range's first primitive and coefficient); grp: the point's group in the
-// item.
-template <int LA, bool GRAD, bool ALLG = false, typename T, class Put>
-__device__ __forceinline__ void basis_atom(const RangeLds<T> &A, int sb, int se, int e0, int c0,
-                                           T x, T y, T z, const Put &put, int grp) {
-  constexpr int NLM = (LA + 1) * (LA + 1);
-  T C[NLM], Cx[NLM], Cy[NLM], Cz[NLM];
-  sh_eval<LA, T>(x, y, z, C, Cx, Cy, Cz);
-  const T r2 = x * x + y * y + z * z;
-  for (int s = sb; s < se; ++s) {
-    const int f = A.fl[s][grp];
-    if (!(f & 1)) continue;  // no stage reads the shell's values on this group
-    const bool wg = GRAD && (ALLG || (f & 2));  // ALLG: gradients wherever values are formed
-    // every lane reads the same shell: its fields are uniform over the wave,
-    // so the loops over its primitives and functions run on scalar counters
-    ShellD sh = A.sh[s];
-    sh.l = __builtin_amdgcn_readfirstlane(sh.l);
-    sh.n_exp = __builtin_amdgcn_readfirstlane(sh.n_exp);
-    sh.n_unc = __builtin_amdgcn_readfirstlane(sh.n_unc);
-    sh.n_contr = __builtin_amdgcn_readfirstlane(sh.n_contr);
-    sh.exp_off = __builtin_amdgcn_readfirstlane(sh.exp_off);
-    sh.contr_off = __builtin_amdgcn_readfirstlane(sh.contr_off);
-    sh.func_off = __builtin_amdgcn_readfirstlane(sh.func_off);
-    const T *ex = A.ex + (sh.exp_off - e0), *nm = A.nm + (sh.exp_off - e0);
-    const T *ct = A.ct + (sh.contr_off - c0);
-    switch (sh.l) {
-      case 0: shell_emit<0, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put, wg); break;
-      case 1: if constexpr (LA >= 1) shell_emit<1, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put, wg); break;
-      case 2: if constexpr (LA >= 2) shell_emit<2, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put, wg); break;
-      case 3: if constexpr (LA >= 3) shell_emit<3, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put, wg); break;
-      case 4: if constexpr (LA >= 4) shell_emit<4, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put, wg); break;
-    }
-  }
-}
 
 // -------------------------------------------------------------- functional
 // Closed-shell terms; each returns F, dF/drho, dF/dgamma added into (f, fr, fg).
@@ -624,94 +173,6 @@ __device__ __forceinline__ long item_at(const int *__restrict__ order, long L, l
 // on no global load.  Screened units (bscreen) walk their list of the
 // (block, range) pairs whose values a later stage reads, and write only the
 // shells read on each point's group; dense units write every shell.
-// A basis item staged: its first point, the range's first primitive and
-// coefficient, its atom count, and the point's coordinates.
-struct BasisItem {
-  long p;
-  int e0, c0, n_atoms;
-  double gx, gy, gz;
-};
-
-// Stages basis item `local` of unit U in A (every thread calls it; starts
-// and ends with a barrier).
-template <bool GRAD, typename T>
-__device__ __forceinline__ BasisItem stage_basis_item(const UnitD &U, long local, RangeLds<T> &A) {
-  const int tid = threadIdx.x;
-  long blk;
-  int rng;
-  if (U.bscreen) {
-    const uint32_t e = U.bitems[local];
-    blk = e >> 16;
-    rng = (int)(e & 0xffffu);
-  } else {
-    rng = (int)(local % U.n_ranges);
-    blk = local / U.n_ranges;
-  }
-  const RangeD R = U.ranges[rng];
-  BasisItem it;
-  it.e0 = R.exp_begin;
-  it.c0 = R.contr_begin;
-  it.n_atoms = R.n_atoms;
-  it.p = blk * kThreads + tid;
-  // the point's coordinates in FP64, loads in flight across the staging
-  it.gx = gld(U.gx + it.p);
-  it.gy = gld(U.gy + it.p);
-  it.gz = gld(U.gz + it.p);
-  __syncthreads();  // the previous item's reads of A are done
-  for (int i = tid; i < R.n_shells; i += kThreads) A.sh[i] = U.shells[R.shell_begin + i];
-  for (int i = tid; i < R.n_exp; i += kThreads) {
-    A.ex[i] = (T)gld(U.exps + it.e0 + i);
-    A.nm[i] = (T)gld(U.norms + it.e0 + i);
-  }
-  for (int i = tid; i < R.n_contr; i += kThreads) A.ct[i] = (T)gld(U.contr + it.c0 + i);
-  if (tid < R.n_atoms) {
-    const AtomD at = U.atoms[gld(U.ratoms + R.atom_begin + tid)];
-    A.ax[tid] = at.x;
-    A.ay[tid] = at.y;
-    A.az[tid] = at.z;
-    A.s0[tid] = at.shell_begin - R.shell_begin;
-    A.s1[tid] = at.shell_end - R.shell_begin;
-    A.lm[tid] = at.lmax;
-  }
-  if (tid < R.n_shells * (kThreads / kGroup)) {  // flag of (shell tid / 8, group tid % 8)
-    uint32_t f = GRAD ? 3u : 1u;
-    if (U.bscreen) {
-      const uint32_t *fw = U.bflags + 16 * local;
-      f = ((fw[tid >> 5] >> (tid & 31)) & 1u) |
-          (GRAD ? ((fw[8 + (tid >> 5)] >> (tid & 31)) & 1u) << 1 : 0u);
-    }
-    A.fl[tid / (kThreads / kGroup)][tid % (kThreads / kGroup)] = (uint8_t)f;
-  }
-  __syncthreads();
-  return it;
-}
-
-// The staged range's atoms in turn at the thread's point, each shell written
-// on the point's group handed to put (ALLG: with its gradients wherever its
-// values are).
-template <bool GRAD, bool ALLG, int LMAX, typename T, class Put>
-__device__ __forceinline__ void eval_basis_item(const RangeLds<T> &A, const BasisItem &it,
-                                                const Put &put) {
-  const int grp = threadIdx.x / kGroup;
-  const int na = __builtin_amdgcn_readfirstlane(it.n_atoms);
-  for (int a = 0; a < na; ++a) {
-    const int sb = __builtin_amdgcn_readfirstlane(A.s0[a]), se = __builtin_amdgcn_readfirstlane(A.s1[a]);
-    bool any = false;
-    for (int s = sb; s < se; ++s) any = any || (A.fl[s][grp] & 1);
-    if (!any) continue;  // no stage reads this atom's values on the point's group
-    const T x = (T)(it.gx - A.ax[a]), y = (T)(it.gy - A.ay[a]), z = (T)(it.gz - A.az[a]);
-    // the kernel holds the registers of its largest case, so it is built
-    // for the largest angular momentum of the list (every atom's lmax <= LMAX)
-    switch (__builtin_amdgcn_readfirstlane(A.lm[a])) {
-      case 0: basis_atom<0, GRAD, ALLG>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 1: if constexpr (LMAX >= 1) basis_atom<1, GRAD, ALLG>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 2: if constexpr (LMAX >= 2) basis_atom<2, GRAD, ALLG>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 3: if constexpr (LMAX >= 3) basis_atom<3, GRAD, ALLG>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      default: if constexpr (LMAX >= 4) basis_atom<4, GRAD, ALLG>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-    }
-  }
-}
-
 template <bool GRAD, typename T, int LMAX>
 __global__ __launch_bounds__(kThreads) void k_basis(const UnitD *__restrict__ units, int nu,
                                                     const long *__restrict__ base,
@@ -721,9 +182,9 @@ __global__ __launch_bounds__(kThreads) void k_basis(const UnitD *__restrict__ un
     const long item = item_at(order, L, total);
     const int u = find_unit(base, nu, item);
     const UnitD &U = units[u];
-    const BasisItem it = stage_basis_item<GRAD>(U, item - base[u], A);
+    const BasisItem it = stage_basis_item(U, item - base[u], A);
     const StorePhi<T> put{(T *)U.phi, U.Mc, (long)U.NP * U.Mc, (int)it.p};
-    eval_basis_item<GRAD, false, LMAX>(A, it, put);
+    eval_basis_item<GRAD, LMAX>(A, it, put);
   }
 }
 
@@ -739,7 +200,7 @@ struct StoreWSplit {
   template <int L, bool GRAD>
   __device__ __forceinline__ void emit(long f0, int nf, float r0, float r1, float x, float y,
                                        float z, const float *C, const float *Cx, const float *Cy,
-                                       const float *Cz, bool) const {
+                                       const float *Cz) const {
 #pragma unroll
     for (int m = 0; m < 2 * L + 1; ++m) {
       const long q = (f0 + (long)m * nf) * Mc + p;
@@ -775,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void k_wbasis(const UnitD *__restrict__ u
     const long item = item_at(order, L, total);
     const int u = find_unit(base, nu, item);
     const UnitD &U = units[u];
-    const BasisItem it = stage_basis_item<GRAD>(U, item - base[u], A);
+    const BasisItem it = stage_basis_item(U, item - base[u], A);
     const long Mc = U.Mc, cs = (long)U.NP * Mc;
     StoreWSplit<NS> put;
     put.Mc = Mc;
@@ -791,12 +252,9 @@ __global__ __launch_bounds__(kThreads) void k_wbasis(const UnitD *__restrict__ u
       put.b1[sp] = GRAD ? gld(cf + 2 * Mc + it.p) : 0.0;
       put.b2[sp] = GRAD ? gld(cf + 3 * Mc + it.p) : 0.0;
     }
-    eval_basis_item<GRAD, true, LMAX>(A, it, put);
+    eval_basis_item<GRAD, LMAX>(A, it, put);
   }
 }
-
-// ----------------------------------------------------------------- density
-constexpr int kDBM = 128;
 
 // item = 256-point block of a unit
 template <bool GGA>
@@ -1514,96 +972,6 @@ void launch_basis(hipStream_t s, bool grad, const StageList &L) {
     case 2: basis_l<T, 2>(s, grad, L); break;
     case 3: basis_l<T, 3>(s, grad, L); break;
     default: basis_l<T, 4>(s, grad, L); break;
-  }
-}
-
-// ---------------------------------------------------- gradient products
-// The products of the nuclear gradient, X = Phi P and Y_c = (d/dc Phi) P
-// (P the density matrix of the last build), over the density contraction's
-// items: 128-point tile x pair of chunks of the tile's functions, K over the
-// tile's runs, the same GEMM with P for D.  Written to XY[plane][f][p] for
-// the tile's functions f only: the gradient's per-point terms take X_f, Y_f
-// where phi_f is not cut off.  nplanes: 1 (X, LDA) or 4.  Units u with
-// u % nspin == spin only (a plan lists a molecule's spins as consecutive
-// units; their items are the same tiles).
-template <int BN, int VAR>
-__global__ __launch_bounds__(kThreads) void k_xy(const StageList S, const double *__restrict__ P,
-                                                 double *__restrict__ XY, int nplanes, int nspin,
-                                                 int spin) {
-  typedef double T;
-  constexpr int BM = kDBM, BK = Var<VAR>::BK, ST = Var<VAR>::ST, TM = BM / 32, TN = BN / 32;
-  __shared__ T As[lds_elems<T, BM, BK, ST, false>()];
-  __shared__ __attribute__((aligned(16))) T Bs[lds_elems<T, BN, BK, ST, true>()];
-  __shared__ uint16_t kl[kMaxRuns];
-  __shared__ uint16_t cl[2 * BN];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, wm = wave >> 1, wn = wave & 1;
-  for (long L = blockIdx.x; L < S.total; L += gridDim.x) {
-    const long it = item_at(S.order, L, S.total);
-    const int u = find_unit(S.base, S.nu, it);
-    if (u % nspin != spin) continue;  // uniform over the workgroup
-    const UnitD &U = S.units[u];
-    const uint32_t e = U.ditems[it - S.base[u]];
-    const int tile = (int)(e >> 8), pair = (int)(e & 255);
-    const long m0 = (long)tile * BM, Mc = U.Mc, NP = U.NP, cs = NP * Mc;
-    const int off = U.tl_off[tile], c8 = U.tl_off[tile + 1] - off;
-    const int foff = U.tf_off[tile] + 2 * pair * BN, nf = U.tf_off[tile + 1] - foff;
-    __syncthreads();  // the previous item's readers of kl and cl are done
-    for (int i = threadIdx.x; i < min(2 * BN, nf); i += kThreads) cl[i] = gld(U.tfl + foff + i);
-    lds_list(U.tl + off, c8, kl);
-    const int ksteps = (c8 * kRun + BK - 1) / BK;
-    const T *phi = (const T *)U.phi;
-    for (int h = 0; h < 2 && h * BN < nf; ++h) {
-      const uint16_t *cfn = cl + h * BN;
-      const int ncol = min(BN, nf - h * BN);
-      auto baddr = [&](int n, int kt, int kk) -> long {
-        const long f = run_fn(kl, c8, kt * BK + kk);
-        return (f < 0 || n >= ncol) ? -1 : (long)cfn[min(n, ncol - 1)] * NP + f;
-      };
-      for (int c = 0; c < nplanes; ++c) {
-        auto aaddr = [&](int m, int kt, int kk) -> long {
-          const long f = run_fn(kl, c8, kt * BK + kk);
-          return f < 0 ? -1 : c * cs + f * Mc + m;
-        };
-        typename MF<T>::acc acc[TM][TN];
-        gemm_tile<T, BM, BN, BK, ST, false, true>(phi + m0, P, ksteps, aaddr, baddr, As, Bs, acc);
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          const int n = wn * (BN / 2) + j * 16 + mf_col(lane);
-          if (n >= ncol) continue;
-          double *xy = XY + c * cs + (long)cfn[n] * Mc + m0;
-#pragma unroll
-          for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) gst(xy + wm * (BM / 2) + i * 16 + MF<T>::row(lane, r), acc[i][j][r]);
-        }
-      }
-    }
-  }
-}
-
-template <int BN>
-static void xy_bn(hipStream_t s, int var, const StageList &L, const double *P, double *XY, int np,
-                  int ns, int sp) {
-  dim3 g(persistent_grid(L.total, 2));
-  switch (var) {
-    case 1: hipLaunchKernelGGL((k_xy<BN, 1>), g, dim3(kThreads), 0, s, L, P, XY, np, ns, sp); break;
-    case 2: hipLaunchKernelGGL((k_xy<BN, 2>), g, dim3(kThreads), 0, s, L, P, XY, np, ns, sp); break;
-    default: hipLaunchKernelGGL((k_xy<BN, 0>), g, dim3(kThreads), 0, s, L, P, XY, np, ns, sp); break;
-  }
-}
-
-void launch_xy(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XY,
-               int nplanes, int nspin, int spin) {
-  if (!L.total) return;
-  StageList W = L;  // a plain static walk (no queues, no schedule order, no log)
-  W.ctr = nullptr;
-  W.qbeg = nullptr;
-  W.order = nullptr;
-  W.tlog = nullptr;
-  switch (tf) {
-    case 64: xy_bn<64>(s, var, W, P, XY, nplanes, nspin, spin); break;
-    case 96: xy_bn<96>(s, var, W, P, XY, nplanes, nspin, spin); break;
-    default: xy_bn<128>(s, var, W, P, XY, nplanes, nspin, spin); break;
   }
 }
 

@@ -45,3 +45,30 @@ def test_equidistant_centres():
     own = np.arange(8, dtype=np.int32)
     w = becke_weights(xyz, np.zeros((8, 3)), own, np.full(8, 3.0))
     assert np.max(np.abs(w - 3.0 / 8)) < 1e-15
+
+
+@pytest.mark.parametrize("na", [1, 2, 9, 40])
+@pytest.mark.parametrize("spins", [1, 2])
+def test_moving_grid_gradient_against_fixed_grid_sums(na, spins):
+    """The moving-grid gradient where the Becke derivatives keep every centre,
+    a few and a small part of them: it is invariant under translation of the
+    molecule with its grid, exactly, and one centre alone has none at all."""
+    from pgxc import XCBuilder, basis
+    els, xyz = systems.random_molecule(na, seed=21) if na > 1 else (["O"], np.zeros((1, 3)))
+    b = basis.seeded_basis(els, xyz, seed=22, shell_set="small")
+    g = grid.molecular_grid(els, xyz, nrad=8, nang=194)
+    own = grid.owners(els, 8, 194)
+    rng = np.random.default_rng(na)
+    n = max(2, b.nbas // 5)
+    C = [np.linalg.qr(rng.normal(size=(b.nbas, n)))[0] for _ in range(spins)]
+    with XCBuilder(b, g, chunk_points=4096) as xc:
+        if spins == 1:
+            xc.set_orbitals(C[0], np.ones(n))
+        else:
+            xc.set_orbitals(np.stack(C, axis=2), np.ones((n, 2)))
+        xc.build("PBE", "fp64", fetch=False)
+        f, again = xc.gradient_grid(own), xc.gradient_grid(own)
+    assert np.array_equal(f, again)
+    # the sum over atoms cancels terms of the size of the per-point sums (about
+    # npts of order 1 to 10 each) to FP64 rounding
+    assert np.max(np.abs(f.sum(axis=0))) < 1e-16 * 10 * len(own)
