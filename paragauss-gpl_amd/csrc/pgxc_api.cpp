@@ -70,10 +70,12 @@ struct pgxc_ctx {
   std::string err;
   // sizes
   int n_atoms = 0, n_shells = 0, nbas = 0, NP = 0, veclen = 128, tf = 128;
+  int pt = 0;  // chunk of the potential contraction: the tile asked for, else setup_screen's choice
   int lmax = 0;  // largest angular momentum of the basis
   int var[2] = {0, 1};  // contraction variant for FP64 and for FP32 builds
   long npts = 0, npad = 0, Mc = 0;
-  int nchunks = 0, nsplit = 1, ntiles = 0;  // nsplit: the chunk rounding's blocks (pgxc_layout)
+  int icols = 128;  // most columns of a density item (setup_screen)
+  int nchunks = 0, nsplit = 1, nparts = 0;  // nsplit: the chunk rounding's blocks (pgxc_layout)
   int nsp = 1;  // point splits of the potential contraction per chunk (setup_screen)
   long nblk_total = 0;
   // device: geometry and basis
@@ -139,7 +141,7 @@ struct pgxc_ctx {
   double last_terms[5] = {0, 0, 0, 0, 0};
   double exps_per_point = 0;
   // screening and work tables over the padded grid (setup_screen)
-  int screen = 0, n8 = 0, nw8 = 0, CH = 0;
+  int screen = 0, n8 = 0, nw8 = 0;
   int *nbt = nullptr;
   uint32_t *sig8 = nullptr;
   ScreenShell *sshells = nullptr;
@@ -209,6 +211,16 @@ int dalloc(pgxc_ctx *c, T **p, size_t count) {
   }
   return PGXC_OK;
 }
+
+// potential partials held at a time per molecule and spin, and work items of
+// their sum below which it is cut into segments
+constexpr long kPartialBytes = 4L << 30, kFoldItems = 1536;
+// items that all run at once (two workgroups a CU): walked without queues, whose
+// claims a launch of one item per workgroup waits for and gains nothing from
+// (water, mixed step: density 54 -> 15 us, potential 34 -> 13)
+constexpr long kResident = 512;
+constexpr double kWideTile = 384.0;    // setup_screen: mean functions of a tile for wide density items
+constexpr double kSplitItems = 256.0;  // setup_screen: potential items a chunk has at least
 
 const uint32_t kSupported = PGXC_XC_PBE;
 const int kTiles[3] = {64, 96, 128};
@@ -320,14 +332,14 @@ long unit_items(const UnitD &U, ItemKind k, int tf) {
 // kdense: the dense K length.
 static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int precision,
                                std::vector<double> &feat, std::vector<double> &flops) {
-  const int tf = c->tf;
+  const int tf = c->pt;
   const int var = precision == PGXC_PREC_FP64 ? c->var[0] : precision == PGXC_PREC_FP32 ? c->var[1] : 0;
   auto push = [&](int kd, double kact, double kdense, bool active, double fl) {
     const double f[PGXC_NFEATURES] = {(double)kd,
                                       precision == PGXC_PREC_FP64 ? 1.0 : 0.0,
                                       precision == PGXC_PREC_FP32 ? 1.0 : 0.0,
                                       precision == PGXC_PREC_BF16X3 ? 1.0 : 0.0,
-                                      tf / 128.0,
+                                      c->tf / 128.0,
                                       std::log2(1.0 + kact) / 16.0,
                                       std::log2(1.0 + kdense) / 16.0,
                                       active ? 1.0 : 0.0,
@@ -342,7 +354,9 @@ static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int p
       const long T = T0 + (e >> 8);
       const int pr = (int)(e & 255), c8 = c->h_tl_off[(size_t)T + 1] - c->h_tl_off[(size_t)T];
       const int nf = c->h_tf_off[(size_t)T + 1] - c->h_tf_off[(size_t)T];
-      const double cols = (double)std::min(2 * tf, nf - 2 * pr * tf);
+      const int cc = (int)round_up(nf, 16) / 16, ni = (nf + c->icols - 1) / c->icols;
+      const int share = 16 * ((cc + ni - 1) / ni);
+      const double cols = (double)std::min(share, nf - pr * share);
       push(0, (double)c8 * kRun, c->NP, true, 2.0 * kScreenTile * cols * c8 * kRun);
     }
   } else {
@@ -452,7 +466,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       P.frow = plan->feat.size() / PGXC_NFEATURES;
       for (int m : um) unit_item_features(mols[m], step, kind, precision, plan->feat, flops);
     }
-    if (contr && queues && P.total > 0) {
+    if (contr && queues && P.total > kResident) {
       P.has_queues = true;  // queue bounds filled in once every cost is known
     } else {
       std::vector<double> pr;
@@ -496,7 +510,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.phi = (char *)c->phi_base + (c->phi_stride ? (size_t)k * c->phi_stride : (size_t)lane * c->phi_lane);
       U.W = (char *)c->W + (size_t)lane * c->w_lane;
       U.D = c->D;
-      U.part = c->part + (size_t)lane * c->ntiles * 4 * c->Mc;
+      U.part = c->part + (size_t)lane * c->nparts * 4 * c->Mc;
       U.coef = c->coef + (size_t)lane * 4 * c->Mc;
       U.state = c->state + p0;
       U.epart = c->epart + 2 * (p0 / kThreads);
@@ -509,11 +523,11 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.npad = c->npad;
       U.n_atoms = c->n_atoms;
       U.NP = c->NP;
-      U.ntiles = c->ntiles;
       U.nsplit = c->nsp;
       U.incremental = incr[m];
       U.mask = functional;
-      U.CH = c->CH;
+      U.icols = c->icols;
+      U.dcols = precision == PGXC_PREC_BF16X3 ? c->icols : kPartCols;
       U.ditems = c->di + c->h_di_off[k];
       U.pitems = c->pi + c->h_pi_off[k];
       U.ndi = c->h_di_off[k + 1] - c->h_di_off[k];
@@ -535,7 +549,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
         UnitD B = U;
         B.W = (char *)c->beta.W + (size_t)lane * c->w_lane;
         B.D = c->beta.D;
-        B.part = c->beta.part + (size_t)lane * c->ntiles * 4 * c->Mc;
+        B.part = c->beta.part + (size_t)lane * c->nparts * 4 * c->Mc;
         B.coef = c->beta.coef + (size_t)lane * 4 * c->Mc;
         B.state = c->beta.state + p0;
         B.Hc = c->beta.Hc + hslot * c->hstride;
@@ -595,6 +609,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       for (int m : wm) pend[k].back().lmax = std::max(pend[k].back().lmax, mols[m]->lmax);
     }
     const int cls = precision == PGXC_PREC_FP64 ? 0 : 1;
+    const bool x3 = precision == PGXC_PREC_BF16X3;
     for (int kind = 0; kind < 2; ++kind)
       for (int li = 0; li < kLists; ++li) {
         const int t = li / kNumVariants, v = li % kNumVariants;
@@ -602,7 +617,9 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
         std::vector<int> subm;
         for (size_t i = 0; i < units.size(); ++i) {
           const pgxc_ctx *c = mols[umol[i]];
-          if (c->tf == kTiles[t] && c->var[cls] == v) {
+          const bool mine = kind == 0 && x3 ? li == (c->icols == 128 ? 0 : 1)  // split-BF16: by item width
+                                            : (kind == 0 ? c->tf : c->pt) == kTiles[t] && c->var[cls] == v;
+          if (mine) {
             sub.push_back(units[i]);
             subm.push_back(umol[i]);
           }
@@ -869,9 +886,8 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
                         const Plan &pl, bool gga, std::vector<hipEvent_t> *ev) {
   const bool x3 = pl.precision == PGXC_PREC_BF16X3;
   const bool two = pl.nlanes > 1 && pl.steps.size() > 1;
-  if (pl.nctr) launch_zero_ints(s, pl.d_ctr, pl.nctr);
   launch_prep(s, pl.d_pack, pl.nmol, pl.d_prep_base, pl.prep_total,
-              x3 ? 2 : std::is_same<T, double>::value ? 0 : 1, false);
+              x3 ? 2 : std::is_same<T, double>::value ? 0 : 1, pl.d_ctr, (int)pl.nctr);
   if (two) {
     (void)hipEventRecord(fork, s);
     (void)hipStreamWaitEvent(s2, fork, 0);
@@ -884,14 +900,14 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
     launch_basis<T>(t, gga, S.basis);
     if (E) (void)hipEventRecord(E[1], t);
     for (int li = 0; li < kLists; ++li) {
-      const int tf = kTiles[li / kNumVariants], v = li % kNumVariants;
+      const int v = li % kNumVariants;
       if constexpr (std::is_same<T, float>::value) {
         if (x3) {
-          launch_density_bf16x3(t, gga, tf, S.dens[li]);
+          launch_density_bf16x3(t, gga, li == 0 ? 128 : 256, S.dens[li]);
           continue;
         }
       }
-      launch_density<T>(t, gga, tf, v, S.dens[li]);
+      launch_density<T>(t, gga, v, S.dens[li]);
     }
     if (E) (void)hipEventRecord(E[2], t);
     if (pl.energy) {
@@ -929,8 +945,7 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
   if (pl.energy) return;
   if (ev) (void)hipEventRecord((*ev)[kEvPack], s);
   launch_fold(s, pl.fold.d, pl.fold.n, pl.fold.base, pl.fold.total);
-  launch_pack(s, pl.d_pack, pl.nmol, pl.d_pack_base, pl.pack_total);
-  launch_prep(s, pl.d_pack, pl.nmol, pl.d_prep_base, pl.prep_total, 0, true);
+  launch_pack(s, pl.d_pack, pl.nmol, pl.d_pack_base, pl.pack_total, pl.d_prep_base, pl.prep_total);
   if (ev) (void)hipEventRecord((*ev)[kEvEnd], s);
 }
 
@@ -1196,11 +1211,6 @@ static int upload(pgxc_ctx *c, V **dst, const std::vector<V> &src) {
   return PGXC_OK;
 }
 
-// potential partials held at a time per molecule and spin, and work items of
-// their sum below which it is cut into segments
-constexpr long kPartialBytes = 4L << 30, kFoldItems = 1536;
-constexpr double kSplitItems = 256.0;  // setup_screen: potential items a chunk has at least
-
 static int alloc_partials(pgxc_ctx *c, double **Hc, double **HS) {
   int rc = dalloc(c, Hc, (size_t)c->hslots * c->hstride);
   if (rc) return rc;
@@ -1212,7 +1222,6 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
   const double n = (double)c->nbas;
   c->flops_dense = 4.0 * c->npts * n * n + 16.0 * c->npts * n;
   c->n8 = c->NP / kRun;
-  c->CH = c->tf / kRun;
   c->screen = on;
   c->nw8 = (c->n8 + 31) / 32;
   const int n8 = c->n8, nw8 = c->nw8;
@@ -1313,7 +1322,14 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
   {
     long spts = kSplitPts;
     const double nt = (double)c->h_tfl.size() / (double)std::max<long>(1, (c->npts + kScreenTile - 1) / kScreenTile);
-    const double nch = std::ceil(1.1 * nt / c->tf);
+    // chunks of 96 functions, or of 64 or 128 where one holds a split's functions
+    // (1.3 times a tile's): split-BF16 stage at 64 / 96 / 128, one lane, (H2O)16
+    // 0.71 / 0.60 / 0.65 ms, (H2O)32 2.40 / 1.90 / 2.41, (H2O)128 and solute 127 /
+    // 89 / 90; FP64 23-atom molecule at 96 / 128 0.30 / 0.15 ms
+    if (!c->pt) c->pt = 1.3 * nt <= 64.0 ? 64 : 1.3 * nt <= 128.0 ? 128 : 96;
+    const double nch = std::ceil(1.1 * nt / c->pt);
+    // density items of 128 columns while a tile has few functions, else 256
+    c->icols = nt > kWideTile ? 256 : 128;
     while (spts > kMinSplitPts && (double)(c->Mc / spts) * nch * nch < kSplitItems &&
            (double)(c->npad / spts) * 4.0 * c->NP <= 268435456.0)  // the places: 256 MiB
       spts /= 2;
@@ -1411,14 +1427,13 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
     for (long t = 0; t < tpc; ++t) {
       const long T = k * tpc + t;
       const int nf = c->h_tf_off[(size_t)T + 1] - c->h_tf_off[(size_t)T];
-      // density items: pairs of column chunks (tf functions) of the tile's functions
-      for (int pr = 0; pr < (nf + 2 * c->tf - 1) / (2 * c->tf); ++pr)
-        c->h_di.push_back((uint32_t)(t << 8 | pr));
+      // density items: shares of at most icols of the tile's functions
+      for (int pr = 0; pr < (nf + c->icols - 1) / c->icols; ++pr) c->h_di.push_back((uint32_t)(t << 8 | pr));
     }
     c->h_di_off.push_back((long)c->h_di.size());
     for (int sl = 0; sl < c->nsp; ++sl) {
       const long S = (long)k * c->nsp + sl;
-      const int nu = c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S], nch = (nu + c->tf - 1) / c->tf;
+      const int nu = c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S], nch = (nu + c->pt - 1) / c->pt;
       for (int ci = 0; ci < nch; ++ci)
         for (int cj = 0; cj < nch; ++cj)
           c->h_pi.push_back((uint32_t)sl << 20 | (uint32_t)ci << 10 | (uint32_t)cj);
@@ -1559,7 +1574,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   function_order(sh, exps, atom_xyz, n_atoms, c->fpos);
   // function tile: requested, or the one of 128 / 96 / 64 that pads nbas least
   if (opt && opt->tile) {
-    c->tf = opt->tile;
+    c->tf = c->pt = opt->tile;
     c->NP = (int)round_up(c->nbas, c->tf);
   } else {
     c->tf = 128;
@@ -1570,7 +1585,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
         c->tf = t;
       }
   }
-  c->ntiles = c->NP / c->tf;
+  c->nparts = (c->NP + kPartCols - 1) / kPartCols;  // density partials of a point at most
 
   // ---- chunking of the grid ----------------------------------------------
   // a chunk holds at most 256 Ki points and 8 GiB of FP64 basis values; a
@@ -1687,7 +1702,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   if ((rc = dalloc(c, &c->epart, 2 * (size_t)c->nblk_total))) return rc;
   if ((rc = dalloc(c, &c->eterm, 5 * (size_t)c->nblk_total))) return rc;
   const size_t L = (size_t)c->nlanes_cap;
-  if ((rc = dalloc(c, &c->part, L * c->ntiles * 4 * c->Mc))) return rc;
+  if ((rc = dalloc(c, &c->part, L * c->nparts * 4 * c->Mc))) return rc;
   if ((rc = dalloc(c, &c->coef, L * 4 * c->Mc))) return rc;
   // a slot for every chunk where they fit kPartialBytes, else as many per lane
   // as do (summed whenever they are full); sums in enough segments of the splits
@@ -1700,7 +1715,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   const long ns = (long)c->nchunks * c->nsp;
   c->nseg = (int)std::min<long>({std::max<long>(kFoldItems / pairs, (ns + 63) / 64), (ns + 3) / 4, 32L});
   if ((rc = alloc_partials(c, &c->Hc, &c->HS))) return rc;
-  HIPCHK(c, hipMemset(c->part, 0, L * c->ntiles * 4 * c->Mc * 8));
+  HIPCHK(c, hipMemset(c->part, 0, L * c->nparts * 4 * c->Mc * 8));
   HIPCHK(c, hipMemset(c->coef, 0, L * 4 * c->Mc * 8));
   return PGXC_OK;
 }
@@ -1737,13 +1752,13 @@ static int alloc_beta(pgxc_ctx *c) {
   if ((rc = dalloc(c, &B.P, np2)) || (rc = dalloc(c, &B.Pref, np2))) return rc;
   HIPCHK(c, hipMalloc(&B.D, np2 * 8));
   if ((rc = dalloc(c, &B.state, (size_t)S_NSLOT * c->npad)) || (rc = dalloc(c, &B.Vstate, npk)) ||
-      (rc = dalloc(c, &B.Vout, npk)) || (rc = dalloc(c, &B.part, L * c->ntiles * 4 * c->Mc)) ||
+      (rc = dalloc(c, &B.Vout, npk)) || (rc = dalloc(c, &B.part, L * c->nparts * 4 * c->Mc)) ||
       (rc = dalloc(c, &B.coef, L * 4 * c->Mc)) || (rc = alloc_partials(c, &B.Hc, &B.HS)))
     return rc;
   HIPCHK(c, hipMemset(B.P, 0, np2 * 8));
   HIPCHK(c, hipMemset(B.Pref, 0, np2 * 8));
   HIPCHK(c, hipMemset(B.state, 0, (size_t)S_NSLOT * c->npad * 8));
-  HIPCHK(c, hipMemset(B.part, 0, L * c->ntiles * 4 * c->Mc * 8));
+  HIPCHK(c, hipMemset(B.part, 0, L * c->nparts * 4 * c->Mc * 8));
   HIPCHK(c, hipMemset(B.coef, 0, L * 4 * c->Mc * 8));
   return PGXC_OK;
 }
@@ -1969,7 +1984,7 @@ static int gradient_impl(pgxc_ctx *c, double *pm) {
     for (int sp = 0; sp < c->ispin; ++sp) {
       // X = Phi P, Z = W P with P of the last build (P_ref)
       for (int li = 0; li < kLists; ++li)
-        launch_xz(s, kTiles[li / kNumVariants], li % kNumVariants, S.dens[li], sp ? c->beta.Pref : c->Pref,
+        launch_xz(s, li % kNumVariants, S.dens[li], sp ? c->beta.Pref : c->Pref,
                   c->gXZ, gga ? 2 : 1, c->ispin, sp);
       launch_bracket(s, gga, c->lmax, unit, Mc, c->n_ranges, c->gXZ,
                      (sp ? c->beta.state : c->state) + p0, np, pm ? pm + p0 : nullptr, c->gpart, c->gsum);

@@ -61,7 +61,7 @@ struct UnitD {
   void *phi;        // [4][NP][Mc] values, d/dx, d/dy, d/dz (T)
   void *W;          // [NP][Mc] (T); split-BF16 builds: bf16 hi / lo planes [2][NP][Mc]
   const void *D;    // [NP][NP] density operand (T); split-BF16: transposed hi / lo planes
-  double *part;     // [NP/tf][4][Mc] density partials
+  double *part;     // [shares of the columns][4][Mc] density partials
   double *coef;     // [4][Mc] potential coefficients a, b
   double *state;    // [S_NSLOT][npad] molecule state, offset to the unit's first point
   double *epart;    // [Mc/256][2] block sums of w f and w rho (offset to the unit)
@@ -76,12 +76,12 @@ struct UnitD {
   const long *ho;   // its functions x its functions (padded to blocks of 16)
   // Work of the contractions, over gathered runs of 8 functions and gathered
   // functions (all of them when screening is off).  ditems / pitems: the
-  // unit's density items (tile << 8 | pair of column chunks) and potential
+  // unit's density items (tile << 8 | share of its columns) and potential
   // items (split << 20 | row chunk << 10 | column chunk).  tl_off / tl: per
   // 128-point tile of the unit, its ascending run list, the density's K
   // (tl_off offset to the unit's first tile, values index tl); tf_off / tfl:
   // the same for its functions (those of the shells not cut off on the
-  // tile), the density's output columns in chunks of tile functions.
+  // tile), the density's output columns.
   // su_off / su: per point split of the unit, the union of its tiles'
   // functions, the potential's rows and columns in chunks of tile functions.
   const uint32_t *ditems, *pitems;
@@ -104,9 +104,9 @@ struct UnitD {
   const uint32_t *bitems, *bflags;
   long nbi;
   long Mc, npad;
-  int n_atoms, n_ranges, NP, ntiles, nsplit, incremental, pad_n;
+  int n_atoms, n_ranges, NP, nsplit, incremental, pad_n;
   uint32_t mask;
-  int CH, pad_c;
+  int icols, dcols;  // most columns of a density item, and of a partial: kPartCols or (split-BF16) icols
   long ndi, npi;  // density / potential items of the unit
 };
 
@@ -170,7 +170,7 @@ void launch_wbasis(hipStream_t s, bool grad, bool two, const StageList &L);
 // var = contraction variant: 0 (K step 16, 2 LDS stages), 1 (32, 1), 2 (32, 2)
 constexpr int kNumVariants = 3;
 template <typename T>
-void launch_density(hipStream_t s, bool grad, int tf, int var, const StageList &L);
+void launch_density(hipStream_t s, bool grad, int var, const StageList &L);
 void launch_functional(hipStream_t s, bool gga, const StageList &L);
 void launch_functional_spin(hipStream_t s, bool gga, const StageList &L);
 // energy terms only (no coefficients, state untouched); spin: open-shell units
@@ -181,19 +181,20 @@ template <typename T>
 void launch_wmat(hipStream_t s, bool grad, bool split, bool two, const StageList &L);
 template <typename T>
 void launch_potential(hipStream_t s, int tf, int var, const StageList &L);
-void launch_density_bf16x3(hipStream_t s, bool grad, int tf, const StageList &L);
+void launch_density_bf16x3(hipStream_t s, bool grad, int icols, const StageList &L);
 void launch_potential_bf16x3(hipStream_t s, int tf, const StageList &L);
 void launch_fold(hipStream_t s, const FoldD *folds, int n, const long *base, long total);
-void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total);
-void launch_zero_ints(hipStream_t s, int *p, long n);
+void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total,
+                 const long *prep_base, long prep_total);
 unsigned contraction_grid(const StageList &L, int per_cu);
 
 // cost model internals used by the planner (cost_model.hip)
 long costmodel_version(const pgxc_costmodel *m);
 int costmodel_features(const pgxc_costmodel *m);
-// mode of the density operand: 0 FP64, 1 FP32, 2 split-BF16 planes of D^T
+// mode of the density operand: 0 FP64, 1 FP32, 2 split-BF16 planes of D^T; also
+// clears the nctr queue counters of the plan
 void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, long total,
-                 int mode, bool finish);
+                 int mode, int *ctr, int nctr);
 
 // item counts per unit, shared by the planner and the kernels' decoding
 inline long items_functional(long Mc) { return Mc / kThreads; }
@@ -215,6 +216,10 @@ constexpr int kMinSplitPts = 256;
 constexpr int kGroup = 32;
 constexpr int kRun = 8;
 constexpr int kScreenTile = 128;       // point tile of the density contraction
+// A density item takes at most 128 or 256 of its tile's functions as columns (a
+// context's choice, UnitD::icols); the FP64/FP32 kernels form them in chunks of
+// kPartCols, a partial each.
+constexpr int kPartCols = 64;
 constexpr int kMaxRuns = 1024;         // runs of 8 functions per molecule (NP <= 8192)
 constexpr int kMaxShells = 8192;       // shells per molecule
 constexpr double kCutoff = 50.0 * (1.0 + 1.0e-6);  // margin: a superset in every precision
@@ -235,7 +240,7 @@ void launch_form_density(hipStream_t s, const double *C, const double *occ, int 
 // Nuclear gradient.  launch_xz: X = Phi P (plane 0) and, for nplanes = 2, Z = W P
 // (plane 1) into XZ[plane][f][p] over a density list's items (tile x function
 // chunks), for the tiles' functions only; units u with u % nspin == spin.
-void launch_xz(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XZ,
+void launch_xz(hipStream_t s, int var, const StageList &L, const double *P, double *XZ,
                int nplanes, int nspin, int spin);
 // coef = 2 a, b from the per-point state; the W pass over it forms Z's operand
 void launch_bracket_coef(hipStream_t s, long Mc, const double *st, long np, double *coef);

@@ -146,14 +146,6 @@ struct DensTile {
   }
 };
 
-// Column chunks of a tile of nf functions, BN at most per chunk: as many chunks
-// as BN needs, their 16-column blocks shared out evenly (a chunk of few columns
-// would stage every point of the tile for little work).
-__device__ __forceinline__ int chunk_cols(int nf, int BN) {
-  const int nch = (nf + BN - 1) / BN, nb = (nf + 15) / 16;
-  return 16 * ((nb + nch - 1) / nch);
-}
-
 // Sums of a wave's 32 points over a chunk's columns: part[0] = sum_n Phi X,
 // part[c] = 2 sum_n d_c Phi X.  A lane holds four consecutive points of one
 // column per block: 16-byte loads; the 16 lanes of a block's columns are summed
@@ -197,7 +189,7 @@ __device__ __forceinline__ void density_sums(typename MF<T>::acc (&acc)[2][NB],
     }
 }
 
-// item = (128-point tile, pair of column chunks of its functions).  Bound by
+// item = (128-point tile, share of its functions as columns).  Bound by
 // the matrix cores and, about equally, the sums' reads of Phi and d Phi (32
 // bytes per point and function, 14 GB at (H2O)32 in FP64).  The kernel before
 // walked whole runs of 8 functions and 96-column chunks (1.4 times the MFMAs)
@@ -215,15 +207,15 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const Stag
     const int u = unit_of(S.base, S.nu, it);
     const UnitD &U = S.units[u];
     const uint32_t e = U.ditems[it - S.base[u]];
-    const int tile = (int)(e >> 8), pair = (int)(e & 255);
+    const int tile = (int)(e >> 8), item = (int)(e & 255);
     const long m0 = (long)tile * kDBM, Mc = U.Mc, NP = U.NP;
     const int off = U.tf_off[tile], nf = U.tf_off[tile + 1] - off;
     const uint16_t *fl = U.tfl + off;
-    const int cc = chunk_cols(nf, BN), nch = (nf + BN - 1) / BN;
+    const int cc = share_cols(nf, BN), per = U.icols / BN, ch1 = min((item + 1) * per, (nf + BN - 1) / BN);
     const T *phi = (const T *)U.phi + m0, *D = (const T *)U.D;
     int ahead = 0;
-    for (int ch = 2 * pair; ch < min(2 * pair + 2, nch); ++ch) {
-      const bool last = ch + 1 == min(2 * pair + 2, nch);
+    for (int ch = item * per; ch < ch1; ++ch) {
+      const bool last = ch + 1 == ch1;
       const uint16_t *cf = fl + ch * cc;
       const int ncol = min(cc, nf - ch * cc);
       auto go = [&](auto nb) {
@@ -234,13 +226,11 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const Stag
         if (last) ahead = walk_ahead(S);
         density_sums<T, NB, GRAD>(acc, phi, Mc, NP * Mc, cf, ncol, U.part + (long)ch * 4 * Mc + m0);
       };
-      // built for 2 blocks and from half a chunk up (a tile of more than one
-      // chunk has no fewer in any but its last)
       const int nb = (ncol + 15) / 16;
-      if (nb <= 2) go(std::integral_constant<int, 2>{});
-      else if (BN == 96 ? nb <= 4 : nb <= BN / 32 + 1) go(std::integral_constant<int, (BN == 96 ? 4 : BN / 32 + 1)>{});
-      else if (BN > 64 && nb <= BN / 16 - 1) go(std::integral_constant<int, (BN > 64 ? BN / 16 - 1 : 4)>{});
-      else go(std::integral_constant<int, BN / 16>{});
+      if (nb <= 1) go(std::integral_constant<int, 1>{});
+      else if (nb == 2) go(std::integral_constant<int, 2>{});
+      else if (nb == 3) go(std::integral_constant<int, 3>{});
+      else go(std::integral_constant<int, 4>{});
     }
     item_log(S, it, t0);
     L = walk_take(S, L, ahead, &slot);
@@ -264,13 +254,13 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_xz(const StageList
     if (u % nspin != spin) continue;  // uniform over the workgroup
     const UnitD &U = S.units[u];
     const uint32_t e = U.ditems[it - S.base[u]];
-    const int tile = (int)(e >> 8), pair = (int)(e & 255);
+    const int tile = (int)(e >> 8), item = (int)(e & 255);
     const long m0 = (long)tile * kDBM, Mc = U.Mc, NP = U.NP;
     const int off = U.tf_off[tile], nf = U.tf_off[tile + 1] - off;
     const uint16_t *fl = U.tfl + off;
-    const int cc = chunk_cols(nf, BN), nch = (nf + BN - 1) / BN;
+    const int cc = share_cols(nf, BN), per = U.icols / BN, ch1 = min((item + 1) * per, (nf + BN - 1) / BN);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    for (int ch = 2 * pair; ch < min(2 * pair + 2, nch); ++ch) {
+    for (int ch = item * per; ch < ch1; ++ch) {
       const uint16_t *cf = fl + ch * cc;
       const int ncol = min(cc, nf - ch * cc);
       for (int pl = 0; pl < nplanes; ++pl) {
@@ -294,59 +284,41 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_xz(const StageList
           }
         };
         const int nb = (ncol + 15) / 16;
-        if (nb <= BN / 32) go(std::integral_constant<int, BN / 32>{});
-        else go(std::integral_constant<int, BN / 16>{});
+        if (nb <= 2) go(std::integral_constant<int, 2>{});
+        else if (nb == 3) go(std::integral_constant<int, 3>{});
+        else go(std::integral_constant<int, 4>{});
       }
     }
   }
 }
 
-template <int BN>
-static void xz_bn(hipStream_t s, int var, const StageList &L, const double *P, double *XZ, int np,
-                  int ns, int sp) {
+inline void launch_xz_impl(hipStream_t s, int var, const StageList &L, const double *P, double *XZ, int np,
+                           int ns, int sp) {
+  if (!L.total) return;
   dim3 g((unsigned)std::min<long>(L.total, 512));
   switch (var) {
-    case 1: hipLaunchKernelGGL((k_xz<BN, 1>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
-    case 2: hipLaunchKernelGGL((k_xz<BN, 2>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
-    default: hipLaunchKernelGGL((k_xz<BN, 0>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+    case 1: hipLaunchKernelGGL((k_xz<kPartCols, 1>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+    case 2: hipLaunchKernelGGL((k_xz<kPartCols, 2>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
+    default: hipLaunchKernelGGL((k_xz<kPartCols, 0>), g, dim3(kThreads), 0, s, L, P, XZ, np, ns, sp); break;
   }
-}
-
-inline void launch_xz_impl(hipStream_t s, int tf, int var, const StageList &L, const double *P, double *XZ,
-                           int nplanes, int nspin, int spin) {
-  if (!L.total) return;
-  switch (tf) {
-    case 64: xz_bn<64>(s, var, L, P, XZ, nplanes, nspin, spin); break;
-    case 96: xz_bn<96>(s, var, L, P, XZ, nplanes, nspin, spin); break;
-    default: xz_bn<128>(s, var, L, P, XZ, nplanes, nspin, spin); break;
-  }
-}
-
-template <typename T, int BN, int VAR>
-static void density_bn(hipStream_t s, bool grad, const StageList &L) {
-  dim3 g(contraction_grid(L, 2));
-  if (grad)
-    hipLaunchKernelGGL((k_density<T, BN, VAR, true>), g, dim3(kThreads), 0, s, L);
-  else
-    hipLaunchKernelGGL((k_density<T, BN, VAR, false>), g, dim3(kThreads), 0, s, L);
 }
 
 template <typename T, int VAR>
-static void density_var(hipStream_t s, bool grad, int tf, const StageList &L) {
-  switch (tf) {
-    case 64: density_bn<T, 64, VAR>(s, grad, L); break;
-    case 96: density_bn<T, 96, VAR>(s, grad, L); break;
-    default: density_bn<T, 128, VAR>(s, grad, L); break;
-  }
+static void density_var(hipStream_t s, bool grad, const StageList &L) {
+  dim3 g(contraction_grid(L, 2));
+  if (grad)
+    hipLaunchKernelGGL((k_density<T, kPartCols, VAR, true>), g, dim3(kThreads), 0, s, L);
+  else
+    hipLaunchKernelGGL((k_density<T, kPartCols, VAR, false>), g, dim3(kThreads), 0, s, L);
 }
 
 template <typename T>
-void launch_density(hipStream_t s, bool grad, int tf, int var, const StageList &L) {
+void launch_density(hipStream_t s, bool grad, int var, const StageList &L) {
   if (!L.total) return;
   switch (var) {
-    case 1: density_var<T, 1>(s, grad, tf, L); break;
-    case 2: density_var<T, 2>(s, grad, tf, L); break;
-    default: density_var<T, 0>(s, grad, tf, L); break;
+    case 1: density_var<T, 1>(s, grad, L); break;
+    case 2: density_var<T, 2>(s, grad, L); break;
+    default: density_var<T, 0>(s, grad, L); break;
   }
 }
 

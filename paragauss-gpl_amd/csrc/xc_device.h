@@ -28,15 +28,23 @@ __device__ __forceinline__ int xcd_remap(int bid, int nblk) {
   return (bid & 7) * per + (bid >> 3);
 }
 
-// A position of a queued list (thread 0 only) from the queues after the
-// workgroup's own (blockIdx.x % kQueues), from `first` on; total when all are
-// drained.
+// A position of a queued list (the first wave calls it) from the queues after
+// the workgroup's own (blockIdx.x % kQueues), from `first` on; total when all
+// are drained.  The lanes look at all counters at once, so a workgroup at the
+// end of the launch waits for one load, not for a claim on every queue in turn.
 __device__ __forceinline__ long walk_claim_queue(const StageList &S, int first) {
-  const int q = (int)(blockIdx.x % kQueues);
-  for (int t = first; t < kQueues; ++t) {
-    const int qq = (q + t) % kQueues;
-    const long c = S.qbeg[qq] + (long)atomicAdd(S.ctr + qq, 1);
-    if (c < S.qbeg[qq + 1]) return c;
+  const int lane = threadIdx.x & 63, t = lane & (kQueues - 1);
+  const int qq = (int)((blockIdx.x + t) % kQueues);
+  const long beg = S.qbeg[qq], end = S.qbeg[qq + 1];
+  const long seen = __hip_atomic_load(S.ctr + qq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned long long open = __ballot(lane < kQueues && lane >= first && beg + seen < end);
+  while (open) {
+    const int u = __builtin_ctzll(open);
+    open &= open - 1;
+    int c = 0;
+    if (lane == u) c = atomicAdd(S.ctr + qq, 1);
+    const long p = S.qbeg[(blockIdx.x + u) % kQueues] + __builtin_amdgcn_readlane(c, u);
+    if (p < S.qbeg[(blockIdx.x + u) % kQueues + 1]) return p;
   }
   return S.total;
 }
@@ -47,7 +55,14 @@ __device__ __forceinline__ long walk_claim_queue(const StageList &S, int first) 
 // of the workgroup calls it.
 __device__ __forceinline__ long walk_next(const StageList &S, long prev, long *slot) {
   if (!S.ctr) return prev < 0 ? (long)blockIdx.x : prev + (long)gridDim.x;
-  if (threadIdx.x == 0) *slot = walk_claim_queue(S, 0);
+  if (threadIdx.x < 64) {
+    const int q = (int)(blockIdx.x % kQueues);
+    int raw = 0;
+    if (threadIdx.x == 0) raw = atomicAdd(S.ctr + q, 1);
+    long p = S.qbeg[q] + (long)__builtin_amdgcn_readfirstlane(raw);
+    if (p >= S.qbeg[q + 1]) p = walk_claim_queue(S, 1);
+    if (threadIdx.x == 0) *slot = p;
+  }
   __syncthreads();
   const long p = *slot;
   __syncthreads();
@@ -70,10 +85,11 @@ __device__ __forceinline__ long walk_take(const StageList &S, long cur, int raw,
   // the claim's value is first read here: an empty asm that takes it keeps
   // the compiler from converting it (and so waiting for it) where it arrives
   asm volatile("" : "+v"(raw));
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     const int q = (int)(blockIdx.x % kQueues);
-    const long p = S.qbeg[q] + (long)raw;
-    *slot = p < S.qbeg[q + 1] ? p : walk_claim_queue(S, 1);
+    long p = S.qbeg[q] + (long)__builtin_amdgcn_readfirstlane(raw);
+    if (p >= S.qbeg[q + 1]) p = walk_claim_queue(S, 1);
+    if (threadIdx.x == 0) *slot = p;
   }
   __syncthreads();
   return *slot;
@@ -222,94 +238,11 @@ __device__ __forceinline__ double group_reduce(double (&v)[M], int lane, int &in
   return v[0];
 }
 
-// Epilogue of X = Phi D for one point tile x gathered column chunk:
-// contributions rho += sum_n Phi(p,n) X(p,n), grad rho += 2 sum_n dPhi(p,n)
-// X(p,n), summed over the chunk's columns in a fixed order (j, then the
-// 16-lane group reduction) and written to part[ch][c][p].  Column n of the
-// chunk is function cfn[n] for n < ncol (absent columns add nothing).  With
-// the FP32 result placement a lane holds four consecutive points of one
-// column, read as one 16-byte load per component.  A lane's columns are looked up once; the loads of IB row
-// blocks (IB divides the wave's row blocks) are issued together and
-// unconditionally (an absent column reads function 0 and adds nothing), so
-// their latencies overlap instead of following one another.  Waves as in
-// gemm_tile_bf16x3 (NT threads, WGN wave columns); every two wave columns
-// make one partial slot: slot ch + s sums wave columns 2s and 2s + 1, and
-// the first nslots slots are written.
-template <typename T, typename ACC, int BM, int BN, bool GRAD, int IB = 1, int NT = kThreads,
-          int WGN = 2>
-__device__ __forceinline__ void density_epilogue(
-    const ACC (&acc)[BM / (NT / 64 / WGN) / 16][BN / WGN / 16], const T *__restrict__ phi,
-    long Mc, int NP, long m0, const uint16_t *cfn, int ncol, int ch, double *__restrict__ part,
-    double (&red)[WGN][4][BM], int nslots = 1) {
-  constexpr int WGM = NT / 64 / WGN, WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
-  constexpr int NC = GRAD ? 4 : 1, SLOTS = WGN / 2;
-  static_assert(MF<T>::kQuadRows, "a lane's results are four consecutive points");
-  static_assert(TM % IB == 0 && WGN % 2 == 0, "whole rounds of row blocks, wave column pairs");
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WGN, wn = wave % WGN;
-  const long cs = (long)NP * Mc;
-  long col[TN];
-  bool live[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) {
-    const int e = wn * WN + j * 16 + mf_col(lane);
-    live[j] = e < ncol;
-    col[j] = live[j] ? (long)cfn[min(e, ncol - 1)] * Mc : 0;
-  }
-#pragma unroll
-  for (int i0 = 0; i0 < TM; i0 += IB) {
-    T v[IB][TN][NC][4];
-#pragma unroll
-    for (int ii = 0; ii < IB; ++ii)
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        const long q0 = col[j] + m0 + wm * WM + (i0 + ii) * 16;
-        const long q = q0 + MF<T>::row(lane, 0);
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          const f4 t = gld((const f4 *)(phi + c * cs + q));
-          v[ii][j][c][0] = t.x; v[ii][j][c][1] = t.y; v[ii][j][c][2] = t.z; v[ii][j][c][3] = t.w;
-        }
-      }
-#pragma unroll
-    for (int ii = 0; ii < IB; ++ii) {
-      const int i = i0 + ii;
-      double s[NC][4];
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[c][r] = 0.0;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-        if (!live[j]) continue;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const double xv = (double)acc[i][j][r];
-          s[0][r] += (double)v[ii][j][0][r] * xv;
-#pragma unroll
-          for (int c = 1; c < NC; ++c) s[c][r] += 2.0 * (double)v[ii][j][c][r] * xv;
-        }
-      }
-      double w[NC * 4];
-#pragma unroll
-      for (int c = 0; c < NC; ++c)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) w[c * 4 + r] = s[c][r];
-      int idx;
-      const double tot = group_reduce<NC * 4>(w, lane, idx);
-      if (NC == 4 || (lane & 3) == 0) {
-        const int c = idx / 4, r = idx % 4;
-        red[wn][c][wm * WM + i * 16 + MF<T>::row(lane, r)] = tot;
-      }
-    }
-  }
-  __syncthreads();
-  for (int idx = tid; idx < SLOTS * NC * BM; idx += NT) {
-    const int sl = idx / (NC * BM), c = (idx / BM) % NC, row = idx % BM;
-    if (sl < nslots)
-      gst(part + ((long)(ch + sl) * 4 + c) * Mc + m0 + row,
-          red[2 * sl][c][row] + red[2 * sl + 1][c][row]);
-  }
+// Columns of a share of a tile's nf functions: as many shares as `most` needs,
+// their 16-column blocks dealt out evenly.
+__device__ __forceinline__ int share_cols(int nf, int most) {
+  const int n = (nf + most - 1) / most, nb = (nf + 15) / 16;
+  return 16 * ((nb + n - 1) / n);
 }
 
 // Functions of a split, padded to whole 16-function blocks: the leading

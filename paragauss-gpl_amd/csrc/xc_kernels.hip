@@ -275,7 +275,7 @@ __global__ __launch_bounds__(kThreads) void k_functional(const UnitD *__restrict
     double rho = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
     // partial sums of the density items of this point's tile, one per chunk
     const int tile = (int)(p / kScreenTile);
-    const int tf = U.CH * kRun, nch = (U.tf_off[tile + 1] - U.tf_off[tile] + tf - 1) / tf;
+    const int nch = (U.tf_off[tile + 1] - U.tf_off[tile] + U.dcols - 1) / U.dcols;
     for (int t = 0; t < nch; ++t) {
       rho += part[((long)t * 4 + 0) * Mc + p];
       if (GGA) {
@@ -515,7 +515,7 @@ __global__ __launch_bounds__(kThreads) void k_functional_spin(const UnitD *__res
     double *coef[2] = {U.coef, U.coef2};
     double rho[2], g[2][3];
     const int tile = (int)(p / kScreenTile);
-    const int tf = U.CH * kRun, nch = (U.tf_off[tile + 1] - U.tf_off[tile] + tf - 1) / tf;
+    const int nch = (U.tf_off[tile + 1] - U.tf_off[tile] + U.dcols - 1) / U.dcols;
     for (int sp = 0; sp < 2; ++sp) {
       double r = 0.0, g0 = 0.0, g1 = 0.0, g2 = 0.0;
       for (int t = 0; t < nch; ++t) {
@@ -632,7 +632,7 @@ __global__ __launch_bounds__(kThreads) void k_energy(const UnitD *__restrict__ u
     const long blk = it - base[u];
     const long p = blk * kThreads + tid, Mc = U.Mc;
     const int tile = (int)(p / kScreenTile);
-    const int tf = U.CH * kRun, nch = (U.tf_off[tile + 1] - U.tf_off[tile] + tf - 1) / tf;
+    const int nch = (U.tf_off[tile + 1] - U.tf_off[tile] + U.dcols - 1) / U.dcols;
     double rho[2] = {0.0, 0.0}, g[2][3] = {{0.0, 0.0, 0.0}, {0.0, 0.0, 0.0}};
     for (int sp = 0; sp < (SPIN ? 2 : 1); ++sp) {
       const double *part = sp ? U.part2 : U.part;
@@ -866,11 +866,21 @@ __global__ __launch_bounds__(kThreads) void k_fold(const FoldD *__restrict__ fol
 
 // item = 256 packed elements of one molecule (caller's function order):
 // V = base + S at the functions' internal rows (S folded above, symmetric,
-// read from its lower tiles, summed over its segments); then the molecule's state for the next
-// incremental build: V_state = V.
+// read from its lower tiles, summed over its segments); then the molecule's
+// state for the next incremental build: V_state = V.  Items from total on: 256
+// elements of P_ref = P (the density operand's list), in the same launch.
 __global__ __launch_bounds__(kThreads) void k_pack(const PackD *__restrict__ mols, int nm,
-                                                   const long *__restrict__ base, long total) {
-  for (long L = blockIdx.x; L < total; L += gridDim.x) {
+                                                   const long *__restrict__ base, long total,
+                                                   const long *__restrict__ prep_base,
+                                                   long prep_total) {
+  for (long L = blockIdx.x; L < total + prep_total; L += gridDim.x) {
+    if (L >= total) {
+      const int m = find_unit(prep_base, nm, L - total);
+      const PackD &M = mols[m];
+      const long i = (L - total - prep_base[m]) * kThreads + threadIdx.x;
+      if (i < M.NP * M.NP) M.Pref[i] = M.P[i];
+      continue;
+    }
     const int m = find_unit(base, nm, L);
     const PackD &M = mols[m];
     const long idx = (L - base[m]) * kThreads + threadIdx.x;
@@ -883,6 +893,7 @@ __global__ __launch_bounds__(kThreads) void k_pack(const PackD *__restrict__ mol
     const long pj = M.fpos[j], pk = M.fpos[k];  // internal rows of caller functions j, k
     const long r = pj > pk ? pj : pk, c = pj > pk ? pk : pj;
     double v = 0.0;
+#pragma unroll 4
     for (int s = 0; s < M.nseg; ++s) v += M.HS[((long)s * NP + r) * NP + c];
     const double out = M.incremental ? M.Vstate[idx] + v : v;
     M.Vout[idx] = out;
@@ -891,30 +902,29 @@ __global__ __launch_bounds__(kThreads) void k_pack(const PackD *__restrict__ mol
 }
 
 // Density operand of one molecule: D = P - P_ref (incremental) or P, in the
-// contraction precision; afterwards P_ref = P.  item = 256 elements.
+// contraction precision.  item = 256 elements.  The first workgroup also clears
+// the plan's queue counters.
 __global__ __launch_bounds__(kThreads) void k_prep(const PackD *__restrict__ mols, int nm,
                                                    const long *__restrict__ base, long total,
-                                                   int mode, int finish) {
+                                                   int mode, int *__restrict__ ctr, int nctr) {
+  if (blockIdx.x == 0)
+    for (int i = threadIdx.x; i < nctr; i += kThreads) ctr[i] = 0;
   for (long L = blockIdx.x; L < total; L += gridDim.x) {
     const int m = find_unit(base, nm, L);
     const PackD &M = mols[m];
     const long i = (L - base[m]) * kThreads + threadIdx.x;
     if (i >= (long)M.NP * M.NP) continue;
-    if (finish) {
-      M.Pref[i] = M.P[i];
+    const double d = M.incremental ? M.P[i] - M.Pref[i] : M.P[i];
+    if (mode == 2) {  // split planes of D^T: element (r, c) goes to (c, r)
+      const long np2 = M.NP * M.NP, r = i / M.NP, c = i % M.NP;
+      __bf16 hi, lo;
+      split_bf16((float)d, hi, lo);
+      ((__bf16 *)M.D)[c * M.NP + r] = hi;
+      ((__bf16 *)M.D)[np2 + c * M.NP + r] = lo;
+    } else if (mode == 1) {
+      ((float *)M.D)[i] = (float)d;
     } else {
-      const double d = M.incremental ? M.P[i] - M.Pref[i] : M.P[i];
-      if (mode == 2) {  // split planes of D^T: element (r, c) goes to (c, r)
-        const long np2 = M.NP * M.NP, r = i / M.NP, c = i % M.NP;
-        __bf16 hi, lo;
-        split_bf16((float)d, hi, lo);
-        ((__bf16 *)M.D)[c * M.NP + r] = hi;
-        ((__bf16 *)M.D)[np2 + c * M.NP + r] = lo;
-      } else if (mode == 1) {
-        ((float *)M.D)[i] = (float)d;
-      } else {
-        ((double *)M.D)[i] = d;
-      }
+      ((double *)M.D)[i] = d;
     }
   }
 }
@@ -1040,32 +1050,23 @@ void launch_wmat(hipStream_t s, bool grad, bool split, bool two, const StageList
 #undef PGXC_WMAT
 }
 
-__global__ __launch_bounds__(kThreads) void k_zero_ints(int *p, long n) {
-  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)gridDim.x * kThreads)
-    p[i] = 0;
-}
-
-void launch_zero_ints(hipStream_t s, int *p, long n) {
-  if (n <= 0) return;
-  hipLaunchKernelGGL(k_zero_ints, dim3(persistent_grid((n + kThreads - 1) / kThreads, 1)),
-                     dim3(kThreads), 0, s, p, n);
-}
-
 void launch_fold(hipStream_t s, const FoldD *folds, int n, const long *base, long total) {
   if (!total) return;
   hipLaunchKernelGGL(k_fold, dim3(persistent_grid(total, 8)), dim3(kThreads), 0, s, folds, n, base, total);
 }
 
-void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total) {
+void launch_pack(hipStream_t s, const PackD *mols, int nm, const long *base, long total,
+                 const long *prep_base, long prep_total) {
   if (!total) return;
-  hipLaunchKernelGGL(k_pack, dim3(persistent_grid(total, 8)), dim3(kThreads), 0, s, mols, nm, base, total);
+  hipLaunchKernelGGL(k_pack, dim3(persistent_grid(total + prep_total, 8)), dim3(kThreads), 0, s, mols, nm, base,
+                     total, prep_base, prep_total);
 }
 
 void launch_prep(hipStream_t s, const PackD *mols, int nm, const long *base, long total,
-                 int mode, bool finish) {
+                 int mode, int *ctr, int nctr) {
   if (!total) return;
   hipLaunchKernelGGL(k_prep, dim3(persistent_grid(total, 8)), dim3(kThreads), 0, s, mols, nm, base,
-                     total, mode, (int)finish);
+                     total, mode, ctr, nctr);
 }
 
 #define PGXC_INST(T)                                                                  \

@@ -1,0 +1,105 @@
+"""The contractions at the edges of their shares, blocks and lists: function
+counts around 16, 64, 96, 128 and 256 columns, point counts that leave part of a
+tile, chunk and split, tiles of many functions (wide split-BF16 items), and
+partials that do not all fit (summed while the build runs)."""
+import numpy as np
+import pytest
+
+import oracle
+from pgxc import XCBuilder, basis, grid, systems
+from pgxc.basis import Basis, Shell
+
+pytestmark = pytest.mark.gpu
+
+
+def _basis(n, rng):
+    """n functions on a line of atoms: s shells of up to 12 functions and, from
+    the second atom on, a p shell where it fits."""
+    shells, xyz, left = [], [], n
+    while left > 0:
+        a = len(xyz)
+        xyz.append((1.9 * a, 0.3 * (a % 3), 0.2 * (a % 2)))
+        k = min(left, 12)
+        shells.append(Shell(a, 0, np.sort(np.exp(rng.uniform(np.log(0.2), np.log(30.0), k))), k, np.zeros((k, 0))))
+        left -= k
+        if a and left >= 3:
+            shells.append(Shell(a, 1, np.array([rng.uniform(0.2, 2.0)]), 1, np.zeros((1, 0))))
+            left -= 3
+    b = Basis(np.array(xyz))
+    b.shells = shells
+    assert b.nbas == n
+    return b
+
+
+def _grid(b, npts, rng):
+    own = rng.integers(0, b.n_atoms, npts)
+    d = rng.normal(size=(npts, 3))
+    r = rng.uniform(0.1, 3.0, npts)
+    pts = b.atom_xyz[own] + r[:, None] * d / np.linalg.norm(d, axis=1)[:, None]
+    return np.asfortranarray(np.column_stack([pts, rng.uniform(0.01, 0.1, npts)]))
+
+
+def _check(got, ref, rel):
+    v = np.max(np.abs(ref[0]))
+    # FP64: sums of some hundred points and functions; the mixed contractions of
+    # a full density carry their operands' rounding (2^-24, 2^-17) into V
+    assert abs(got[1] - ref[1]) <= 1e-9 + rel * abs(ref[1])
+    assert np.max(np.abs(got[0] - ref[0])) <= 1e-10 + 10 * rel * v
+    assert abs(got[2] - ref[2]) <= 1e-9 + rel * abs(ref[2])
+
+
+@pytest.mark.parametrize("n,npts", [(1, 129), (15, 31), (16, 300), (17, 1000), (64, 700), (65, 700),
+                                    (95, 257), (97, 511), (127, 300), (128, 300), (129, 640),
+                                    (193, 300), (257, 385), (420, 300)])
+@pytest.mark.parametrize("spins", [1, 2])
+def test_function_counts(n, npts, spins):
+    rng = np.random.default_rng(1000 * n + spins)
+    b = _basis(n, rng)
+    g = _grid(b, npts, rng)
+    m = max(1, n // 6)
+    C = [np.linalg.qr(rng.normal(size=(n, m)))[0] for _ in range(spins)]
+    P = C[0] @ C[0].T if spins == 1 else np.stack([c @ c.T for c in C], axis=2)
+    ref = {f: oracle.xc_build(b, g, mask, P=P, nthreads=4, ispin=spins)
+           for f, mask in (("PBE", oracle.MASK_PBE), ("LDA", oracle.MASK_LDA))}
+    for screen in (True, False):
+        with XCBuilder(b, g, screen=screen) as xc:
+            xc.set_density(P)
+            for f in ("PBE", "LDA"):
+                for prec, rel in (("fp64", 0.0), ("fp32", 2e-6), ("bf16x3", 5e-5)):
+                    _check(xc.build(f, prec), ref[f], rel)
+
+
+@pytest.mark.parametrize("tile", [64, 96, 128])
+@pytest.mark.parametrize("variant", [0, 1, 2])
+def test_tiles_and_variants(tile, variant):
+    rng = np.random.default_rng(10 * tile + variant)
+    b = _basis(150, rng)
+    g = _grid(b, 5000, rng)
+    C = np.linalg.qr(rng.normal(size=(150, 20)))[0]
+    ref = oracle.xc_build(b, g, oracle.MASK_PBE, C=C, occ=np.ones(20), nthreads=4)
+    with XCBuilder(b, g, tile=tile, variants=(variant, variant), chunk_points=2048) as xc:
+        xc.set_orbitals(C, np.ones(20))
+        for prec, rel in (("fp64", 0.0), ("fp32", 2e-6), ("bf16x3", 5e-5)):
+            _check(xc.build("PBE", prec), ref, rel)
+
+
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_partials_summed_during_the_build(lanes):
+    """Without screening every split holds every function and the partials of
+    all chunks pass 4 GiB, so they are summed as they fill their slots; with
+    screening they fit.  Both are the same sums."""
+    els, xyz = systems.water_cluster(45, seed=3, jitter_a=0.2)
+    b = basis.seeded_basis(els, xyz, seed=12, shell_set="medium")
+    g = grid.molecular_grid(els, xyz, nrad=16, nang=302, partition="gpu")
+    C, occ = systems.random_orbitals(b.nbas, 40, seed=5)
+    out = []
+    for screen in (True, False):
+        with XCBuilder(b, g, screen=screen, chunk_points=4096, basis_cache=False) as xc:
+            xc.set_lanes(lanes)
+            lay = xc.layout()
+            if not screen:
+                assert 8.0 * b.nbas ** 2 * lay["npad"] / 2048 > 4 * 2 ** 30
+            xc.set_orbitals(C, occ)
+            out.append(xc.build("PBE", "fp64"))
+    (h0, e0, q0), (h1, e1, q1) = out
+    assert np.max(np.abs(h0 - h1)) <= 1e-10 and abs(e0 - e1) <= 1e-9 and abs(q0 - q1) <= 1e-9
