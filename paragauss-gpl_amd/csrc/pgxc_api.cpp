@@ -219,6 +219,7 @@ constexpr long kPartialBytes = 4L << 30, kFoldItems = 1536;
 // claims a launch of one item per workgroup waits for and gains nothing from
 // (water, mixed step: density 54 -> 15 us, potential 34 -> 13)
 constexpr long kResident = 512;
+constexpr long kBasisItems = 2048;
 constexpr double kWideTile = 384.0;    // setup_screen: mean functions of a tile for wide density items
 constexpr double kSplitItems = 256.0;  // setup_screen: potential items a chunk has at least
 
@@ -598,7 +599,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     // W: split-BF16 builds evaluate the basis again over the basis items
     // (test switch PGXC_W_READ=1: they read the stored values back instead,
     // the same bits)
-    const bool wb = precision == PGXC_PREC_BF16X3 && !getenv("PGXC_W_READ");
+    const bool wb = !getenv("PGXC_W_READ");
     plan->wbasis = wb ? 1 : 0;
     const ItemKind wkind = wb ? K_WBASIS : K_WMAT;
     {  // closed-shell units; the open-shell ones in wmat2 below
@@ -918,8 +919,8 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
     launch_functional(t, gga, S.func);
     launch_functional_spin(t, gga, S.func2);
     if (pl.wbasis) {
-      launch_wbasis(t, gga, false, S.wmat);
-      launch_wbasis(t, gga, true, S.wmat2);
+      launch_wbasis<T>(t, gga, x3, false, S.wmat);
+      launch_wbasis<T>(t, gga, x3, true, S.wmat2);
     } else {
       launch_wmat<T>(t, gga, x3, false, S.wmat);
       launch_wmat<T>(t, gga, x3, true, S.wmat2);
@@ -1612,8 +1613,10 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
   HIPCHK(c, hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
   HIPCHK(c, hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
-  // atom ranges of the basis stage: consecutive atoms in shell order, as
-  // many as the kernel's LDS image holds
+  // atom ranges of the basis stage: consecutive atoms in shell order, as many
+  // as the kernel's LDS image holds, fewer where a chunk's blocks would give the
+  // device less than kBasisItems items
+  const int ra_most = (int)std::min<long>(kRangeAtoms, std::max<long>(1, n_atoms * (c->Mc / kThreads) / kBasisItems));
   std::vector<int> ratoms;
   for (int a = 0; a < n_atoms; ++a)
     if (at[a].shell_end > at[a].shell_begin) ratoms.push_back(a);
@@ -1623,7 +1626,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   for (size_t i = 0; i < ratoms.size(); ++i) {
     const AtomD &a = at[ratoms[i]];
     const int ns = a.shell_end - a.shell_begin;
-    if (c->h_ranges.empty() || c->h_ranges.back().n_atoms == kRangeAtoms ||
+    if (c->h_ranges.empty() || c->h_ranges.back().n_atoms == ra_most ||
         c->h_ranges.back().n_shells + ns > kRangeShells ||
         c->h_ranges.back().n_exp + a.n_exp > kRangePrims ||
         c->h_ranges.back().n_contr + a.n_contr > kRangeContr) {
@@ -1977,8 +1980,13 @@ static int gradient_impl(pgxc_ctx *c, double *pm) {
       for (int sp = 0; sp < c->ispin; ++sp)
         launch_bracket_coef(s, Mc, (sp ? c->beta.state : c->state) + p0, np,
                             (sp ? c->beta.coef : c->coef) + (size_t)lane * 4 * Mc);
-      launch_wmat<double>(s, true, false, false, S.wmat);
-      launch_wmat<double>(s, true, false, true, S.wmat2);
+      if (gp.wbasis) {
+        launch_wbasis<double>(s, true, false, false, S.wmat);
+        launch_wbasis<double>(s, true, false, true, S.wmat2);
+      } else {
+        launch_wmat<double>(s, true, false, false, S.wmat);
+        launch_wmat<double>(s, true, false, true, S.wmat2);
+      }
     }
     const UnitD *unit = c->ispin == 2 ? S.func2.units : S.func.units;
     for (int sp = 0; sp < c->ispin; ++sp) {
