@@ -182,7 +182,7 @@ struct pgxc_ctx {
   std::vector<long> h_bi_off;
   std::vector<int> fpos;          // internal position of each caller function
   std::vector<double> axyz;       // atom positions (bohr), caller order
-  int *d_fpos = nullptr;
+  int *d_fpos = nullptr, *d_finv = nullptr;  // and its inverse, caller function of each position
   Sched sched;
 };
 
@@ -1687,6 +1687,11 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   }
   if ((rc = dalloc(c, &c->d_fpos, c->nbas))) return rc;
   HIPCHK(c, hipMemcpy(c->d_fpos, c->fpos.data(), sizeof(int) * c->nbas, hipMemcpyHostToDevice));
+  {
+    std::vector<int> finv((size_t)c->nbas);
+    for (int f = 0; f < c->nbas; ++f) finv[(size_t)c->fpos[f]] = f;
+    if ((rc = upload(c, &c->d_finv, finv))) return rc;
+  }
   HIPCHK(c, hipMemcpy(c->exps, exps, 8 * eoff, hipMemcpyHostToDevice));
   HIPCHK(c, hipMemcpy(c->norms, norms, 8 * eoff, hipMemcpyHostToDevice));
   if (coff > 0) HIPCHK(c, hipMemcpy(c->contr, contr, 8 * coff, hipMemcpyHostToDevice));
@@ -1828,25 +1833,18 @@ extern "C" int pgxc_set_orbitals(pgxc_ctx *c, int32_t ispin, int32_t nbas, int32
   const int n = c->nbas;
   double *dC = nullptr, *docc = nullptr;
   ScopedDev tmp;  // dC and docc, freed on every return below
-  for (int sp = 0; sp < ispin; ++sp)
-    HIPCHK(c, hipMemsetAsync(sp ? c->beta.P : c->P, 0, (size_t)c->NP * c->NP * 8, c->stream));
   if (nocc > 0) {
     HIPCHK(c, hipMalloc((void **)&dC, (size_t)ispin * n * nocc * 8));
     tmp.keep(dC);
     HIPCHK(c, hipMalloc((void **)&docc, (size_t)ispin * nocc * 8));
     tmp.keep(docc);
-    std::vector<double> Cp((size_t)ispin * n * nocc);  // rows in the internal function order
-    for (int sp = 0; sp < ispin; ++sp)
-      for (int k = 0; k < nocc; ++k)
-        for (int i = 0; i < n; ++i)
-          Cp[(size_t)c->fpos[i] + ((size_t)sp * nocc + k) * n] = C[(size_t)i + ((size_t)sp * nocc + k) * n];
-    HIPCHK(c, hipMemcpy(dC, Cp.data(), Cp.size() * 8, hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(dC, C, (size_t)ispin * n * nocc * 8, hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(docc, occ, (size_t)ispin * nocc * 8, hipMemcpyHostToDevice));
-    for (int sp = 0; sp < ispin; ++sp)
-      launch_form_density(c->stream, dC + (size_t)sp * n * nocc, docc + (size_t)sp * nocc, n, nocc,
-                          c->NP, sp ? c->beta.P : c->P);
-    HIPCHK(c, hipGetLastError());
   }
+  for (int sp = 0; sp < ispin; ++sp)  // nocc = 0: P = 0
+    launch_form_density(c->stream, dC + (size_t)sp * n * nocc, docc + (size_t)sp * nocc, c->d_finv, n, nocc,
+                        c->NP, sp ? c->beta.P : c->P);
+  HIPCHK(c, hipGetLastError());
   HIPCHK(c, hipStreamSynchronize(c->stream));
   c->have_density = 1;
   c->density_mode = mode;
@@ -2210,7 +2208,7 @@ int pgxc_destroy(pgxc_ctx *c) {
   }
   void *bufs[] = {c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->exps, c->norms, c->contr, c->P, c->Pref,
                   c->D, c->phi, c->W, c->part, c->coef, c->Hc, c->HS, c->state,
-                  c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos,
+                  c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos, c->d_finv,
                   c->phic[0], c->phic[1], c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,
                   c->ho, c->pos, c->rbits, c->di, c->pi, c->bi, c->bfl, c->gXZ, c->gpart, c->gsum, c->gpm, c->gmov, c->perm_d, c->beta.P, c->beta.Pref, c->beta.D,
                   c->beta.W, c->beta.part, c->beta.coef, c->beta.Hc, c->beta.HS, c->beta.state,

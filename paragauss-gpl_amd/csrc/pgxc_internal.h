@@ -233,10 +233,10 @@ void launch_screen(hipStream_t s, long ntiles_pts, const double *gx, const doubl
                    const ScreenShell *shells, int n8, int *nb, uint32_t *sig8,
                    uint32_t *smark);
 
-// P = C diag(occ) C^T into an NP x NP padded array
-void launch_form_density(hipStream_t s, const double *C, const double *occ, int n,
+// P = C diag(occ) C^T into an NP x NP padded array (C in caller order; finv:
+// caller index of each internal function)
+void launch_form_density(hipStream_t s, const double *C, const double *occ, const int *finv, int n,
                          int nocc, int NP, double *P);
-
 
 // Nuclear gradient.  launch_xz: X = Phi P (plane 0) and, for nplanes = 2, Z = W P
 // (plane 1) into XZ[plane][f][p] over a density list's items (tile x function

@@ -103,3 +103,27 @@ def test_partials_summed_during_the_build(lanes):
             out.append(xc.build("PBE", "fp64"))
     (h0, e0, q0), (h1, e1, q1) = out
     assert np.max(np.abs(h0 - h1)) <= 1e-10 and abs(e0 - e1) <= 1e-9 and abs(q0 - q1) <= 1e-9
+
+
+@pytest.mark.parametrize("n,nocc", [(1, 1), (3, 0), (17, 5), (63, 15), (64, 16), (65, 17), (130, 33), (200, 1)])
+@pytest.mark.parametrize("spins", [1, 2])
+def test_density_from_orbitals(n, nocc, spins):
+    """P formed on the device from orbitals and occupations (tiles of 64, 16
+    orbitals a step, caller order) gives the builds of the same P as a matrix."""
+    rng = np.random.default_rng(n + 7 * nocc)
+    b = _basis(n, rng)
+    g = _grid(b, 200, rng)
+    shape = (n, nocc) if spins == 1 else (n, nocc, 2)
+    C, occ = rng.normal(size=shape) / np.sqrt(n), rng.uniform(0.1, 2.0, shape[1:])
+    if spins == 1:
+        P = (C * occ) @ C.T
+    else:
+        P = np.stack([(C[:, :, s] * occ[:, s]) @ C[:, :, s].T for s in range(2)], axis=2)
+    with XCBuilder(b, g) as xc:
+        xc.set_density(P)
+        h0, e0, q0 = xc.build("PBE", "fp64")
+        xc.set_orbitals(C, occ)
+        h1, e1, q1 = xc.build("PBE", "fp64")
+    # sums of at most 33 products of order 1 in both: P to some 1e-15
+    assert np.max(np.abs(h0 - h1)) <= 1e-12 * max(1.0, np.max(np.abs(h0)))
+    assert abs(e0 - e1) <= 1e-12 * max(1.0, abs(e0)) and abs(q0 - q1) <= 1e-12 * max(1.0, abs(q0))
