@@ -59,8 +59,50 @@ struct ScopedDev {
 
 }  // namespace
 
+// Host memory the device copies to and from directly, in two halves that take
+// turns: one is filled by the copy engine while the host empties the other.
+// 1 MiB a half: a copy of it takes longer than starting one.
+struct PinnedPair {
+  static constexpr size_t kHalf = 1 << 20;
+  char *buf = nullptr;
+  hipEvent_t ev[2] = {nullptr, nullptr};
+  hipError_t init() {
+    hipError_t e = hipHostMalloc((void **)&buf, 2 * kHalf);
+    for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
+    return e;
+  }
+  void release() {
+    if (buf) (void)hipHostFree(buf);
+    for (auto &v : ev)
+      if (v) (void)hipEventDestroy(v);
+    buf = nullptr;
+  }
+  // n doubles at dev, in order, to take(first, count, values); waits for the
+  // stream's earlier work
+  template <class Take>
+  hipError_t fetch(hipStream_t s, const double *dev, size_t n, Take take) {
+    const size_t per = kHalf / 8, parts = (n + per - 1) / per;
+    hipError_t e = hipSuccess;
+    auto len = [&](size_t i) { return std::min(per, n - i * per); };
+    for (size_t i = 0; i <= parts && e == hipSuccess; ++i) {
+      if (i < parts) {
+        e = hipMemcpyAsync(buf + (i & 1) * kHalf, dev + i * per, 8 * len(i), hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(ev[i & 1], s);
+      }
+      if (i > 0 && e == hipSuccess) {
+        e = hipEventSynchronize(ev[(i - 1) & 1]);
+        if (e == hipSuccess) take((i - 1) * per, len(i - 1), (const double *)(buf + ((i - 1) & 1) * kHalf));
+      }
+    }
+    return e;
+  }
+};
+
 struct pgxc_ctx {
   int device = 0;
+  PinnedPair pin;
+  double *orb = nullptr;  // orbitals and occupations of the last pgxc_set_orbitals
+  size_t orb_n = 0;
   hipStream_t stream = nullptr;
   // chunks alternate between two lanes (this stream and stream2, each with its
   // own work buffers) so one chunk's stages overlap the next chunk's
@@ -1100,14 +1142,13 @@ static void set_stats(pgxc_ctx *c, int precision) {
 }
 
 static int collect(pgxc_ctx *c, hipStream_t s, uint32_t functional, int precision) {
-  std::vector<double> ep(2 * (size_t)c->nblk_total);
-  HIPCHK(c, hipMemcpyAsync(ep.data(), c->epart, ep.size() * 8, hipMemcpyDeviceToHost, s));
-  HIPCHK(c, hipStreamSynchronize(s));
   double e = 0.0, q = 0.0;
-  for (long b = 0; b < c->nblk_total; ++b) {
-    e += ep[2 * b];
-    q += ep[2 * b + 1];
-  }
+  HIPCHK(c, c->pin.fetch(s, c->epart, 2 * (size_t)c->nblk_total, [&](size_t, size_t n, const double *v) {
+    for (size_t b = 0; b < n; b += 2) {
+      e += v[b];
+      q += v[b + 1];
+    }
+  }));
   c->last_exc = e;
   c->last_charge = q;
   c->have_state = 1;
@@ -1611,6 +1652,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
   c->nlanes = c->nlanes_cap = c->nchunks > 1 ? 2 : 1;
   HIPCHK(c, hipStreamCreateWithFlags(&c->stream2, hipStreamNonBlocking));
+  HIPCHK(c, c->pin.init());
   HIPCHK(c, hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
   HIPCHK(c, hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
   // atom ranges of the basis stage: consecutive atoms in shell order, as many
@@ -1822,8 +1864,6 @@ extern "C" int pgxc_set_density(pgxc_ctx *c, int32_t ispin, int32_t nbas, const 
   return PGXC_OK;
 }
 
-// Temporary device buffers of a call, freed when the call returns on any path.
-
 extern "C" int pgxc_set_orbitals(pgxc_ctx *c, int32_t ispin, int32_t nbas, int32_t nocc,
                                  const double *C, const double *occ, int32_t mode) {
   int rc = check_density_args(c, ispin, nbas, mode);
@@ -1831,15 +1871,24 @@ extern "C" int pgxc_set_orbitals(pgxc_ctx *c, int32_t ispin, int32_t nbas, int32
   if (nocc < 0 || (nocc > 0 && (!C || !occ)))
     return fail(c, PGXC_ERR_ARG, "pgxc_set_orbitals: bad nocc or null C/occ");
   const int n = c->nbas;
-  double *dC = nullptr, *docc = nullptr;
-  ScopedDev tmp;  // dC and docc, freed on every return below
-  if (nocc > 0) {
-    HIPCHK(c, hipMalloc((void **)&dC, (size_t)ispin * n * nocc * 8));
-    tmp.keep(dC);
-    HIPCHK(c, hipMalloc((void **)&docc, (size_t)ispin * nocc * 8));
-    tmp.keep(docc);
-    HIPCHK(c, hipMemcpy(dC, C, (size_t)ispin * n * nocc * 8, hipMemcpyHostToDevice));
-    HIPCHK(c, hipMemcpy(docc, occ, (size_t)ispin * nocc * 8, hipMemcpyHostToDevice));
+  const size_t nC = (size_t)ispin * n * nocc, no = (size_t)ispin * nocc;
+  if (c->orb_n < nC + no) {
+    dfree(c->orb);
+    c->orb = nullptr;
+    c->orb_n = 0;
+    HIPCHK(c, hipMalloc((void **)&c->orb, (nC + no) * 8));
+    c->orb_n = nC + no;
+  }
+  double *dC = c->orb, *docc = c->orb + nC;
+  if ((nC + no) * 8 <= 2 * PinnedPair::kHalf) {  // one copy from pinned memory
+    if (nC) {
+      memcpy(c->pin.buf, C, nC * 8);
+      memcpy(c->pin.buf + nC * 8, occ, no * 8);
+      HIPCHK(c, hipMemcpyAsync(dC, c->pin.buf, (nC + no) * 8, hipMemcpyHostToDevice, c->stream));
+    }
+  } else {
+    HIPCHK(c, hipMemcpy(dC, C, nC * 8, hipMemcpyHostToDevice));
+    HIPCHK(c, hipMemcpy(docc, occ, no * 8, hipMemcpyHostToDevice));
   }
   for (int sp = 0; sp < ispin; ++sp)  // nocc = 0: P = 0
     launch_form_density(c->stream, dC + (size_t)sp * n * nocc, docc + (size_t)sp * nocc, c->d_finv, n, nocc,
@@ -1877,7 +1926,13 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   else
     launch_plan<float>(s, c->stream2, c->fork, c->join, *c->plan, gga, &c->ev);
   HIPCHK(c, hipGetLastError());
-  HIPCHK(c, hipStreamSynchronize(s));
+  // waits for the build; a small V comes along in the same wait
+  const size_t npk = (size_t)c->nbas * (c->nbas + 1) / 2;
+  const bool along = ham && c->ispin == 1 && 8 * npk <= PinnedPair::kHalf &&
+                     16 * (size_t)c->nblk_total <= PinnedPair::kHalf;
+  const double *v = (const double *)(c->pin.buf + PinnedPair::kHalf);
+  if (along) HIPCHK(c, hipMemcpyAsync((void *)v, c->Vout, 8 * npk, hipMemcpyDeviceToHost, s));
+  if ((rc = collect(c, s, functional, precision))) return rc;
   for (int k = 0; k < 4; ++k) c->timing[k] = 0.0;
   float t = 0;
   for (size_t k = 0; k < c->plan->steps.size(); ++k) {
@@ -1892,7 +1947,10 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   HIPCHK(c, hipEventElapsedTime(&t, c->ev[kEvStart], c->ev[kEvEnd]));
   c->timing[5] = t;
   mark_basis_cached(c, elem, precision, gga);
-  if ((rc = collect(c, s, functional, precision))) return rc;
+  if (along) {
+    for (size_t i = 0; i < npk; ++i) ham[i] += v[i];
+    ham = nullptr;
+  }
   return pgxc_get_result(c, ham, exc, charge);
 }
 
@@ -1901,10 +1959,14 @@ int pgxc_get_result(pgxc_ctx *c, double *ham, double *exc, double *charge) {
   if (!c->have_state) return fail(c, PGXC_ERR_STATE, "no build has run on this context");
   if (ham) {  // ispin = 2: alpha / beta at even / odd positions
     const size_t npk = (size_t)c->nbas * (c->nbas + 1) / 2, is = (size_t)c->ispin;
-    std::vector<double> v(npk);
     for (size_t sp = 0; sp < is; ++sp) {
-      HIPCHK(c, hipMemcpy(v.data(), sp ? c->beta.Vout : c->Vout, npk * 8, hipMemcpyDeviceToHost));
-      for (size_t i = 0; i < npk; ++i) ham[i * is + sp] += v[i];
+      double *h = ham + sp;
+      HIPCHK(c, c->pin.fetch(c->stream, sp ? c->beta.Vout : c->Vout, npk, [&](size_t i0, size_t n, const double *v) {
+        if (is == 1)
+          for (size_t i = 0; i < n; ++i) h[i0 + i] += v[i];
+        else
+          for (size_t i = 0; i < n; ++i) h[(i0 + i) * 2] += v[i];
+      }));
     }
   }
   if (exc) *exc += c->last_exc;
@@ -1930,12 +1992,11 @@ int pgxc_energy(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ter
   else
     launch_plan<float>(s, c->stream2, c->fork, c->join, *c->plan_e, gga, nullptr);
   HIPCHK(c, hipGetLastError());
-  std::vector<double> et(5 * (size_t)c->nblk_total);
-  HIPCHK(c, hipMemcpyAsync(et.data(), c->eterm, et.size() * 8, hipMemcpyDeviceToHost, s));
-  HIPCHK(c, hipStreamSynchronize(s));
   double t[5] = {0, 0, 0, 0, 0};
-  for (long b = 0; b < c->nblk_total; ++b)
-    for (int k = 0; k < 5; ++k) t[k] += et[5 * b + k];
+  size_t at = 0;
+  HIPCHK(c, c->pin.fetch(s, c->eterm, 5 * (size_t)c->nblk_total, [&](size_t, size_t n, const double *v) {
+    for (size_t i = 0; i < n; ++i, ++at) t[at % 5] += v[i];
+  }));
   memcpy(c->last_terms, t, sizeof(t));
   mark_basis_cached(c, elem, precision, gga);
   if (terms4) memcpy(terms4, t, 4 * sizeof(double));
@@ -2206,7 +2267,7 @@ int pgxc_destroy(pgxc_ctx *c) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     g_cache_bytes[c->device] -= c->phic_bytes[0] + c->phic_bytes[1];
   }
-  void *bufs[] = {c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->exps, c->norms, c->contr, c->P, c->Pref,
+  void *bufs[] = {c->orb, c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->exps, c->norms, c->contr, c->P, c->Pref,
                   c->D, c->phi, c->W, c->part, c->coef, c->Hc, c->HS, c->state,
                   c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos, c->d_finv,
                   c->phic[0], c->phic[1], c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,
@@ -2220,6 +2281,7 @@ int pgxc_destroy(pgxc_ctx *c) {
   if (c->stream2) (void)hipStreamDestroy(c->stream2);
   if (c->fork) (void)hipEventDestroy(c->fork);
   if (c->join) (void)hipEventDestroy(c->join);
+  c->pin.release();
   delete c;
   return PGXC_OK;
 }
@@ -2415,6 +2477,8 @@ int pgxc_batch_destroy(pgxc_batch *b) {
   return PGXC_OK;
 }
 
+constexpr int64_t kBeckePart = 1 << 18;
+
 int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, const double *pts,
                        const int32_t *owner, const double *w_atomic, double *w_out) {
   if (n_atoms <= 0 || npts < 0 || !atom_xyz ||
@@ -2430,42 +2494,60 @@ int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, co
       const double dz = atom_xyz[3 * i + 2] - atom_xyz[3 * k + 2];
       if (!(dx * dx + dy * dy + dz * dz > 0.0)) return PGXC_ERR_ARG;  // coincident centres
     }
-  const size_t ninv = (size_t)n_atoms * n_atoms;
-  double *d_a = nullptr, *d_inv = nullptr, *d_p = nullptr, *d_w = nullptr, *d_o = nullptr;
-  int *d_own = nullptr;
-  hipStream_t s = nullptr;
+  // Points go in parts of kBeckePart: a part's upload (from the caller's pageable
+  // memory, which the copy has read when it returns) runs while the parts before
+  // it are computed, and its weights come back while those after it are.
+  const size_t ninv = (size_t)n_atoms * n_atoms, na3 = 3 * (size_t)n_atoms;
+  const int64_t parts = (npts + kBeckePart - 1) / kBeckePart;
+  double *dev = nullptr;  // centres, inverse distances, points (3), weights in, weights out; owners
+  hipStream_t s = nullptr, sc = nullptr;
+  std::vector<hipEvent_t> up((size_t)parts, nullptr), done((size_t)parts, nullptr);
   int rc = PGXC_OK;
   auto chk = [&](hipError_t e) {
     if (e != hipSuccess && rc == PGXC_OK)
       rc = e == hipErrorOutOfMemory ? PGXC_ERR_NOMEM : PGXC_ERR_HIP;
+    return rc == PGXC_OK;
   };
   chk(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  chk(hipMalloc((void **)&d_a, 24 * (size_t)n_atoms));
-  chk(hipMalloc((void **)&d_inv, ninv * 8));
-  chk(hipMalloc((void **)&d_p, 24 * (size_t)npts));
-  chk(hipMalloc((void **)&d_w, 8 * (size_t)npts));
-  chk(hipMalloc((void **)&d_o, 8 * (size_t)npts));
-  chk(hipMalloc((void **)&d_own, 4 * (size_t)npts));
-  if (rc == PGXC_OK) {
-    chk(hipMemcpyAsync(d_a, atom_xyz, 24 * (size_t)n_atoms, hipMemcpyHostToDevice, s));
-    chk(hipMemcpyAsync(d_p, pts, 24 * (size_t)npts, hipMemcpyHostToDevice, s));
-    chk(hipMemcpyAsync(d_w, w_atomic, 8 * (size_t)npts, hipMemcpyHostToDevice, s));
-    chk(hipMemcpyAsync(d_own, owner, 4 * (size_t)npts, hipMemcpyHostToDevice, s));
+  chk(hipStreamCreateWithFlags(&sc, hipStreamNonBlocking));
+  chk(hipMalloc((void **)&dev, 8 * (na3 + ninv) + 44 * (size_t)npts + 8));
+  for (int64_t i = 0; i < parts && rc == PGXC_OK; ++i) {
+    chk(hipEventCreateWithFlags(&up[(size_t)i], hipEventDisableTiming));
+    chk(hipEventCreateWithFlags(&done[(size_t)i], hipEventDisableTiming));
   }
+  double *d_a = dev, *d_inv = d_a + na3, *d_p = d_inv + ninv, *d_w = d_p + 3 * npts, *d_o = d_w + npts;
+  int *d_own = (int *)(d_o + npts);
   if (rc == PGXC_OK) {
+    chk(hipMemcpyAsync(d_a, atom_xyz, 8 * na3, hipMemcpyHostToDevice, s));
     launch_inv_dist(s, n_atoms, d_a, d_inv);
-    launch_becke(s, n_atoms, d_a, d_inv, (long)npts, d_p, d_own, d_w, d_o);
-    chk(hipGetLastError());
-    chk(hipMemcpyAsync(w_out, d_o, 8 * (size_t)npts, hipMemcpyDeviceToHost, s));
-    chk(hipStreamSynchronize(s));
   }
-  dfree(d_a);
-  dfree(d_inv);
-  dfree(d_p);
-  dfree(d_w);
-  dfree(d_o);
-  dfree(d_own);
+  for (int64_t i = 0; i < parts + 2 && rc == PGXC_OK; ++i) {
+    if (i < parts) {
+      const int64_t p0 = i * kBeckePart, n = std::min<int64_t>(kBeckePart, npts - p0);
+      for (int d = 0; d < 3; ++d)
+        chk(hipMemcpyAsync(d_p + d * npts + p0, pts + d * npts + p0, 8 * (size_t)n, hipMemcpyHostToDevice, sc));
+      chk(hipMemcpyAsync(d_w + p0, w_atomic + p0, 8 * (size_t)n, hipMemcpyHostToDevice, sc));
+      chk(hipMemcpyAsync(d_own + p0, owner + p0, 4 * (size_t)n, hipMemcpyHostToDevice, sc));
+      chk(hipEventRecord(up[(size_t)i], sc));
+      chk(hipStreamWaitEvent(s, up[(size_t)i], 0));
+      launch_becke(s, n_atoms, d_a, d_inv, (long)n, (long)npts, d_p + p0, d_own + p0, d_w + p0, d_o + p0);
+      chk(hipGetLastError());
+      chk(hipEventRecord(done[(size_t)i], s));
+    }
+    if (i >= 2) {
+      const int64_t p0 = (i - 2) * kBeckePart, n = std::min<int64_t>(kBeckePart, npts - p0);
+      chk(hipStreamWaitEvent(sc, done[(size_t)(i - 2)], 0));
+      chk(hipMemcpyAsync(w_out + p0, d_o + p0, 8 * (size_t)n, hipMemcpyDeviceToHost, sc));
+    }
+  }
+  if (sc) chk(hipStreamSynchronize(sc));
+  if (s) chk(hipStreamSynchronize(s));
+  dfree(dev);
+  for (auto *v : {&up, &done})
+    for (hipEvent_t e : *v)
+      if (e) (void)hipEventDestroy(e);
   if (s) (void)hipStreamDestroy(s);
+  if (sc) (void)hipStreamDestroy(sc);
   return rc;
 }
 
@@ -2510,7 +2592,7 @@ int pgxc_becke_weights_noalloc(int32_t n_atoms, const double *atom_xyz, int64_t 
   }
   hipStream_t s = (hipStream_t)stream;
   launch_inv_dist(s, n_atoms, atom_xyz, ptr);  // every entry rewritten: nothing to clear
-  launch_becke(s, n_atoms, atom_xyz, ptr, (long)npts, pts, owner, w_atomic, w_out);
+  launch_becke(s, n_atoms, atom_xyz, ptr, (long)npts, (long)npts, pts, owner, w_atomic, w_out);
   if (hipGetLastError() != hipSuccess)
     return free_fail(PGXC_ERR_HIP, "pgxc_becke_weights_noalloc: kernel launch failed");
   return PGXC_OK;

@@ -266,7 +266,8 @@ void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *
 
 // Becke partition weights of points owned by atoms (grid generation)
 void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv);
+// npts points with coordinates stride apart
 void launch_becke(hipStream_t s, int na, const double *axyz, const double *inv_dist, long npts,
-                  const double *pts, const int *owner, const double *wat, double *wout);
+                  long stride, const double *pts, const int *owner, const double *wat, double *wout);
 
 }  // namespace pgxc

@@ -35,13 +35,14 @@ constexpr double kNegligible = 5.421010862427522e-20;  // 2^-64
 
 __global__ __launch_bounds__(kThreads) void k_becke(int na, const double *__restrict__ axyz,
                                                     const double *__restrict__ inv_dist,
-                                                    long npts, const double *__restrict__ pts,
+                                                    long npts, long stride,
+                                                    const double *__restrict__ pts,
                                                     const int *__restrict__ owner,
                                                     const double *__restrict__ wat,
                                                     double *__restrict__ wout) {
   const long p = (long)blockIdx.x * kThreads + threadIdx.x;
   if (p >= npts) return;
-  const double x = pts[p], y = pts[npts + p], z = pts[2 * npts + p];
+  const double x = pts[p], y = pts[stride + p], z = pts[2 * stride + p];
   const int own = owner[p];
   auto dist = [&](int i) {
     const double dx = axyz[3 * i] - x, dy = axyz[3 * i + 1] - y, dz = axyz[3 * i + 2] - z;
@@ -154,8 +155,8 @@ void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv) {
 }
 
 void launch_becke(hipStream_t s, int na, const double *axyz, const double *inv_dist, long npts,
-                  const double *pts, const int *owner, const double *wat, double *wout) {
+                  long stride, const double *pts, const int *owner, const double *wat, double *wout) {
   hipLaunchKernelGGL(k_becke, dim3((unsigned)((npts + kThreads - 1) / kThreads)), dim3(kThreads),
-                     0, s, na, axyz, inv_dist, npts, pts, owner, wat, wout);
+                     0, s, na, axyz, inv_dist, npts, stride, pts, owner, wat, wout);
 }
 }  // namespace pgxc
