@@ -128,7 +128,8 @@ struct pgxc_ctx {
   int *ratoms = nullptr;     // atoms in shell order
   int n_ranges = 0;
   std::vector<RangeD> h_ranges;
-  double *exps = nullptr, *norms = nullptr, *contr = nullptr;
+  double *tabd = nullptr;  // shell tables (exponents, norms, coefficients), FP64 and FP32
+  float *tabf = nullptr;
   // device: density (NP x NP); D holds the operand in the build's precision
   double *P = nullptr, *Pref = nullptr;
   void *D = nullptr;
@@ -546,9 +547,8 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.ranges = c->ranges;
       U.ratoms = c->ratoms;
       U.n_ranges = c->n_ranges;
-      U.exps = c->exps;
-      U.norms = c->norms;
-      U.contr = c->contr;
+      U.tabd = c->tabd;
+      U.tabf = c->tabf;
       const int lane = k % lanes_of(c);  // work buffers of chunk k: its stream's lane
       U.phi = (char *)c->phi_base + (c->phi_stride ? (size_t)k * c->phi_stride : (size_t)lane * c->phi_lane);
       U.W = (char *)c->W + (size_t)lane * c->w_lane;
@@ -586,7 +586,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.su = c->su;
       U.sumask = c->sumask;
       U.bitems = c->bi + c->h_bi_off[k];
-      U.bflags = c->bfl + 8 * c->h_bi_off[k];
+      U.bflags = c->bfl + 2 * c->h_bi_off[k];
       U.nbi = c->h_bi_off[k + 1] - c->h_bi_off[k];
       if (c->ispin == 2) {  // the beta spin's unit: same points and basis values
         UnitD B = U;
@@ -941,7 +941,7 @@ static void launch_plan(hipStream_t s, hipStream_t s2, hipEvent_t fork, hipEvent
     hipEvent_t *E = ev ? ev->data() + kEvStep + 5 * k : nullptr;
     if (E) (void)hipEventRecord(E[0], t);
     launch_basis<T>(t, gga, S.basis);
-    if (E) (void)hipEventRecord(E[1], t);
+    if (E && S.basis.total) (void)hipEventRecord(E[1], t);  // cached values: no stage, no mark
     for (int li = 0; li < kLists; ++li) {
       const int v = li % kNumVariants;
       if constexpr (std::is_same<T, float>::value) {
@@ -1432,17 +1432,17 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
       for (long b = 0; b < c->Mc / kThreads; ++b) {
         const uint32_t *m0 = smark.data() + (size_t)((g0 + b * gpb) / 4) * nws, *m1 = m0 + nws;
         for (int ri = 0; ri < nr; ++ri) {
-          // per (shell j of the range, group g of the block): read
-          uint32_t fw[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+          // the range's shells read on each tile of the block
+          uint32_t fw[2] = {0, 0};
           const RangeD &R = c->h_ranges[(size_t)ri];
           for (int j = 0; j < R.n_shells; ++j) {
             const int sg = R.shell_begin + j;
-            const uint32_t a = (m0[sg / 32] >> (sg % 32)) & 1u, z = (m1[sg / 32] >> (sg % 32)) & 1u;
-            fw[j / 4] |= (0xfu * a | 0xf0u * z) << (8 * (j % 4));
+            fw[0] |= ((m0[sg / 32] >> (sg % 32)) & 1u) << j;
+            fw[1] |= ((m1[sg / 32] >> (sg % 32)) & 1u) << j;
           }
-          if (!(fw[0] | fw[1] | fw[2] | fw[3] | fw[4] | fw[5] | fw[6] | fw[7])) continue;
+          if (!(fw[0] | fw[1])) continue;
           bi.push_back((uint32_t)(b << 16 | ri));
-          bfl.insert(bfl.end(), fw, fw + 8);
+          bfl.insert(bfl.end(), fw, fw + 2);
         }
       }
       c->h_bi_off.push_back((long)bi.size());
@@ -1548,9 +1548,10 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
     at[a].shell_begin = at[a].shell_end = 0;
     at[a].lmax = 0;
     at[a].pad = 0;
-    at[a].exp_begin = at[a].n_exp = at[a].contr_begin = at[a].n_contr = 0;
   }
   long eoff = 0, coff = 0, foff = 0;
+  std::vector<double> tab;
+  std::map<std::pair<int, std::string>, int> tabs;
   int prev_atom = -1;
   std::vector<int> seen(n_atoms, 0);
   for (int s = 0; s < n_shells; ++s) {
@@ -1583,8 +1584,24 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
     at[d.atom].lmax = std::max(at[d.atom].lmax, d.l);
     c->lmax = std::max(c->lmax, d.l);
     d.exp_off = (int)eoff;
-    d.contr_off = (int)coff;
     d.func_off = (int)foff;
+    {  // blocks of kPB primitives: exponents (padded with the last one), norms and each
+       // contraction's coefficients; shells with the same contents share a table, so that a large
+       // system's few kinds of shell stay in the scalar cache (16 KiB for two CUs)
+      const int row = (d.n_exp + kPB - 1) / kPB * kPB;
+      std::vector<double> t((size_t)(2 + d.n_contr) * row, 0.0);
+      for (int e = 0; e < row; ++e) {
+        double *q = t.data() + (2 + d.n_contr) * (e / kPB * kPB) + e % kPB;
+        q[0] = exps[eoff + std::min(e, d.n_exp - 1)];
+        if (e >= d.n_exp) continue;
+        q[kPB] = norms[eoff + e];
+        for (int k = 0; k < d.n_contr; ++k) q[(2 + k) * kPB] = contr[coff + (long)k * d.n_exp + e];
+      }
+      const std::string key((const char *)t.data(), t.size() * sizeof(double));
+      const auto ins = tabs.insert({{d.n_contr, key}, (int)tab.size()});
+      if (ins.second) tab.insert(tab.end(), t.begin(), t.end());
+      d.tab = ins.first->second;
+    }
     eoff += d.n_exp;
     coff += (long)d.n_exp * d.n_contr;
     foff += (long)(2 * d.l + 1) * (d.n_unc + d.n_contr);
@@ -1595,13 +1612,6 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
       np += sh[s].n_exp;
       nc += (long)sh[s].n_exp * sh[s].n_contr;
     }
-    if (at[a].shell_end > at[a].shell_begin) {
-      const ShellD &f = sh[at[a].shell_begin];
-      at[a].exp_begin = f.exp_off;
-      at[a].contr_begin = f.contr_off;
-    }
-    at[a].n_exp = (int)np;
-    at[a].n_contr = (int)nc;
     if (at[a].shell_end - at[a].shell_begin > kAtomShells || np > kAtomPrims || nc > kAtomContr)
       return fail(c, PGXC_ERR_UNSUPPORTED,
                   "pgxc_create: atom " + std::to_string(a) + " has more than " +
@@ -1655,9 +1665,9 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   HIPCHK(c, c->pin.init());
   HIPCHK(c, hipEventCreateWithFlags(&c->fork, hipEventDisableTiming));
   HIPCHK(c, hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
-  // atom ranges of the basis stage: consecutive atoms in shell order, as many
-  // as the kernel's LDS image holds, fewer where a chunk's blocks would give the
-  // device less than kBasisItems items
+  // atom ranges of the basis stage: consecutive atoms in shell order, at most
+  // kRangeAtoms (half as many: FP32 basis stage of (H2O)32 1.50 -> 1.64 ms), fewer
+  // where a chunk's blocks would give the device less than kBasisItems items
   const int ra_most = (int)std::min<long>(kRangeAtoms, std::max<long>(1, n_atoms * (c->Mc / kThreads) / kBasisItems));
   std::vector<int> ratoms;
   for (int a = 0; a < n_atoms; ++a)
@@ -1669,21 +1679,15 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
     const AtomD &a = at[ratoms[i]];
     const int ns = a.shell_end - a.shell_begin;
     if (c->h_ranges.empty() || c->h_ranges.back().n_atoms == ra_most ||
-        c->h_ranges.back().n_shells + ns > kRangeShells ||
-        c->h_ranges.back().n_exp + a.n_exp > kRangePrims ||
-        c->h_ranges.back().n_contr + a.n_contr > kRangeContr) {
+        c->h_ranges.back().n_shells + ns > kRangeShells) {
       RangeD r{};
       r.atom_begin = (int)i;
       r.shell_begin = a.shell_begin;
-      r.exp_begin = a.exp_begin;
-      r.contr_begin = a.contr_begin;
       c->h_ranges.push_back(r);
     }
     RangeD &r = c->h_ranges.back();
     ++r.n_atoms;
     r.n_shells += ns;
-    r.n_exp += a.n_exp;
-    r.n_contr += a.n_contr;
   }
   c->n_ranges = (int)c->h_ranges.size();
   int rc;
@@ -1692,9 +1696,12 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   if ((rc = dalloc(c, &c->shells, n_shells))) return rc;
   if ((rc = dalloc(c, &c->ranges, std::max<size_t>(c->h_ranges.size(), 1)))) return rc;
   if ((rc = dalloc(c, &c->ratoms, std::max<size_t>(ratoms.size(), 1)))) return rc;
-  if ((rc = dalloc(c, &c->exps, eoff))) return rc;
-  if ((rc = dalloc(c, &c->norms, eoff))) return rc;
-  if ((rc = dalloc(c, &c->contr, std::max<long>(coff, 1)))) return rc;
+  tab.insert(tab.end(), 2 * kPB, 0.0);  // a block is read with two contractions
+  if ((rc = upload(c, &c->tabd, tab))) return rc;
+  {
+    std::vector<float> t32(tab.begin(), tab.end());
+    if ((rc = upload(c, &c->tabf, t32))) return rc;
+  }
   // grid in space-filling-curve order, padded with far points of zero weight
   std::vector<long> perm;
   morton_order(grid, npts, npts, 1, perm);
@@ -1734,9 +1741,6 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
     for (int f = 0; f < c->nbas; ++f) finv[(size_t)c->fpos[f]] = f;
     if ((rc = upload(c, &c->d_finv, finv))) return rc;
   }
-  HIPCHK(c, hipMemcpy(c->exps, exps, 8 * eoff, hipMemcpyHostToDevice));
-  HIPCHK(c, hipMemcpy(c->norms, norms, 8 * eoff, hipMemcpyHostToDevice));
-  if (coff > 0) HIPCHK(c, hipMemcpy(c->contr, contr, 8 * coff, hipMemcpyHostToDevice));
   if ((rc = setup_screen(c, sh, exps, !(opt && opt->no_screen)))) return rc;
   const size_t np2 = (size_t)c->NP * c->NP;
   if ((rc = dalloc(c, &c->P, np2))) return rc;
@@ -1937,8 +1941,9 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   float t = 0;
   for (size_t k = 0; k < c->plan->steps.size(); ++k) {
     const hipEvent_t *E = c->ev.data() + kEvStep + 5 * k;
-    for (int j = 0; j < 4; ++j) {
-      HIPCHK(c, hipEventElapsedTime(&t, E[j], E[j + 1]));
+    const bool cached = !c->plan->steps[k].basis.total;
+    for (int j = cached ? 1 : 0; j < 4; ++j) {
+      HIPCHK(c, hipEventElapsedTime(&t, E[cached && j == 1 ? 0 : j], E[j + 1]));
       c->timing[j] += t;
     }
   }
@@ -2267,7 +2272,7 @@ int pgxc_destroy(pgxc_ctx *c) {
     std::lock_guard<std::mutex> lk(g_cache_mu);
     g_cache_bytes[c->device] -= c->phic_bytes[0] + c->phic_bytes[1];
   }
-  void *bufs[] = {c->orb, c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->exps, c->norms, c->contr, c->P, c->Pref,
+  void *bufs[] = {c->orb, c->grid, c->atoms, c->shells, c->ranges, c->ratoms, c->tabd, c->tabf, c->P, c->Pref,
                   c->D, c->phi, c->W, c->part, c->coef, c->Hc, c->HS, c->state,
                   c->Vstate, c->Vout, c->epart, c->nbt, c->sig8, c->sshells, c->d_fpos, c->d_finv,
                   c->phic[0], c->phic[1], c->tl_off, c->tl, c->tf_off, c->tfl, c->tfb, c->tlm, c->su_off, c->su, c->sumask,

@@ -15,34 +15,28 @@ constexpr int kMaxContr = 8;  // contracted functions per shell
 // per atom at most: shells, primitives and contraction coefficients
 constexpr int kAtomShells = 16, kAtomPrims = 256, kAtomContr = 1024;
 // A basis item evaluates one 256-point block against a range of atoms,
-// consecutive in shell order, whose basis data the kernel stages in LDS
-// together: at most kRangeAtoms atoms, kRangeShells shells, kRangePrims
-// primitives and kRangeContr contraction coefficients (an atom of the
-// per-atom maximum fits alone).
-constexpr int kRangeAtoms = 8, kRangeShells = 32, kRangePrims = 256, kRangeContr = 1024;
+// consecutive in shell order: at most kRangeAtoms atoms and kRangeShells shells
+// (a word of flags; an atom of the per-atom maximum fits).
+constexpr int kRangeAtoms = 8, kRangeShells = 32;
+constexpr int kPB = 4;  // rows of a shell's table are padded to this many primitives
 constexpr int kThreads = 256; // 4 wave64 per workgroup everywhere
 constexpr double kFar = 1.0e6;  // coordinate of padding points (all exps cut off)
 
 // One shell = one (atom, l) block of unique_atom_basis_type.
 struct ShellD {
-  int atom, l, n_exp, n_unc, n_contr, exp_off, contr_off, func_off;
+  int atom, l, n_exp, n_unc, n_contr, exp_off, tab, func_off;  // tab: its table in tabd / tabf
 };
 
-// One centre with the contiguous shell range it carries, and the contiguous
-// ranges of its shells' primitives (exp_begin, n_exp) and contraction
-// coefficients (contr_begin, n_contr).
+// One centre with the contiguous shell range it carries.
 struct AtomD {
   double x, y, z;
   int shell_begin, shell_end, lmax, pad;
-  int exp_begin, n_exp, contr_begin, n_contr;
 };
 
 // A range of atoms for the basis stage: ratoms[atom_begin .. +n_atoms) are
-// its atoms, in shell order; their shells (shell_begin, n_shells), primitives
-// and contraction coefficients are contiguous.
+// its atoms, in shell order; their shells (shell_begin, n_shells) are contiguous.
 struct RangeD {
   int atom_begin, n_atoms, shell_begin, n_shells;
-  int exp_begin, n_exp, contr_begin, n_contr;
 };
 
 // Per-point state kept across builds (incremental mode), SoA of length npad.
@@ -55,7 +49,8 @@ struct UnitD {
   const double *gx, *gy, *gz, *gw;  // grid of the unit's points (offset to its first point)
   const AtomD *atoms;
   const ShellD *shells;
-  const double *exps, *norms, *contr;
+  const double *tabd;  // the shells' exponents, norms and coefficients, in FP64
+  const float *tabf;   // and in FP32
   const RangeD *ranges;  // the basis stage's atom ranges
   const int *ratoms;     // atoms in shell order (the ranges index it)
   void *phi;        // [4][NP][Mc] values, d/dx, d/dy, d/dz (T)
@@ -99,8 +94,8 @@ struct UnitD {
   int nwf, pad_f;
   // Basis stage over the blocks the other stages read.  bitems: basis items
   // (256-point block << 16 | atom range) that write some block, block by block,
-  // with bflags: 8 words per item, bit 8 j + g: the values and gradients of the
-  // range's shell j are read on group g of the block.
+  // with bflags: per item a word for each of the block's two tiles, bit j: the
+  // values and gradients of the range's shell j are read there.
   const uint32_t *bitems, *bflags;
   long nbi;
   long Mc, npad;

@@ -1,6 +1,6 @@
 // Basis evaluation on the device, shared by the basis and W stages and the
-// nuclear gradient: solid harmonics, a range of atoms' data staged in LDS, and
-// the walk over a staged range.
+// nuclear gradient: solid harmonics, the shells' radial parts from scalar
+// tables, and the walk over a basis item.
 #pragma once
 #include "pgxc_internal.h"
 #include "xc_device.h"
@@ -97,79 +97,108 @@ __device__ __forceinline__ void fn_values(int m, T r0, T r1, T x, T y, T z, cons
 }
 
 // Emitter of the basis stage: stores a shell's values (and gradients) at
-// point p of the [4][NP][Mc] planes.  Global (not flat) stores: a flat
-// store also counts against the LDS wait counter, so every wait for the
-// staged shell data would wait for the stores issued before it.
+// point p of the [4][NP][Mc] planes: the row's address is the wave's (scalar, a
+// step per function), the lane adds its point's 32-bit offset in the store.
 template <typename T>
 struct StorePhi {
   T *phi;
   long Mc, cs;
-  int p;
+  unsigned p;
   template <int L, bool GRAD>
   __device__ __forceinline__ void emit(long f0, int nf, T r0, T r1, T x, T y, T z, const T *C,
                                        const T *Cx, const T *Cy, const T *Cz) const {
+    T *row = phi + f0 * Mc;
+    const long step = nf * Mc;
 #pragma unroll
-    for (int m = 0; m < 2 * L + 1; ++m) {
-      const long q = (f0 + (long)m * nf) * Mc + p;
+    for (int m = 0; m < 2 * L + 1; ++m, row += step) {
       T v, gx = T(0), gy = T(0), gz = T(0);
       fn_values<L, false>(m, r0, r1, x, y, z, C, Cx, Cy, Cz, v, gx, gy, gz);
-      gst(phi + q, v);
+      gst_row(row, p, v);
       if (GRAD) {
         fn_values<L, true>(m, r0, r1, x, y, z, C, Cx, Cy, Cz, v, gx, gy, gz);
-        gst(phi + cs + q, gx);
-        gst(phi + 2 * cs + q, gy);
-        gst(phi + 3 * cs + q, gz);
+        gst_row(row + cs, p, gx);
+        gst_row(row + 2 * cs, p, gy);
+        gst_row(row + 3 * cs, p, gz);
       }
     }
   }
 };
 
-// A range of atoms' basis data staged in LDS for a basis item: the shells,
-// their exponents, norms and contraction coefficients in the evaluation
-// precision, per atom its centre, shell range (relative to the range's
-// first shell) and largest l, and per (shell, 32-point group of the item)
-// whether to write its values (and gradients).
+// Reads of tables that no kernel writes, at addresses that are the same for the
+// whole wave: scalar loads into scalar registers (the constant address space
+// says so; through an ordinary pointer from a descriptor the compiler has to
+// expect the stores in between to change them).
 template <typename T>
-struct RangeLds {
-  ShellD sh[kRangeShells];
-  T ex[kRangePrims], nm[kRangePrims], ct[kRangeContr];
-  double ax[kRangeAtoms], ay[kRangeAtoms], az[kRangeAtoms];
-  int s0[kRangeAtoms], s1[kRangeAtoms], lm[kRangeAtoms];
-  uint8_t fl[kRangeShells][kThreads / kGroup];
+__device__ __forceinline__ T cld(const T *p) {
+  return *(const __attribute__((address_space(4))) T *)p;
+}
+
+// The units' shell tables in T: per shell its primitives in blocks of kPB (padded
+// with the last exponent, norm and coefficients 0), a block's exponents, norms and
+// the coefficients of each contraction in turn.
+template <typename T>
+__device__ __forceinline__ const T *shell_tables(const UnitD &U);
+template <>
+__device__ __forceinline__ const double *shell_tables<double>(const UnitD &U) { return U.tabd; }
+template <>
+__device__ __forceinline__ const float *shell_tables<float>(const UnitD &U) { return U.tabf; }
+
+__device__ __forceinline__ ShellD shell_at(const ShellD *p) {
+  ShellD s;
+  s.atom = cld(&p->atom);
+  s.l = cld(&p->l);
+  s.n_exp = cld(&p->n_exp);
+  s.n_unc = cld(&p->n_unc);
+  s.n_contr = cld(&p->n_contr);
+  s.tab = cld(&p->tab);
+  s.func_off = cld(&p->func_off);
+  return s;
+}
+
+// A block of a shell's table: loaded at once, so that a wave waits once for it
+// (scalar loads return out of order: each wait is for all of them), with the
+// first two contractions (the table ends with as much room); the others as used.
+template <typename T>
+struct PrimBlock {
+  const T *p;
+  T al[kPB], nv[kPB], c[2][kPB];
+  __device__ __forceinline__ PrimBlock(const T *tab, int nc, int e0) : p(tab + (2 + nc) * e0) {
+#pragma unroll
+    for (int i = 0; i < kPB; ++i) {
+      al[i] = cld(p + i);
+      nv[i] = cld(p + kPB + i);
+      c[0][i] = cld(p + 2 * kPB + i);
+      c[1][i] = cld(p + 3 * kPB + i);
+    }
+  }
+  __device__ __forceinline__ T coeff(int k, int i) const { return k < 2 ? c[k][i] : cld(p + (2 + k) * kPB + i); }
 };
 
-// ex, nm: the shell's primitives; ct: its n_exp x n_contr coefficients.
-// Primitives go in blocks of kPB: the block's exponents, norms and
-// coefficients are read from LDS together (one wait, not one per read), its
-// radial factors formed without a branch per primitive (a block whose
-// primitives are all cut off on the wave's points skips the exponentials),
-// then added into the contractions in primitive order.
-constexpr int kPB = 4;
+// tab: the shell's table.  Primitives go in blocks of kPB: radial factors formed
+// without a branch per primitive (a block whose primitives are all cut off on
+// the wave's points skips the exponentials and adds nothing), then added into
+// the contractions in primitive order.
 template <int L, bool GRAD, typename T, class Put>
-__device__ __forceinline__ void shell_emit(const ShellD &sh, const T *ex, const T *nm, const T *ct,
-                                           T x, T y, T z, T r2, const T *C, const T *Cx,
-                                           const T *Cy, const T *Cz, const Put &put) {
+__device__ __forceinline__ void shell_emit(const ShellD &sh, const T *tab, T x, T y, T z, T r2,
+                                           const T *C, const T *Cx, const T *Cy, const T *Cz,
+                                           const Put &put) {
   const int ne = sh.n_exp, nu = sh.n_unc, nc = sh.n_contr, nf = nu + nc;
   T rc0[kMaxContr], rc1[kMaxContr];
 #pragma unroll
   for (int k = 0; k < kMaxContr; ++k) rc0[k] = rc1[k] = T(0);
   for (int e0 = 0; e0 < ne; e0 += kPB) {
-    T al[kPB], ar2[kPB], nv[kPB], r0[kPB], r1[kPB];
+    const PrimBlock<T> q(tab, nc, e0);
+    T r0[kPB], r1[kPB];
     bool any = false;
 #pragma unroll
-    for (int i = 0; i < kPB; ++i) {
-      const int e = min(e0 + i, ne - 1);  // past the shell: a repeat, never used
-      al[i] = ex[e];
-      nv[i] = nm[e];
-      ar2[i] = al[i] * r2;
-      any = any || (e0 + i < ne && ar2[i] < T(50));
-    }
-    if (__ballot(any)) {
+    for (int i = 0; i < kPB; ++i) any = any || q.al[i] * r2 < T(50);
+    const bool live = __ballot(any) != 0;
+    if (live) {
 #pragma unroll
       for (int i = 0; i < kPB; ++i) {
-        const T v = nv[i] * exp(-ar2[i]);
-        r0[i] = (e0 + i < ne && ar2[i] < T(50)) ? v : T(0);  // primitive cut-off of radial1()
-        r1[i] = (T(-2) * al[i]) * r0[i];
+        const T ar2 = q.al[i] * r2, v = q.nv[i] * exp(-ar2);
+        r0[i] = ar2 < T(50) ? v : T(0);  // primitive cut-off of radial1()
+        r1[i] = (T(-2) * q.al[i]) * r0[i];
       }
     } else {
 #pragma unroll
@@ -179,18 +208,16 @@ __device__ __forceinline__ void shell_emit(const ShellD &sh, const T *ex, const 
     for (int i = 0; i < kPB; ++i)
       if (e0 + i < nu)
         put.template emit<L, GRAD>(sh.func_off + e0 + i, nf, r0[i], r1[i], x, y, z, C, Cx, Cy, Cz);
+    if (!live) continue;
 #pragma unroll
     for (int k = 0; k < kMaxContr; ++k)
       if (k < nc) {
-        T c[kPB];
 #pragma unroll
-        for (int i = 0; i < kPB; ++i) c[i] = ct[k * ne + min(e0 + i, ne - 1)];
-#pragma unroll
-        for (int i = 0; i < kPB; ++i)
-          if (e0 + i < ne) {
-            rc0[k] += r0[i] * c[i];
-            rc1[k] += r1[i] * c[i];
-          }
+        for (int i = 0; i < kPB; ++i) {
+          const T c = q.coeff(k, i);
+          rc0[k] += r0[i] * c;
+          rc1[k] += r1[i] * c;
+        }
       }
   }
 #pragma unroll
@@ -199,110 +226,77 @@ __device__ __forceinline__ void shell_emit(const ShellD &sh, const T *ex, const 
       put.template emit<L, GRAD>(sh.func_off + nu + k, nf, rc0[k], rc1[k], x, y, z, C, Cx, Cy, Cz);
 }
 
-// One atom's shells sb .. se-1 of the LDS image A at one point (e0, c0: the
-// range's first primitive and coefficient); grp: the point's group in the
-// item.
+// The shells `live` (bits, from shell s0 on) of one atom at the thread's point.
 template <int LA, bool GRAD, typename T, class Put>
-__device__ __forceinline__ void basis_atom(const RangeLds<T> &A, int sb, int se, int e0, int c0,
-                                           T x, T y, T z, const Put &put, int grp) {
+__device__ __forceinline__ void basis_atom(const UnitD &U, int s0, unsigned live, T x, T y, T z,
+                                           const Put &put) {
   constexpr int NLM = (LA + 1) * (LA + 1);
   T C[NLM], Cx[NLM], Cy[NLM], Cz[NLM];
   sh_eval<LA, T>(x, y, z, C, Cx, Cy, Cz);
   const T r2 = x * x + y * y + z * z;
-  for (int s = sb; s < se; ++s) {
-    if (!(A.fl[s][grp] & 1)) continue;  // no stage reads the shell's values on this group
-    // every lane reads the same shell: its fields are uniform over the wave,
-    // so the loops over its primitives and functions run on scalar counters
-    ShellD sh = A.sh[s];
-    sh.l = __builtin_amdgcn_readfirstlane(sh.l);
-    sh.n_exp = __builtin_amdgcn_readfirstlane(sh.n_exp);
-    sh.n_unc = __builtin_amdgcn_readfirstlane(sh.n_unc);
-    sh.n_contr = __builtin_amdgcn_readfirstlane(sh.n_contr);
-    sh.exp_off = __builtin_amdgcn_readfirstlane(sh.exp_off);
-    sh.contr_off = __builtin_amdgcn_readfirstlane(sh.contr_off);
-    sh.func_off = __builtin_amdgcn_readfirstlane(sh.func_off);
-    const T *ex = A.ex + (sh.exp_off - e0), *nm = A.nm + (sh.exp_off - e0);
-    const T *ct = A.ct + (sh.contr_off - c0);
+  for (; live; live &= live - 1) {
+    const ShellD sh = shell_at(U.shells + s0 + __builtin_ctz(live));
+    const T *tab = shell_tables<T>(U) + sh.tab;
     switch (sh.l) {
-      case 0: shell_emit<0, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put); break;
-      case 1: if constexpr (LA >= 1) shell_emit<1, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put); break;
-      case 2: if constexpr (LA >= 2) shell_emit<2, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put); break;
-      case 3: if constexpr (LA >= 3) shell_emit<3, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put); break;
-      case 4: if constexpr (LA >= 4) shell_emit<4, GRAD>(sh, ex, nm, ct, x, y, z, r2, C, Cx, Cy, Cz, put); break;
+      case 0: shell_emit<0, GRAD>(sh, tab, x, y, z, r2, C, Cx, Cy, Cz, put); break;
+      case 1: if constexpr (LA >= 1) shell_emit<1, GRAD>(sh, tab, x, y, z, r2, C, Cx, Cy, Cz, put); break;
+      case 2: if constexpr (LA >= 2) shell_emit<2, GRAD>(sh, tab, x, y, z, r2, C, Cx, Cy, Cz, put); break;
+      case 3: if constexpr (LA >= 3) shell_emit<3, GRAD>(sh, tab, x, y, z, r2, C, Cx, Cy, Cz, put); break;
+      case 4: if constexpr (LA >= 4) shell_emit<4, GRAD>(sh, tab, x, y, z, r2, C, Cx, Cy, Cz, put); break;
     }
   }
 }
 
-// A basis item staged: its first point, the range's first primitive and
-// coefficient, its atom count, and the point's coordinates.
-struct BasisItem {
-  long p;
-  int e0, c0, n_atoms;
-  double gx, gy, gz;
+// One atom of a basis item on the wave's tile: its centre, first shell, largest
+// l, and its shells that are not cut off there (bits from the first shell on).
+struct ItemAtom {
+  double x, y, z;
+  int s0, lmax;
+  unsigned live;
 };
-
-// Stages basis item `local` of unit U in A (every thread calls it; starts
-// and ends with a barrier).
-template <typename T>
-__device__ __forceinline__ BasisItem stage_basis_item(const UnitD &U, long local, RangeLds<T> &A) {
-  const int tid = threadIdx.x;
-  const uint32_t e = U.bitems[local];
-  const long blk = e >> 16;
-  const int rng = (int)(e & 0xffffu);
-  const RangeD R = U.ranges[rng];
-  BasisItem it;
-  it.e0 = R.exp_begin;
-  it.c0 = R.contr_begin;
-  it.n_atoms = R.n_atoms;
-  it.p = blk * kThreads + tid;
-  // the point's coordinates in FP64, loads in flight across the staging
-  it.gx = gld(U.gx + it.p);
-  it.gy = gld(U.gy + it.p);
-  it.gz = gld(U.gz + it.p);
-  __syncthreads();  // the previous item's reads of A are done
-  for (int i = tid; i < R.n_shells; i += kThreads) A.sh[i] = U.shells[R.shell_begin + i];
-  for (int i = tid; i < R.n_exp; i += kThreads) {
-    A.ex[i] = (T)gld(U.exps + it.e0 + i);
-    A.nm[i] = (T)gld(U.norms + it.e0 + i);
-  }
-  for (int i = tid; i < R.n_contr; i += kThreads) A.ct[i] = (T)gld(U.contr + it.c0 + i);
-  if (tid < R.n_atoms) {
-    const AtomD at = U.atoms[gld(U.ratoms + R.atom_begin + tid)];
-    A.ax[tid] = at.x;
-    A.ay[tid] = at.y;
-    A.az[tid] = at.z;
-    A.s0[tid] = at.shell_begin - R.shell_begin;
-    A.s1[tid] = at.shell_end - R.shell_begin;
-    A.lm[tid] = at.lmax;
-  }
-  if (tid < R.n_shells * (kThreads / kGroup))  // flag of (shell tid / 8, group tid % 8)
-    A.fl[tid / (kThreads / kGroup)][tid % (kThreads / kGroup)] =
-        (uint8_t)((U.bflags[8 * local + (tid >> 5)] >> (tid & 31)) & 1u);
-  __syncthreads();
-  return it;
+__device__ __forceinline__ ItemAtom item_atom(const UnitD &U, int rng, int a, unsigned mask) {
+  const RangeD *R = U.ranges + rng;
+  const AtomD *at = U.atoms + cld(U.ratoms + cld(&R->atom_begin) + a);
+  ItemAtom q;
+  q.s0 = cld(&at->shell_begin);
+  const int n = cld(&at->shell_end) - q.s0;  // at most kAtomShells
+  q.live = (mask >> (q.s0 - cld(&R->shell_begin))) & ((1u << n) - 1u);
+  q.x = cld(&at->x);
+  q.y = cld(&at->y);
+  q.z = cld(&at->z);
+  q.lmax = cld(&at->lmax);
+  return q;
 }
 
-// The staged range's atoms in turn at the thread's point, each shell written
-// on the point's group handed to put.
+// The basis items' walk: item `local` of unit U is a 256-point block and a range
+// of atoms; the shells of the range not cut off on a tile of the block are the
+// bits of bflags[2 local + tile].  A wave's 64 points lie in one tile, so which
+// shells it evaluates, and every table read, is uniform: scalar registers, no
+// LDS, and waves that wait for no other.
+__device__ __forceinline__ long item_point(const UnitD &U, long local) {
+  return (long)(cld(U.bitems + local) >> 16) * kThreads + threadIdx.x;
+}
+__device__ __forceinline__ unsigned item_mask(const UnitD &U, long local) {
+  return cld(U.bflags + 2 * local + (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >> 1));
+}
 template <bool GRAD, int LMAX, typename T, class Put>
-__device__ __forceinline__ void eval_basis_item(const RangeLds<T> &A, const BasisItem &it,
-                                                const Put &put) {
-  const int grp = threadIdx.x / kGroup;
-  const int na = __builtin_amdgcn_readfirstlane(it.n_atoms);
+__device__ __forceinline__ void eval_basis_item(const UnitD &U, long local, long p, const Put &put) {
+  const unsigned mask = item_mask(U, local);
+  if (!mask) return;
+  const int rng = (int)(cld(U.bitems + local) & 0xffffu), na = cld(&U.ranges[rng].n_atoms);
+  const double gx = gld(U.gx + p), gy = gld(U.gy + p), gz = gld(U.gz + p);
   for (int a = 0; a < na; ++a) {
-    const int sb = __builtin_amdgcn_readfirstlane(A.s0[a]), se = __builtin_amdgcn_readfirstlane(A.s1[a]);
-    bool any = false;
-    for (int s = sb; s < se; ++s) any = any || (A.fl[s][grp] & 1);
-    if (!any) continue;  // no stage reads this atom's values on the point's group
-    const T x = (T)(it.gx - A.ax[a]), y = (T)(it.gy - A.ay[a]), z = (T)(it.gz - A.az[a]);
+    const ItemAtom q = item_atom(U, rng, a, mask);
+    if (!q.live) continue;  // no stage reads this atom's values on the wave's tile
+    const T x = (T)(gx - q.x), y = (T)(gy - q.y), z = (T)(gz - q.z);
     // the kernel holds the registers of its largest case, so it is built
     // for the largest angular momentum of the list (every atom's lmax <= LMAX)
-    switch (__builtin_amdgcn_readfirstlane(A.lm[a])) {
-      case 0: basis_atom<0, GRAD>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 1: if constexpr (LMAX >= 1) basis_atom<1, GRAD>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 2: if constexpr (LMAX >= 2) basis_atom<2, GRAD>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      case 3: if constexpr (LMAX >= 3) basis_atom<3, GRAD>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
-      default: if constexpr (LMAX >= 4) basis_atom<4, GRAD>(A, sb, se, it.e0, it.c0, x, y, z, put, grp); break;
+    switch (q.lmax) {
+      case 0: basis_atom<0, GRAD>(U, q.s0, q.live, x, y, z, put); break;
+      case 1: if constexpr (LMAX >= 1) basis_atom<1, GRAD>(U, q.s0, q.live, x, y, z, put); break;
+      case 2: if constexpr (LMAX >= 2) basis_atom<2, GRAD>(U, q.s0, q.live, x, y, z, put); break;
+      case 3: if constexpr (LMAX >= 3) basis_atom<3, GRAD>(U, q.s0, q.live, x, y, z, put); break;
+      default: if constexpr (LMAX >= 4) basis_atom<4, GRAD>(U, q.s0, q.live, x, y, z, put); break;
     }
   }
 }

@@ -4,13 +4,13 @@
 //   hi = bf16(x), lo = bf16(x - hi)
 // and a product is formed from three v_mfma_f32_16x16x32_bf16 passes,
 //   a*b ~ a_lo*b_hi + a_hi*b_lo + a_hi*b_hi,   FP32 accumulation,
-// dropping a_lo*b_lo (relative 2^-16).  W (k_wmat) and D^T (k_prep) are
+// dropping a_lo*b_lo (relative 2^-16).  W (k_wbasis) and D^T (k_prep) are
 // stored split and k-contiguous, so their staging is a copy of 16-byte
 // vectors into LDS; the basis values are read in FP32 (as stored, points
 // contiguous) and split while they are staged, k-contiguous for the
 // potential and transposed for the density.
-// Same tiles and epilogues as the FP32/FP64 contractions (xc_kernels.hip);
-// K advances 32 per MFMA.
+// Items, partials and lists as for the FP32 and FP64 contractions
+// (xc_contract.h); K advances 32 per MFMA.
 #include <type_traits>
 
 #include "pgxc_internal.h"

@@ -18,6 +18,24 @@ template <typename T>
 __device__ __forceinline__ void gst(T *p, T v) {
   *(__attribute__((address_space(1))) T *)p = v;
 }
+// Access at column p of a row whose address is the same for the whole wave: the
+// instruction takes the scalar base and the lane's 32-bit byte offset (a unit has
+// at most 2^24 points), no address arithmetic per lane.
+template <typename T>
+__device__ __forceinline__ void gst_row(T *row, unsigned p, T v) {
+  auto *base = (__attribute__((address_space(1))) char *)row;
+  unsigned off = p * (unsigned)sizeof(T);
+  asm("" : "+v"(off));  // widened here, where the store's form is chosen
+  *(__attribute__((address_space(1))) T *)(base + off) = v;
+}
+
+template <typename T>
+__device__ __forceinline__ T gld_row(const T *row, unsigned p) {
+  const auto *base = (const __attribute__((address_space(1))) char *)row;
+  unsigned off = p * (unsigned)sizeof(T);
+  asm("" : "+v"(off));
+  return *(const __attribute__((address_space(1))) T *)(base + off);
+}
 
 // Workgroups are dispatched round-robin over the 8 XCDs; give every XCD a
 // contiguous range of tile ids so that tiles sharing an operand panel share
@@ -111,6 +129,9 @@ __device__ __forceinline__ void item_log(const StageList &S, long it, uint64_t t
 
 // x = hi + lo with hi = bf16(x), lo = bf16(x - hi)
 __device__ __forceinline__ void split_bf16(float x, __bf16 &hi, __bf16 &lo) {
+  // x stays a float: a conversion from FP64 before it must not be merged into
+  // the one to bf16, which the hardware has only from FP32 (9 instructions more)
+  asm("" : "+v"(x));
   hi = (__bf16)x;
   lo = (__bf16)(x - (float)hi);
 }

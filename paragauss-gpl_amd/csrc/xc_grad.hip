@@ -87,11 +87,12 @@ __device__ __forceinline__ void sh_along(Du x, Du y, Du z, Du *C, Du *Cx, Du *Cy
   }
 }
 
-// One point's inputs of the bracket: X and Z at the point's functions (stride
-// Mc; LDA: Z = 2 a X), b, and where the sum goes.
+// One point's inputs of the bracket: X and Z (rows of Mc, read at column p;
+// LDA: Z = 2 a X) and b.
 struct Bracket {
   const double *X, *Z;
   long Mc;
+  unsigned p;
   double a2, b[3];
 };
 
@@ -107,8 +108,8 @@ __device__ __forceinline__ void bracket_fn(const Bracket &B, long f0, int nf, do
 #pragma unroll
   for (int m = 0; m < 2 * L + 1; ++m) {
     const long q = (f0 + (long)m * nf) * B.Mc;
-    X[m] = gld(B.X + q);
-    Z[m] = GGA ? gld(B.Z + q) : B.a2 * X[m];
+    X[m] = gld_row(B.X + q, B.p);
+    Z[m] = GGA ? gld_row(B.Z + q, B.p) : B.a2 * X[m];
   }
   double u0[3] = {0.0, 0.0, 0.0}, u1[3] = {0.0, 0.0, 0.0}, zs = 0.0, xs = 0.0, xg = 0.0;
 #pragma unroll
@@ -138,28 +139,48 @@ __device__ __forceinline__ void bracket_fn(const Bracket &B, long f0, int nf, do
 }
 
 template <int L, bool GGA>
-__device__ __forceinline__ void bracket_shell(const Bracket &B, const ShellD &sh, const double *ex,
-                                              const double *nm, const double *ct, double x,
-                                              double y, double z, const Du *C, const Du *Cx,
+__device__ __forceinline__ void bracket_shell(const Bracket &B, const ShellD &sh, const double *tab,
+                                              double x, double y, double z, const Du *C, const Du *Cx,
                                               const Du *Cy, const Du *Cz, double (&t)[3]) {
   const int ne = sh.n_exp, nu = sh.n_unc, nc = sh.n_contr, nf = nu + nc;
   const double rr = x * x + y * y + z * z, bx = GGA ? B.b[0] * x + B.b[1] * y + B.b[2] * z : 0.0;
   double s0[kMaxContr], s1[kMaxContr], s2[kMaxContr];
 #pragma unroll
   for (int k = 0; k < kMaxContr; ++k) s0[k] = s1[k] = s2[k] = 0.0;
-  for (int e = 0; e < ne; ++e) {
-    const double al = ex[e], ar2 = al * rr;
-    double r0 = 0.0;
-    if (ar2 < 50.0) r0 = nm[e] * exp(-ar2);  // the value evaluation's cut-off
-    const double r1 = -2.0 * al * r0, r2 = -2.0 * al * r1;
-    if (e < nu) bracket_fn<L, GGA>(B, sh.func_off + e, nf, r0, r1, r2, x, y, z, bx, C, Cx, Cy, Cz, t);
+  for (int e0 = 0; e0 < ne; e0 += kPB) {  // as shell_emit
+    const PrimBlock<double> q(tab, nc, e0);
+    double r0[kPB], r1[kPB], r2[kPB];
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < kPB; ++i) any = any || q.al[i] * rr < 50.0;
+    const bool live = __ballot(any) != 0;
+#pragma unroll
+    for (int i = 0; i < kPB; ++i) r0[i] = 0.0;
+    if (live) {
+#pragma unroll
+      for (int i = 0; i < kPB; ++i) {
+        const double ar2 = q.al[i] * rr, v = q.nv[i] * exp(-ar2);
+        r0[i] = ar2 < 50.0 ? v : 0.0;  // the value evaluation's cut-off
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kPB; ++i) {
+      r1[i] = -2.0 * q.al[i] * r0[i];
+      r2[i] = -2.0 * q.al[i] * r1[i];
+      if (e0 + i < nu)
+        bracket_fn<L, GGA>(B, sh.func_off + e0 + i, nf, r0[i], r1[i], r2[i], x, y, z, bx, C, Cx, Cy, Cz, t);
+    }
+    if (!live) continue;
 #pragma unroll
     for (int k = 0; k < kMaxContr; ++k)
       if (k < nc) {
-        const double c = ct[k * ne + e];
-        s0[k] += r0 * c;
-        s1[k] += r1 * c;
-        s2[k] += r2 * c;
+#pragma unroll
+        for (int i = 0; i < kPB; ++i) {
+          const double c = q.coeff(k, i);
+          s0[k] += r0[i] * c;
+          s1[k] += r1[i] * c;
+          s2[k] += r2[i] * c;
+        }
       }
   }
 #pragma unroll
@@ -168,32 +189,22 @@ __device__ __forceinline__ void bracket_shell(const Bracket &B, const ShellD &sh
       bracket_fn<L, GGA>(B, sh.func_off + nu + k, nf, s0[k], s1[k], s2[k], x, y, z, bx, C, Cx, Cy, Cz, t);
 }
 
-// The brackets of one staged atom's shells at the thread's point.
+// The brackets of one atom's live shells at the thread's point.
 template <int LA, bool GGA>
-__device__ __forceinline__ void bracket_atom(const RangeLds<double> &A, int sb, int se, int e0, int c0,
-                                             int grp, const Bracket &B, double x, double y, double z,
-                                             double (&t)[3]) {
+__device__ __forceinline__ void bracket_atom(const UnitD &U, int s0, unsigned live, const Bracket &B,
+                                             double x, double y, double z, double (&t)[3]) {
   constexpr int NLM = (LA + 1) * (LA + 1);
   Du C[NLM], Cx[NLM], Cy[NLM], Cz[NLM];
   sh_along<LA>({x, B.b[0]}, {y, B.b[1]}, {z, B.b[2]}, C, Cx, Cy, Cz);
-  for (int s = sb; s < se; ++s) {
-    if (!(A.fl[s][grp] & 1)) continue;  // cut off on the point's tile
-    ShellD sh = A.sh[s];
-    sh.l = __builtin_amdgcn_readfirstlane(sh.l);
-    sh.n_exp = __builtin_amdgcn_readfirstlane(sh.n_exp);
-    sh.n_unc = __builtin_amdgcn_readfirstlane(sh.n_unc);
-    sh.n_contr = __builtin_amdgcn_readfirstlane(sh.n_contr);
-    sh.exp_off = __builtin_amdgcn_readfirstlane(sh.exp_off);
-    sh.contr_off = __builtin_amdgcn_readfirstlane(sh.contr_off);
-    sh.func_off = __builtin_amdgcn_readfirstlane(sh.func_off);
-    const double *ex = A.ex + (sh.exp_off - e0), *nm = A.nm + (sh.exp_off - e0);
-    const double *ct = A.ct + (sh.contr_off - c0);
+  for (; live; live &= live - 1) {
+    const ShellD sh = shell_at(U.shells + s0 + __builtin_ctz(live));
+    const double *tab = U.tabd + sh.tab;
     switch (sh.l) {
-      case 0: bracket_shell<0, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
-      case 1: if constexpr (LA >= 1) bracket_shell<1, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
-      case 2: if constexpr (LA >= 2) bracket_shell<2, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
-      case 3: if constexpr (LA >= 3) bracket_shell<3, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
-      case 4: if constexpr (LA >= 4) bracket_shell<4, GGA>(B, sh, ex, nm, ct, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 0: bracket_shell<0, GGA>(B, sh, tab, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 1: if constexpr (LA >= 1) bracket_shell<1, GGA>(B, sh, tab, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 2: if constexpr (LA >= 2) bracket_shell<2, GGA>(B, sh, tab, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 3: if constexpr (LA >= 3) bracket_shell<3, GGA>(B, sh, tab, x, y, z, C, Cx, Cy, Cz, t); break;
+      case 4: if constexpr (LA >= 4) bracket_shell<4, GGA>(B, sh, tab, x, y, z, C, Cx, Cy, Cz, t); break;
     }
   }
 }
@@ -212,49 +223,52 @@ __device__ __forceinline__ double wave_sum(double v) {
 // atom) when pm is given.  XZ = [2][NP][Mc] at the tiles' functions; st: the
 // build's coefficients a, b (planes stride np apart).  Bound by the reads of X
 // and Z and the registers of their use (two waves a SIMD; one: 0.80 ms).  Per
-// (H2O)16 chunk of 245 760 points 0.47 ms; storing the six second-derivative
-// planes of every function and point and reading 13 planes back twice, once per
-// sum, took 2.7 ms.
+// (H2O)16 chunk of 245 760 points 0.38 ms (0.48 with a range staged in LDS and a
+// branch per primitive; 0.67 when the items came through loads the compiler takes
+// for different lanes' and everything after them went per lane); storing the six
+// second-derivative planes of every function and point and reading 13 planes back
+// twice, once per sum, took 2.7 ms.
 template <bool GGA, int LMAX>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(LMAX <= 2 ? 2 : 1))) void k_bracket(const UnitD *__restrict__ unit,
                                                       const double *__restrict__ XZ,
                                                       const double *__restrict__ st, long np,
                                                       double *__restrict__ pm,
                                                       double *__restrict__ part) {
-  __shared__ RangeLds<double> A;
   const UnitD &U = *unit;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, grp = tid / kGroup;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long Mc = U.Mc, cs = (long)U.NP * Mc;
   for (long blk = blockIdx.x; blk < Mc / kThreads; blk += gridDim.x) {
     long i0 = 0, hi = U.nbi;  // the block's items: they are listed block by block
     while (i0 < hi) {
       const long mid = (i0 + hi) >> 1;
-      if ((long)(U.bitems[mid] >> 16) < blk) i0 = mid + 1; else hi = mid;
+      if ((long)(cld(U.bitems + mid) >> 16) < blk) i0 = mid + 1; else hi = mid;
     }
     const long p = blk * kThreads + tid;
     Bracket B;
-    B.X = XZ + p;
-    B.Z = XZ + cs + p;
+    B.X = XZ;
+    B.Z = XZ + cs;
     B.Mc = Mc;
+    B.p = (unsigned)p;
     B.a2 = 2.0 * st[(S_A)*np + p];
     for (int d = 0; d < 3; ++d) B.b[d] = GGA ? st[(S_BX + d) * np + p] : 0.0;
+    const double r[3] = {gld(U.gx + p), gld(U.gy + p), gld(U.gz + p)};
     double tp[3] = {0.0, 0.0, 0.0};
-    for (long item = i0; item < U.nbi && (long)(U.bitems[item] >> 16) == blk; ++item) {
-      const BasisItem it = stage_basis_item(U, item, A);
-      const int na = __builtin_amdgcn_readfirstlane(it.n_atoms);
+    for (long item = i0; item < U.nbi && (long)(cld(U.bitems + item) >> 16) == blk; ++item) {
+      const unsigned mask = item_mask(U, item);
+      const int rng = (int)(cld(U.bitems + item) & 0xffffu), na = cld(&U.ranges[rng].n_atoms);
       for (int a = 0; a < na; ++a) {
-        const int sb = __builtin_amdgcn_readfirstlane(A.s0[a]), se = __builtin_amdgcn_readfirstlane(A.s1[a]);
-        bool any = false;
-        for (int s = sb; s < se; ++s) any = any || (A.fl[s][grp] & 1);
+        const ItemAtom q = item_atom(U, rng, a, mask);
         double t[3] = {0.0, 0.0, 0.0};
-        if (any) {
-          const double x = it.gx - A.ax[a], y = it.gy - A.ay[a], z = it.gz - A.az[a];
-          switch (__builtin_amdgcn_readfirstlane(A.lm[a])) {
-            case 0: bracket_atom<0, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
-            case 1: bracket_atom<1, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
-            case 2: if constexpr (LMAX >= 2) bracket_atom<2, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
-            default: if constexpr (LMAX >= 4) bracket_atom<4, GGA>(A, sb, se, it.e0, it.c0, grp, B, x, y, z, t); break;
-          }
+        if (!q.live) {
+          if (lane < 3) part[((item * kRangeAtoms + a) * 4 + wave) * 3 + lane] = 0.0;
+          continue;
+        }
+        const double x = r[0] - q.x, y = r[1] - q.y, z = r[2] - q.z;
+        switch (q.lmax) {
+          case 0: bracket_atom<0, GGA>(U, q.s0, q.live, B, x, y, z, t); break;
+          case 1: bracket_atom<1, GGA>(U, q.s0, q.live, B, x, y, z, t); break;
+          case 2: if constexpr (LMAX >= 2) bracket_atom<2, GGA>(U, q.s0, q.live, B, x, y, z, t); break;
+          default: if constexpr (LMAX >= 4) bracket_atom<4, GGA>(U, q.s0, q.live, B, x, y, z, t); break;
         }
         for (int d = 0; d < 3; ++d) {
           tp[d] += t[d];

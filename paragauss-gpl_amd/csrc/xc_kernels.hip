@@ -6,7 +6,7 @@
 //                 2421-2619; solid harmonics modules/solid_harmonics_module.f90:369-568)
 //   k_functional  Slater + PW92 + PBE-x + PBE-c in FP64, closed-form derivatives
 //                 (modules/xc_func.f90:187-305 and the term modules)
-//   k_wmat        W = a Phi + b . grad Phi  (modules/xc_hamiltonian.f90:1429-1483)
+//   k_wbasis      W = a Phi + b . grad Phi  (modules/xc_hamiltonian.f90:1429-1483)
 //   k_pack        V = H + H^T into the packed lower triangle (:1561-1567)
 #include <type_traits>
 
@@ -166,24 +166,23 @@ __device__ __forceinline__ long item_at(const int *__restrict__ order, long L, l
 }
 
 // ------------------------------------------------------------------- basis
-// item = (256-point block, range of atoms) of a unit; one thread per point,
-// walking the range's atoms.  The workgroup first stages the range's shells,
-// primitives, coefficients and atom centres and the per-(shell, group) write
-// flags in LDS, all loads in flight together, so the evaluation itself waits
-// on no global load.  The items are the (block, range) pairs whose values a
-// later stage reads; only the shells read on each point's group are written.
+// item = (256-point block, range of atoms) of a unit, of the pairs whose values a
+// later stage reads; one thread per point, walking the range's atoms.  The tables
+// are read by scalar loads (a shell's block of four primitives in one wait), rows
+// addressed by the wave; staging a range in LDS behind two barriers, with row
+// addresses per lane, took for an (H2O)32 build, one lane, 1.67 ms in FP32 (now
+// 1.50: the writes, 7.0 GB a build, at 4.6 TB/s) and 3.06 in FP64 (2.88).
 template <bool GRAD, typename T, int LMAX>
 __global__ __launch_bounds__(kThreads) void k_basis(const UnitD *__restrict__ units, int nu,
                                                     const long *__restrict__ base,
                                                     const int *__restrict__ order, long total) {
-  __shared__ RangeLds<T> A;
   for (long L = blockIdx.x; L < total; L += gridDim.x) {
     const long item = item_at(order, L, total);
     const int u = find_unit(base, nu, item);
     const UnitD &U = units[u];
-    const BasisItem it = stage_basis_item(U, item - base[u], A);
-    const StorePhi<T> put{(T *)U.phi, U.Mc, (long)U.NP * U.Mc, (int)it.p};
-    eval_basis_item<GRAD, LMAX>(A, it, put);
+    const long local = item - base[u], p = item_point(U, local);
+    const StorePhi<T> put{(T *)U.phi, U.Mc, (long)U.NP * U.Mc, (unsigned)p};
+    eval_basis_item<GRAD, LMAX, T>(U, local, p, put);
   }
 }
 
@@ -194,14 +193,15 @@ template <typename T, bool SPLIT, int NS>
 struct StoreW {
   void *w[2];
   long Mc, cs;
-  int p;
+  unsigned p;
   double a[2], b0[2], b1[2], b2[2];
   template <int L, bool GRAD>
   __device__ __forceinline__ void emit(long f0, int nf, T r0, T r1, T x, T y, T z, const T *C,
                                        const T *Cx, const T *Cy, const T *Cz) const {
+    long row = f0 * Mc;  // rows' addresses are the wave's, the lane's point a 32-bit offset
+    const long step = nf * Mc;
 #pragma unroll
-    for (int m = 0; m < 2 * L + 1; ++m) {
-      const long q = (f0 + (long)m * nf) * Mc + p;
+    for (int m = 0; m < 2 * L + 1; ++m, row += step) {
       T v, gx = T(0), gy = T(0), gz = T(0);
       fn_values<L, GRAD>(m, r0, r1, x, y, z, C, Cx, Cy, Cz, v, gx, gy, gz);
 #pragma unroll
@@ -212,10 +212,10 @@ struct StoreW {
         if constexpr (SPLIT) {
           __bf16 h, l;
           split_bf16((float)u, h, l);
-          gst((uint16_t *)w[sp] + q, __builtin_bit_cast(uint16_t, h));
-          gst((uint16_t *)w[sp] + cs + q, __builtin_bit_cast(uint16_t, l));
+          gst_row((uint16_t *)w[sp] + row, p, __builtin_bit_cast(uint16_t, h));
+          gst_row((uint16_t *)w[sp] + row + cs, p, __builtin_bit_cast(uint16_t, l));
         } else {
-          gst((T *)w[sp] + q, (T)u);
+          gst_row((T *)w[sp] + row, p, (T)u);
         }
       }
     }
@@ -228,33 +228,34 @@ struct StoreW {
 // potential reads (TWO: both spins of an open-shell unit).  Trades the reads of
 // four planes for the evaluation: functional and W of an (H2O)32 build, one
 // lane, FP64 4.48 -> 2.64 ms, FP32 2.28 -> 1.77; 14-atom open shell 284 -> 140
-// us, 23-atom LDA 127 -> 92; one water 23 -> 23.
+// us, 23-atom LDA 127 -> 92; one water 23 -> 23.  Bound by vector instructions (50
+// a wave and function, a third of them exponentials): with tables from scalar
+// loads, rows addressed by the wave and one conversion to bf16 instead of an
+// emulated one from FP64, FP64 1.71 ms, FP32 1.23, split BF16 2.02 -> 1.32.
 template <typename T, bool SPLIT, bool GRAD, bool TWO, int LMAX>
 __global__ __launch_bounds__(kThreads) void k_wbasis(const UnitD *__restrict__ units, int nu,
                                                      const long *__restrict__ base,
                                                      const int *__restrict__ order, long total) {
-  __shared__ RangeLds<T> A;
   constexpr int NS = TWO ? 2 : 1;
   for (long L = blockIdx.x; L < total; L += gridDim.x) {
     const long item = item_at(order, L, total);
     const int u = find_unit(base, nu, item);
     const UnitD &U = units[u];
-    const BasisItem it = stage_basis_item(U, item - base[u], A);
-    const long Mc = U.Mc;
+    const long local = item - base[u], p = item_point(U, local), Mc = U.Mc;
     StoreW<T, SPLIT, NS> put;
     put.Mc = Mc;
     put.cs = (long)U.NP * Mc;
-    put.p = (int)it.p;
+    put.p = (unsigned)p;
 #pragma unroll
     for (int sp = 0; sp < NS; ++sp) {
       const double *cf = sp ? U.coef2 : U.coef;
       put.w[sp] = sp ? U.W2 : U.W;
-      put.a[sp] = gld(cf + it.p);
-      put.b0[sp] = GRAD ? gld(cf + Mc + it.p) : 0.0;
-      put.b1[sp] = GRAD ? gld(cf + 2 * Mc + it.p) : 0.0;
-      put.b2[sp] = GRAD ? gld(cf + 3 * Mc + it.p) : 0.0;
+      put.a[sp] = gld(cf + p);
+      put.b0[sp] = GRAD ? gld(cf + Mc + p) : 0.0;
+      put.b1[sp] = GRAD ? gld(cf + 2 * Mc + p) : 0.0;
+      put.b2[sp] = GRAD ? gld(cf + 3 * Mc + p) : 0.0;
     }
-    eval_basis_item<GRAD, LMAX>(A, it, put);
+    eval_basis_item<GRAD, LMAX, T>(U, local, p, put);
   }
 }
 

@@ -127,3 +127,41 @@ def test_density_from_orbitals(n, nocc, spins):
     # sums of at most 33 products of order 1 in both: P to some 1e-15
     assert np.max(np.abs(h0 - h1)) <= 1e-12 * max(1.0, np.max(np.abs(h0)))
     assert abs(e0 - e1) <= 1e-12 * max(1.0, abs(e0)) and abs(q0 - q1) <= 1e-12 * max(1.0, abs(q0))
+
+
+def _shell_basis(lmax, rng):
+    """Three atoms; the first with the most shells an atom may have: 1 to 9
+    primitives (blocks of 4 and their remainders), 0 to 8 contractions."""
+    shells = []
+    for a, count in ((0, 16), (1, 3), (2, 1)):
+        for s in range(count):
+            ne, nc = 1 + (5 * s + a) % 9, (3 * s + 2 * a) % 9
+            nu = 1 if nc == 0 else s % 2
+            l = s % (lmax + 1)
+            ex = np.sort(np.exp(rng.uniform(np.log(0.3), np.log(20.0), ne)))[::-1].copy()
+            shells.append(Shell(a, l, ex, min(nu, ne), rng.uniform(-0.6, 0.6, (ne, nc))))
+    b = Basis(np.array([(0.0, 0.0, 0.0), (1.1, 0.2, -0.3), (-0.4, 1.3, 0.9)]))
+    b.shells = shells
+    return b
+
+
+@pytest.mark.parametrize("lmax", [0, 2, 3, 4])
+@pytest.mark.parametrize("spins", [1, 2])
+def test_shell_tables(lmax, spins):
+    """Every count of primitives and contractions a block of a shell's table can
+    end with, on both tiles of a block, in the basis, W and gradient stages."""
+    from test_gpu_gradient import check, fd_gradient
+    rng = np.random.default_rng(31 * lmax + spins)
+    b = _shell_basis(lmax, rng)
+    g = _grid(b, 300, rng)
+    n, m = b.nbas, 3
+    C = [np.linalg.qr(rng.normal(size=(n, m)))[0] for _ in range(spins)]
+    P = C[0] @ C[0].T if spins == 1 else np.stack([c @ c.T for c in C], axis=2)
+    with XCBuilder(b, g) as xc:
+        xc.set_density(P)
+        for f, mask in (("LDA", oracle.MASK_LDA), ("PBE", oracle.MASK_PBE)):
+            ref = oracle.xc_build(b, g, mask, P=P, nthreads=4, ispin=spins)
+            for prec, rel in (("fp32", 2e-6), ("bf16x3", 5e-5), ("fp64", 0.0)):
+                _check(xc.build(f, prec), ref, rel)
+            if spins == 1 and lmax in (2, 4):
+                check(xc.gradient(), fd_gradient(b, g, mask, P=P))
