@@ -669,10 +669,10 @@ def main():
     flops = stats["flops"] / 2.0
     achieved = flops / (st[dom] * 1e-3) / 1e12
     if best == "bf16x3":
-        kname = "k_%s_bf16x3<%d%s>" % (dom, tf, ",true" if dom == "density" else "")
+        kname = "k_density_bf16x3<true,128>" if dom == "density" else "k_potential_bf16x3<%d>" % tf
     else:
         v = layout["variant_fp32"]
-        kname = "k_%s<float,%d,%d%s>" % (dom, tf, v, ",true" if dom == "density" else "")
+        kname = "k_density<float,64,%d,true>" % v if dom == "density" else "k_potential<float,%d,%d>" % (tf, v)
     mfma = {"achieved": achieved, "peak": peak,
             "unit": "TFLOP/s" + (" (FP32-equivalent: BF16 peak / 3 passes)" if best == "bf16x3" else ""),
             "frac": achieved / peak,
