@@ -148,13 +148,14 @@ struct pgxc_ctx {
   size_t phi_stride = 0;
   int skip_basis = 0;        // the current build reads cached basis values
   double *part = nullptr, *coef = nullptr;
-  // potential partials: slots of one chunk's splits each (hstride doubles),
-  // hslots of them over all lanes; every chunk its own slot, or (hflush) as
-  // many as kPartialBytes hold, summed into HS whenever a lane's are full.
+  // potential partials (hsize doubles): those of all chunks, or (hflush, when
+  // they pass kPartialBytes) of as many chunks as a lane's share holds, summed
+  // into HS whenever it is full: after the chunks k with h_flush[lanes - 1][k].
   // HS: [nseg][NP][NP] their symmetric sums
   double *Hc = nullptr, *HS = nullptr;
-  long hstride = 0;
-  int hslots = 0, hflush = 0, nseg = 1;
+  long hsize = 0;
+  int hflush = 0, nseg = 1;
+  std::vector<char> h_flush[2];
   // open shell (ispin = 2): the fields above and below serve the alpha spin,
   // these the beta spin (allocated with the first open-shell density; the
   // basis values and the work tables are shared)
@@ -558,10 +559,8 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       U.state = c->state + p0;
       U.epart = c->epart + 2 * (p0 / kThreads);
       U.eterm = c->eterm + 5 * (p0 / kThreads);
-      const int L = lanes_of(c), R = c->hslots / L;  // the lane's share of the slots
-      const size_t hslot = (size_t)(k % L) * R + (k / L) % R;
-      U.Hc = c->Hc + hslot * c->hstride;
-      U.ho = c->ho + (long)k * c->nsp;
+      U.Hc = c->Hc;
+      U.ho = c->ho + ((long)(lanes_of(c) - 1) * c->nchunks + k) * c->nsp;
       U.Mc = c->Mc;
       U.npad = c->npad;
       U.n_atoms = c->n_atoms;
@@ -595,7 +594,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
         B.part = c->beta.part + (size_t)lane * c->nparts * 4 * c->Mc;
         B.coef = c->beta.coef + (size_t)lane * 4 * c->Mc;
         B.state = c->beta.state + p0;
-        B.Hc = c->beta.Hc + hslot * c->hstride;
+        B.Hc = c->beta.Hc;
         U.part2 = B.part;
         U.coef2 = B.coef;
         U.state2 = B.state;
@@ -759,25 +758,21 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     pbase[q + 1] = pbase[q] + (npk + kThreads - 1) / kThreads;
     qbase[q + 1] = qbase[q] + (Q.NP * Q.NP + kThreads - 1) / kThreads;
   }
-  // sums of the potential partials: after the step that fills a lane's slots
-  // or ends the lane (molecules with more chunks than slots), else all at the
-  // end, in segments of the splits
+  // sums of the potential partials: after the steps that fill a lane's share or
+  // end the lane (hflush), else all at the end, in segments of the splits
   auto fold_of = [&](const pgxc_ctx *c, int sp) {
     FoldD F;
     memset(&F, 0, sizeof(F));
     F.Hc = sp ? c->beta.Hc : c->Hc;
-    F.ho = c->ho;
+    F.ho = c->ho + (long)(lanes_of(c) - 1) * c->nchunks * c->nsp;
     F.su_off = c->su_off;
     F.pos = c->pos;
     F.rbits = c->rbits;
     F.out = sp ? c->beta.HS : c->HS;
-    F.stride = c->hstride;
     F.NP = c->NP;
     F.nsplit = c->nsp;
     F.bytes_c = (c->nsp + 7) / 8;
     F.nbytes = F.bytes_c * c->nchunks;
-    F.lanes = lanes_of(c);
-    F.slots = c->hslots / F.lanes;
     return F;
   };
   struct FoldOff {
@@ -815,18 +810,20 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
         }
         continue;
       }
-      F.step = F.lanes;
+      F.step = lanes_of(c);
       F.nseg = 1;
       double *out = F.out;
-      for (int k = 0; k < c->nchunks; ++k) {
-        const int j = k / F.lanes, ln = k % F.lanes;
-        if ((j + 1) % F.slots != 0 && k + F.lanes < c->nchunks) continue;
-        const int j0 = j / F.slots * F.slots;
+      for (int ln = 0; ln < F.step; ++ln) {
         F.out = out + (size_t)ln * c->NP * c->NP;
-        F.chunk0 = j0 * F.lanes + ln;
-        F.nchunks = j - j0 + 1;
-        F.acc = j0 > 0;
-        flush[(size_t)k].push_back(F);
+        F.chunk0 = ln;
+        F.acc = 0;
+        for (int k = ln; k < c->nchunks; k += F.step) {
+          if (!c->h_flush[F.step - 1][(size_t)k]) continue;
+          F.nchunks = (k - F.chunk0) / F.step + 1;
+          flush[(size_t)k].push_back(F);
+          F.chunk0 = k + F.step;
+          F.acc = 1;
+        }
       }
     }
   }
@@ -1254,7 +1251,7 @@ static int upload(pgxc_ctx *c, V **dst, const std::vector<V> &src) {
 }
 
 static int alloc_partials(pgxc_ctx *c, double **Hc, double **HS) {
-  int rc = dalloc(c, Hc, (size_t)c->hslots * c->hstride);
+  int rc = dalloc(c, Hc, (size_t)c->hsize);
   if (rc) return rc;
   return dalloc(c, HS, (size_t)std::max(c->nseg, c->nlanes_cap) * c->NP * c->NP);
 }
@@ -1385,10 +1382,9 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
   c->h_su_off.assign(1, 0);
   c->h_su.clear();
   c->h_sumask.clear();
-  std::vector<long> ho((size_t)NS);
+  std::vector<long> ho((size_t)(2 * NS)), hc((size_t)c->nchunks);  // ho: for one and for two lanes
   std::vector<uint16_t> pos((size_t)NS * c->NP, 0xffff);
   std::vector<uint8_t> rbits((size_t)(c->NP / 32) * bpc * c->nchunks, 0);
-  c->hstride = 1;
   {
     std::vector<uint32_t> tm((size_t)c->NP);
     long at = 0;
@@ -1411,8 +1407,44 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
       ho[(size_t)S] = at;
       const long ld = round_up((long)(c->h_su.size() - u0), 16);
       at += ld * ld;
-      c->hstride = std::max(c->hstride, at);
+      hc[(size_t)(S / c->nsp)] = at;
     }
+  }
+  // Room for all chunks' partials, or kPartialBytes shared by the lanes (at least
+  // a chunk each): a lane's chunks lie one behind the other until the next does
+  // not fit.  Chunks differ (outer points need more functions): by their own sizes
+  // the 159 chunks of (H2O)128 and solute fill it 21 times on two lanes, in slots of the largest
+  // 54 times, and every sum reads and writes the N^2 sums (fold kernels of a build
+  // 49 -> 35 ms, two builds of a step 506 -> 485 ms).
+  {
+    const long cap = kPartialBytes / 8, most = *std::max_element(hc.begin(), hc.end());
+    const long total = std::accumulate(hc.begin(), hc.end(), 0L);
+    c->hflush = total > cap;
+    c->hsize = c->hflush ? c->nlanes_cap * std::max(most, cap / c->nlanes_cap) : std::max(total, 1L);
+    const std::vector<long> rel(ho.begin(), ho.begin() + NS);
+    for (int lanes = 1; lanes <= 2; ++lanes) {
+      std::vector<char> &fl = c->h_flush[lanes - 1];
+      fl.assign((size_t)c->nchunks, 0);
+      const long share = c->hsize / std::min(lanes, c->nlanes_cap);
+      for (int ln = 0; ln < lanes; ++ln) {
+        long at = 0;
+        for (int k = ln; k < c->nchunks; k += lanes) {
+          if (c->hflush && at + hc[(size_t)k] > share) {
+            fl[(size_t)(k - lanes)] = 1;
+            at = 0;
+          }
+          const long base = c->hflush ? ln * share + at : std::accumulate(hc.begin(), hc.begin() + k, 0L);
+          for (int j = 0; j < c->nsp; ++j)
+            ho[(size_t)((lanes - 1) * NS + (long)k * c->nsp + j)] = base + rel[(size_t)((long)k * c->nsp + j)];
+          at += hc[(size_t)k];
+          if (k + lanes >= c->nchunks) fl[(size_t)k] = 1;
+        }
+      }
+    }
+    if (getenv("PGXC_DEBUG"))
+      fprintf(stderr, "pgxc: partials %.4g bytes in %.4g, sums %d times on one lane, %d on two\n", 8.0 * total,
+              8.0 * c->hsize, (int)std::count(c->h_flush[0].begin(), c->h_flush[0].end(), 1),
+              (int)std::count(c->h_flush[1].begin(), c->h_flush[1].end(), 1));
   }
   if ((rc = upload(c, &c->ho, ho))) return rc;
   if ((rc = upload(c, &c->pos, pos))) return rc;
@@ -1454,9 +1486,9 @@ static int setup_screen(pgxc_ctx *c, const std::vector<ShellD> &sh, const double
       for (size_t t = 0; t + 1 < c->h_tf_off.size(); ++t) ev += (double)kScreenTile * (c->h_tf_off[t + 1] - c->h_tf_off[t]);
       for (long S = 0; S < NS; ++S) hu += c->h_su_off[(size_t)S + 1] - c->h_su_off[(size_t)S];
       fprintf(stderr, "pgxc: basis items %zu (of %ld), elements per build %.4g; %ld splits of %ld points, "
-                      "%.1f functions each; partials of a chunk %.4g bytes\n",
+                      "%.1f functions each\n",
               bi.size(), (long)c->nchunks * (c->Mc / kThreads) * c->n_ranges, ev, NS, c->Mc / c->nsp,
-              hu / NS, 8.0 * c->hstride);
+              hu / NS);
     }
   }
   // work items per chunk
@@ -1758,13 +1790,7 @@ int pgxc_create_opt(pgxc_ctx **out, int32_t n_atoms, const double *atom_xyz, int
   const size_t L = (size_t)c->nlanes_cap;
   if ((rc = dalloc(c, &c->part, L * c->nparts * 4 * c->Mc))) return rc;
   if ((rc = dalloc(c, &c->coef, L * 4 * c->Mc))) return rc;
-  // a slot for every chunk where they fit kPartialBytes, else as many per lane
-  // as do (summed whenever they are full); sums in enough segments of the splits
-  // that a small matrix still fills the device
-  const long slot_b = 8 * c->hstride;
-  const long want = round_up(c->nchunks, (long)L);
-  c->hflush = want * slot_b > kPartialBytes;
-  c->hslots = (int)(c->hflush ? std::max<long>(1, kPartialBytes / slot_b / (long)L) * (long)L : want);
+  // sums in enough segments of the splits that a small matrix still fills the device
   const long nb32 = c->NP / 32, pairs = nb32 * (nb32 + 1) / 2;
   const long ns = (long)c->nchunks * c->nsp;
   c->nseg = (int)std::min<long>({std::max<long>(kFoldItems / pairs, (ns + 63) / 64), (ns + 3) / 4, 32L});

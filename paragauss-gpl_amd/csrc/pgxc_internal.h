@@ -119,8 +119,8 @@ struct PackD {
 
 // Sums of a molecule's potential partials (k_fold): chunks chunk0, chunk0 +
 // step, ... (nchunks of them), of their mask bytes the share seg of nseg, into
-// out[NP][NP] (added to it when acc is set).  Chunk k's partials lie in slot
-// (k % lanes) * slots + (k / lanes) % slots of Hc.  pos[split][NP]: a
+// out[NP][NP] (added to it when acc is set).  Split s's partial lies at ho[s]
+// of Hc.  pos[split][NP]: a
 // function's place in the split's list (0xffff: absent); rbits[row block of 32
 // functions][nbytes]: a bit per split, whether it has any of the block's
 // functions (bytes_c bytes per chunk).
@@ -131,8 +131,8 @@ struct FoldD {
   const uint16_t *pos;
   const uint8_t *rbits;
   double *out;
-  long stride, NP;
-  int nsplit, bytes_c, nbytes, lanes, slots, chunk0, step, nchunks, seg, nseg, acc, pad;
+  long NP;
+  int nsplit, bytes_c, nbytes, chunk0, step, nchunks, seg, nseg, acc, pad;
 };
 
 // One launch's items: prefix offsets base[0..nu] over units, optional order.

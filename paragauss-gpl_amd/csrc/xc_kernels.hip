@@ -815,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void k_fold(const FoldD *__restrict__ fol
           const long S = (long)k * F.nsplit + sl;
           ls[q] = (int)S;
           ld[q] = split_ld(F.su_off[S + 1] - F.su_off[S]);
-          hp[q] = F.Hc + (long)((k % F.lanes) * F.slots + (k / F.lanes) % F.slots) * F.stride + F.ho[S];
+          hp[q] = F.Hc + F.ho[S];
         }
         if (tid == 0) cnt = __popcll(lv);
       }

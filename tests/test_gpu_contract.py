@@ -165,3 +165,27 @@ def test_shell_tables(lmax, spins):
                 _check(xc.build(f, prec), ref, rel)
             if spins == 1 and lmax in (2, 4):
                 check(xc.gradient(), fd_gradient(b, g, mask, P=P))
+
+
+def test_partials_of_uneven_chunks(monkeypatch, capfd):
+    """Chunks of different sizes laid one behind the other in a lane's share of
+    the partials: one lane and two, which sum them after different chunks, agree
+    with the sums over every function (all chunks the same size)."""
+    monkeypatch.setenv("PGXC_DEBUG", "1")
+    els, xyz = systems.water_cluster(64, seed=4, jitter_a=0.2)
+    b = basis.seeded_basis(els, xyz, seed=13, shell_set="medium")
+    g = grid.molecular_grid(els, xyz, nrad=40, nang=302, partition="gpu")
+    C, occ = systems.random_orbitals(b.nbas, 40, seed=6)
+    out = []
+    for screen, lanes in ((True, 1), (True, 2), (False, 2)):
+        with XCBuilder(b, g, screen=screen, chunk_points=16384, basis_cache=False) as xc:
+            if screen:
+                said = [l for l in capfd.readouterr().err.splitlines() if "sums" in l][-1].split()
+                one, two = int(said[said.index("sums") + 1]), int(said[-3])
+                assert one > 1 and two > 2, said
+            xc.set_lanes(lanes)
+            xc.set_orbitals(C, occ)
+            out.append(xc.build("PBE", "fp64"))
+    for h, e, q in out[1:]:
+        assert np.max(np.abs(h - out[0][0])) <= 1e-10
+        assert abs(e - out[0][1]) <= 1e-9 and abs(q - out[0][2]) <= 1e-9
