@@ -261,6 +261,10 @@ void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *
 
 // Becke partition weights of points owned by atoms (grid generation)
 void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv);
+// up to kAllPairs centres every pair is formed: kernel on molecules' grids of 15 to
+// 300 thousand points, all pairs / near centres first, 3 atoms 9 / 10.5 us, 8
+// 19 / 24, 11 40 / 47, 12 46 / 49, 13 54 / 55, 14 73 / 69, 16 94 / 80, 24 263 / 172
+constexpr int kAllPairs = 12;
 // npts points with coordinates stride apart
 void launch_becke(hipStream_t s, int na, const double *axyz, const double *inv_dist, long npts,
                   long stride, const double *pts, const int *owner, const double *wat, double *wout);

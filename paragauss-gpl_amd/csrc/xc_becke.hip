@@ -17,6 +17,38 @@ __device__ __forceinline__ double becke_s(double mu) {
   return 0.5 - n3 * (1.0 / 16384.0);
 }
 
+// Every cell's product over all pairs of centres, one point per thread: for few
+// centres (launch_becke), where the search for the near ones costs more than it
+// leaves out.  A lone centre takes the whole weight at any point.
+__global__ __launch_bounds__(kThreads) void k_becke_all(int na, const double *__restrict__ axyz,
+                                                        const double *__restrict__ inv_dist,
+                                                        long npts, long stride,
+                                                        const double *__restrict__ pts,
+                                                        const int *__restrict__ owner,
+                                                        const double *__restrict__ wat,
+                                                        double *__restrict__ wout) {
+  const long p = (long)blockIdx.x * kThreads + threadIdx.x;
+  if (p >= npts) return;
+  const double x = pts[p], y = pts[stride + p], z = pts[2 * stride + p];
+  const int own = owner[p];
+  auto dist = [&](int i) {
+    const double dx = axyz[3 * i] - x, dy = axyz[3 * i + 1] - y, dz = axyz[3 * i + 2] - z;
+    return sqrt(dx * dx + dy * dy + dz * dz);
+  };
+  double sum = 0.0, pown = 0.0;
+  for (int i = 0; i < na; ++i) {
+    const double ri = dist(i);
+    double pi = 1.0;
+    for (int k = 0; k < na; ++k) {
+      if (k == i) continue;
+      pi *= becke_s((ri - dist(k)) * inv_dist[(long)i * na + k]);
+    }
+    sum += pi;
+    if (i == own) pown = pi;
+  }
+  wout[p] = wat[p] * (pown / sum);
+}
+
 // One point per thread.  Written out, P_i = prod_k s(mu_ik) over all pairs is
 // FP64 arithmetic on n^2 pairs a point, and almost all of the P_i are too small
 // to change a bit of their sum: a centre far from the point has a factor of
@@ -156,7 +188,8 @@ void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv) {
 
 void launch_becke(hipStream_t s, int na, const double *axyz, const double *inv_dist, long npts,
                   long stride, const double *pts, const int *owner, const double *wat, double *wout) {
-  hipLaunchKernelGGL(k_becke, dim3((unsigned)((npts + kThreads - 1) / kThreads)), dim3(kThreads),
-                     0, s, na, axyz, inv_dist, npts, stride, pts, owner, wat, wout);
+  hipLaunchKernelGGL(na <= kAllPairs ? k_becke_all : k_becke,
+                     dim3((unsigned)((npts + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, na, axyz, inv_dist,
+                     npts, stride, pts, owner, wat, wout);
 }
 }  // namespace pgxc

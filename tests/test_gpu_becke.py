@@ -72,3 +72,27 @@ def test_moving_grid_gradient_against_fixed_grid_sums(na, spins):
     # the sum over atoms cancels terms of the size of the per-point sums (about
     # npts of order 1 to 10 each) to FP64 rounding
     assert np.max(np.abs(f.sum(axis=0))) < 1e-16 * 10 * len(own)
+
+
+def test_lone_centre_takes_the_whole_weight():
+    """One centre: its weights are the one-centre weights at every point, also
+    where the distance overflows or is no number."""
+    pts = np.zeros((70, 3))
+    pts[1:6] = [[1e200, 0, 0], [0, -1e160, 2], [np.inf, 1, 1], [0, 0, np.nan], [1e-300, 0, 0]]
+    wat = np.linspace(0.1, 2.0, 70)
+    w = becke_weights(np.zeros((1, 3)), pts, np.zeros(70, dtype=np.int32), wat)
+    assert np.array_equal(w, wat)
+
+
+@pytest.mark.parametrize("na", [11, 12, 13, 14])
+@pytest.mark.parametrize("npts", [1, 63, 257, 4097])
+def test_weights_where_the_kernel_changes(na, npts):
+    """Up to 12 centres every pair is formed, above that the near ones first."""
+    xyz = systems.random_molecule(14, seed=3)[1][:na]
+    rng = np.random.default_rng(100 * na + npts)
+    pts, own = _points(rng, xyz, max(npts, na + 1))
+    pts, own = pts[:npts], own[:npts]
+    wat = rng.uniform(0.1, 2.0, npts)
+    got = becke_weights(xyz, pts, own, wat)
+    ref = grid.becke_numpy(xyz, pts, own, wat)
+    assert np.max(np.abs(got - ref) / wat) < 1e-13 * 27 / 16 * na  # as above
