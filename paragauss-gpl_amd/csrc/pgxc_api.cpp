@@ -2525,14 +2525,19 @@ int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, co
       const double dz = atom_xyz[3 * i + 2] - atom_xyz[3 * k + 2];
       if (!(dx * dx + dy * dy + dz * dz > 0.0)) return PGXC_ERR_ARG;  // coincident centres
     }
-  // Points go in parts of kBeckePart: a part's upload (from the caller's pageable
-  // memory, which the copy has read when it returns) runs while the parts before
-  // it are computed, and its weights come back while those after it are.
+  // Many centres and points go in parts of kBeckePart: a part's upload (from the
+  // caller's pageable memory, which the copy has read when it returns) runs while
+  // the parts before it are computed, and its weights come back while those after
+  // it are.  The kernel of few centres is a small share of its transfers, and one
+  // part has nothing to overlap: one stream and no events then (a call of 3 atoms
+  // with 41 000 points 250 us with them, 173 without).
+  const int64_t per = n_atoms > kAllPairs ? kBeckePart : std::max<int64_t>(npts, 1);
   const size_t ninv = (size_t)n_atoms * n_atoms, na3 = 3 * (size_t)n_atoms;
-  const int64_t parts = (npts + kBeckePart - 1) / kBeckePart;
+  const int64_t parts = (npts + per - 1) / per;
+  const bool overlap = parts > 1;
   double *dev = nullptr;  // centres, inverse distances, points (3), weights in, weights out; owners
-  hipStream_t s = nullptr, sc = nullptr;
-  std::vector<hipEvent_t> up((size_t)parts, nullptr), done((size_t)parts, nullptr);
+  hipStream_t s = nullptr, s2 = nullptr;
+  std::vector<hipEvent_t> up((size_t)(overlap ? parts : 0), nullptr), done(up);
   int rc = PGXC_OK;
   auto chk = [&](hipError_t e) {
     if (e != hipSuccess && rc == PGXC_OK)
@@ -2540,12 +2545,13 @@ int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, co
     return rc == PGXC_OK;
   };
   chk(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
-  chk(hipStreamCreateWithFlags(&sc, hipStreamNonBlocking));
+  if (overlap) chk(hipStreamCreateWithFlags(&s2, hipStreamNonBlocking));
   chk(hipMalloc((void **)&dev, 8 * (na3 + ninv) + 44 * (size_t)npts + 8));
-  for (int64_t i = 0; i < parts && rc == PGXC_OK; ++i) {
-    chk(hipEventCreateWithFlags(&up[(size_t)i], hipEventDisableTiming));
-    chk(hipEventCreateWithFlags(&done[(size_t)i], hipEventDisableTiming));
+  for (size_t i = 0; i < up.size() && rc == PGXC_OK; ++i) {
+    chk(hipEventCreateWithFlags(&up[i], hipEventDisableTiming));
+    chk(hipEventCreateWithFlags(&done[i], hipEventDisableTiming));
   }
+  hipStream_t sc = overlap ? s2 : s;  // the transfers' stream
   double *d_a = dev, *d_inv = d_a + na3, *d_p = d_inv + ninv, *d_w = d_p + 3 * npts, *d_o = d_w + npts;
   int *d_own = (int *)(d_o + npts);
   if (rc == PGXC_OK) {
@@ -2554,31 +2560,34 @@ int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, co
   }
   for (int64_t i = 0; i < parts + 2 && rc == PGXC_OK; ++i) {
     if (i < parts) {
-      const int64_t p0 = i * kBeckePart, n = std::min<int64_t>(kBeckePart, npts - p0);
-      for (int d = 0; d < 3; ++d)
-        chk(hipMemcpyAsync(d_p + d * npts + p0, pts + d * npts + p0, 8 * (size_t)n, hipMemcpyHostToDevice, sc));
+      const int64_t p0 = i * per, n = std::min<int64_t>(per, npts - p0);
+      const int nd = overlap ? 3 : 1;  // the coordinates of all points lie in one piece
+      for (int d = 0; d < nd; ++d)
+        chk(hipMemcpyAsync(d_p + d * npts + p0, pts + d * npts + p0, 24 * (size_t)n / nd, hipMemcpyHostToDevice, sc));
       chk(hipMemcpyAsync(d_w + p0, w_atomic + p0, 8 * (size_t)n, hipMemcpyHostToDevice, sc));
       chk(hipMemcpyAsync(d_own + p0, owner + p0, 4 * (size_t)n, hipMemcpyHostToDevice, sc));
-      chk(hipEventRecord(up[(size_t)i], sc));
-      chk(hipStreamWaitEvent(s, up[(size_t)i], 0));
+      if (overlap) {
+        chk(hipEventRecord(up[(size_t)i], sc));
+        chk(hipStreamWaitEvent(s, up[(size_t)i], 0));
+      }
       launch_becke(s, n_atoms, d_a, d_inv, (long)n, (long)npts, d_p + p0, d_own + p0, d_w + p0, d_o + p0);
       chk(hipGetLastError());
-      chk(hipEventRecord(done[(size_t)i], s));
+      if (overlap) chk(hipEventRecord(done[(size_t)i], s));
     }
     if (i >= 2) {
-      const int64_t p0 = (i - 2) * kBeckePart, n = std::min<int64_t>(kBeckePart, npts - p0);
-      chk(hipStreamWaitEvent(sc, done[(size_t)(i - 2)], 0));
+      const int64_t p0 = (i - 2) * per, n = std::min<int64_t>(per, npts - p0);
+      if (overlap) chk(hipStreamWaitEvent(sc, done[(size_t)(i - 2)], 0));
       chk(hipMemcpyAsync(w_out + p0, d_o + p0, 8 * (size_t)n, hipMemcpyDeviceToHost, sc));
     }
   }
-  if (sc) chk(hipStreamSynchronize(sc));
+  if (s2) chk(hipStreamSynchronize(s2));
   if (s) chk(hipStreamSynchronize(s));
   dfree(dev);
   for (auto *v : {&up, &done})
     for (hipEvent_t e : *v)
       if (e) (void)hipEventDestroy(e);
   if (s) (void)hipStreamDestroy(s);
-  if (sc) (void)hipStreamDestroy(sc);
+  if (s2) (void)hipStreamDestroy(s2);
   return rc;
 }
 

@@ -96,3 +96,30 @@ def test_weights_where_the_kernel_changes(na, npts):
     got = becke_weights(xyz, pts, own, wat)
     ref = grid.becke_numpy(xyz, pts, own, wat)
     assert np.max(np.abs(got - ref) / wat) < 1e-13 * 27 / 16 * na  # as above
+
+
+@pytest.mark.parametrize("na", [12, 13])
+@pytest.mark.parametrize("npts", [0, 1, (1 << 18) - 1, 1 << 18, (1 << 18) + 1, (1 << 19) + 130])
+def test_weights_in_one_part_and_in_several(na, npts):
+    """Grids above 2^18 points of more than 12 centres go through the device in
+    parts: each part's weights are those of a call with its points alone, and
+    the output array may be the input's."""
+    import ctypes
+    from pgxc import _lib
+    xyz = np.ascontiguousarray(systems.random_molecule(14, seed=3)[1][:na])
+    rng = np.random.default_rng(npts + na)
+    n = max(npts, 64)
+    own = rng.integers(0, na, n).astype(np.int32)[:npts]
+    pts = np.asfortranarray(xyz[own] + rng.normal(size=(npts, 3)))
+    wat = rng.uniform(0.1, 2.0, n)[:npts]
+    got = becke_weights(xyz, pts, own, wat)
+    per = 1 << 18
+    for p in range(0, npts, per):
+        q = slice(p, min(p + per, npts))
+        assert np.array_equal(got[q], becke_weights(xyz, pts[q], own[q], wat[q]))
+    io = wat.copy()
+    dp, ip = ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int32)
+    P = lambda a: a.ctypes.data_as(dp)
+    assert _lib.load().pgxc_becke_weights(na, P(xyz), npts, P(pts), own.ctypes.data_as(ip), P(io),
+                                          P(io)) == 0
+    assert np.array_equal(io, got)
