@@ -15,6 +15,7 @@
 #include <cstdio>
 #include <cstring>
 #include <map>
+#include <memory>
 #include <mutex>
 #include <numeric>
 #include <string>
@@ -426,10 +427,11 @@ static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int p
   }
 }
 
-// Build (or reuse) the plan of a set of molecules for one configuration.
+// Make (or reuse) the plan of a set of molecules for one configuration.  A plan
+// that could not be made whole leaves the slot empty.
 static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int precision,
                     const std::vector<int> &incr, const std::vector<double> &unit_prio,
-                    long order_version, const Sched &sc, Plan *&plan, pgxc_ctx *errc,
+                    long order_version, const Sched &sc, Plan *&slot, pgxc_ctx *errc,
                     int energy = 0) {
   const int smode = sc.model ? sc.mode : std::min(sc.mode, (int)PGXC_SCHED_ANALYTIC);
   std::vector<int> lanes, spins;
@@ -437,16 +439,17 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
     lanes.push_back(c->nlanes);
     spins.push_back(c->ispin);
   }
-  if (plan && plan->functional == functional && plan->precision == precision &&
-      plan->incr == incr && plan->lanes == lanes && plan->spins == spins &&
-      plan->energy == energy &&
-      plan->order_version == order_version &&
-      plan->sched_mode == smode &&
-      plan->log == sc.log && plan->model == sc.model &&
-      plan->model_version == costmodel_version(sc.model))
+  if (slot && slot->functional == functional && slot->precision == precision &&
+      slot->incr == incr && slot->lanes == lanes && slot->spins == spins &&
+      slot->energy == energy &&
+      slot->order_version == order_version &&
+      slot->sched_mode == smode &&
+      slot->log == sc.log && slot->model == sc.model &&
+      slot->model_version == costmodel_version(sc.model))
     return PGXC_OK;
-  free_plan(plan);
-  plan = new Plan();
+  free_plan(slot);
+  std::unique_ptr<Plan> made(new Plan());
+  Plan *plan = made.get();
   plan->functional = functional;
   plan->precision = precision;
   plan->incr = incr;
@@ -880,6 +883,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
   plan->d_prep_base = (long *)(B + qb_off);
   plan->pack_total = pbase[npack];
   plan->prep_total = qbase[npack];
+  slot = made.release();
   return PGXC_OK;
 }
 

@@ -1,0 +1,86 @@
+"""The library's host code over a stand-in HIP runtime (tests/fake_hip.cpp, host
+memory, no kernels): what it keeps and frees between calls, on paths where a
+mistake would be a fault on the device.  Each test runs in a process of its own,
+which loads the stand-in before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, sys
+hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+hip.fake_stale.restype = hip.fake_live.restype = ctypes.c_long
+hip.fake_fail_in.argtypes = [ctypes.c_long]
+import numpy as np
+from pgxc import Batch, XCBuilder, _lib, basis, grid, systems
+from pgxc.costmodel import CostModel
+from pgxc.xc import BF16X3, FP32, FP64, LDA, PBE
+
+ARG, UNSUPPORTED, HIP, NOMEM, STATE = range(1, 6)
+
+def builder(n=1, seed=0, **kw):
+    els, xyz = systems.h2o() if n == 1 else systems.water_cluster(n, seed=seed)
+    b = basis.seeded_basis(els, xyz, seed=1, shell_set="small")
+    g = grid.molecular_grid(els, xyz, nrad=10, nang=194)
+    xc = XCBuilder(b, g, chunk_points=2048, **kw)
+    xc.set_orbitals(*systems.random_orbitals(b.nbas, 5, seed=2))
+    return xc
+
+def raises(code, fn):
+    try:
+        fn()
+    except _lib.PgxcError as e:
+        assert e.code == code, (e.code, str(e))
+    else:
+        raise AssertionError("no error")
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfakehip.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-o", so,
+                    os.path.join(ROOT, "tests", "fake_hip.cpp")], check=True)
+    return so
+
+
+def run(fake, code):
+    env = dict(os.environ, PYTHONPATH=os.path.join(ROOT, "paragauss-gpl_amd"))
+    r = subprocess.run([sys.executable, "-c", PRELUDE + code, fake], env=env, text=True,
+                       capture_output=True, timeout=120)
+    assert r.returncode == 0, r.stdout + r.stderr
+
+
+def test_build_fails_again_after_a_failed_plan(fake):
+    """A plan that could not be made (a cost model of another feature count, no
+    memory for its tables) is not taken for a made one by the next call."""
+    run(fake, """
+for n in (1, 2):
+    xs = [builder(k + 1) for k in range(n)]
+    call = xs[0] if n == 1 else Batch(xs)
+    calls = [lambda: call.build(PBE, FP64)]
+    if n == 1:
+        calls.append(lambda: xs[0].energy(PBE, FP64))
+    model = CostModel(_lib.NFEATURES - 1)
+    call.set_schedule(_lib.SCHED_MODEL, model)
+    for c in calls + calls:
+        raises(ARG, c)
+        raises(ARG, c)
+    raises(STATE, xs[0].result)  # no build has run
+    call.set_schedule(_lib.SCHED_ANALYTIC)
+    for c in calls + [xs[0].gradient]:
+        c()
+    call.set_schedule(_lib.SCHED_STATIC)  # another plan for each, and for the gradient:
+    for c in [lambda: call.build(LDA, FP64)] + calls[1:] + [xs[0].gradient]:
+        for _ in range(2):
+            hip.fake_fail_in(1)  # the plan's tables
+            raises(NOMEM, c)
+            hip.hipGetLastError()
+        c()
+    call.close()
+assert hip.fake_stale() == 0
+""")
