@@ -217,9 +217,11 @@ int cm_fail(pgxc_costmodel *m, int code, const std::string &msg) {
 #define CMCHK(m, call)                                                                 \
   do {                                                                                 \
     hipError_t e_ = (call);                                                            \
-    if (e_ != hipSuccess)                                                              \
+    if (e_ != hipSuccess) {                                                            \
+      (void)hipGetLastError(); /* reported here, not by the next check of a launch */  \
       return cm_fail(m, e_ == hipErrorOutOfMemory ? PGXC_ERR_NOMEM : PGXC_ERR_HIP,     \
                      std::string(#call) + ": " + hipGetErrorString(e_));               \
+    }                                                                                  \
   } while (0)
 
 // splitmix64 (Steele, Lea & Flood, 2014): a deterministic initialisation

@@ -238,12 +238,16 @@ int fail(pgxc_ctx *c, int code, const std::string &msg) {
   return code;
 }
 
+// An error that goes back to the caller leaves the runtime's record too, where
+// the next call's check of its launches would find it and fail as well.
 #define HIPCHK(ctx, call)                                                              \
   do {                                                                                 \
     hipError_t e_ = (call);                                                            \
-    if (e_ != hipSuccess)                                                              \
+    if (e_ != hipSuccess) {                                                            \
+      (void)hipGetLastError();                                                         \
       return fail(ctx, e_ == hipErrorOutOfMemory ? PGXC_ERR_NOMEM : PGXC_ERR_HIP,       \
                   std::string(#call) + ": " + hipGetErrorString(e_));                  \
+    }                                                                                  \
   } while (0)
 
 template <typename T>
@@ -252,6 +256,7 @@ int dalloc(pgxc_ctx *c, T **p, size_t count) {
   hipError_t e = hipMalloc((void **)p, sizeof(T) * std::max<size_t>(count, 1));
   if (e != hipSuccess) {
     *p = nullptr;
+    (void)hipGetLastError();
     return fail(c, PGXC_ERR_NOMEM, std::string("hipMalloc: ") + hipGetErrorString(e));
   }
   return PGXC_OK;
@@ -2370,6 +2375,7 @@ int pgxc_batch_create(pgxc_batch **out, int32_t n, pgxc_ctx *const *ctxs) {
       hipEventCreateWithFlags(&b->fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&b->join, hipEventDisableTiming) != hipSuccess ||
       hipEventCreate(&b->e0) != hipSuccess || hipEventCreate(&b->e1) != hipSuccess) {
+    (void)hipGetLastError();
     b->err = "pgxc_batch_create: stream/event creation failed";
     return PGXC_ERR_HIP;
   }
@@ -2431,13 +2437,19 @@ int pgxc_batch_build(pgxc_batch *b, uint32_t functional, int32_t precision, int3
       if (e == hipSuccess) e = hipGraphInstantiate(&pl.graph, pl.graph_src, nullptr, nullptr, 0);
     }
     if (e != hipSuccess) {
+      (void)hipGetLastError();
       b->err = std::string("hipGraph capture: ") + hipGetErrorString(e);
       return PGXC_ERR_HIP;
     }
   }
-  if (hipEventRecord(b->e0, s) != hipSuccess) return PGXC_ERR_HIP;
+  if (hipEventRecord(b->e0, s) != hipSuccess) {
+    (void)hipGetLastError();
+    b->err = "hipEventRecord failed";
+    return PGXC_ERR_HIP;
+  }
   if (use_graph) {
     if (hipGraphLaunch(pl.graph, s) != hipSuccess) {
+      (void)hipGetLastError();
       b->err = "hipGraphLaunch failed";
       return PGXC_ERR_HIP;
     }
@@ -2450,6 +2462,7 @@ int pgxc_batch_build(pgxc_batch *b, uint32_t functional, int32_t precision, int3
   hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) {
+    (void)hipGetLastError();
     b->err = std::string("batch build: ") + hipGetErrorString(e);
     return PGXC_ERR_HIP;
   }
@@ -2544,6 +2557,7 @@ int pgxc_becke_weights(int32_t n_atoms, const double *atom_xyz, int64_t npts, co
   std::vector<hipEvent_t> up((size_t)(overlap ? parts : 0), nullptr), done(up);
   int rc = PGXC_OK;
   auto chk = [&](hipError_t e) {
+    if (e != hipSuccess) (void)hipGetLastError();
     if (e != hipSuccess && rc == PGXC_OK)
       rc = e == hipErrorOutOfMemory ? PGXC_ERR_NOMEM : PGXC_ERR_HIP;
     return rc == PGXC_OK;
@@ -2606,6 +2620,7 @@ static __device__ __align__(256) double scratch[(size_t)kNoAllocMaxAtoms * kNoAl
 static std::mutex g_scratch_mu;
 static double *g_scratch_ptr[kNoAllocMaxDevices];
 static int free_fail(int code, const char *msg) {
+  if (code == PGXC_ERR_HIP) (void)hipGetLastError();
   snprintf(g_free_err, sizeof(g_free_err), "%s", msg);
   return code;
 }

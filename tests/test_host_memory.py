@@ -79,8 +79,34 @@ for n in (1, 2):
         for _ in range(2):
             hip.fake_fail_in(1)  # the plan's tables
             raises(NOMEM, c)
-            hip.hipGetLastError()
+            hip.hipGetLastError()  # what the calls leave behind is the next test's
         c()
     call.close()
 assert hip.fake_stale() == 0
+""")
+
+
+def test_an_error_is_reported_once(fake):
+    """A failed allocation fails its own call; the same call made again, and the
+    calls after it, find no trace of it."""
+    run(fake, """
+xc = builder()
+for call in (lambda: xc.build(PBE, FP64), lambda: xc.energy(PBE, FP64), xc.gradient,
+             lambda: xc.gradient_grid(grid.owners(["O", "H", "H"], 10, 194)),
+             lambda: xc.set_orbitals(np.eye(xc.nbas), np.ones(xc.nbas)), lambda: xc.build(LDA, FP64)):
+    hip.fake_fail_in(1)
+    raises(NOMEM, call)
+    call()
+hip.fake_fail_in(20)
+raises(NOMEM, builder)
+builder().build(PBE, FP64)
+m = CostModel(9)
+hip.fake_fail_in(1)
+raises(NOMEM, lambda: m.predict(np.ones((4, 9))))
+m.predict(np.ones((4, 9)))
+from pgxc import becke_weights
+args = np.eye(3), np.ones((5, 3)), np.zeros(5, dtype=np.int32), np.ones(5)
+hip.fake_fail_in(1)
+raises(NOMEM, lambda: becke_weights(*args))
+becke_weights(*args)
 """)
