@@ -294,6 +294,18 @@ struct StepPlan {
   StageList dens[kLists], pot[kLists];
 };
 
+// The work buffers of a molecule that a plan's units hold (ensure_work makes and
+// moves them).
+struct WorkBufs {
+  const void *phi, *W, *W2;
+  size_t phi_stride, phi_lane, w_lane;
+  int skip_basis;
+  bool operator==(const WorkBufs &o) const {
+    return phi == o.phi && W == o.W && W2 == o.W2 && phi_stride == o.phi_stride && phi_lane == o.phi_lane &&
+           w_lane == o.w_lane && skip_basis == o.skip_basis;
+  }
+};
+
 struct Plan {
   uint32_t functional = 0;
   int precision = 0;
@@ -315,6 +327,7 @@ struct Plan {
   int nlanes = 1;  // 2: chunk k runs on lane k % 2 (two streams)
   std::vector<int> lanes;  // lanes in use per molecule when the plan was made
   std::vector<int> spins;  // ispin per molecule when the plan was made
+  std::vector<WorkBufs> bufs;  // and its work buffers
   PackD *d_pack = nullptr;
   long *d_pack_base = nullptr, *d_prep_base = nullptr;
   long pack_total = 0, prep_total = 0;
@@ -440,12 +453,15 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
                     int energy = 0) {
   const int smode = sc.model ? sc.mode : std::min(sc.mode, (int)PGXC_SCHED_ANALYTIC);
   std::vector<int> lanes, spins;
+  std::vector<WorkBufs> bufs;  // a call on a member alone may have moved them
   for (auto *c : mols) {
     lanes.push_back(c->nlanes);
     spins.push_back(c->ispin);
+    bufs.push_back({c->phi_base, c->W, c->ispin == 2 ? c->beta.W : nullptr, c->phi_stride, c->phi_lane, c->w_lane,
+                    c->skip_basis});
   }
   if (slot && slot->functional == functional && slot->precision == precision &&
-      slot->incr == incr && slot->lanes == lanes && slot->spins == spins &&
+      slot->incr == incr && slot->lanes == lanes && slot->spins == spins && slot->bufs == bufs &&
       slot->energy == energy &&
       slot->order_version == order_version &&
       slot->sched_mode == smode &&
@@ -460,6 +476,7 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
   plan->incr = incr;
   plan->lanes = lanes;
   plan->spins = spins;
+  plan->bufs = bufs;
   plan->energy = energy;
   plan->order_version = order_version;
   plan->sched_mode = smode;
@@ -1029,14 +1046,12 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
   const size_t need_phi = phi_elem_bytes(elem) * (size_t)c->NP * c->Mc;
   const size_t need_w = (size_t)c->NP * c->Mc * elem * c->nlanes_cap;
   c->w_lane = (size_t)c->NP * c->Mc * elem;
-  bool moved = false;
   if (c->w_bytes < need_w) {
     dfree(c->W);
     c->W = nullptr;
     c->w_bytes = 0;
     HIPCHK(c, hipMalloc(&c->W, need_w));
     c->w_bytes = need_w;
-    moved = true;
   }
   if (c->ispin == 2 && c->beta.w_bytes < need_w) {
     dfree(c->beta.W);
@@ -1044,7 +1059,6 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
     c->beta.w_bytes = 0;
     HIPCHK(c, hipMalloc(&c->beta.W, need_w));
     c->beta.w_bytes = need_w;
-    moved = true;
   }
   // basis cache: every chunk's values, when they take at most a quarter of
   // the device, leave 32 GiB free, and the caches of all contexts on the
@@ -1090,16 +1104,9 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
   void *base = c->phic[e] ? c->phic[e] : c->phi;
   const size_t stride = c->phic[e] ? need_phi : 0;
   // an LDA pass writes only the value planes: a GGA build after it evaluates again
-  const int skip = c->phic[e] && c->phic_valid[e] && (c->phic_grad[e] || !grad);
-  if (base != c->phi_base || stride != c->phi_stride || skip != c->skip_basis) moved = true;
   c->phi_base = base;
   c->phi_stride = stride;
-  c->skip_basis = skip;
-  if (moved) {  // their unit descriptors hold the old pointers
-    free_plan(c->plan);
-    free_plan(c->plan_e);
-    free_plan(c->plan_g);
-  }
+  c->skip_basis = c->phic[e] && c->phic_valid[e] && (c->phic_grad[e] || !grad);
   return PGXC_OK;
 }
 
@@ -2406,19 +2413,14 @@ int pgxc_batch_build(pgxc_batch *b, uint32_t functional, int32_t precision, int3
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
   const size_t elem = precision == PGXC_PREC_FP64 ? 8 : 4;
   hipStream_t s = b->stream;
-  bool moved = false;
   for (int m = 0; m < nm; ++m) {
     pgxc_ctx *c = b->mols[m];
-    const void *phi0 = c->phi_base, *w0 = c->W, *wb0 = c->beta.W;
-    const int skip0 = c->skip_basis;
     int rc = ensure_work(c, elem, precision, s, gga);
     if (rc) {
       b->err = "molecule " + std::to_string(m) + ": " + c->err;
       return rc;
     }
-    moved = moved || phi0 != c->phi_base || w0 != c->W || wb0 != c->beta.W || skip0 != c->skip_basis;
   }
-  if (moved) free_plan(b->plan);
   int rc = get_plan(b->mols, functional, precision, incr, b->prio, b->order_version, b->sched,
                     b->plan, b->mols[0]);
   if (rc) {

@@ -109,3 +109,26 @@ def test_batch_with_mixed_lane_counts(mols):
                 assert np.array_equal(r[0], s[0]) and r[1] == s[1] and r[2] == s[2]
     for xb in bs:
         xb.close()
+
+
+@pytest.mark.parametrize("cache", [True, False])
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_after_a_members_build_in_another_precision(mols, cache, graph):
+    """A member's own FP64 build or gradient moves the work buffers of its mixed
+    builds; batches before and after it give the same bits."""
+    bs = []
+    for (b, g, C, occ) in mols[:2]:
+        bs.append(XCBuilder(b, g, chunk_points=2048, basis_cache=cache))
+        bs[-1].set_orbitals(C, occ)
+    with Batch(bs) as batch:
+        for _ in range(2):
+            batch.build(PBE, FP32, graph=graph)
+        ref = batch.results()
+        for between in (lambda x: x.gradient(), lambda x: (x.build(PBE, FP64), x.build(PBE, FP32))):
+            for x in bs:
+                between(x)
+                batch.build(PBE, FP32, graph=graph)
+                for r, s in zip(batch.results(), ref):
+                    assert np.array_equal(r[0], s[0]) and r[1] == s[1] and r[2] == s[2]
+    for xb in bs:
+        xb.close()

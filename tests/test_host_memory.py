@@ -110,3 +110,37 @@ hip.fake_fail_in(1)
 raises(NOMEM, lambda: becke_weights(*args))
 becke_weights(*args)
 """)
+
+
+@pytest.mark.parametrize("cache", [True, False])
+@pytest.mark.parametrize("graph", [False, True])
+def test_batch_after_its_members_own_builds(fake, cache, graph):
+    """A member's own build or gradient in another precision moves its work
+    buffers; the batch's next build must not use the tables (or the graph) that
+    name the old ones.  The calls in between return to the batch's precision,
+    so that the batch's own call moves nothing."""
+    run(fake, """
+cache, graph = %r, %r
+for prec in (FP32, BF16X3):
+    for between in (lambda x: x.gradient(),
+                    lambda x: (x.build(PBE, FP64), x.build(PBE, prec)),
+                    lambda x: (x.gradient(), x.build(PBE, prec)),
+                    lambda x: (x.energy(LDA, FP64), x.energy(LDA, prec)),
+                    lambda x: (x.set_orbitals(np.ones((x.nbas, 4, 2)), np.ones((4, 2))), x.build(PBE, FP64),
+                               x.build(PBE, prec), x.set_orbitals(np.ones((x.nbas, 4)), np.ones(4)))):
+        xs = [builder(1, basis_cache=cache), builder(2, basis_cache=cache)]
+        bt, other = Batch(xs), Batch(xs[::-1])
+        bt.build(PBE, prec, graph=graph)
+        bt.build(PBE, prec, graph=graph)  # from kept basis values, if they are kept
+        for k in (0, 1, 0):
+            between(xs[k])
+            assert hip.fake_stale() == 0
+            bt.build(PBE, prec, graph=graph)
+            assert hip.fake_stale() == 0
+            other.build(PBE, FP64, graph=graph)
+            bt.build(PBE, prec, graph=graph)
+            assert hip.fake_stale() == 0
+        bt.close(), other.close()
+        for x in xs:
+            x.close()
+""" % (cache, graph))
