@@ -166,6 +166,7 @@ struct pgxc_ctx {
     double *state = nullptr, *Vstate = nullptr, *Vout = nullptr;
     void *D = nullptr, *W = nullptr;
     size_t w_bytes = 0;
+    int ready = 0;  // every buffer but W is there
   } beta;
   // device: state and results
   double *state = nullptr;                    // [S_NSLOT][npad]
@@ -1841,12 +1842,12 @@ int pgxc_layout(const pgxc_ctx *c, int64_t *out8) {
 // Buffers of the beta spin, zeroed like the alpha spin's at creation.
 static int alloc_beta(pgxc_ctx *c) {
   auto &B = c->beta;
-  if (B.P) return PGXC_OK;
+  if (B.ready) return PGXC_OK;
   const size_t np2 = (size_t)c->NP * c->NP, npk = (size_t)c->nbas * (c->nbas + 1) / 2;
   const size_t L = (size_t)c->nlanes_cap;
   int rc;
   if ((rc = dalloc(c, &B.P, np2)) || (rc = dalloc(c, &B.Pref, np2))) return rc;
-  HIPCHK(c, hipMalloc(&B.D, np2 * 8));
+  if (!B.D) HIPCHK(c, hipMalloc(&B.D, np2 * 8));
   if ((rc = dalloc(c, &B.state, (size_t)S_NSLOT * c->npad)) || (rc = dalloc(c, &B.Vstate, npk)) ||
       (rc = dalloc(c, &B.Vout, npk)) || (rc = dalloc(c, &B.part, L * c->nparts * 4 * c->Mc)) ||
       (rc = dalloc(c, &B.coef, L * 4 * c->Mc)) || (rc = alloc_partials(c, &B.Hc, &B.HS)))
@@ -1856,6 +1857,7 @@ static int alloc_beta(pgxc_ctx *c) {
   HIPCHK(c, hipMemset(B.state, 0, (size_t)S_NSLOT * c->npad * 8));
   HIPCHK(c, hipMemset(B.part, 0, L * c->nparts * 4 * c->Mc * 8));
   HIPCHK(c, hipMemset(B.coef, 0, L * 4 * c->Mc * 8));
+  B.ready = 1;  // a call that failed before here goes on with those it lacks
   return PGXC_OK;
 }
 

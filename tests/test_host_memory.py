@@ -144,3 +144,32 @@ for prec in (FP32, BF16X3):
         for x in xs:
             x.close()
 """ % (cache, graph))
+
+
+def test_open_shell_buffers_after_a_failed_allocation(fake):
+    """The beta spin's buffers: whichever of them cannot be had, the call fails,
+    the context stays closed shell, and the same call made again has them all."""
+    run(fake, """
+def live_after(fail):
+    xc = builder()
+    C, occ = systems.random_orbitals(xc.nbas, 5, seed=2)
+    P = np.stack([(C * occ) @ C.T] * 2, axis=2)
+    xc.build(PBE, FP64)
+    before = xc.save_state()
+    if fail:
+        hip.fake_fail_in(fail)
+        raises(NOMEM, lambda: xc.set_density(P))
+        assert xc.save_state() == before
+    xc.set_density(P)
+    n = hip.fake_live()
+    xc.build(PBE, FP64)
+    xc.close()
+    assert hip.fake_live() == 0
+    return n
+want = live_after(0)
+for k in range(1, 11):
+    assert live_after(k) == want, k
+xc = builder()
+hip.fake_fail_in(11)  # the tenth was the last
+xc.set_density(np.ones((xc.nbas, xc.nbas, 2)))
+""")
