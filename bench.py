@@ -629,9 +629,9 @@ def main():
     xc.set_schedule(sched_mode, model)
     warm = timed(xc, "basis cached")
     st1w, _ = one_lane(xc, warm["best"])
-    # work the contraction kernels execute (gathered runs of 8 functions,
-    # whole function tiles): counted from the item log of one more build of
-    # each mixed form
+    # work the contraction kernels execute (the columns and K of every density
+    # item, whole chunks of functions in the potential): counted from the item
+    # log of one more build of each mixed form
     executed = {}
     xc.set_item_log(True)
     for prec in precs:
@@ -639,11 +639,13 @@ def main():
         xc.build(PBE, PRECISIONS[prec], fetch=False)
         F, _ = xc.item_log()
         k = np.exp2(16.0 * F[:, 5]) - 1.0
-        # density item: 128 points x a pair of function tiles (both computed
-        # by the split-BF16 kernel); potential item: function tile x tile
-        tile = F[:, 4] * 128.0
-        rows = np.where(F[:, 0] == 0, 128.0, tile)
-        cols = np.where(F[:, 0] == 0, 2.0 * tile, tile)
+        # density item: 128 points x its columns (in FP32 a tile's K functions
+        # over its items; split BF16 pads its shares to blocks of 16);
+        # potential item: chunk x chunk
+        cols = F[:, 4] * 128.0
+        if prec == "fp32":
+            cols = np.where(F[:, 0] == 0, k / np.ceil(np.rint(k) / cols), cols)
+        rows = np.where(F[:, 0] == 0, 128.0, cols)
         fl = 2.0 * rows * cols * k
         executed[prec] = {"density": float(fl[F[:, 0] == 0].sum()),
                           "potential": float(fl[F[:, 0] == 1].sum())}

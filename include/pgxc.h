@@ -66,10 +66,11 @@ extern "C" {
 
 /* Features of one work item, in this order (pgxc_item_log, cost model):
  * kind (0 density, 1 potential contraction), precision one-hot (FP64, FP32,
- * BF16x3), function tile / 128, log2(1 + K length left after screening) / 16,
- * log2(1 + dense K length) / 16, 1 if any block is left after screening,
- * variant / 2.  (K: functions of the density contraction, points of the
- * potential contraction.) */
+ * BF16x3), columns / 128 (density: the share of its tile's functions that an
+ * item takes, in whole blocks of 16; potential: the functions of a chunk), log2(1 + K length left after screening) / 16, log2(1 + dense K
+ * length) / 16, 1 if any block is left after screening, variant / 2.  (K:
+ * functions of the density contraction, in whole runs of 8 for BF16x3; points
+ * of the potential contraction.) */
 #define PGXC_NFEATURES 9
 
 typedef struct pgxc_ctx pgxc_ctx;

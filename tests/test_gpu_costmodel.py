@@ -172,3 +172,36 @@ def test_network_beats_counted_flops(case, trained):
     print("held-out rms error of log(item time): network %.4f, counted flops %.4f"
           % (e_net, e_count), flush=True)
     assert e_net < e_count
+
+
+@pytest.mark.parametrize("exp_range,chunk", [((0.1, 5000.0), 8192), ((0.1, 0.5), 2048)],
+                         ids=["few functions", "wide tiles"])
+def test_features_count_the_work_of_the_items(exp_range, chunk):
+    """Density items: the FP64 and FP32 kernels take a tile's own functions as K
+    and as columns, split BF16 whole runs of 8 as K.  A tile's items share its
+    columns in blocks of 16, so from K and the share follow how many items the
+    tile has, and the sum over them of columns x K is that of the tiles' squared
+    function counts, which the statistics hold."""
+    els, xyz = systems.water_cluster(14, seed=2)
+    b = basis.seeded_basis(els, xyz, seed=33, shell_set="medium", exp_range=exp_range)
+    g = grid.molecular_grid(els, xyz, nrad=6, nang=194)
+    C, occ = systems.random_orbitals(b.nbas, 10, seed=32)
+    with XCBuilder(b, g, chunk_points=chunk) as xc:
+        xc.set_orbitals(C, occ)
+        xc.set_item_log(True)
+        log = {}
+        for prec in (FP64, FP32, BF16X3):
+            xc.build(PBE, prec, fetch=False)
+            Z = xc.item_log()[0]
+            d, p = Z[Z[:, 0] == 0], Z[Z[:, 0] == 1]
+            assert set(np.unique(p[:, 4])) <= {0.5, 0.75, 1.0}
+            log[prec] = 128.0 * d[:, 4], np.exp2(16.0 * d[:, 5]) - 1.0
+        n2 = xc.stats()["n2"]
+    for share, K in log.values():
+        assert np.all(share >= 16) and np.all(share <= 256) and np.all(share % 16 == 0)
+    share, K = log[FP64]
+    items = np.ceil(np.rint(K) / share)
+    assert abs(np.sum(K * K / items) - n2) <= 1e-9 * n2
+    assert np.array_equal(log[FP32][0], share) and np.array_equal(log[FP32][1], K)
+    runs = log[BF16X3][1]
+    assert np.all(np.abs(runs / 8 - np.rint(runs / 8)) < 1e-9) and np.all(np.rint(runs) >= np.rint(K))
