@@ -2149,14 +2149,14 @@ int pgxc_gradient_grid(pgxc_ctx *c, const int32_t *owner, double *grad) {
   // inverse distances, per-wave cells, sums and centre lists
   const long waves = becke_grad_waves(na, np);
   size_t off[8] = {0}, bytes[7] = {4 * (size_t)npts, 4 * (size_t)np, 8 * (size_t)np, 8 * inv.size(),
-                                   512 * (size_t)waves * na, 24 * (size_t)waves * na, 2 * (size_t)waves * na};
+                                   512 * (size_t)waves * na, 24 * (size_t)waves * na, 4 * (size_t)waves * na};
   for (int i = 0; i < 7; ++i) off[i + 1] = off[i] + (size_t)round_up((long)bytes[i], 256);
   int rc;
   if ((rc = dalloc(c, &c->gmov, off[7])) || (rc = dalloc(c, &c->gpm, 3 * (size_t)np))) return rc;
   int *d_caller = (int *)(c->gmov + off[0]), *d_own = (int *)(c->gmov + off[1]);
   double *fp = (double *)(c->gmov + off[2]), *d_inv = (double *)(c->gmov + off[3]);
   double *scr = (double *)(c->gmov + off[4]), *part = (double *)(c->gmov + off[5]);
-  uint16_t *list = (uint16_t *)(c->gmov + off[6]);
+  int *list = (int *)(c->gmov + off[6]);
   hipStream_t s = c->stream;
   HIPCHK(c, hipMemsetAsync(c->gpm, 0, 24 * (size_t)np, s));
   HIPCHK(c, hipMemcpyAsync(d_inv, inv.data(), 8 * inv.size(), hipMemcpyHostToDevice, s));

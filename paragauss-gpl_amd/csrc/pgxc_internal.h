@@ -257,7 +257,7 @@ void launch_point_f(hipStream_t s, bool gga, bool spin, uint32_t mask, long Mc, 
 long becke_grad_waves(int na, long np);
 void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long np,
                        const double *grid, const double *fp, const int *owner, long waves,
-                       double *scr, uint16_t *list, double *part, double *grad);
+                       double *scr, int *list, double *part, double *grad);
 
 // Becke partition weights of points owned by atoms (grid generation)
 void launch_inv_dist(hipStream_t s, int na, const double *axyz, double *inv);

@@ -1,6 +1,7 @@
 // Becke partition weights for gfx950: the cell weights of a molecular grid's
 // points, FP64, from a table of inverse centre distances.
 #include "pgxc_internal.h"
+#include "xc_device.h"
 
 namespace pgxc {
 // Becke partition weight of the owning atom (J. Chem. Phys. 88, 2547 (1988)),
@@ -55,15 +56,15 @@ __global__ __launch_bounds__(kThreads) void k_becke_all(int na, const double *__
 // 1e-2 to 1e-10 with each centre near the point.  So the kNear nearest centres
 // are found first, P of the nearest one is formed in full (it is at most the
 // sum), and a centre whose product over just the kNear nearest ones is at or
-// below 2^-64 of that is left out of the sum (at most 1024 terms of them: below
-// half an ulp), unless it owns the point.  The rest are formed in full, over
+// below 2^-64 of that (2^-54 over their number for more than 1024 centres) is left
+// out of the sum, unless it owns the point: all of them together are below half
+// an ulp of it.  The rest are formed in full, over
 // the centres in order, kForm at a time so that a centre's distance is found
 // once for all of them; a wave forms the centres any of its points needs.
 // Bound by FP64 arithmetic.  (H2O)32, 96 centres, 1 961 792 points: 33 centres
 // a wave are formed in full (14 for a single point), 5.0 ms; every product over
 // all centres took 21.9 ms.
 constexpr int kNear = 8, kForm = 8;
-constexpr double kNegligible = 5.421010862427522e-20;  // 2^-64
 
 __global__ __launch_bounds__(kThreads) void k_becke(int na, const double *__restrict__ axyz,
                                                     const double *__restrict__ inv_dist,
@@ -105,7 +106,7 @@ __global__ __launch_bounds__(kThreads) void k_becke(int na, const double *__rest
       }
   }
   // here and below a centre's factor with itself is s(0) = 1/2: starts at 2
-  double floor_p = 2.0 * kNegligible;
+  double floor_p = 2.0 * becke_negligible(na);
 #pragma unroll 2
   for (int k = 0; k < na; ++k) {
     floor_p *= becke_s((rn[0] - dist(k)) * inv_dist[(long)in[0] * na + k]);

@@ -270,6 +270,12 @@ __device__ __forceinline__ int share_cols(int nf, int most) {
 // dimension of its potential partial.
 __device__ __forceinline__ int split_ld(int n) { return (n + 15) & ~15; }
 
+// Share of the nearest centre's Becke cell at or below which a centre's cell is
+// left out: na of them are at most 2^-54, a quarter of an ulp of the cells' sum.
+__device__ __forceinline__ double becke_negligible(int na) {
+  return na <= 1024 ? 5.421010862427522e-20 /* 2^-64 */ : 5.551115123125783e-17 /* 2^-54 */ / na;
+}
+
 // One 16 x 16 block of H = W^T Phi into the split's partial.
 template <typename T>
 __device__ __forceinline__ void put_block(const typename MF<T>::acc &acc, double *H, int ld) {

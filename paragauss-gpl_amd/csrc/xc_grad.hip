@@ -424,7 +424,7 @@ __device__ __forceinline__ double dist(const AtomD &A, Pt r) {
 // One wave per workgroup, a point per lane, groups of 64 points in turn: the
 // wave's sums over its points of w f d log w / dR into part[wave][na][3].  As the
 // weights themselves, only the centres C whose P_C can matter to a point of the
-// wave (above 2^-64 of the nearest centre's, or the owner) are formed and
+// wave (above becke_negligible of the nearest centre's, or the owner) are formed and
 // differentiated: their P in scr[wave][listed centre][64], their indices in
 // list[wave][na].  For each of them every other centre D takes
 // k_C sigma d mu_CD / dR_D, C the same with d mu_CD / dR_C, and the owner
@@ -433,7 +433,6 @@ __device__ __forceinline__ double dist(const AtomD &A, Pt r) {
 // two kernels) 21 ms.
 // LDS: the wave's sums are kept there (na up to kLdsAtoms), else in part.
 constexpr int kNearQ = 8, kFormQ = 4, kLdsAtoms = 1024;
-constexpr double kNegligibleQ = 5.421010862427522e-20;  // 2^-64
 template <bool LDS>
 __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restrict__ atoms,
                                                    const double *__restrict__ inv_dist, long np,
@@ -441,12 +440,12 @@ __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restri
                                                    const double *__restrict__ fp,
                                                    const int *__restrict__ owner,
                                                    double *__restrict__ scr,
-                                                   uint16_t *__restrict__ list,
+                                                   int *__restrict__ list,
                                                    double *__restrict__ part) {
   extern __shared__ double lacc[];  // 3 na
   double *acc = LDS ? lacc : part + (long)blockIdx.x * na * 3;
   double *P = scr + (long)blockIdx.x * na * 64;
-  uint16_t *ls = list + (long)blockIdx.x * na;
+  int *ls = list + (long)blockIdx.x * na;
   const int lane = threadIdx.x;
   for (int j = lane; j < 3 * na; j += 64) acc[j] = 0.0;
   __syncthreads();
@@ -480,7 +479,7 @@ __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restri
           id = ti;
         }
     }
-    double floor_p = 2.0 * kNegligibleQ;  // 2: a centre's cell with itself is 1/2
+    double floor_p = 2.0 * becke_negligible(na);  // 2: a centre's cell with itself is 1/2
     for (int k = 0; k < na; ++k)
       floor_p *= becke_cell((rn[0] - dist(atoms[k], r)) * inv_dist[(long)in[0] * na + k]);
     int nl = 0;  // listed centres, the same for the wave
@@ -491,7 +490,7 @@ __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restri
       for (int t = 0; t < kNearQ; ++t)
         if (t < na) pi *= becke_cell((ri - rn[t]) * inv_dist[(long)i * na + in[t]]);
       if (!__any(on && (!(pi <= floor_p) || i == own))) continue;
-      if (lane == 0) ls[nl] = (uint16_t)i;
+      if (lane == 0) ls[nl] = i;
       ++nl;
     }
     __syncthreads();
@@ -501,7 +500,7 @@ __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restri
       int c[kFormQ];
 #pragma unroll
       for (int m = 0; m < kFormQ; ++m) {
-        c[m] = __builtin_amdgcn_readfirstlane((int)ls[min(c0 + m, nl - 1)]);
+        c[m] = __builtin_amdgcn_readfirstlane(ls[min(c0 + m, nl - 1)]);
         ri[m] = dist(atoms[c[m]], r);
         pi[m] = 2.0;
       }
@@ -525,7 +524,7 @@ __global__ __launch_bounds__(64) void k_becke_grad(int na, const AtomD *__restri
 #pragma unroll
       for (int m = 0; m < kFormQ; ++m) {
         const bool there = c0 + m < nl;
-        c[m] = __builtin_amdgcn_readfirstlane((int)ls[min(c0 + m, nl - 1)]);
+        c[m] = __builtin_amdgcn_readfirstlane(ls[min(c0 + m, nl - 1)]);
         rc[m] = dist(atoms[c[m]], r, ec[m]);
         kc[m] = on && there ? wf * ((c[m] == own ? 1.0 : 0.0) - P[min(c0 + m, nl - 1) * 64 + lane] * iz) : 0.0;
         ac[m][0] = ac[m][1] = ac[m][2] = 0.0;
@@ -606,7 +605,7 @@ void launch_bracket(hipStream_t s, bool gga, int lmax, const UnitD *unit, long M
 long becke_grad_waves(int na, long np) {
   // one wave each, as many as fill the device a few times over and 256 MiB of
   // scratch allow
-  const long per = (long)na * (64 * 8 + 2 + 24);
+  const long per = (long)na * (64 * 8 + 4 + 24);
   return std::max<long>(1, std::min<long>({np / 64, 4096L, (256L << 20) / per}));
 }
 
@@ -618,7 +617,7 @@ void launch_owner_sum(hipStream_t s, int na, long np, const int *owner, const do
 
 void launch_becke_grad(hipStream_t s, int na, const AtomD *atoms, const double *inv_dist, long np,
                        const double *grid, const double *fp, const int *owner, long waves,
-                       double *scr, uint16_t *list, double *part, double *grad) {
+                       double *scr, int *list, double *part, double *grad) {
   auto k = na <= kLdsAtoms ? k_becke_grad<true> : k_becke_grad<false>;
   hipLaunchKernelGGL(k, dim3((unsigned)waves), dim3(64), na <= kLdsAtoms ? 24 * na : 0, s, na, atoms, inv_dist,
                      np, grid, fp, owner, scr, list, part);

@@ -123,3 +123,24 @@ def test_weights_in_one_part_and_in_several(na, npts):
     assert _lib.load().pgxc_becke_weights(na, P(xyz), npts, P(pts), own.ctypes.data_as(ip), P(io),
                                           P(io)) == 0
     assert np.array_equal(io, got)
+
+
+@pytest.mark.parametrize("na", [1024, 1025, 1500])
+def test_weights_of_many_centres(na):
+    """Above 1024 centres what is left out of the sum shrinks with their number."""
+    xyz = np.array([[i, j, k] for i in range(12) for j in range(12) for k in range(11)])[:na] * 2.5
+    xyz = xyz + np.random.default_rng(na).uniform(-0.5, 0.5, xyz.shape)
+    rng = np.random.default_rng(1)
+    own = rng.integers(0, na, 130).astype(np.int32)
+    pts = xyz[own] + rng.normal(size=(130, 3))
+    D = np.linalg.norm(xyz[:, None] - xyz[None], axis=2) + np.eye(na)
+    ref = np.empty(130)
+    for p in range(130):
+        r = np.linalg.norm(pts[p] - xyz, axis=1)
+        mu = (r[:, None] - r[None]) / D
+        for _ in range(3):
+            mu = mu * (3.0 - mu * mu) / 2.0
+        P = np.prod(np.where(np.eye(na, dtype=bool), 1.0, (1.0 - mu) / 2.0), axis=1)
+        ref[p] = P[own[p]] / P.sum()
+    got = becke_weights(xyz, pts, own, np.ones(130))
+    assert np.max(np.abs(got - ref)) < 1e-13 * 27 / 16 * na  # as above
