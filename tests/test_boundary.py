@@ -119,3 +119,16 @@ def test_product_has_no_cpu_fallback():
             if f.endswith((".py", ".cpp", ".hip", ".h", ".f90")):
                 src = open(os.path.join(dirpath, f)).read()
                 assert "import oracle" not in src and "liboracle" not in src, f
+
+
+def test_build_takes_an_empty_reference_folder_for_none(tmp_path):
+    """The reference's modules are built where they are, not where their folder is
+    there and empty (their makefile has no rule for a file that is missing)."""
+    import __graft_entry__ as entry
+    assert not entry.has_reference(str(tmp_path / "none")) and not entry.has_reference(str(tmp_path))
+    (tmp_path / "modules").mkdir()
+    assert not entry.has_reference(str(tmp_path))
+    # the file looked for is one the makefile builds
+    assert "$(REF)/modules/type_module.f90" in open(os.path.join(ROOT, "oracle", "ref.mk")).read()
+    (tmp_path / "modules" / "type_module.f90").write_text("")
+    assert entry.has_reference(str(tmp_path))
