@@ -266,10 +266,15 @@ int dalloc(pgxc_ctx *c, T **p, size_t count) {
 // potential partials held at a time per molecule and spin, and work items of
 // their sum below which it is cut into segments
 constexpr long kPartialBytes = 4L << 30, kFoldItems = 1536;
-// items that all run at once (two workgroups a CU): walked without queues, whose
+// A contraction of at most kQueueItems items is walked without queues, whose
 // claims a launch of one item per workgroup waits for and gains nothing from
-// (water, mixed step: density 54 -> 15 us, potential 34 -> 13)
-constexpr long kResident = 512;
+// (water, mixed step: density 54 -> 15 us, potential 34 -> 13): two workgroups
+// on each of the 256 CUs.  The split-BF16 density with wide items has one
+// workgroup a CU, and above 256 items the walk deals a second round before the
+// first has ended.  The other lane's launches fill that gap; on one lane the
+// queues take it (290 to 400 items a chunk, 1320 functions: density stage 2.99 ->
+// 2.64 and 2.90 -> 2.58 ms, on two lanes energies 2.05 -> 2.10 ms).
+constexpr long kQueueItems = 512, kQueueItemsWide = 256;
 constexpr long kBasisItems = 2048;
 constexpr double kWideTile = 384.0;    // setup_screen: mean functions of a tile for wide density items
 constexpr double kSplitItems = 256.0;  // setup_screen: potential items a chunk has at least
@@ -544,7 +549,8 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       P.frow = plan->feat.size() / PGXC_NFEATURES;
       for (int m : um) unit_item_features(mols[m], step, kind, precision, plan->feat, flops);
     }
-    if (contr && queues && P.total > kResident) {
+    const bool wide = kind == K_DENS && precision == PGXC_PREC_BF16X3 && !um.empty() && mols[um[0]]->icols > 128;
+    if (contr && queues && P.total > (wide && plan_lanes == 1 ? kQueueItemsWide : kQueueItems)) {
       P.has_queues = true;  // queue bounds filled in once every cost is known
     } else {
       std::vector<double> pr;

@@ -205,3 +205,24 @@ def test_features_count_the_work_of_the_items(exp_range, chunk):
     assert np.array_equal(log[FP32][0], share) and np.array_equal(log[FP32][1], K)
     runs = log[BF16X3][1]
     assert np.all(np.abs(runs / 8 - np.rint(runs / 8)) < 1e-9) and np.all(np.rint(runs) >= np.rint(K))
+
+
+@pytest.mark.parametrize("chunk", [14336, 16384, 18432, 32768, 34816])
+@pytest.mark.parametrize("lanes", [1, 2])
+def test_wide_items_around_the_queue_limits(chunk, lanes):
+    """The split-BF16 density with wide items (two a tile here) just below and above
+    256 items a chunk, where one lane takes the queues, and 512, where two do: the
+    same bits as the static walk."""
+    els, xyz = systems.water_cluster(14, seed=2)
+    b = basis.seeded_basis(els, xyz, seed=33, shell_set="medium", exp_range=(0.1, 0.5))
+    g = grid.molecular_grid(els, xyz, nrad=6, nang=194)
+    C, occ = systems.random_orbitals(b.nbas, 10, seed=32)
+    out = []
+    for mode in (_lib.SCHED_STATIC, _lib.SCHED_ANALYTIC):
+        with XCBuilder(b, g, chunk_points=chunk) as xc:
+            assert xc.layout()["chunks"] > 1
+            xc.set_lanes(lanes)
+            xc.set_schedule(mode)
+            xc.set_orbitals(C, occ)
+            out.append(xc.build(PBE, BF16X3))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1:] == out[1][1:]
