@@ -1056,7 +1056,7 @@ static hipError_t poison_basis(const pgxc_ctx *c, void *base, size_t elem, size_
 }
 
 // grad: the build reads the gradient planes of the basis values (GGA)
-static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, bool grad) {
+static int ensure_work(pgxc_ctx *c, size_t elem, hipStream_t s, bool grad) {
   const size_t need_phi = phi_elem_bytes(elem) * (size_t)c->NP * c->Mc;
   const size_t need_w = (size_t)c->NP * c->Mc * elem * c->nlanes_cap;
   c->w_lane = (size_t)c->NP * c->Mc * elem;
@@ -1125,7 +1125,7 @@ static int ensure_work(pgxc_ctx *c, size_t elem, int precision, hipStream_t s, b
 }
 
 // after a build: the cache of this element type now holds valid values
-static void mark_basis_cached(pgxc_ctx *c, size_t elem, int precision, bool grad) {
+static void mark_basis_cached(pgxc_ctx *c, size_t elem, bool grad) {
   const int e = elem == 8 ? 0 : 1;
   if (c->phic[e]) {
     c->phic_valid[e] = 1;
@@ -1971,7 +1971,7 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
   hipStream_t s = c->stream;
   const size_t elem = precision == PGXC_PREC_FP64 ? 8 : 4;
-  if ((rc = ensure_work(c, elem, precision, s, gga))) return rc;
+  if ((rc = ensure_work(c, elem, s, gga))) return rc;
   std::vector<pgxc_ctx *> mols{c};
   std::vector<int> incrv{incr};
   if ((rc = get_plan(mols, functional, precision, incrv, {}, -1, c->sched, c->plan, c))) return rc;
@@ -2008,7 +2008,7 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   c->timing[4] = t;
   HIPCHK(c, hipEventElapsedTime(&t, c->ev[kEvStart], c->ev[kEvEnd]));
   c->timing[5] = t;
-  mark_basis_cached(c, elem, precision, gga);
+  mark_basis_cached(c, elem, gga);
   if (along) {
     for (size_t i = 0; i < npk; ++i) ham[i] += v[i];
     ham = nullptr;
@@ -2045,7 +2045,7 @@ int pgxc_energy(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ter
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
   hipStream_t s = c->stream;
   const size_t elem = precision == PGXC_PREC_FP64 ? 8 : 4;
-  if ((rc = ensure_work(c, elem, precision, s, gga))) return rc;
+  if ((rc = ensure_work(c, elem, s, gga))) return rc;
   std::vector<pgxc_ctx *> mols{c};
   std::vector<int> full{0};
   if ((rc = get_plan(mols, functional, precision, full, {}, -1, c->sched, c->plan_e, c, 1))) return rc;
@@ -2060,7 +2060,7 @@ int pgxc_energy(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ter
     for (size_t i = 0; i < n; ++i, ++at) t[at % 5] += v[i];
   }));
   memcpy(c->last_terms, t, sizeof(t));
-  mark_basis_cached(c, elem, precision, gga);
+  mark_basis_cached(c, elem, gga);
   if (terms4) memcpy(terms4, t, 4 * sizeof(double));
   if (charge) *charge = t[4];
   return PGXC_OK;
@@ -2074,7 +2074,7 @@ static int gradient_impl(pgxc_ctx *c, double *pm) {
   const bool gga = (functional & (PGXC_XC_PBEX | PGXC_XC_PBEC)) != 0;
   hipStream_t s = c->stream;
   int rc;
-  if ((rc = ensure_work(c, 8, PGXC_PREC_FP64, s, true))) return rc;
+  if ((rc = ensure_work(c, 8, s, true))) return rc;
   // an FP64 plan for its basis and W stages: chunk k's values land where its
   // unit points (the FP64 cache, or the lane's work buffer when there is none)
   std::vector<pgxc_ctx *> mols{c};
@@ -2120,7 +2120,7 @@ static int gradient_impl(pgxc_ctx *c, double *pm) {
     }
   }
   if (hipGetLastError() != hipSuccess) return fail(c, PGXC_ERR_HIP, "pgxc_gradient: launch failed");
-  mark_basis_cached(c, 8, PGXC_PREC_FP64, true);
+  mark_basis_cached(c, 8, true);
   return PGXC_OK;
 }
 
@@ -2430,7 +2430,7 @@ int pgxc_batch_build(pgxc_batch *b, uint32_t functional, int32_t precision, int3
   hipStream_t s = b->stream;
   for (int m = 0; m < nm; ++m) {
     pgxc_ctx *c = b->mols[m];
-    int rc = ensure_work(c, elem, precision, s, gga);
+    int rc = ensure_work(c, elem, s, gga);
     if (rc) {
       b->err = "molecule " + std::to_string(m) + ": " + c->err;
       return rc;
@@ -2494,7 +2494,7 @@ int pgxc_batch_build(pgxc_batch *b, uint32_t functional, int32_t precision, int3
       return rc;
     }
     c->timing[5] = t;
-    mark_basis_cached(c, elem, precision, gga);
+    mark_basis_cached(c, elem, gga);
   }
   return PGXC_OK;
 }

@@ -76,10 +76,6 @@ struct PSOperand {
   // rowf(r): element offset of row r (k = 0), or -1; maskf(r): the 128-k
   // tiles from k = kb on where row r can be nonzero (bit t: tile t, at most
   // 32 tiles); a row's steps on other tiles stage zeros without reading it
-  template <class RowF>
-  __device__ __forceinline__ void init(const Src &S, const RowF &rowf) {
-    init(S, rowf, [](int) { return ~0u; }, 0);
-  }
   template <class RowF, class MaskF>
   __device__ __forceinline__ void init(const Src &S, const RowF &rowf, const MaskF &maskf, long kb) {
     dummy = S.hi;
@@ -139,10 +135,6 @@ struct PFOperand {
   f4 v[2][PER];
   unsigned ok[2];
 
-  template <class RowF>
-  __device__ __forceinline__ void init(const float *plane, const RowF &rowf) {
-    init(plane, rowf, [](int) { return ~0u; }, 0);
-  }
   template <class RowF, class MaskF>
   __device__ __forceinline__ void init(const float *plane, const RowF &rowf, const MaskF &maskf,
                                        long kb) {
@@ -300,15 +292,6 @@ __device__ __forceinline__ void gemm_tile_bf16x3(
     }
     if (kt < ksteps) step(s0, s1, kt);
   }
-}
-
-__device__ __forceinline__ int find_unit_x3(const long *__restrict__ base, int nu, long it) {
-  int lo = 0, hi = nu - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (base[mid] <= it) lo = mid; else hi = mid - 1;
-  }
-  return lo;
 }
 
 
@@ -481,7 +464,7 @@ __global__ __launch_bounds__(kDensThreads) __attribute__((amdgpu_waves_per_eu(IC
   for (long L = walk_next(S, -1, &slot); L < S.total;) {
     const uint64_t t0 = S.tlog ? wall_clock64() : 0;
     const long it = walk_item(S, L);
-    const int u = find_unit_x3(S.base, S.nu, it);
+    const int u = find_unit(S.base, S.nu, it);
     const UnitD &U = S.units[u];
     const uint32_t e = U.ditems[it - S.base[u]];
     const int tile = (int)(e >> 8), item = (int)(e & 255);
@@ -542,7 +525,7 @@ __attribute__((amdgpu_waves_per_eu(BT == 128 ? 4 : 2))) void k_potential_bf16x3(
   for (long L = walk_next(S, -1, &slot); L < S.total;) {
     const uint64_t t0 = S.tlog ? wall_clock64() : 0;
     const long it = walk_item(S, L);
-    const int u = find_unit_x3(S.base, S.nu, it);
+    const int u = find_unit(S.base, S.nu, it);
     const UnitD &U = S.units[u];
     const uint32_t e = U.pitems[it - S.base[u]];
     const int sl = (int)(e >> 20), ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);

@@ -20,15 +20,6 @@
 
 namespace pgxc {
 
-__device__ __forceinline__ int unit_of(const long *__restrict__ base, int nu, long it) {
-  int lo = 0, hi = nu - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (base[mid] <= it) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
 template <typename T>
 struct V2 {
   typedef T type __attribute__((ext_vector_type(2)));
@@ -50,14 +41,15 @@ constexpr int kLPad = 16;  // LDS row padding: the four k rows an MFMA operand
 // NB 16-column blocks, f and c entries of the tile's function list: four waves,
 // each 32 points x all columns.  Both operands are staged [k][row] as they lie
 // in memory: a wave takes whole k rows (its index is uniform, so their addresses
-// are scalar), a lane two points of Phi and one or two columns of D (symmetric,
-// so row f(k) is read along the columns).  Rows past the list repeat its last
+// are scalar), a lane two points of Phi and one column of D (symmetric, so row
+// f(k) is read along the columns).  Rows past the list repeat its last
 // function, and their D is 0; columns past it repeat its last one and are not
 // used.  The list entries of a step are read a step ahead of its loads.
 //
 // ST = 2: two LDS stages, one barrier per step; ST = 1: one stage.
 template <typename T, int BN, int VAR>
 struct DensTile {
+  static_assert(BN <= 64, "a column per lane");
   static constexpr int BK = Var<VAR>::BK, ST = Var<VAR>::ST;
   static constexpr int SA = kDBM + kLPad, SB = BN + kLPad, R = BK / 4;
   static constexpr int kLds = ST * BK * (SA + SB);
@@ -70,13 +62,11 @@ struct DensTile {
                                              const uint16_t *__restrict__ fl, int K,
                                              const uint16_t *__restrict__ cf, int ncol, T *lds,
                                              acc_t (&acc)[2][NB]) {
-    constexpr bool TWO = NB > 4;  // a second column per lane
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ksteps = (K + BK - 1) / BK;
-    const int c0 = gld(cf + min(lane, ncol - 1)), c1 = TWO ? gld(cf + min(64 + lane, ncol - 1)) : 0;
-    const bool in1 = 64 + lane < BN;
+    const int c0 = gld(cf + min(lane, ncol - 1));
     v2 ra[R];
-    T rb0[R], rb1[R];
+    T rb[R];
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -87,8 +77,7 @@ struct DensTile {
       for (int e = 0; e < R; ++e) {
         const long f = __builtin_amdgcn_readlane(fk, wave + 4 * e);
         ra[e] = gld((const v2 *)(phi + f * Mc) + lane);
-        rb0[e] = gld(D + f * NP + c0);
-        if constexpr (TWO) rb1[e] = gld(D + f * NP + c1);
+        rb[e] = gld(D + f * NP + c0);
       }
     };
     auto store = [&](int buf, int kt) {
@@ -98,9 +87,7 @@ struct DensTile {
         const int r = wave + 4 * e;
         const bool live = kt * BK + r < K;
         *(v2 *)(as + r * SA + 2 * lane) = ra[e];
-        bs[r * SB + lane] = live ? rb0[e] : T(0);
-        if constexpr (TWO)
-          if (in1) bs[r * SB + 64 + lane] = live ? rb1[e] : T(0);
+        bs[r * SB + lane] = live ? rb[e] : T(0);
       }
     };
     const int ar = 32 * wave + row_point<T>(lane & 15), br = lane & 15, kg = lane >> 4;
@@ -184,7 +171,7 @@ __device__ __forceinline__ void density_sums(typename MF<T>::acc (&acc)[2][NB],
 #pragma unroll
         for (int r = 0; r < 4; ++r) t[r] += (double)v[j][r / E][r % E] * (double)acc[i][j][r];
       int idx;
-      const double tot = group_reduce<4>(t, lane, idx);
+      const double tot = group_reduce(t, lane, idx);
       if ((lane & 3) == 0) gst(part + (long)c * Mc + p0 + 16 * i + idx, c ? 2.0 * tot : tot);
     }
 }
@@ -204,7 +191,7 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const Stag
   for (long L = walk_next(S, -1, &slot); L < S.total;) {
     const uint64_t t0 = S.tlog ? wall_clock64() : 0;
     const long it = walk_item(S, L);
-    const int u = unit_of(S.base, S.nu, it);
+    const int u = find_unit(S.base, S.nu, it);
     const UnitD &U = S.units[u];
     const uint32_t e = U.ditems[it - S.base[u]];
     const int tile = (int)(e >> 8), item = (int)(e & 255);
@@ -250,7 +237,7 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_xz(const StageList
   __shared__ __attribute__((aligned(16))) double lds[G::kLds];
   for (long L = blockIdx.x; L < S.total; L += gridDim.x) {
     const long it = (long)xcd_remap((int)L, (int)S.total);
-    const int u = unit_of(S.base, S.nu, it);
+    const int u = find_unit(S.base, S.nu, it);
     if (u % nspin != spin) continue;  // uniform over the workgroup
     const UnitD &U = S.units[u];
     const uint32_t e = U.ditems[it - S.base[u]];
@@ -462,7 +449,7 @@ __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_potential(const St
   for (long L = walk_next(S, -1, &slot); L < S.total;) {
     const uint64_t t0 = S.tlog ? wall_clock64() : 0;
     const long it = walk_item(S, L);
-    const int u = unit_of(S.base, S.nu, it);
+    const int u = find_unit(S.base, S.nu, it);
     const UnitD &U = S.units[u];
     const uint32_t e = U.pitems[it - S.base[u]];
     const int sl = (int)(e >> 20), ci = (int)((e >> 10) & 1023), cj = (int)(e & 1023);

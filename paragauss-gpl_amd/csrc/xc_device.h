@@ -1,6 +1,7 @@
-// Device helpers shared by the contraction kernels (FP64/FP32 MFMA and
-// split-BF16): MFMA traits and result placement, XCD-aware tile order, and
-// the two GEMM epilogues (density contraction, potential accumulation).
+// Device helpers shared by the kernels: memory access, the walk over work lists
+// (XCD-aware order, queues), MFMA traits and result placement, the split into
+// bf16 parts, and what the contractions have in common (a potential item's live
+// blocks, sums over a result block's columns, the store of a block).
 #pragma once
 #include "pgxc_internal.h"
 
@@ -35,6 +36,16 @@ __device__ __forceinline__ T gld_row(const T *row, unsigned p) {
   unsigned off = p * (unsigned)sizeof(T);
   asm("" : "+v"(off));
   return *(const __attribute__((address_space(1))) T *)(base + off);
+}
+
+// Unit whose items hold item `it` (base: the units' first items).
+__device__ __forceinline__ int find_unit(const long *__restrict__ base, int nu, long it) {
+  int lo = 0, hi = nu - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (base[mid] <= it) lo = mid; else hi = mid - 1;
+  }
+  return lo;
 }
 
 // Workgroups are dispatched round-robin over the 8 XCDs; give every XCD a
@@ -177,16 +188,6 @@ __device__ __forceinline__ void lds_list(const uint16_t *__restrict__ src, int n
   __syncthreads();
 }
 
-// Function (row of Phi / W / D) of entry e of a gathered run list, or -1
-// past the list's n runs.
-// The list read is unconditional (clamped into the list), so the lookup
-// compiles to a select rather than a branch.
-__device__ __forceinline__ long run_fn(const uint16_t *runs, int n, int e) {
-  const int r = e >> 3;
-  const long v = (long)runs[min(r, max(n - 1, 0))] * kRun + (e & 7);
-  return r < n ? v : -1;
-}
-
 // Potential item (row chunk x column chunk of a split's functions, both within
 // BT): per 16-function block and 128-point tile of the split (at most 32)
 // whether some function of the block is in the tile's list, as bits of rb[t]
@@ -224,38 +225,26 @@ __device__ __forceinline__ int potential_tiles(const uint32_t *__restrict__ rm, 
   return *n;
 }
 
-// Sum of M per-lane values (M = 4 or 16) over the 16 lanes of each lane
-// group (the 16 columns of an MFMA result block) by recursive halving: at the
-// exchange with lane l ^ o a lane keeps half of the values it still holds
-// and sends the other half, so M = 16 values take 8 + 4 + 2 + 1 shuffles
-// instead of 4 x 16.  Returns the total of value `index` in this lane
-// (index = l & 15 for M = 16; for M = 4 the groups of 4 lanes l & ~3 share
-// index (l & 12) / 4).  The addition order is fixed.
-template <int O, int m>
-struct GroupStep {  // one exchange with lane ^ O while m values are held
-  template <int M>
-  __device__ static __forceinline__ void run(double (&v)[M], int lane, int &index) {
-    if constexpr (m > 1) {
-      const bool hi = (lane & O) != 0;
-#pragma unroll
-      for (int k = 0; k < m / 2; ++k) {
-        const double send = hi ? v[k] : v[k + m / 2];
-        const double keep = hi ? v[k + m / 2] : v[k];
-        v[k] = keep + __shfl_xor(send, O);
-      }
-      if (hi) index += m / 2;
-    } else {
-      v[0] += __shfl_xor(v[0], O);
-    }
-    if constexpr (O > 1) GroupStep<O / 2, (m > 1 ? m / 2 : 1)>::run(v, lane, index);
-  }
-};
-
-template <int M>
-__device__ __forceinline__ double group_reduce(double (&v)[M], int lane, int &index) {
-  static_assert(M == 4 || M == 16, "4 or 16 values");
+// Sums of 4 per-lane values over the 16 lanes of each lane group (the 16 columns
+// of an MFMA result block) by recursive halving: at the first two exchanges a
+// lane keeps half of the values it still holds and sends the other half, so they
+// take 2 + 1 + 1 + 1 shuffles instead of 4 x 4.  Returns the total of value
+// `index` in this lane (the groups of 4 lanes l & ~3 share index (l & 12) / 4).
+// The addition order is fixed.
+__device__ __forceinline__ double group_reduce(double (&v)[4], int lane, int &index) {
   index = 0;
-  GroupStep<8, M>::run(v, lane, index);
+#pragma unroll
+  for (int m = 2; m >= 1; m >>= 1) {  // m values kept, exchange with lane ^ 4 m
+    const bool hi = (lane & (4 * m)) != 0;
+#pragma unroll
+    for (int k = 0; k < m; ++k) {
+      const double send = hi ? v[k] : v[k + m], keep = hi ? v[k + m] : v[k];
+      v[k] = keep + __shfl_xor(send, 4 * m);
+    }
+    if (hi) index += m;
+  }
+  v[0] += __shfl_xor(v[0], 2);
+  v[0] += __shfl_xor(v[0], 1);
   return v[0];
 }
 

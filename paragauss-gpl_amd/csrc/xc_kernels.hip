@@ -152,15 +152,6 @@ __device__ __forceinline__ double sum4(const double (&e)[4]) { return ((e[0] + e
 // XCD-blocked order so that neighbouring tiles share an XCD's L2.  Items write
 // disjoint outputs, so the order never changes a result bit.
 
-__device__ __forceinline__ int find_unit(const long *__restrict__ base, int nu, long it) {
-  int lo = 0, hi = nu - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (base[mid] <= it) lo = mid; else hi = mid - 1;
-  }
-  return lo;
-}
-
 __device__ __forceinline__ long item_at(const int *__restrict__ order, long L, long total) {
   return order ? (long)order[L] : (long)xcd_remap((int)L, (int)total);
 }
