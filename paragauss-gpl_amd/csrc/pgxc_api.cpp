@@ -62,10 +62,13 @@ struct ScopedDev {
 
 // Host memory the device copies to and from directly, in two halves that take
 // turns: one is filled by the copy engine while the host empties the other.
-// 1 MiB a half: a copy of it takes longer than starting one.
+// 1 MiB a half: a copy of it takes longer than starting one.  A thread may read a
+// build's results while others read them or set the next orbitals: whoever uses
+// the halves holds mu until their contents are taken.
 struct PinnedPair {
   static constexpr size_t kHalf = 1 << 20;
   char *buf = nullptr;
+  std::recursive_mutex mu;
   hipEvent_t ev[2] = {nullptr, nullptr};
   hipError_t init() {
     hipError_t e = hipHostMalloc((void **)&buf, 2 * kHalf);
@@ -82,6 +85,7 @@ struct PinnedPair {
   // stream's earlier work
   template <class Take>
   hipError_t fetch(hipStream_t s, const double *dev, size_t n, Take take) {
+    std::lock_guard<std::recursive_mutex> lk(mu);
     const size_t per = kHalf / 8, parts = (n + per - 1) / per;
     hipError_t e = hipSuccess;
     auto len = [&](size_t i) { return std::min(per, n - i * per); };
@@ -1941,6 +1945,7 @@ extern "C" int pgxc_set_orbitals(pgxc_ctx *c, int32_t ispin, int32_t nbas, int32
     c->orb_n = nC + no;
   }
   double *dC = c->orb, *docc = c->orb + nC;
+  std::lock_guard<std::recursive_mutex> lk(c->pin.mu);  // to the wait below
   if ((nC + no) * 8 <= 2 * PinnedPair::kHalf) {  // one copy from pinned memory
     if (nC) {
       memcpy(c->pin.buf, C, nC * 8);
@@ -1988,6 +1993,7 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
     launch_plan<float>(s, c->stream2, c->fork, c->join, *c->plan, gga, &c->ev);
   HIPCHK(c, hipGetLastError());
   // waits for the build; a small V comes along in the same wait
+  std::unique_lock<std::recursive_mutex> lk(c->pin.mu);
   const size_t npk = (size_t)c->nbas * (c->nbas + 1) / 2;
   const bool along = ham && c->ispin == 1 && 8 * npk <= PinnedPair::kHalf &&
                      16 * (size_t)c->nblk_total <= PinnedPair::kHalf;
@@ -2013,6 +2019,7 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
     for (size_t i = 0; i < npk; ++i) ham[i] += v[i];
     ham = nullptr;
   }
+  lk.unlock();
   return pgxc_get_result(c, ham, exc, charge);
 }
 
