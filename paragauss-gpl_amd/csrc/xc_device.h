@@ -231,20 +231,27 @@ __device__ __forceinline__ int potential_tiles(const uint32_t *__restrict__ rm, 
 // take 2 + 1 + 1 + 1 shuffles instead of 4 x 4.  Returns the total of value
 // `index` in this lane (the groups of 4 lanes l & ~3 share index (l & 12) / 4).
 // The addition order is fixed.
+template <int O, int m>
+struct GroupStep {  // one exchange with lane ^ O while m values are held
+  __device__ static __forceinline__ void run(double (&v)[4], int lane, int &index) {
+    if constexpr (m > 1) {
+      const bool hi = (lane & O) != 0;
+#pragma unroll
+      for (int k = 0; k < m / 2; ++k) {
+        const double send = hi ? v[k] : v[k + m / 2];
+        const double keep = hi ? v[k + m / 2] : v[k];
+        v[k] = keep + __shfl_xor(send, O);
+      }
+      if (hi) index += m / 2;
+    } else {
+      v[0] += __shfl_xor(v[0], O);
+    }
+    if constexpr (O > 1) GroupStep<O / 2, (m > 1 ? m / 2 : 1)>::run(v, lane, index);
+  }
+};
 __device__ __forceinline__ double group_reduce(double (&v)[4], int lane, int &index) {
   index = 0;
-#pragma unroll
-  for (int m = 2; m >= 1; m >>= 1) {  // m values kept, exchange with lane ^ 4 m
-    const bool hi = (lane & (4 * m)) != 0;
-#pragma unroll
-    for (int k = 0; k < m; ++k) {
-      const double send = hi ? v[k] : v[k + m], keep = hi ? v[k + m] : v[k];
-      v[k] = keep + __shfl_xor(send, 4 * m);
-    }
-    if (hi) index += m;
-  }
-  v[0] += __shfl_xor(v[0], 2);
-  v[0] += __shfl_xor(v[0], 1);
+  GroupStep<8, 4>::run(v, lane, index);
   return v[0];
 }
 
