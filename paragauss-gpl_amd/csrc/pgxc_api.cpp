@@ -427,16 +427,16 @@ static void unit_item_features(const pgxc_ctx *c, int step, ItemKind kind, int p
     for (long i = c->h_di_off[step]; i < c->h_di_off[step + 1]; ++i) {
       const uint32_t e = c->h_di[(size_t)i];
       const long T = T0 + (e >> 8);
-      const int item = (int)(e & 255), nf = c->h_tf_off[(size_t)T + 1] - c->h_tf_off[(size_t)T];
-      // the columns as the kernels take them: n chunks of cc (at most dcols), per an
-      // item.  The feature is the share that a tile's items have in common, not
-      // what is left for the last one: items of equal predicted cost keep their
-      // natural order, and a tile's items read its values together ((H2O)32 in
-      // FP64, the model's schedule: 15.77 ms with each item's own columns, 15.58
-      // with the share)
+      const int nf = c->h_tf_off[(size_t)T + 1] - c->h_tf_off[(size_t)T];
+      // The columns as the kernels take them: n chunks of cc (at most dcols), per an
+      // item.  Feature and cost are the same for all items of a tile, its share and
+      // its flops over its items, not those of what is left for the last one: items
+      // of equal cost keep their natural order in a queue, and a tile's items then
+      // read its values together.  (H2O)32 in FP64, counted flops 15.6 -> 15.3 ms,
+      // the model 15.8 -> 15.5.
       const int dcols = precision == PGXC_PREC_BF16X3 ? c->icols : kPartCols, per = c->icols / dcols;
       const int n = (nf + dcols - 1) / dcols, cc = 16 * (((nf + 15) / 16 + n - 1) / n);
-      const double cols = std::min(nf, (item + 1) * per * cc) - item * per * cc;
+      const double cols = (double)nf / ((n + per - 1) / per);
       const double K = precision == PGXC_PREC_BF16X3 ? kRun * (c->h_tl_off[(size_t)T + 1] - c->h_tl_off[(size_t)T]) : nf;
       push(0, std::min(per, n) * cc, K, c->NP, true, 2.0 * kScreenTile * cols * K);
     }
