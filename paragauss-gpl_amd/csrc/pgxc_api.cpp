@@ -61,17 +61,21 @@ struct ScopedDev {
 }  // namespace
 
 // Host memory the device copies to and from directly, in two halves that take
-// turns: one is filled by the copy engine while the host empties the other.
-// 1 MiB a half: a copy of it takes longer than starting one.  A thread may read a
-// build's results while others read them or set the next orbitals: whoever uses
-// the halves holds mu until their contents are taken.
+// turns: one is filled by the device while the host empties the other.  1 MiB a
+// half: a copy of it takes longer than starting one.  The copies are kernels:
+// from 32 KiB on, hipMemcpyAsync takes the copy engine, which for some contexts
+// starts 110 us late behind each build (V of 132 functions 26 or 124 us, by kernel
+// 23; orbitals of 132 functions 35 or 138, by kernel 35; (H2O)32's V 737, by kernel
+// 219; through pageable memory 19, 58 and 451).  A thread may read a build's results while others read them or set
+// the next orbitals: whoever uses the halves holds mu until their contents are
+// taken.
 struct PinnedPair {
   static constexpr size_t kHalf = 1 << 20;
   char *buf = nullptr;
   std::recursive_mutex mu;
   hipEvent_t ev[2] = {nullptr, nullptr};
   hipError_t init() {
-    hipError_t e = hipHostMalloc((void **)&buf, 2 * kHalf);
+    hipError_t e = hipHostMalloc((void **)&buf, 2 * kHalf, hipHostMallocCoherent);
     for (int i = 0; i < 2 && e == hipSuccess; ++i) e = hipEventCreateWithFlags(&ev[i], hipEventDisableTiming);
     return e;
   }
@@ -91,7 +95,8 @@ struct PinnedPair {
     auto len = [&](size_t i) { return std::min(per, n - i * per); };
     for (size_t i = 0; i <= parts && e == hipSuccess; ++i) {
       if (i < parts) {
-        e = hipMemcpyAsync(buf + (i & 1) * kHalf, dev + i * per, 8 * len(i), hipMemcpyDeviceToHost, s);
+        launch_copy(s, dev + i * per, (double *)(buf + (i & 1) * kHalf), (long)len(i));
+        e = hipGetLastError();
         if (e == hipSuccess) e = hipEventRecord(ev[i & 1], s);
       }
       if (i > 0 && e == hipSuccess) {
@@ -1950,7 +1955,7 @@ extern "C" int pgxc_set_orbitals(pgxc_ctx *c, int32_t ispin, int32_t nbas, int32
     if (nC) {
       memcpy(c->pin.buf, C, nC * 8);
       memcpy(c->pin.buf + nC * 8, occ, no * 8);
-      HIPCHK(c, hipMemcpyAsync(dC, c->pin.buf, (nC + no) * 8, hipMemcpyHostToDevice, c->stream));
+      launch_copy(c->stream, (const double *)c->pin.buf, dC, (long)(nC + no));
     }
   } else {
     HIPCHK(c, hipMemcpy(dC, C, nC * 8, hipMemcpyHostToDevice));
@@ -1997,8 +2002,8 @@ int pgxc_build(pgxc_ctx *c, uint32_t functional, int32_t precision, double *ham,
   const size_t npk = (size_t)c->nbas * (c->nbas + 1) / 2;
   const bool along = ham && c->ispin == 1 && 8 * npk <= PinnedPair::kHalf &&
                      16 * (size_t)c->nblk_total <= PinnedPair::kHalf;
-  const double *v = (const double *)(c->pin.buf + PinnedPair::kHalf);
-  if (along) HIPCHK(c, hipMemcpyAsync((void *)v, c->Vout, 8 * npk, hipMemcpyDeviceToHost, s));
+  double *v = (double *)(c->pin.buf + PinnedPair::kHalf);
+  if (along) launch_copy(s, c->Vout, v, (long)npk);
   if ((rc = collect(c, s, functional, precision))) return rc;
   for (int k = 0; k < 4; ++k) c->timing[k] = 0.0;
   float t = 0;

@@ -230,6 +230,7 @@ void launch_screen(hipStream_t s, long ntiles_pts, const double *gx, const doubl
 
 // P = C diag(occ) C^T into an NP x NP padded array (C in caller order; finv:
 // caller index of each internal function)
+void launch_copy(hipStream_t s, const double *src, double *dst, long n);
 void launch_form_density(hipStream_t s, const double *C, const double *occ, const int *finv, int n,
                          int nocc, int NP, double *P);
 

@@ -8,6 +8,7 @@
 //                 (modules/xc_func.f90:187-305 and the term modules)
 //   k_wbasis      W = a Phi + b . grad Phi  (modules/xc_hamiltonian.f90:1429-1483)
 //   k_pack        V = H + H^T into the packed lower triangle (:1561-1567)
+#include <algorithm>
 #include <type_traits>
 
 #include "pgxc_internal.h"
@@ -1233,6 +1234,19 @@ void launch_form_density(hipStream_t s, const double *C, const double *occ, cons
   const long nt = (NP + kFT - 1) / kFT;
   hipLaunchKernelGGL(k_form_density, dim3((unsigned)(nt * (nt + 1) / 2)), dim3(kThreads), 0, s, C, occ, finv, n,
                      nocc, NP, P);
+}
+
+// n doubles from src to dst, one of them pinned host memory: bound by the link
+// (1 MiB to the host in 49 us, 21 GB/s; 2 KiB in 3 us).
+__global__ __launch_bounds__(kThreads) void k_copy(const double *__restrict__ src, double *__restrict__ dst,
+                                                   long n) {
+  for (long i = (long)blockIdx.x * kThreads + threadIdx.x; i < n; i += (long)gridDim.x * kThreads) dst[i] = src[i];
+}
+
+void launch_copy(hipStream_t s, const double *src, double *dst, long n) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_copy, dim3((unsigned)std::min<long>(512, (n + kThreads - 1) / kThreads)), dim3(kThreads), 0,
+                     s, src, dst, n);
 }
 
 }  // namespace pgxc

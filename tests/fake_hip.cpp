@@ -4,6 +4,8 @@
 // is kept mapped and remembered, so that a table which still names it can be
 // found: fake_stale() counts the words of the launched plans' tables that point
 // into freed memory.  fake_fail_in(n): the n-th allocation from now on fails.
+// fake_engine() counts the copies of pinned memory large enough for the runtime
+// to give them to a copy engine.
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
@@ -16,8 +18,8 @@ typedef int err_t;  // hipError_t
 constexpr err_t kOk = 0, kInvalid = 1, kNoMem = 2;
 std::map<uintptr_t, size_t> live, dead;
 std::map<const void *, std::string> names;
-std::set<uintptr_t> captured;
-long fail_in = 0, stale = 0;
+std::set<uintptr_t> captured, pinned;
+long fail_in = 0, stale = 0, engine = 0;
 bool capturing = false;
 err_t last = kOk;
 int token;
@@ -44,6 +46,7 @@ err_t set(err_t e) {
 
 extern "C" {
 long fake_stale() { return stale; }
+long fake_engine() { return engine; }
 long fake_live() { return (long)live.size(); }
 void fake_fail_in(long n) { fail_in = n; }
 
@@ -107,14 +110,21 @@ err_t hipFree(void *p) {
   live.erase(it);
   return kOk;
 }
-err_t hipHostMalloc(void **p, size_t n, unsigned) { return hipMalloc(p, n); }
+err_t hipHostMalloc(void **p, size_t n, unsigned) {
+  const err_t e = hipMalloc(p, n);
+  if (e == kOk) pinned.insert((uintptr_t)*p);
+  return e;
+}
 err_t hipHostFree(void *p) { return hipFree(p); }
 err_t hipMemcpy(void *d, const void *s, size_t n, int) {
   if (n && (!d || !s)) return set(kInvalid);
   memcpy(d, s, n);
   return kOk;
 }
-err_t hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *) { return hipMemcpy(d, s, n, k); }
+err_t hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *) {
+  for (const void *p : {(const void *)d, s}) engine += n > 16384 && pinned.count(owner(live, (uintptr_t)p));
+  return hipMemcpy(d, s, n, k);
+}
 err_t hipMemset(void *d, int v, size_t n) {
   if (n && !d) return set(kInvalid);
   if (v || owner(live, (uintptr_t)d) != (uintptr_t)d) memset(d, v, n);

@@ -13,7 +13,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PRELUDE = """
 import ctypes, sys
 hip = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
-hip.fake_stale.restype = hip.fake_live.restype = ctypes.c_long
+hip.fake_stale.restype = hip.fake_live.restype = hip.fake_engine.restype = ctypes.c_long
 hip.fake_fail_in.argtypes = [ctypes.c_long]
 import numpy as np
 from pgxc import Batch, XCBuilder, _lib, basis, grid, systems
@@ -173,3 +173,21 @@ xc = builder()
 hip.fake_fail_in(11)  # the tenth was the last
 xc.set_density(np.ones((xc.nbas, xc.nbas, 2)))
 """)
+
+
+@pytest.mark.parametrize("ispin", [1, 2])
+def test_no_call_waits_for_a_copy_engine(fake, ispin):
+    """Orbitals, V and energy terms of more than 16 KB go through the pinned
+    memory by kernels: a copy engine may start 100 us late behind a build."""
+    run(fake, """
+for n in (1, 4, 16):
+    xc = builder(n)
+    C, occ = systems.random_orbitals(xc.nbas, 5 * n, seed=2)
+    if %d == 2:
+        C, occ = np.stack([C, C], axis=2), np.stack([occ, occ], axis=1)
+    xc.set_orbitals(C, occ)
+    xc.build(PBE, FP64)
+    xc.result()
+    xc.energy(PBE, FP64)
+    assert hip.fake_engine() == 0, n
+""" % ispin)
