@@ -67,28 +67,31 @@ extern "C" {
 /* Features of one work item, in this order (pgxc_item_log, cost model):
  * kind (0 density, 1 potential contraction), precision one-hot (FP64, FP32,
  * BF16x3), columns / 128 (density: the share of its tile's functions that an
- * item takes, in whole blocks of 16; potential: the functions of a chunk), log2(1 + K length left after screening) / 16, log2(1 + dense K
- * length) / 16, 1 if any block is left after screening, variant / 2.  (K:
- * functions of the density contraction, in whole runs of 8 for BF16x3; points
- * of the potential contraction.) */
+ * item takes, in whole blocks of 16; potential: the functions of a chunk),
+ * log2(1 + K length left after screening) / 16, log2(1 + dense K length) / 16,
+ * 1 if any block is left after screening, variant / 2.  (K: functions of the
+ * density contraction, in whole runs of 8 for BF16x3; points of the potential
+ * contraction.) */
 #define PGXC_NFEATURES 9
 
 typedef struct pgxc_ctx pgxc_ctx;
 typedef struct pgxc_batch pgxc_batch;
 typedef struct pgxc_costmodel pgxc_costmodel;
 
-/* Layout options of a context (pgxc_create_opt).  tile: function tile of the
- * MFMA contractions, 64, 96 or 128 (0: the one padding nbas least).
+/* Layout options of a context (pgxc_create_opt).  tile: 64, 96 or 128: nbas is
+ * padded to a multiple of it, and the potential contraction takes its functions
+ * in chunks of it (0: the padding is the least of the three, the chunks follow
+ * the functions a point split has).
  * chunk_points: largest number of grid points held in one work chunk, a
  * multiple of 2048 (0: at most 256 Ki points and 8 GiB of FP64 basis values).
  * variant_fp64 / variant_fp32: contraction kernel variant for FP64 and FP32
  * builds, 0 (K step 16, two LDS stages), 1 (K step 32, one LDS stage),
  * 2 (K step 32, two LDS stages); -1 keeps the default.  pgxc/autotune.py picks
  * tile and variants by timing them.  no_screen: 1 runs the contractions over
- * every basis function and point; 0 (default) skips the 32-function x
- * 32-point blocks on which the radial cut-off alpha r^2 >= 50
- * (modules/orbital_module.f90:1839-1855) makes every basis value exactly zero,
- * which leaves every result bit unchanged.  no_basis_cache: 1 evaluates the
+ * every basis function and point; 0 (default) leaves out, per tile of 128
+ * points, the shells whose every value there the radial cut-off
+ * alpha r^2 >= 50 (modules/orbital_module.f90:1839-1855) makes exactly zero:
+ * only the rounding of the regrouped sums differs.  no_basis_cache: 1 evaluates the
  * basis values in every build; 0 (default) keeps the values of every grid
  * chunk on the device after the first build of each precision and reuses
  * them (the role of ParaGauss's orbital store across SCF cycles,
@@ -221,8 +224,8 @@ int pgxc_gradient(pgxc_ctx *ctx, double *grad);
  * owner[npts] (caller point order): the atom whose atomic grid holds the
  * point; the grid's weights must be the Becke partition of those atomic
  * grids.  grad (n_atoms x 3) receives dE_xc/dR, at the last build's density
- * and coefficients, FP64.  The first call allocates 36 bytes per point and at
- * most 256 MiB of scratch, which the context keeps.
+ * and coefficients, FP64.  The first call allocates 40 bytes per point, 8 per
+ * pair of atoms and at most 256 MiB of scratch, which the context keeps.
  */
 int pgxc_gradient_grid(pgxc_ctx *ctx, const int32_t *owner, double *grad);
 
@@ -296,7 +299,10 @@ int pgxc_destroy(pgxc_ctx *ctx);
  * loop of xc_build calls.  Each context keeps its own results
  * (pgxc_get_result) and incremental state, exactly as after pgxc_build.
  * Results do not depend on the schedule: every work item writes its own
- * partial sums, reduced in a fixed order.
+ * partial sums, reduced in a fixed order.  Every context keeps its own work
+ * memory while it lives: a chunk's W and (uncached) basis values per lane, the
+ * potential's partial sums (those of all its chunks, up to 4 GiB per spin) and
+ * 2 MiB of pinned host memory; a smaller chunk_points makes the first smaller.
  */
 int pgxc_batch_create(pgxc_batch **batch, int32_t n, pgxc_ctx *const *ctxs);
 

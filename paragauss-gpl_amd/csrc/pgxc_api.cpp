@@ -328,7 +328,7 @@ struct Plan {
   long order_version = -1;
   int sched_mode = 0, log = 0;
   int energy = 0;  // energy terms only: no W, potential, fold or packing
-  int wbasis = 0;  // split-BF16 W from the basis evaluated again (k_wbasis)
+  int wbasis = 0;  // W from the basis evaluated again (k_wbasis)
   const pgxc_costmodel *model = nullptr;
   long model_version = -1;
   int *d_ctr = nullptr;  // queue counters of every contraction list
@@ -685,9 +685,8 @@ static int get_plan(std::vector<pgxc_ctx *> &mols, uint32_t functional, int prec
       pick(0, [](const pgxc_ctx *c) { return c->ispin == 1; }, fu, fm);
       pend[k].push_back(stage(fu, fm, K_FUNC, 0, k));
     }
-    // W: split-BF16 builds evaluate the basis again over the basis items
-    // (test switch PGXC_W_READ=1: they read the stored values back instead,
-    // the same bits)
+    // W: the basis evaluated again over the basis items (test switch
+    // PGXC_W_READ=1: the stored values read back instead, the same bits)
     const bool wb = !getenv("PGXC_W_READ");
     plan->wbasis = wb ? 1 : 0;
     const ItemKind wkind = wb ? K_WBASIS : K_WMAT;

@@ -155,15 +155,17 @@ struct StageList {
   int lmax;  // basis lists: the largest angular momentum of their atoms
 };
 
-// ---- launchers (kernels live in xc_kernels.hip / xc_bf16x3.hip) -----------
+// ---- launchers (kernels: xc_kernels.hip; the contractions' xc_contract.h and
+// xc_bf16x3.hip) --------------------------------------------------------------
 template <typename T>
 void launch_basis(hipStream_t s, bool grad, const StageList &L);
 // W over the basis items, the basis evaluated again (split: stored as bf16 hi / lo
 // planes; two: both spins of open-shell units)
 template <typename T>
 void launch_wbasis(hipStream_t s, bool grad, bool split, bool two, const StageList &L);
-// tf = function tile (64, 96 or 128) shared by every unit of the list;
-// var = contraction variant: 0 (K step 16, 2 LDS stages), 1 (32, 1), 2 (32, 2)
+// var = contraction variant: 0 (K step 16, 2 LDS stages), 1 (32, 1), 2 (32, 2);
+// tf = chunk of functions of the potential (64, 96 or 128) and icols = columns of
+// the split-BF16 density's items (128 or 256), the same for every unit of a list
 constexpr int kNumVariants = 3;
 template <typename T>
 void launch_density(hipStream_t s, bool grad, int var, const StageList &L);
@@ -171,8 +173,8 @@ void launch_functional(hipStream_t s, bool gga, const StageList &L);
 void launch_functional_spin(hipStream_t s, bool gga, const StageList &L);
 // energy terms only (no coefficients, state untouched); spin: open-shell units
 void launch_energy(hipStream_t s, bool gga, bool spin, const StageList &L);
-// two: open-shell alpha units, whose W pass writes both spins' W (W, W2 from
-// coef, coef2) from one read of the basis values
+// W from the stored basis values (two: both spins' W, W2 from coef, coef2, from
+// one read)
 template <typename T>
 void launch_wmat(hipStream_t s, bool grad, bool split, bool two, const StageList &L);
 template <typename T>

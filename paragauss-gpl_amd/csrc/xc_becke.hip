@@ -62,8 +62,10 @@ __global__ __launch_bounds__(kThreads) void k_becke_all(int na, const double *__
 // the centres in order, kForm at a time so that a centre's distance is found
 // once for all of them; a wave forms the centres any of its points needs.
 // Bound by FP64 arithmetic.  (H2O)32, 96 centres, 1 961 792 points: 33 centres
-// a wave are formed in full (14 for a single point), 5.0 ms; every product over
-// all centres took 21.9 ms.
+// a wave are formed in full (14 for a single point), 5.0 ms in one launch; every
+// product over all centres took 21.9 ms.  pgxc_becke_weights launches it per part
+// of 2^18 points, 1024 workgroups, half of what the device holds: 7.3 ms in all,
+// beside the transfers they overlap.
 constexpr int kNear = 8, kForm = 8;
 
 __global__ __launch_bounds__(kThreads) void k_becke(int na, const double *__restrict__ axyz,

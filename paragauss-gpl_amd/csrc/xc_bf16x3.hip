@@ -446,9 +446,10 @@ __device__ __forceinline__ void dens_sums_x3(const f4 (&acc)[4][TN], const float
 // the staging of Phi.  Bound by the sums' HBM reads (16 bytes per point and
 // function) and, for many functions, by LDS.  Stage of an (H2O)32 build, one
 // lane, 228 functions a tile: 3.48 ms with one workgroup of 192 columns per CU
-// and the values read in the MFMA blocks' layout, 3.38 with two of 128, 2.95
+// and the values read in the MFMA blocks' layout, 3.38 with two of 128, 2.8
 // with the values read by column; (H2O)128 and solute, 916 a tile: 171 ms of
-// two-lane stage time at IC = 128, 150 at 256.
+// two-lane stage time at IC = 128, 150 at 256.  At IC = 128 the 128 registers of
+// four waves a SIMD are 9 too few (32 bytes of scratch a lane).
 template <bool GRAD, int IC>
 __global__ __launch_bounds__(kDensThreads) __attribute__((amdgpu_waves_per_eu(IC == 128 ? 4 : 2))) void k_density_bf16x3(const StageList S) {
   // the sums' X and reduction reuse the staging LDS
@@ -510,7 +511,8 @@ void launch_density_bf16x3(hipStream_t s, bool grad, int icols, const StageList 
   else density_x3<256>(s, grad, L);
 }
 
-// item = (point split, function tile pair), as k_potential
+// item = (point split, function tile pair), as k_potential (chunks of 128: four
+// waves a SIMD, 20 registers spilled, 84 bytes a lane)
 constexpr int pot_threads(int BT) { return BT == 128 ? 512 : 256; }
 template <int BT>
 __global__ __launch_bounds__(pot_threads(BT))

@@ -181,7 +181,8 @@ __device__ __forceinline__ void density_sums(typename MF<T>::acc (&acc)[2][NB],
 // bytes per point and function, 14 GB at (H2O)32 in FP64).  The kernel before
 // walked whole runs of 8 functions and 96-column chunks (1.4 times the MFMAs)
 // and looked every operand vector up in the run list as it loaded it: FP64
-// density stage of an (H2O)32 build, one lane, 10.8 ms; now 6.5.
+// density stage of an (H2O)32 build, one lane, 10.8 ms; now 6.3 (variant 1 6.6,
+// 2 8.5).
 template <typename T, int BN, int VAR, bool GRAD>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_density(const StageList S) {
@@ -437,7 +438,8 @@ struct PotTile {
 // build, one lane: 10.1 -> 6.1 ms; 23-atom molecule (233 000 points) 852 -> 150
 // us, its 57 splits of 4096 points now 456 of 512.  Variants 0 and 1 keep
 // their LDS stages under 80 KB: two workgroups share a CU and hide each other's
-// waits.
+// waits.  With FP64 chunks of 128, 16 result blocks and a step's operands pass the
+// 256 registers: variant 0 spills 13 (56 bytes of scratch a lane), variant 1 103.
 template <typename T, int BT, int VAR>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(VAR == 2 ? 1 : 2))) void k_potential(const StageList S) {

@@ -222,7 +222,8 @@ __device__ __forceinline__ double wave_sum(double v) {
 // functions into pm[d][p] += 2 t (w grad f at the point: its motion with its
 // atom) when pm is given.  XZ = [2][NP][Mc] at the tiles' functions; st: the
 // build's coefficients a, b (planes stride np apart).  Bound by the reads of X
-// and Z and the registers of their use (two waves a SIMD; one: 0.80 ms).  Per
+// and Z and the registers of their use (two waves a SIMD; one: 0.80 ms; with f and
+// g shells one, 14 registers spilled in the GGA kernel).  Per
 // (H2O)16 chunk of 245 760 points 0.38 ms (0.48 with a range staged in LDS and a
 // branch per primitive; 0.67 when the items came through loads the compiler takes
 // for different lanes' and everything after them went per lane); storing the six

@@ -223,7 +223,11 @@ struct StoreW {
 // us, 23-atom LDA 127 -> 92; one water 23 -> 23.  Bound by vector instructions (50
 // a wave and function, a third of them exponentials): with tables from scalar
 // loads, rows addressed by the wave and one conversion to bf16 instead of an
-// emulated one from FP64, FP64 1.71 ms, FP32 1.23, split BF16 2.02 -> 1.32.
+// emulated one from FP64, FP64 1.69 ms, FP32 1.22, split BF16 2.02 -> 1.31.  With f
+// and g shells (one or two waves a SIMD in FP64) it is the better one too where the
+// stage takes time: functional and W of (H2O)16 with 784 functions, 391 000 points,
+// evaluated / read in FP64 468 / 1296 us (LDA 291 / 492), FP32 306 / 629 (204 /
+// 223), split BF16 370 / 659 (235 / 229); one water within 9 us, either way.
 template <typename T, bool SPLIT, bool GRAD, bool TWO, int LMAX>
 __global__ __launch_bounds__(kThreads) void k_wbasis(const UnitD *__restrict__ units, int nu,
                                                      const long *__restrict__ base,
@@ -773,9 +777,9 @@ __global__ __launch_bounds__(kThreads) void k_wmat(const UnitD *__restrict__ uni
 // listed in LDS with the places of the two blocks' functions, so the loop over
 // them has only the elements' loads, four splits' at a time, to wait for.  The
 // mirror tile's sums change places through LDS.  Bound by the latency of those
-// loads; a tile all splits hold sets the time, hence the segments of at most
-// 64 splits: (H2O)32, 960 splits, 500 MB, fold and packing 0.30 ms (0.65 with
-// two segments).
+// loads; a tile all splits hold sets the time, hence the segments, of at most 64
+// splits while there are no more than 32 of them: (H2O)32, 960 splits, 500 MB,
+// fold and packing 0.32 ms (0.65 with two segments).
 constexpr int kFoldSplits = 64;
 __global__ __launch_bounds__(kThreads) void k_fold(const FoldD *__restrict__ folds, int n,
                                                    const long *__restrict__ base, long total) {
