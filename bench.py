@@ -630,8 +630,9 @@ def main():
     warm = timed(xc, "basis cached")
     st1w, _ = one_lane(xc, warm["best"])
     # work the contraction kernels execute (the columns and K of every density
-    # item, whole chunks of functions in the potential): counted from the item
-    # log of one more build of each mixed form
+    # item; in the potential whole chunks of functions, of which FP32 leaves out
+    # the blocks without one on a tile): counted from the item log of one more
+    # build of each mixed form
     executed = {}
     xc.set_item_log(True)
     for prec in precs:
@@ -640,15 +641,18 @@ def main():
         F, _ = xc.item_log()
         k = np.exp2(16.0 * F[:, 5]) - 1.0
         # density item: 128 points x its columns (in FP32 a tile's K functions
-        # over its items; split BF16 pads its shares to blocks of 16);
+        # over its items; split BF16 takes 64 columns and K of 32 at a time);
         # potential item: chunk x chunk
         cols = F[:, 4] * 128.0
+        dens = F[:, 0] == 0
         if prec == "fp32":
-            cols = np.where(F[:, 0] == 0, k / np.ceil(np.rint(k) / cols), cols)
-        rows = np.where(F[:, 0] == 0, 128.0, cols)
+            cols = np.where(dens, k / np.ceil(np.rint(k) / cols), cols)
+        else:
+            cols = np.where(dens, 64.0 * np.ceil(cols / 64.0), cols)
+            k = np.where(dens, 32.0 * np.ceil(np.rint(k) / 32.0), k)
+        rows = np.where(dens, 128.0, cols)
         fl = 2.0 * rows * cols * k
-        executed[prec] = {"density": float(fl[F[:, 0] == 0].sum()),
-                          "potential": float(fl[F[:, 0] == 1].sum())}
+        executed[prec] = {"density": float(fl[dens].sum()), "potential": float(fl[~dens].sum())}
     xc.set_item_log(False)
     perr = precision_errors(xc, C, occ, precs)
     log("precision errors per ||dP||_F:", perr)
